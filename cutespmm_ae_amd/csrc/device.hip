@@ -65,6 +65,9 @@ int choose_mfma_shape(uint64_t slots, uint64_t bricks, uint64_t blocks, uint64_t
     return shape;
 }
 
+// Floats per lane of a B or C row: four wherever a row has four (the kernels need no alignment beyond a float).
+inline int lane_floats(uint32_t N) { return N >= 4u ? 4 : N >= 2u ? 2 : 1; }
+
 inline int hip_fail(hipError_t e, const char *what, int line)
 {
     g_hip_error = std::string(hipGetErrorString(e)) + " (" + what + ", device.hip:" + std::to_string(line) + ")";
@@ -817,8 +820,7 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
     // the mean) 25-35 % at N = 16 and 32, geomean over the 43 matrices against the best single kernel 1.18 -> 1.10
     // (N = 16), 1.10 -> 1.04 (N = 32), 1.07 -> 1.03 (N = 128).  With one row per wavefront (N >= 256) the same move
     // loses (HEP-th-new, N = 512: 60 -> 68 us), so it is not made there.
-    const uint32_t row_lane_width = (N % 4 == 0) ? 4u : (N % 2 == 0) ? 2u : 1u;      // floats per lane of the row kernel
-    const bool rows_share_a_wavefront = t.max_row_nnz == 0 && (N + row_lane_width - 1u) / row_lane_width < 64u;
+    const bool rows_share_a_wavefront = t.max_row_nnz == 0 && (N + uint32_t(lane_floats(N)) - 1u) / uint32_t(lane_floats(N)) < 64u;
     uint32_t n_brick = 0, n_rows = 0, n_empty = 0;
     for (uint32_t q = 0; q < d->P; ++q) {
         const uint32_t nblk = d->brp[q + 1] - d->brp[q];
@@ -874,7 +876,7 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
     }
 
     // brick kernel shape
-    p->vec = (N % 4 == 0) ? 4 : (N % 2 == 0) ? 2 : 1;
+    p->vec = lane_floats(N);
     p->rows_vec = p->vec;
     // a brick work item spans 16*VEC columns: for narrow N take the narrowest tile that still covers N
     while (p->vec > 1 && 8u * uint32_t(p->vec) >= N) p->vec /= 2;
@@ -927,8 +929,9 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
         p->shape = choose_mfma_shape(slots, bricks, blocks, uint64_t(d->K) + d->M, d->nnz, N, t.operand_residency, c.cache_bytes);
     }
     if (p->shape == 2 && !(offsets_fit && (d->numQuadVals + 64u) * 4u <= 0xffffffffull)) p->shape = 1;
-    // bf16x3 exists for the rolling brick kernel with four columns per lane; any other shape computes in fp32
-    p->bf16x3 = t.precision == CUTE_PREC_BF16X3 && p->shape == 1 && p->pipeline == 1 && p->vec == 4;
+    // bf16x3 exists for the rolling brick kernel with four columns per lane, and is asked for with N a multiple of four;
+    // any other shape computes in fp32
+    p->bf16x3 = t.precision == CUTE_PREC_BF16X3 && p->shape == 1 && p->pipeline == 1 && p->vec == 4 && N % 4u == 0;
     // The chunk list depends on the MFMA kernel (its work units are blocks or list groups).  It is built,
     // and if the partial tiles of the cut panels then turn out to be more rows than the fast kernels'
     // 24-bit row operand can address, built once more for the pipelined brick kernel, whose stores use
@@ -1291,7 +1294,7 @@ int csr_launch(int alg, const uint32_t *rp, const uint32_t *cl, const float *vl,
                                s, rp, cl, vl, dB, dC, M, N);
             break;
         case 2: {
-            const int vec = (N % 4 == 0) ? 4 : (N % 2 == 0) ? 2 : 1;
+            const int vec = lane_floats(N);
             uint32_t need = (N + vec - 1) / vec, logl = 0;
             while ((1u << logl) < need && logl < 6) ++logl;
             const uint32_t w = (1u << logl) * vec;
