@@ -6,11 +6,20 @@
 // Both layouts are orderings of the matrix entries: the brick tiles hold the entries of a 16-row panel
 // sorted by (column, row) -- active column a of the panel is column a%4 of brick (a%16)/4 of block a/16, and
 // inside a brick the lane-order bitmap runs column-major -- and the quad lists hold the entries of a 4-row
-// strip in the same order.  Rows are sorted and duplicate-free (checked first), so an entry finds its place
-// without any sort: its position is the number of entries of its panel (strip) with a smaller column, which
-// is a sum of binary searches over the panel's 16 rows, plus the rows above it that hold the same column.
-// An entry is the first of its column when no row above it holds that column; a prefix sum over these
-// flags, taken in sorted order, numbers the active columns.  Everything else is a scatter.
+// strip in the same order.  Rows are sorted and duplicate-free (checked first).
+//
+// A panel of up to kPanelCap entries in a window of up to kPanelSpan columns is one work-group's, and nothing is sorted: the
+// window is a bitmap in LDS, the running popcount of its words numbers the active columns, and one word per active column
+// collects which of the 16 rows hold it.  Positions, list places, header lines and records all follow from prefix sums over
+// those words; lines and records are written by the 16 lanes that stand for their 16 columns, so nothing is cleared beforehand
+// and no global atomic is needed.  About six LDS operations an entry; ranking it by binary searches over the panel's other rows
+// takes 50 to 100 (LDS merges of the rows, measured: census 57, strip lists 52 us on the graph below, 44 and 40 on the
+// finite-element matrix).
+// R-MAT graph of 65 536 nodes, 1.24 million entries: census 28 us, strip lists 40, where the entry-parallel kernels
+// over the whole matrix took 226 and 64; finite-element matrix of 24 000 rows, 1.44 million entries: census 13, brick tiles
+// 15 (before: 166 and 37).  What bounds it is latency: a dozen dependent steps a panel, four to six work-groups a compute unit.
+// Other panels (hub rows of a graph, windows too wide for the bitmap) take the entry-parallel path at the end, where an entry's
+// position is a sum of binary searches over the panel's rows in global memory; both write the same words.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -23,25 +32,68 @@ constexpr int kThreads = 256;
 constexpr int kScanItems = 8;                               // entries per thread of a scan block
 constexpr uint32_t kScanBlock = kThreads * kScanItems;      // entries per scan block
 
-enum : int { kErrRange = 1, kErrUnsorted = 2 };
+constexpr uint32_t kPanelCap = 2048;                        // entries of a panel that one work-group holds, eight a thread
+constexpr uint32_t kPanelSmall = kPanelCap / 2;             // list kernel: most panels need half the LDS, twice as many then run at a time
+constexpr uint32_t kPanelSpan = 1u << 17;                   // columns of its window: a bitmap of 16 KB and 8 KB of running counts
+
+enum : uint32_t { kErrRange = 1, kErrUnsorted = 2 };
+
+// What the planner wants to know about a panel; one 48-byte record each, written to host memory.
+struct PanelCensus {
+    uint32_t nnz, maxRow;      // entries, longest row
+    uint32_t cols, span;       // distinct (active) columns, last column - first column + 1
+    uint32_t pairs[4];         // distinct columns of each 4-row strip
+    uint32_t stored;           // entries that are not zero
+    uint32_t error;            // kErrRange | kErrUnsorted; the other fields then mean nothing
+    uint32_t pad[2];
+};
+static_assert(sizeof(PanelCensus) == 48, "written as twelve words");
+
+// The panels beyond kPanelCap or kPanelSpan, in ascending order.
+struct LargePanels {
+    const uint32_t *panel;     // [count]
+    const uint32_t *prefix;    // [count + 1] running number of entries
+    uint32_t count, total;
+};
 
 __device__ __forceinline__ uint64_t global_id() { return uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; }
 
+// Inclusive scan over the 64 lanes of a wavefront by data-parallel-primitive moves: shifts by 1, 2, 4, 8 inside the rows of 16
+// lanes, then the last lane of row 0 (2) to row 1 (3) and of lane 31 to rows 2 and 3.  No LDS round trip a step, which a
+// shuffle is: 29.9 -> 25.2 us for the list kernel, 32.0 -> 27.8 for the census of the graph above.  op(IDENTITY, x) = x.
+template <uint32_t IDENTITY, class Op>
+__device__ __forceinline__ uint32_t wave_scan(uint32_t x, Op op)
+{
+#define CUTE_DPP(ctrl, rows) x = op(x, uint32_t(__builtin_amdgcn_update_dpp(int(IDENTITY), int(x), ctrl, rows, 0xf, false)))
+    CUTE_DPP(0x111, 0xf);                    // row_shr:1
+    CUTE_DPP(0x112, 0xf);
+    CUTE_DPP(0x114, 0xf);
+    CUTE_DPP(0x118, 0xf);
+    CUTE_DPP(0x142, 0xa);                    // row_bcast:15
+    CUTE_DPP(0x143, 0xc);                    // row_bcast:31
+#undef CUTE_DPP
+    return x;
+}
+__device__ __forceinline__ uint32_t wave_add(uint32_t x) { return wave_scan<0u>(x, [](uint32_t a, uint32_t b) { return a + b; }); }
+
 // ------------------------------------------------------------------------------------------------
 // Inclusive prefix sum of uint32 values, in three steps: block sums, their prefix sum (by the same three
-// steps), block-local prefix sums shifted by the sums of the blocks before.
+// steps), block-local prefix sums shifted by the sums of the blocks before.  Several arrays of one length, `pitch` apart, are
+// summed by one launch (grid.y).
 // ------------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(kThreads) void scan_block_sums(const uint32_t *__restrict__ in, uint64_t n, uint32_t *__restrict__ sums)
+__global__ __launch_bounds__(kThreads) void scan_block_sums(const uint32_t *__restrict__ in, uint64_t n, uint64_t pitch, uint32_t *__restrict__ sums,
+                                                            uint64_t sums_pitch)
 {
+    in += blockIdx.y * pitch;
+    sums += blockIdx.y * sums_pitch;
     __shared__ uint32_t wave_sum[kThreads / 64];
     const uint64_t base = uint64_t(blockIdx.x) * kScanBlock + uint64_t(threadIdx.x) * kScanItems;
     uint32_t s = 0;
 #pragma unroll
     for (int i = 0; i < kScanItems; ++i)
         if (base + i < n) s += in[base + i];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-    if ((threadIdx.x & 63) == 0) wave_sum[threadIdx.x >> 6] = s;
+    s = wave_add(s);
+    if ((threadIdx.x & 63) == 63) wave_sum[threadIdx.x >> 6] = s;
     __syncthreads();
     if (threadIdx.x == 0) {
         uint32_t t = 0;
@@ -51,25 +103,21 @@ __global__ __launch_bounds__(kThreads) void scan_block_sums(const uint32_t *__re
     }
 }
 
-// `sums` holds the inclusive prefix sums of the block sums (nullptr when there is one block); in == out is allowed.
-__global__ __launch_bounds__(kThreads) void scan_block_apply(const uint32_t *in, uint32_t *out, uint64_t n, const uint32_t *__restrict__ sums)
+// `sums` holds the inclusive prefix sums of the block sums (nullptr when there is one block).
+__global__ __launch_bounds__(kThreads) void scan_block_apply(uint32_t *data, uint64_t n, uint64_t pitch, const uint32_t *__restrict__ sums, uint64_t sums_pitch)
 {
+    data += blockIdx.y * pitch;
+    if (sums) sums += blockIdx.y * sums_pitch;
     __shared__ uint32_t wave_total[kThreads / 64];
     const uint64_t base = uint64_t(blockIdx.x) * kScanBlock + uint64_t(threadIdx.x) * kScanItems;
     uint32_t v[kScanItems];
     uint32_t t = 0;
 #pragma unroll
     for (int i = 0; i < kScanItems; ++i) {
-        t += base + i < n ? in[base + i] : 0u;
+        t += base + i < n ? data[base + i] : 0u;
         v[i] = t;
     }
-    uint32_t incl = t;                                       // inclusive sum over the lanes of this wavefront
-    const uint32_t lane = threadIdx.x & 63u;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t up = __shfl_up(incl, off, 64);
-        if (lane >= uint32_t(off)) incl += up;
-    }
+    const uint32_t incl = wave_add(t), lane = threadIdx.x & 63u;       // inclusive sum over the lanes of this wavefront
     if (lane == 63u) wave_total[threadIdx.x >> 6] = incl;
     __syncthreads();
     uint32_t offset = (sums && blockIdx.x) ? sums[blockIdx.x - 1] : 0u;
@@ -77,284 +125,691 @@ __global__ __launch_bounds__(kThreads) void scan_block_apply(const uint32_t *in,
     offset += incl - t;
 #pragma unroll
     for (int i = 0; i < kScanItems; ++i)
-        if (base + i < n) out[base + i] = offset + v[i];
+        if (base + i < n) data[base + i] = offset + v[i];
 }
 
-// ------------------------------------------------------------------------------------------------
-// Entry -> row, and the preconditions of the format (data.cu:204,256-258 relies on them; here they are
-// checked): every column below K, strictly increasing inside a row.  rowPtr has been checked on the host.
-// ------------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(kThreads) void row_of_entries(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols,
-                                                           uint32_t M, uint32_t K, uint32_t nnz, uint32_t *__restrict__ rowOf,
-                                                           int *__restrict__ error)
+// The three CSR arrays into the handle's own memory: from the caller's device arrays, or from pinned host memory.
+__global__ __launch_bounds__(kThreads) void copy_words(const uint32_t *__restrict__ src, uint32_t *__restrict__ dst, uint64_t n)
 {
-    const uint64_t e = global_id();
-    if (e >= nnz) return;
-    uint32_t lo = 0, hi = M - 1u;                            // the row r with rowPtr[r] <= e < rowPtr[r+1]
-    while (lo < hi) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (rowPtr[mid + 1] <= e) lo = mid + 1u;
-        else hi = mid;
-    }
-    rowOf[e] = lo;
-    const uint32_t c = cols[e];
-    if (c >= K) atomicOr(error, int(kErrRange));
-    if (e > rowPtr[lo] && cols[e - 1] >= c) atomicOr(error, int(kErrUnsorted));
+    for (uint64_t i = global_id(); i < n; i += uint64_t(gridDim.x) * kThreads) dst[i] = src[i];
 }
 
-__device__ __forceinline__ uint32_t lower_bound(const uint32_t *__restrict__ cols, uint32_t lo, uint32_t hi, uint32_t c)
+__global__ __launch_bounds__(kThreads) void copy_csr(const uint32_t *__restrict__ srcRowPtr, const uint32_t *__restrict__ srcCols,
+                                                     const uint32_t *__restrict__ srcVals, uint32_t M, uint32_t nnz,
+                                                     uint32_t *__restrict__ rowPtr, uint32_t *__restrict__ cols, uint32_t *__restrict__ vals)
 {
+    const uint64_t stride = uint64_t(gridDim.x) * kThreads;
+    for (uint64_t i = global_id(); i < nnz; i += stride) { cols[i] = srcCols[i]; vals[i] = srcVals[i]; }
+    for (uint64_t i = global_id(); i <= M; i += stride) rowPtr[i] = srcRowPtr[i];
+}
+
+__device__ __forceinline__ uint32_t row_in_panel(const uint32_t *rp, uint32_t e)
+{
+    uint32_t lo = 0, hi = 15u;                               // the row r with rp[r] <= e < rp[r+1]
     while (lo < hi) {
         const uint32_t mid = (lo + hi) >> 1;
-        if (cols[mid] < c) lo = mid + 1u;
+        if (rp[mid + 1] <= e) lo = mid + 1u;
         else hi = mid;
     }
     return lo;
 }
 
-// Position of every entry in the (column, row) order of its 16-row panel (posP) and of its 4-row strip (posS),
-// and, at those positions, whether the entry is the first of its column there (firstP, firstS).
-__global__ __launch_bounds__(kThreads) void entry_positions(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols,
-                                                            const uint32_t *__restrict__ rowOf, uint32_t nnz,
-                                                            uint32_t *__restrict__ posP, uint32_t *__restrict__ posS,
-                                                            uint32_t *__restrict__ firstP, uint32_t *__restrict__ firstS)
+// ------------------------------------------------------------------------------------------------
+// A panel in LDS.
+// ------------------------------------------------------------------------------------------------
+struct Two { uint32_t x, y; };
+template <uint32_t CAP> struct PanelLds {
+    uint32_t rp[17];                         // row starts, from the panel's first entry
+    uint32_t lo, hi;                         // first and last column
+    Two waveSum[kThreads / 64];
+    uint32_t col[CAP];                       // active columns
+    uint32_t rows[CAP];                      // and the rows that hold them: bits 0..15 any entry, bits 16..31 one that is not zero
+};
+
+// The entries t, t + 256, .. of a panel in one thread's registers.
+template <uint32_t CAP> struct PanelEntries {
+    static constexpr uint32_t kEach = CAP / kThreads;
+    uint32_t active[kEach];                  // index of the entry's column among the panel's active columns
+    uint32_t row[kEach];
+    float val[kEach];
+};
+
+// Dynamic LDS of the panel kernels: the window's bitmap and the running counts of its words, later reused.
+inline __host__ __device__ uint32_t panel_window_words(uint32_t max_span) { return (max_span + 31u) / 32u; }
+
+// Sum over the threads before this one, and over the whole work-group in `total`, of two words at once.
+template <uint32_t CAP> __device__ __forceinline__ Two block_exclusive(PanelLds<CAP> &l, Two own, Two &total)
 {
-    const uint64_t e = global_id();
-    if (e >= nnz) return;
-    const uint32_t r = rowOf[e], c = cols[e];
-    const uint32_t r0 = r & ~15u, me = r - r0, strip0 = me & ~3u;
-    uint32_t below = 0, above_same = 0, below_s = 0, above_same_s = 0;
-    uint32_t lo = rowPtr[r0];
-    const uint32_t panel_start = lo;
-    uint32_t strip_start = 0;
-    for (uint32_t i = 0; i < 16u; ++i) {
-        const uint32_t hi = rowPtr[r0 + i + 1u];
-        if (i == strip0) strip_start = lo;
-        uint32_t cnt, has = 0;
-        if (i == me) cnt = uint32_t(e) - lo;
-        else {
-            const uint32_t lb = lower_bound(cols, lo, hi, c);
-            cnt = lb - lo;
-            has = (lb < hi && cols[lb] == c) ? 1u : 0u;
-        }
-        below += cnt;
-        if (i < me) above_same += has;
-        if ((i & ~3u) == strip0) {
-            below_s += cnt;
-            if (i < me) above_same_s += has;
-        }
-        lo = hi;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const Two incl = {wave_add(own.x), wave_add(own.y)};
+    if (lane == 63u) l.waveSum[wave] = incl;
+    __syncthreads();
+    Two before = {incl.x - own.x, incl.y - own.y};
+    total = {0u, 0u};
+#pragma unroll
+    for (uint32_t w = 0; w < kThreads / 64u; ++w) {
+        const Two v = l.waveSum[w];
+        if (w < wave) { before.x += v.x; before.y += v.y; }
+        total.x += v.x;
+        total.y += v.y;
     }
-    const uint32_t pp = panel_start + below + above_same, ps = strip_start + below_s + above_same_s;
-    posP[e] = pp;
-    posS[e] = ps;
+    __syncthreads();
+    return before;
+}
+template <uint32_t CAP> __device__ __forceinline__ uint32_t block_exclusive(PanelLds<CAP> &l, uint32_t own, uint32_t &total)
+{
+    Two sum;
+    const uint32_t before = block_exclusive(l, Two{own, 0u}, sum).x;
+    total = sum.x;
+    return before;
+}
+
+// Row starts into LDS; returns the number of entries, or ~0u when the pointers do not ascend within [0, nnz].
+// (every panel checks its own 17, so together they check all of them before anything is indexed through them)
+template <uint32_t CAP> __device__ __forceinline__ uint32_t panel_rows(PanelLds<CAP> &l, const uint32_t *__restrict__ rowPtr, uint32_t p, uint32_t P, uint32_t nnz,
+                                               uint32_t &start)
+{
+    const uint32_t t = threadIdx.x;
+    int bad = 0;
+    const uint32_t s = rowPtr[uint64_t(p) * 16u];
+    if (t < 17u) {
+        const uint32_t v = rowPtr[uint64_t(p) * 16u + t];
+        l.rp[t] = v - s;
+        if (t < 16u) bad = v > rowPtr[uint64_t(p) * 16u + t + 1u];
+        else bad = v > nnz || (p == P - 1u && v != nnz);
+        if (t == 0u && p == 0u && v != 0u) bad = 1;
+    }
+    if (t == 0u) { l.lo = ~0u; l.hi = 0u; }
+    bad = __syncthreads_or(bad);
+    start = s;
+    return bad ? ~0u : l.rp[16];
+}
+
+template <uint32_t CAP> __device__ __forceinline__ bool panel_fits(const PanelLds<CAP> &l, uint32_t max_span) { return l.hi - l.lo < max_span; }
+
+// Loads the entries of a panel of up to CAP of them, finds its column window and clears the LDS that numbers it (while the
+// loads are on their way).  CHECK: returns the error bits of the panel, every thread the same.
+template <bool CHECK, uint32_t CAP>
+__device__ __forceinline__ uint32_t load_panel(PanelLds<CAP> &l, PanelEntries<CAP> &e, uint32_t *window, const uint32_t *__restrict__ cols,
+                                               const float *__restrict__ vals, uint32_t start, uint32_t n, uint32_t K, uint32_t max_span)
+{
+    const uint32_t t = threadIdx.x;
+    int range = 0, unsorted = 0;
+    uint32_t lo = ~0u, hi = 0u;
+#pragma unroll
+    for (uint32_t k = 0; k < PanelEntries<CAP>::kEach; ++k) {
+        if (k * kThreads >= n) break;
+        const uint32_t i = k * kThreads + t;
+        if (i >= n) continue;
+        e.active[k] = cols[uint64_t(start) + i];             // its column until number_columns
+        e.val[k] = vals[uint64_t(start) + i];
+    }
+    for (uint32_t w = t; w < panel_window_words(max_span); w += kThreads) window[w] = 0u;
+    for (uint32_t i = t; i < n; i += kThreads) l.rows[i] = 0u;
+#pragma unroll
+    for (uint32_t k = 0; k < PanelEntries<CAP>::kEach; ++k) {
+        if (k * kThreads >= n) break;
+        const uint32_t i = k * kThreads + t;
+        if (i >= n) continue;
+        e.row[k] = row_in_panel(l.rp, i);
+        const uint32_t c = e.active[k];
+        lo = min(lo, c);
+        hi = max(hi, c);
+        if (CHECK) {
+            range |= c >= K;
+            unsorted |= i > l.rp[e.row[k]] && cols[uint64_t(start) + i - 1u] >= c;
+        }
+    }
+    lo = wave_scan<~0u>(lo, [](uint32_t a, uint32_t b) { return min(a, b); });
+    hi = wave_scan<0u>(hi, [](uint32_t a, uint32_t b) { return max(a, b); });
+    if ((t & 63u) == 63u) { atomicMin(&l.lo, lo); atomicMax(&l.hi, hi); }
+    if (!CHECK) {
+        __syncthreads();
+        return 0u;
+    }
+    if (!__syncthreads_or(range | unsorted)) return 0u;
+    range = __syncthreads_or(range);
+    return (range ? kErrRange : 0u) | (__syncthreads_or(unsorted) ? kErrUnsorted : 0u);
+}
+
+// Numbers the active columns and fills l.col and l.rows; returns how many there are.
+template <uint32_t CAP>
+__device__ __forceinline__ uint32_t number_columns(PanelLds<CAP> &l, PanelEntries<CAP> &e, uint32_t *window, uint32_t n)
+{
+    const uint32_t t = threadIdx.x, lo = l.lo, words = (l.hi - lo) / 32u + 1u;
+    uint16_t *count = reinterpret_cast<uint16_t *>(window + words);
+#pragma unroll
+    for (uint32_t k = 0; k < PanelEntries<CAP>::kEach; ++k) {
+        if (k * kThreads >= n) break;
+        if (k * kThreads + t < n) atomicOr(&window[(e.active[k] - lo) >> 5], 1u << ((e.active[k] - lo) & 31u));
+    }
+    __syncthreads();
+    const uint32_t per = (words + kThreads - 1u) / kThreads, w0 = min(t * per, words), w1 = min(w0 + per, words);
+    uint32_t own = 0;
+    for (uint32_t w = w0; w < w1; ++w) own += uint32_t(__popc(window[w]));
+    uint32_t total;
+    uint32_t run = block_exclusive(l, own, total);
+    for (uint32_t w = w0; w < w1; ++w) { count[w] = uint16_t(run); run += uint32_t(__popc(window[w])); }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t k = 0; k < PanelEntries<CAP>::kEach; ++k) {
+        if (k * kThreads >= n) break;
+        if (k * kThreads + t >= n) continue;
+        const uint32_t c = e.active[k], w = (c - lo) >> 5;
+        const uint32_t a = count[w] + uint32_t(__popc(window[w] & ((1u << ((c - lo) & 31u)) - 1u)));
+        e.active[k] = a;
+        l.col[a] = c;
+        atomicOr(&l.rows[a], (1u << e.row[k]) | (e.val[k] != 0.0f ? 1u << (16u + e.row[k]) : 0u));
+    }
+    __syncthreads();
+    return total;
+}
+
+// Does strip s hold the column?  Strips 0 and 1 in the halves of x, 2 and 3 in those of y; half() takes one out again.
+__device__ __forceinline__ Two strips_of(uint32_t rows)
+{
+    return {(rows & 0xfu ? 1u : 0u) | (rows & 0xf0u ? 0x10000u : 0u), (rows & 0xf00u ? 1u : 0u) | (rows & 0xf000u ? 0x10000u : 0u)};
+}
+__device__ __forceinline__ uint32_t half(const Two &v, uint32_t s) { return ((s & 2u ? v.y : v.x) >> (16u * (s & 1u))) & 0xffffu; }
+
+__global__ __launch_bounds__(kThreads) void panel_census(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols,
+                                                         const float *__restrict__ vals, uint32_t P, uint32_t K, uint32_t nnz, uint32_t max_span,
+                                                         PanelCensus *__restrict__ out)
+{
+    constexpr uint32_t CAP = kPanelCap;
+    extern __shared__ uint32_t window[];
+    __shared__ PanelLds<CAP> l;
+    __shared__ PanelCensus res;
+    const uint32_t p = blockIdx.x, t = threadIdx.x;
+    uint32_t start;
+    if (t < 12u) reinterpret_cast<uint32_t *>(&res)[t] = 0u;
+    const uint32_t n = panel_rows(l, rowPtr, p, P, nnz, start);
+    if (n == ~0u) {
+        if (t == 0u) res.error = kErrRange;
+    } else {
+        if (t < 16u) atomicMax(&res.maxRow, l.rp[t + 1] - l.rp[t]);
+        if (t == 0u) res.nnz = n;
+        if (n > kPanelCap) {
+            if (t < 16u && l.rp[t + 1] > l.rp[t]) {
+                atomicMin(&l.lo, cols[uint64_t(start) + l.rp[t]]);
+                atomicMax(&l.hi, cols[uint64_t(start) + l.rp[t + 1] - 1u]);
+            }
+        } else if (n) {
+            PanelEntries<CAP> e;
+            const uint32_t err = load_panel<true>(l, e, window, cols, vals, start, n, K, max_span);
+            if (err) {
+                if (t == 0u) res.error = err;
+            } else if (panel_fits(l, max_span)) {
+                const uint32_t active = number_columns(l, e, window, n);
+                Two pairs = {0u, 0u};
+                uint32_t stored = 0;
+                for (uint32_t a = t; a < active; a += kThreads) {
+                    const Two here = strips_of(l.rows[a]);
+                    pairs.x += here.x;
+                    pairs.y += here.y;
+                    stored += uint32_t(__popc(l.rows[a] >> 16));
+                }
+                pairs = {wave_add(pairs.x), wave_add(pairs.y)};
+                stored = wave_add(stored);
+                if ((t & 63u) == 63u) {
+#pragma unroll
+                    for (uint32_t s = 0; s < 4u; ++s) atomicAdd(&res.pairs[s], half(pairs, s));
+                    atomicAdd(&res.stored, stored);
+                }
+                if (t == 0u) res.cols = active;
+            }
+        }
+    }
+    __syncthreads();
+    if (t == 0u && n && n != ~0u) res.span = l.hi - l.lo + 1u;
+    __syncthreads();
+    if (t < 12u) reinterpret_cast<uint32_t *>(out + p)[t] = reinterpret_cast<const uint32_t *>(&res)[t];
+}
+
+// Brick tiles of the panels that fit: hdr lines and values (cute_hrpb_retile defines both).  brp: first block of every
+// panel.  Block 0 also writes the wavefront of zeros behind the values.
+__global__ __launch_bounds__(kThreads) void panel_bricks(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols,
+                                                         const float *__restrict__ vals, uint32_t P, uint32_t nnz, uint32_t max_span,
+                                                         const uint32_t *__restrict__ brp, uint32_t *__restrict__ hdr, float *__restrict__ tile_vals)
+{
+    constexpr uint32_t CAP = kPanelCap;
+    extern __shared__ uint32_t window[];
+    __shared__ PanelLds<CAP> l;
+    const uint32_t p = blockIdx.x, t = threadIdx.x;
+    if (p == 0u && t < 64u) tile_vals[uint64_t(nnz) + t] = 0.0f;
+    const uint32_t block0 = brp[p];
+    uint32_t start;
+    const uint32_t n = panel_rows(l, rowPtr, p, P, nnz, start);
+    if (n == 0u || n > kPanelCap) return;
+    PanelEntries<CAP> e;
+    load_panel<false>(l, e, window, cols, vals, start, n, 0u, max_span);
+    if (!panel_fits(l, max_span)) return;
+    const uint32_t active = number_columns(l, e, window, n);
+    uint16_t *first = reinterpret_cast<uint16_t *>(window);   // position of every active column's first entry, and n behind the last
+    {
+        uint32_t own = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < PanelEntries<CAP>::kEach; ++k) {
+            const uint32_t a = t * PanelEntries<CAP>::kEach + k;
+            own += a < active ? uint32_t(__popc(l.rows[a] & 0xffffu)) : 0u;
+        }
+        uint32_t total;
+        uint32_t run = block_exclusive(l, own, total);
+#pragma unroll
+        for (uint32_t k = 0; k < PanelEntries<CAP>::kEach; ++k) {
+            const uint32_t a = t * PanelEntries<CAP>::kEach + k;
+            if (a <= active) first[a] = uint16_t(run);
+            run += a < active ? uint32_t(__popc(l.rows[a] & 0xffffu)) : 0u;
+        }
+        if (t == 0u && active == CAP) first[CAP] = uint16_t(n);
+    }
+    __syncthreads();
+    const uint32_t slots = ((active + 15u) / 16u) * 16u;
+    for (uint32_t a = t; a < slots; a += kThreads) {          // sixteen lanes are the sixteen columns of one block
+        const uint32_t b = first[min(a, active)];
+        const uint32_t mask = a < active ? l.rows[a] & 0xffffu : 0u;
+        const uint32_t slot = a & 15u, j = slot >> 2, k = slot & 3u;
+        uint32_t *h = hdr + (uint64_t(block0) + (a >> 4)) * CUTE_TILED_HDR_WORDS;
+        h[k * 4u + j] = a < active ? l.col[a] : 0u;
+        const uint32_t upper = __shfl_xor(mask, 1);           // bit k*16 + row of the brick's bitmap: two columns to a word
+        if ((k & 1u) == 0u) h[16u + 2u * j + (k >> 1)] = mask | (upper << 16);
+        if (k == 0u) h[24u + j] = start + b;                  // a brick of padding columns only points at the panel's end
+        if (slot < 4u) h[28u + slot] = slot == 0u ? uint32_t(first[min((a | 15u) + 1u, active)]) - first[a & ~15u] : 0u;
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < PanelEntries<CAP>::kEach; ++k) {
+        if (k * kThreads >= n) break;
+        if (k * kThreads + t >= n) continue;
+        const uint32_t a = e.active[k];
+        tile_vals[uint64_t(start) + first[a] + uint32_t(__popc(l.rows[a] & ((1u << e.row[k]) - 1u)))] = e.val[k];
+    }
+}
+
+// Quad lists of the panels that fit (cute_quad_pack defines them).  STRIPS: one list per strip, groups[4p + s] its first group;
+// else four lockstep lists per panel, groups[p].  valBase: first stored value of every panel.  A thread is one
+// (row group, column) pair; the running number of stored values over the pairs of the panel is at once the place of
+// their values and, at a group's first pair, the record's index word.  Block 0 writes the zeros behind the values.
+// list_of: the panels to take (those beyond kPanelSmall: a launch over all panels spends 15 us on work-groups that only leave),
+// nullptr: every panel of up to CAP entries.
+// Dynamic LDS: the window, then (in its place) the list places of every column, four 16-bit numbers each.
+template <bool STRIPS, uint32_t CAP>
+__global__ __launch_bounds__(kThreads) void panel_quads(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols,
+                                                        const float *__restrict__ vals, uint32_t P, uint32_t nnz, uint32_t max_span, const uint32_t *__restrict__ list_of,
+                                                        const uint32_t *__restrict__ groups, const uint32_t *__restrict__ valBase, uint32_t stored,
+                                                        uint32_t *__restrict__ recs, float *__restrict__ packed)
+{
+    extern __shared__ uint32_t window[];
+    __shared__ PanelLds<CAP> l;
+    __shared__ uint16_t list[CAP], place[CAP];    // pair -> active column, and -> its first value from the panel's first
+    const uint32_t p = list_of ? list_of[blockIdx.x] : blockIdx.x, t = threadIdx.x;
+    if (!list_of && p == 0u && t < 64u) packed[uint64_t(stored) + t] = 0.0f;
+    const uint32_t group0 = groups[uint64_t(p) * (STRIPS ? 4u : 1u)], value0 = valBase[p];
+    uint32_t start;
+    const uint32_t n = panel_rows(l, rowPtr, p, P, nnz, start);
+    if (n == 0u || n > CAP) return;
+    PanelEntries<CAP> e;
+    load_panel<false>(l, e, window, cols, vals, start, n, 0u, max_span);
+    if (!panel_fits(l, max_span)) return;
+    const uint32_t active = number_columns(l, e, window, n);
+    Two *before = reinterpret_cast<Two *>(window);            // pairs in front of an active column's, in each strip's list
+    Two lens;
+    {
+        Two own = {0u, 0u};
+#pragma unroll
+        for (uint32_t k = 0; k < PanelEntries<CAP>::kEach; ++k) {
+            const uint32_t a = t * PanelEntries<CAP>::kEach + k;
+            const Two here = strips_of(a < active ? l.rows[a] : 0u);
+            own.x += here.x;
+            own.y += here.y;
+        }
+        Two run = block_exclusive(l, own, lens);
+        // (a strip's pairs stand behind those of the strips in front of it)
+        const uint32_t front = half(lens, 0) + half(lens, 1);
+        run.x += half(lens, 0) << 16;
+        run.y += front | ((front + half(lens, 2)) << 16);
+#pragma unroll
+        for (uint32_t k = 0; k < PanelEntries<CAP>::kEach; ++k) {
+            const uint32_t a = t * PanelEntries<CAP>::kEach + k;
+            if (a >= active) break;
+            const Two here = strips_of(l.rows[a]);
+            before[a] = run;
+#pragma unroll
+            for (uint32_t s = 0; s < 4u; ++s)
+                if (half(here, s)) list[half(run, s)] = uint16_t(a);
+            run.x += here.x;
+            run.y += here.y;
+        }
+    }
+    __syncthreads();
+    uint32_t len[4], list0[4], group_before[4], total = 0;    // list lengths and starts; STRIPS: groups in front of each strip
+#pragma unroll
+    for (uint32_t s = 0; s < 4u; ++s) {
+        len[s] = half(lens, s);
+        list0[s] = s ? list0[s - 1] + len[s - 1] : 0u;
+        group_before[s] = total;
+        total = STRIPS ? total + (len[s] + 15u) / 16u : max(total, (len[s] + 3u) / 4u);
+    }
+    const uint32_t slots = total * 16u;
+    uint32_t base = 0;
+    for (uint32_t x0 = 0; x0 < slots; x0 += kThreads) {
+        const uint32_t x = x0 + t, g = x >> 4, pair = x & 15u;
+        const bool live = x < slots;
+        const uint32_t s = STRIPS ? (g >= group_before[1] ? 1u : 0u) + (g >= group_before[2] ? 1u : 0u) + (g >= group_before[3] ? 1u : 0u) : pair & 3u;
+        auto of_strip = [&](const uint32_t (&v)[4]) { return s == 0u ? v[0] : s == 1u ? v[1] : s == 2u ? v[2] : v[3]; };
+        const uint32_t q = STRIPS ? 16u * (g - of_strip(group_before)) + pair : 4u * g + (pair >> 2);
+        const uint32_t my_len = of_strip(len), my_list = of_strip(list0);
+        uint32_t col = 0, mask = 0;
+        if (live && my_len) {
+            const uint32_t a = list[my_list + min(q, my_len - 1u)];           // padding repeats the last column of its list
+            col = l.col[a];
+            mask = q < my_len ? (l.rows[a] >> (16u + 4u * s)) & 15u : 0u;     // an explicit zero is an empty slot
+        }
+        uint32_t sum;
+        const uint32_t at = base + block_exclusive(l, uint32_t(__popc(mask)), sum);
+        base += sum;
+        uint32_t word = mask << (4u * (pair & 7u));           // slot 4*pair + row: eight pairs to a mask word
+        word |= __shfl_xor(word, 1);
+        word |= __shfl_xor(word, 2);
+        word |= __shfl_xor(word, 4);
+        if (live) {
+            uint32_t *rec = recs + (uint64_t(group0) + g) * CUTE_QUAD_RECORD_WORDS;
+            rec[pair] = col;
+            if (pair == 0u) { rec[16] = word; rec[18] = value0 + at; }
+            if (pair == 8u) { rec[17] = word; rec[19] = 0u; }
+            if (q < my_len) place[my_list + q] = uint16_t(at);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t k = 0; k < PanelEntries<CAP>::kEach; ++k) {
+        if (k * kThreads >= n) break;
+        if (k * kThreads + t >= n || e.val[k] == 0.0f) continue;
+        const uint32_t a = e.active[k], s = e.row[k] >> 2, mask = (l.rows[a] >> (16u + 4u * s)) & 15u;
+        const uint32_t pr = half(before[a], s);
+        packed[uint64_t(value0) + place[pr] + uint32_t(__popc(mask & ((1u << (e.row[k] & 3u)) - 1u)))] = e.val[k];
+    }
+}
+
+// ------------------------------------------------------------------------------------------------
+// The other panels: a thread per entry, searches over the rows in global memory, positions and numbers in temporary
+// arrays over the entries of these panels alone (index id = prefix[k] + position in the panel).
+// ------------------------------------------------------------------------------------------------
+// First index whose column is not below c[k] in each of R sorted ranges [lo[k], lo[k] + len[k]); left in lo.  The searches
+// advance together, so their reads overlap: 57 -> 41 us for the hub panels of the graph above.
+template <int R>
+__device__ __forceinline__ void lower_bounds(const uint32_t *__restrict__ cols, uint32_t (&lo)[R], uint32_t (&len)[R], uint32_t c)
+{
+    uint32_t left;
+    do {
+        left = 0;
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const uint32_t half = len[k] >> 1, probe = len[k] ? lo[k] + half : 0u;
+            const bool less = cols[probe] < c && len[k] != 0u;
+            lo[k] = less ? probe + 1u : lo[k];
+            len[k] = less ? len[k] - half - 1u : half;
+            left |= len[k];
+        }
+    } while (left);
+}
+
+__device__ __forceinline__ uint32_t upper_index(const uint32_t *__restrict__ prefix, uint32_t count, uint32_t id)
+{
+    uint32_t lo = 0, hi = count - 1u;                        // the k with prefix[k] <= id < prefix[k+1]
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (prefix[mid + 1] <= id) lo = mid + 1u;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// Position of every entry in the (column, row) order of its panel (posP) and of its strip (posS), and, at those positions,
+// whether the entry is the first of its column there (firstP, firstS).  Also counts the stored values and checks the columns.
+__global__ __launch_bounds__(kThreads) void large_positions(LargePanels L, const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols,
+                                                            const float *__restrict__ vals, uint32_t K, uint32_t *__restrict__ posP,
+                                                            uint32_t *__restrict__ posS, uint32_t *__restrict__ firstP,
+                                                            uint32_t *__restrict__ firstS, PanelCensus *__restrict__ res)
+{
+    const uint64_t id64 = global_id();
+    const bool live = id64 < L.total;
+    const uint32_t id = live ? uint32_t(id64) : L.total - 1u;
+    const uint32_t k = upper_index(L.prefix, L.count, id), base = L.prefix[k];
+    const uint32_t *rp = rowPtr + uint64_t(L.panel[k]) * 16u;
+    const uint32_t panel_start = rp[0], e = panel_start + (id - base), me = row_in_panel(rp, e), strip0 = me & ~3u;
+    const uint32_t c = cols[e];
+    if (res) {
+        uint32_t err = 0;
+        if (c >= K) err |= kErrRange;
+        if (e > rp[me] && cols[e - 1u] >= c) err |= kErrUnsorted;
+        if (live && err) atomicOr(&res[k].error, err);
+        // one addition per wavefront where its entries belong to one panel, which is nearly always
+        const bool stored = live && vals[e] != 0.0f;
+        const uint32_t k0 = __shfl(k, 0);
+        if (__ballot(k != k0) == 0ull) {
+            const uint64_t m = __ballot(stored);
+            if ((threadIdx.x & 63u) == 0u && m) atomicAdd(&res[k].stored, uint32_t(__popcll(m)));
+        } else if (stored) atomicAdd(&res[k].stored, 1u);
+    }
+    if (!live) return;
+    uint32_t below = 0, above_same = 0, below_s = 0, above_same_s = 0;
+#pragma unroll
+    for (uint32_t i0 = 0; i0 < 16u; i0 += 4u) {              // a strip's rows at a time
+        uint32_t lo[4], len[4];
+#pragma unroll
+        for (uint32_t k = 0; k < 4u; ++k) { lo[k] = rp[i0 + k]; len[k] = rp[i0 + k + 1u] - lo[k]; }
+        lower_bounds<4>(cols, lo, len, c);
+#pragma unroll
+        for (uint32_t k = 0; k < 4u; ++k) {
+            const uint32_t i = i0 + k, cnt = lo[k] - rp[i];  // (the entry's own row counts the entries in front of it)
+            const uint32_t has = (i < me && lo[k] < rp[i + 1u] && cols[lo[k]] == c) ? 1u : 0u;
+            below += cnt;
+            above_same += has;
+            if (i0 == strip0) { below_s += cnt; above_same_s += has; }
+        }
+    }
+    // (columns that are not sorted give positions that mean nothing, but never ones outside the panel: the census refuses them)
+    const uint32_t last = L.prefix[k + 1] - 1u;
+    const uint32_t pp = min(base + below + above_same, last), ps = min(base + (rp[strip0] - panel_start) + below_s + above_same_s, last);
+    posP[id] = pp;
+    posS[id] = ps;
     firstP[pp] = above_same == 0u ? 1u : 0u;
     firstS[ps] = above_same_s == 0u ? 1u : 0u;
 }
 
-// Active columns per panel and list pairs per strip, from the prefix sums DP, DS of the first-of-column flags.
-// Also the width of every panel's column window (last column - first column + 1; rows are sorted).
-__global__ __launch_bounds__(kThreads) void count_columns(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols,
-                                                          const uint32_t *__restrict__ DP, const uint32_t *__restrict__ DS,
-                                                          uint32_t P, uint32_t *__restrict__ panelCols,
-                                                          uint32_t *__restrict__ stripPairs, uint32_t *__restrict__ panelSpan)
+// Active columns and list pairs of the large panels, from the prefix sums DP, DS of the first flags.
+__global__ __launch_bounds__(kThreads) void large_counts(LargePanels L, const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ DP,
+                                                         const uint32_t *__restrict__ DS, const PanelCensus *__restrict__ res, PanelCensus *__restrict__ out)
+{
+    const uint64_t k = global_id();
+    if (k >= L.count) return;
+    const uint32_t p = L.panel[k], base = L.prefix[k], end = L.prefix[k + 1];
+    const uint32_t *rp = rowPtr + uint64_t(p) * 16u;
+    auto run = [](const uint32_t *__restrict__ D, uint32_t b, uint32_t e) { return e > b ? D[e - 1u] - (b ? D[b - 1u] : 0u) : 0u; };
+    out[p].cols = run(DP, base, end);
+    for (uint32_t s = 0; s < 4u; ++s) out[p].pairs[s] = run(DS, base + (rp[4u * s] - rp[0]), base + (rp[4u * s + 4u] - rp[0]));
+    out[p].stored = res[k].stored;
+    out[p].error = res[k].error;
+}
+
+// unit[k]: first block (group) of large panel k in the layout; unitPrefix: running number of blocks (groups) over the large
+// panels.  Clears their header lines (records), which the scatter below fills with atomics.
+__global__ __launch_bounds__(kThreads) void large_clear(const uint32_t *__restrict__ unit, const uint32_t *__restrict__ unitPrefix,
+                                                        uint32_t count, uint32_t words, uint32_t *__restrict__ dst)
 {
     const uint64_t id = global_id();
-    if (id < P) {
-        const uint32_t s = rowPtr[id * 16u], e = rowPtr[id * 16u + 16u];
-        panelCols[id] = e > s ? DP[e - 1u] - DP[s] + 1u : 0u;
-        uint32_t lo = ~0u, hi = 0u;
-        for (uint32_t r = 0; r < 16u; ++r) {
-            const uint32_t rs = rowPtr[id * 16u + r], re = rowPtr[id * 16u + r + 1u];
-            if (re > rs) { lo = min(lo, cols[rs]); hi = max(hi, cols[re - 1u]); }
-        }
-        panelSpan[id] = e > s ? hi - lo + 1u : 0u;
-    }
-    if (id < uint64_t(P) * 4u) {
-        const uint32_t s = rowPtr[id * 4u], e = rowPtr[id * 4u + 4u];
-        stripPairs[id] = e > s ? DS[e - 1u] - DS[s] + 1u : 0u;
-    }
+    if (id >= uint64_t(unitPrefix[count]) * words) return;
+    const uint32_t u = uint32_t(id / words), k = upper_index(unitPrefix, count, u);
+    dst[(uint64_t(unit[k]) + (u - unitPrefix[k])) * words + uint32_t(id % words)] = 0u;
 }
 
-// ------------------------------------------------------------------------------------------------
-// Brick tiles: hdr[nb][32] (zeroed before) and vals[] in (panel, column, row) order.
-// ------------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(kThreads) void brick_scatter(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols,
-                                                          const float *__restrict__ vals, const uint32_t *__restrict__ rowOf,
-                                                          const uint32_t *__restrict__ posP, const uint32_t *__restrict__ DP,
-                                                          const uint32_t *__restrict__ brp, uint32_t nnz, uint32_t *hdr,
-                                                          float *__restrict__ tile_vals)
+__global__ __launch_bounds__(kThreads) void large_bricks(LargePanels L, const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols,
+                                                         const float *__restrict__ vals, const uint32_t *__restrict__ posP,
+                                                         const uint32_t *__restrict__ DP, const uint32_t *__restrict__ unit,
+                                                         uint32_t *hdr, float *__restrict__ tile_vals)
 {
-    const uint64_t e = global_id();
-    if (e >= nnz) return;
-    const uint32_t r = rowOf[e], p = r >> 4, row = r & 15u, pos = posP[e], start = rowPtr[p << 4];
-    const uint32_t a = DP[pos] - DP[start];                  // index of the entry's column among the panel's active columns
+    const uint64_t id = global_id();
+    if (id >= L.total) return;
+    const uint32_t k0 = upper_index(L.prefix, L.count, uint32_t(id)), base = L.prefix[k0];
+    const uint32_t *rp = rowPtr + uint64_t(L.panel[k0]) * 16u;
+    const uint32_t start = rp[0], e = start + (uint32_t(id) - base), row = row_in_panel(rp, e), pos = posP[id];
+    const uint32_t a = DP[pos] - DP[base];                   // index of the entry's column among the panel's active columns
     const uint32_t j = (a >> 2) & 3u, k = a & 3u;
-    uint32_t *h = hdr + (size_t(brp[p]) + (a >> 4)) * CUTE_TILED_HDR_WORDS;
-    tile_vals[pos] = vals[e];
+    uint32_t *h = hdr + (uint64_t(unit[k0]) + (a >> 4)) * CUTE_TILED_HDR_WORDS;
+    tile_vals[start + (pos - base)] = vals[e];
     const uint32_t bit = k * 16u + row;                      // the A operand slot of lane `bit` in v_mfma_f32_16x16x4_f32
     atomicOr(h + 16u + 2u * j + (bit >> 5), 1u << (bit & 31u));
-    if (pos == start || DP[pos] != DP[pos - 1u]) {           // first entry of its column: the column's own words
+    if (pos == base || DP[pos] != DP[pos - 1u]) {            // first entry of its column: the column's own words
         h[k * 4u + j] = cols[e];
-        if (k == 0u) h[24u + j] = pos;
+        if (k == 0u) h[24u + j] = start + (pos - base);
     }
 }
 
-// Per block: value offsets of bricks that hold padding columns only (they point at the end of the block, where
-// a running offset would stand) and the number of entries in the block.
-__global__ __launch_bounds__(kThreads) void brick_finish(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ brp,
-                                                         const uint32_t *__restrict__ panelCols, uint32_t P, uint32_t nb, uint32_t *hdr)
+// Per block of a large panel: value offsets of bricks that hold padding columns only (they point at the end of the block,
+// where a running offset would stand) and the number of entries in the block.
+__global__ __launch_bounds__(kThreads) void large_brick_ends(LargePanels L, const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ unit,
+                                                             const uint32_t *__restrict__ unitPrefix, const uint32_t *__restrict__ panelCols,
+                                                             uint32_t *hdr)
 {
     const uint64_t b = global_id();
-    if (b >= nb) return;
-    uint32_t lo = 0, hi = P - 1u;                            // the panel p with brp[p] <= b < brp[p+1]
-    while (lo < hi) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (brp[mid + 1] <= b) lo = mid + 1u;
-        else hi = mid;
-    }
-    const uint32_t p = lo;
-    uint32_t *h = hdr + size_t(b) * CUTE_TILED_HDR_WORDS;
-    const uint32_t end = (b + 1u == brp[p + 1u]) ? rowPtr[p * 16u + 16u] : hdr[size_t(b + 1u) * CUTE_TILED_HDR_WORDS + 24u];
-    const uint32_t live = min(16u, panelCols[p] - 16u * (uint32_t(b) - brp[p]));
+    if (b >= unitPrefix[L.count]) return;
+    const uint32_t k = upper_index(unitPrefix, L.count, uint32_t(b)), local = uint32_t(b) - unitPrefix[k];
+    uint32_t *h = hdr + (uint64_t(unit[k]) + local) * CUTE_TILED_HDR_WORDS;
+    const bool last = b + 1u == unitPrefix[k + 1u];
+    const uint32_t end = last ? rowPtr[uint64_t(L.panel[k]) * 16u + 16u] : h[CUTE_TILED_HDR_WORDS + 24u];
+    const uint32_t live = min(16u, panelCols[k] - 16u * local);
     for (uint32_t j = 1; j < 4u; ++j)
         if (4u * j >= live) h[24u + j] = end;
     h[28] = end - h[24];
 }
 
-// ------------------------------------------------------------------------------------------------
-// Quad lists: recs[numGroups][20] (zeroed before) and the stored values in slot order.
-// STRIPS: one list per 4-row strip (unit = strip, a group = 16 consecutive pairs); else four lockstep lists
-// per panel (unit = panel, pair 4*step + list).
-// ------------------------------------------------------------------------------------------------
+// Where the pair of an entry of large panel k stands.  STRIPS: one list per 4-row strip (a group = 16 consecutive pairs of one
+// strip, group[4k + s] its first); else four lockstep lists per panel (pair 4*step + list, group[k] the panel's first).
 template <bool STRIPS>
-__device__ __forceinline__ void quad_place(uint32_t r, uint32_t pos, const uint32_t *__restrict__ rowPtr,
-                                           const uint32_t *__restrict__ DS, const uint32_t *__restrict__ qgp, uint32_t &group,
-                                           uint32_t &pair, bool &first)
+__device__ __forceinline__ void large_place(uint32_t k, uint32_t row, uint32_t stripBase, uint32_t pos, const uint32_t *__restrict__ DS,
+                                            const uint32_t *__restrict__ group, uint32_t &g, uint32_t &pair, bool &first)
 {
-    const uint32_t s = r >> 2, start = rowPtr[s << 2];
-    const uint32_t q = DS[pos] - DS[start];                  // index of the entry's column in the strip's list
+    const uint32_t s = row >> 2;
+    const uint32_t q = DS[pos] - DS[stripBase];              // index of the entry's column in the strip's list
     if (STRIPS) {
-        group = qgp[s] + (q >> 4);
+        g = group[4u * k + s] + (q >> 4);
         pair = q & 15u;
     } else {
-        group = qgp[r >> 4] + (q >> 2);
-        pair = 4u * (q & 3u) + (s & 3u);
+        g = group[k] + (q >> 2);
+        pair = 4u * (q & 3u) + s;
     }
-    first = pos == start || DS[pos] != DS[pos - 1u];
+    first = pos == stripBase || DS[pos] != DS[pos - 1u];
 }
 
-template <bool STRIPS>
-__global__ __launch_bounds__(kThreads) void quad_scatter(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols,
-                                                         const float *__restrict__ vals, const uint32_t *__restrict__ rowOf,
-                                                         const uint32_t *__restrict__ posS, const uint32_t *__restrict__ DS,
-                                                         const uint32_t *__restrict__ qgp, uint32_t nnz, uint32_t *recs)
-{
-    const uint64_t e = global_id();
-    if (e >= nnz) return;
-    const uint32_t r = rowOf[e];
-    uint32_t g, pair;
-    bool first;
-    quad_place<STRIPS>(r, posS[e], rowPtr, DS, qgp, g, pair, first);
-    uint32_t *rec = recs + size_t(g) * CUTE_QUAD_RECORD_WORDS;
-    const uint32_t slot = 4u * pair + (r & 3u);
-    if (vals[e] != 0.0f) atomicOr(rec + 16u + (slot >> 5), 1u << (slot & 31u));   // an explicit zero is an empty slot
-    if (first) rec[pair] = cols[e];
-}
-
-// Per group: the number of stored values (for the prefix sum that gives each group its first value) and the
-// columns of padding pairs, which repeat the last column of their list (0 for an empty list).
-template <bool STRIPS>
-__global__ __launch_bounds__(kThreads) void quad_groups(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols,
-                                                        const uint32_t *__restrict__ qgp, uint32_t U,
-                                                        const uint32_t *__restrict__ stripPairs, uint32_t numGroups, uint32_t *recs,
-                                                        uint32_t *__restrict__ counts)
-{
-    const uint64_t g = global_id();
-    if (g >= numGroups) return;
-    uint32_t lo = 0, hi = U - 1u;                            // the unit u with qgp[u] <= g < qgp[u+1]
-    while (lo < hi) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (qgp[mid + 1] <= g) lo = mid + 1u;
-        else hi = mid;
-    }
-    const uint32_t u = lo, local = uint32_t(g) - qgp[u];
-    uint32_t *rec = recs + size_t(g) * CUTE_QUAD_RECORD_WORDS;
-    counts[g] = uint32_t(__popc(rec[16]) + __popc(rec[17]));
-    const uint32_t lists = STRIPS ? 1u : 4u;
-    for (uint32_t l = 0; l < lists; ++l) {
-        const uint32_t strip = STRIPS ? u : 4u * u + l;
-        const uint32_t len = stripPairs[strip];
-        // steps of this list inside the group: 16 (strips) or 4 (lockstep)
-        const uint32_t per = STRIPS ? 16u : 4u, first_step = local * per;
-        if (first_step + per <= len) continue;               // no padding in this list here
-        uint32_t last = 0;
-        if (len)
-            for (uint32_t i = 0; i < 4u; ++i) {
-                const uint32_t s = rowPtr[strip * 4u + i], e = rowPtr[strip * 4u + i + 1u];
-                if (e > s) last = max(last, cols[e - 1u]);
-            }
-        for (uint32_t t = 0; t < per; ++t)
-            if (first_step + t >= len) rec[STRIPS ? t : 4u * t + l] = last;
-    }
-}
-
-// counts holds the inclusive prefix sums of the stored values per group: word 18 of a record is the index of
-// the group's first stored value.
-__global__ __launch_bounds__(kThreads) void quad_first_values(const uint32_t *__restrict__ counts, uint32_t numGroups, uint32_t *recs)
-{
-    const uint64_t g = global_id();
-    if (g >= numGroups) return;
-    recs[size_t(g) * CUTE_QUAD_RECORD_WORDS + 18u] = g ? counts[g - 1u] : 0u;
-}
-
-template <bool STRIPS>
-__global__ __launch_bounds__(kThreads) void quad_values(const uint32_t *__restrict__ rowPtr, const float *__restrict__ vals,
-                                                        const uint32_t *__restrict__ rowOf, const uint32_t *__restrict__ posS,
-                                                        const uint32_t *__restrict__ DS, const uint32_t *__restrict__ qgp,
-                                                        uint32_t nnz, const uint32_t *__restrict__ recs, float *__restrict__ packed)
-{
-    const uint64_t e = global_id();
-    if (e >= nnz) return;
-    const float v = vals[e];
-    if (v == 0.0f) return;
-    const uint32_t r = rowOf[e];
-    uint32_t g, pair;
-    bool first;
-    quad_place<STRIPS>(r, posS[e], rowPtr, DS, qgp, g, pair, first);
-    const uint32_t *rec = recs + size_t(g) * CUTE_QUAD_RECORD_WORDS;
-    const uint32_t slot = 4u * pair + (r & 3u);
-    const uint64_t mask = (uint64_t(rec[17]) << 32) | rec[16];
-    const uint32_t rank = uint32_t(__popcll(mask & ((1ull << slot) - 1ull)));
-    packed[rec[18] + rank] = v;
-}
-
-// One 128-byte head per work item of a quad plan: its descriptor and a copy of its first group's record.
-__global__ __launch_bounds__(kThreads) void quad_heads(const uint4 *__restrict__ chunks, uint32_t numChunks,
-                                                       const uint32_t *__restrict__ recs, uint32_t head_words, uint32_t *__restrict__ heads)
+// VALUES false: columns and slot masks of the records (cleared before); true: the stored values, once the records are whole.
+template <bool STRIPS, bool VALUES>
+__global__ __launch_bounds__(kThreads) void large_quads(LargePanels L, const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols,
+                                                        const float *__restrict__ vals, const uint32_t *__restrict__ posS,
+                                                        const uint32_t *__restrict__ DS, const uint32_t *__restrict__ group,
+                                                        uint32_t *recs, float *__restrict__ packed)
 {
     const uint64_t id = global_id();
-    const uint64_t i = id / head_words;
-    const uint32_t w = uint32_t(id % head_words);
-    if (i >= numChunks) return;
-    const uint4 ck = chunks[i];
-    uint32_t v = 0;
-    if (w == 0) v = ck.x;
-    else if (w == 1) v = ck.y;
-    else if (w == 2) v = ck.z;
-    else if (w == 3) v = ck.w;
-    else if (w < 4u + CUTE_QUAD_RECORD_WORDS && ck.x < ck.y) v = recs[size_t(ck.x) * CUTE_QUAD_RECORD_WORDS + (w - 4u)];
-    heads[id] = v;
+    if (id >= L.total) return;
+    const uint32_t k = upper_index(L.prefix, L.count, uint32_t(id)), base = L.prefix[k];
+    const uint32_t *rp = rowPtr + uint64_t(L.panel[k]) * 16u;
+    const uint32_t e = rp[0] + (uint32_t(id) - base), row = row_in_panel(rp, e);
+    const float v = vals[e];
+    if (VALUES && v == 0.0f) return;
+    uint32_t g, pair;
+    bool first;
+    large_place<STRIPS>(k, row, base + (rp[row & ~3u] - rp[0]), posS[id], DS, group, g, pair, first);
+    uint32_t *rec = recs + uint64_t(g) * CUTE_QUAD_RECORD_WORDS;
+    const uint32_t slot = 4u * pair + (row & 3u);
+    if (VALUES) {
+        const uint64_t mask = (uint64_t(rec[17]) << 32) | rec[16];
+        packed[rec[18] + uint32_t(__popcll(mask & ((1ull << slot) - 1ull)))] = v;
+    } else {
+        if (v != 0.0f) atomicOr(rec + 16u + (slot >> 5), 1u << (slot & 31u));   // an explicit zero is an empty slot
+        if (first) rec[pair] = cols[e];
+    }
 }
 
-// The row kernel's list of a mixed plan: every listed row with its row pointers, {row, first entry, end, 0}.
-__global__ __launch_bounds__(kThreads) void pack_row_list(const uint32_t *__restrict__ rows, uint32_t numRows,
-                                                          const uint32_t *__restrict__ rowPtr, uint4 *__restrict__ out)
+// Per group of a large panel: the number of stored values (counts, for the prefix sum that gives each group its first value)
+// and the columns of padding pairs, which repeat the last column of their list (0 for an empty list).
+template <bool STRIPS>
+__global__ __launch_bounds__(kThreads) void large_groups(LargePanels L, const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols,
+                                                         const uint32_t *__restrict__ group, const uint32_t *__restrict__ groupPrefix,
+                                                         const uint32_t *__restrict__ stripPairs, uint32_t *recs, uint32_t *__restrict__ counts)
 {
-    const uint64_t i = global_id();
-    if (i >= numRows) return;
-    const uint32_t r = rows[i];
-    out[i] = make_uint4(r, rowPtr[r], rowPtr[r + 1u], 0u);
+    const uint64_t id = global_id();
+    if (id >= groupPrefix[L.count]) return;
+    const uint32_t k = upper_index(groupPrefix, L.count, uint32_t(id)), local = uint32_t(id) - groupPrefix[k];
+    const uint32_t g = (STRIPS ? group[4u * k] : group[k]) + local;
+    uint32_t *rec = recs + uint64_t(g) * CUTE_QUAD_RECORD_WORDS;
+    counts[id] = uint32_t(__popc(rec[16]) + __popc(rec[17]));
+    for (uint32_t s = 0; s < 4u; ++s) {
+        const uint32_t len = stripPairs[4u * k + s];
+        uint32_t first_step, per;                            // steps of this list inside the group: 16 (strips) or 4 (lockstep)
+        if (STRIPS) {
+            const uint32_t g0 = group[4u * k + s];
+            if (g < g0 || g >= g0 + (len + 15u) / 16u) continue;
+            first_step = 16u * (g - g0); per = 16u;
+        } else { first_step = 4u * local; per = 4u; }
+        if (first_step + per <= len) continue;               // no padding in this list here
+        uint32_t last = 0;
+        const uint32_t *rp = rowPtr + uint64_t(L.panel[k]) * 16u + 4u * s;
+        if (len)
+            for (uint32_t i = 0; i < 4u; ++i)
+                if (rp[i + 1u] > rp[i]) last = max(last, cols[rp[i + 1u] - 1u]);
+        for (uint32_t x = 0; x < per; ++x)
+            if (first_step + x >= len) rec[STRIPS ? x : 4u * x + s] = last;
+    }
+}
+
+// counts holds the inclusive prefix sums of the stored values per group: word 18 of a record is the index of the group's first.
+__global__ __launch_bounds__(kThreads) void large_first_values(const uint32_t *__restrict__ unit, const uint32_t *__restrict__ groupPrefix, const uint32_t *__restrict__ valBase,
+                                                               uint32_t count, const uint32_t *__restrict__ counts, uint32_t *recs)
+{
+    const uint64_t id = global_id();
+    if (id >= groupPrefix[count]) return;
+    const uint32_t k = upper_index(groupPrefix, count, uint32_t(id)), b = groupPrefix[k];
+    const uint32_t before = (id ? counts[id - 1u] : 0u) - (b ? counts[b - 1u] : 0u);
+    recs[(uint64_t(unit[k]) + (uint32_t(id) - b)) * CUTE_QUAD_RECORD_WORDS + 18u] = valBase[k] + before;
+}
+
+// The tables of a plan, from its staged host copy, in one launch: chunk descriptors -- or, for the quad kernels (recs given),
+// one 128-byte head per work item: its descriptor and a copy of its first group's record --, the list of cut panels, and the
+// row kernel's list of a mixed plan, expanded from panels: every row with its row pointers, {row, first entry, end, 0}.
+struct PlanTables {
+    const uint4 *chunks;       // staged
+    const uint4 *fixups;
+    const uint32_t *rowPanels;
+    uint32_t numChunks, numFixups, numRowPanels;
+    uint4 *dChunks;            // device
+    uint32_t *dHeads;
+    uint4 *dFixups, *dRowList;
+};
+
+__global__ __launch_bounds__(kThreads) void plan_tables(PlanTables T, const uint32_t *__restrict__ recs, uint32_t head_words,
+                                                        const uint32_t *__restrict__ rowPtr)
+{
+    uint64_t id = global_id();
+    const uint64_t chunk_items = uint64_t(T.numChunks) * (recs ? head_words : 1u);
+    if (id < chunk_items) {
+        if (!recs) { T.dChunks[id] = T.chunks[id]; return; }
+        const uint32_t w = uint32_t(id % head_words);
+        const uint4 ck = T.chunks[id / head_words];
+        uint32_t v = 0;
+        if (w == 0) v = ck.x;
+        else if (w == 1) v = ck.y;
+        else if (w == 2) v = ck.z;
+        else if (w == 3) v = ck.w;
+        else if (w < 4u + CUTE_QUAD_RECORD_WORDS && ck.x < ck.y) v = recs[uint64_t(ck.x) * CUTE_QUAD_RECORD_WORDS + (w - 4u)];
+        T.dHeads[id] = v;
+        return;
+    }
+    id -= chunk_items;
+    if (id < T.numFixups) { T.dFixups[id] = T.fixups[id]; return; }
+    id -= T.numFixups;
+    if (id < uint64_t(T.numRowPanels) * 16u) {
+        const uint32_t r = T.rowPanels[id >> 4] * 16u + uint32_t(id & 15u);
+        T.dRowList[id] = make_uint4(r, rowPtr[r], rowPtr[r + 1u], 0u);
+    }
 }
 
 // Hub plans (hrpb_quad_hub_f32): how often every column occurs in the quad records, and a copy of the records in

@@ -3,8 +3,11 @@
 
 #include <cmath>
 #include <cstdio>
+#include <functional>
 #include <mutex>
+#include <queue>
 #include <string>
+#include <unordered_map>
 
 #include "common.hpp"
 #include "kernels.hip.hpp"
@@ -171,6 +174,8 @@ struct cute_hrpb_dev {
     // the CSR arrays the first time a plan asks for it.  `lock` guards those late builds.
     std::mutex lock;
     bool haveBricks = false, haveQuads = false;
+    // one allocation each: the CSR arrays, the brick tiles, the quad lists
+    void *csrMemory = nullptr, *brickMemory = nullptr, *quadMemory = nullptr;
     uint32_t *dHdr = nullptr;           // brick tiles: one 128-byte header line per block
     float *dVals = nullptr;             // brick tiles: values in lane order, then 64 zeros
     uint32_t *dRowPtr = nullptr, *dCols = nullptr;
@@ -188,7 +193,10 @@ struct cute_hrpb_dev {
     std::vector<uint32_t> panelCols;    // active columns per row panel
     std::vector<uint32_t> panelMaxRow;  // longest row of each panel
     std::vector<uint32_t> panelSpan;    // width of each panel's column window (last column - first column + 1)
+    std::vector<uint32_t> panelStored;  // entries of each panel that are not zero (what the quad lists store)
 };
+
+namespace { void give_device_memory(void *p); }
 
 struct cute_spmm_plan {
     const cute_hrpb_dev *d = nullptr;
@@ -199,7 +207,8 @@ struct cute_spmm_plan {
     bool bf16x3 = false;                // brick kernel on the bf16 matrix pipeline (three products of bf16 hi/lo parts)
     int rows_vec = 4, rows_logl = 6;    // row kernel shape
     uint32_t rows_slabs = 1;
-    uint4 *dChunks = nullptr;
+    void *memory = nullptr;             // one allocation for the tables and the partial tiles below
+    uint4 *dChunks = nullptr;           // brick kernels
     uint32_t *dHeads = nullptr;         // quad kernels: per chunk, the descriptor and the record of its first group
     // hub plans: the most referenced B rows are staged in LDS by persistent work-groups (hrpb_quad_hub_f32)
     uint32_t numHub = 0;
@@ -246,11 +255,17 @@ bool deal_chunks(std::vector<uint4> &chunks, uint32_t num_slabs, uint32_t cus_pe
         const uint32_t s = y * per_xcd + pos / wpg;
         return (s % cus_per_xcd) * 4u + (pos % wpg + s / cus_per_xcd) % 4u;
     };
+    std::vector<uint32_t> lane(span * num_slabs);            // the SIMDs a position meets, slab by slab
+    for (uint32_t pos = 0; pos < span; ++pos)
+        for (uint32_t y = 0; y < num_slabs; ++y) lane[size_t(pos) * num_slabs + y] = simd_of(pos, y);
     std::vector<uint4> dealt(chunks);
     uint64_t before = 0, after = 0;
     std::vector<uint64_t> load(simds);
     std::vector<uint32_t> order;
-    std::vector<uint8_t> taken;
+    // Positions by the load of their fullest SIMD, then by position.  Loads only grow, so an entry's stored load is a lower
+    // bound: one that has grown goes back with its new load, and the first that has not is the position to take.
+    typedef std::pair<uint64_t, uint32_t> Place;
+    std::priority_queue<Place, std::vector<Place>, std::greater<Place>> places;
     for (uint32_t x = 0; x < cute_dev::kNumXcd; ++x) {
         const size_t b = std::min(chunks.size(), x * span), e = std::min(chunks.size(), (x + 1) * span);
         if (e <= b) continue;
@@ -258,26 +273,26 @@ bool deal_chunks(std::vector<uint4> &chunks, uint32_t num_slabs, uint32_t cus_pe
         auto cost = [&](uint32_t i) { return uint64_t(chunks[b + i].y - chunks[b + i].x) + 2u; };
         std::fill(load.begin(), load.end(), 0);
         for (uint32_t i = 0; i < n; ++i)
-            for (uint32_t y = 0; y < num_slabs; ++y) load[simd_of(i, y)] += cost(i);
+            for (uint32_t y = 0; y < num_slabs; ++y) load[lane[size_t(i) * num_slabs + y]] += cost(i);
         before = std::max(before, *std::max_element(load.begin(), load.end()));
         order.resize(n);
         for (uint32_t i = 0; i < n; ++i) order[i] = i;
         std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t c2) { return cost(a) > cost(c2); });
         std::fill(load.begin(), load.end(), 0);
-        taken.assign(n, 0);
+        for (uint32_t pos = 0; pos < n; ++pos) places.emplace(uint64_t(0), pos);
         for (uint32_t i : order) {
-            uint32_t best = n;
-            uint64_t best_peak = ~uint64_t(0);
-            for (uint32_t pos = 0; pos < n; ++pos) {
-                if (taken[pos]) continue;
+            uint32_t pos;
+            for (;;) {
+                const Place top = places.top();
+                places.pop();
+                pos = top.second;
                 uint64_t peak = 0;
-                for (uint32_t y = 0; y < num_slabs; ++y) peak = std::max(peak, load[simd_of(pos, y)]);
-                if (peak < best_peak) { best_peak = peak; best = pos; }
-                if (peak == 0) break;                                      // nothing beats an idle SIMD
+                for (uint32_t y = 0; y < num_slabs; ++y) peak = std::max(peak, load[lane[size_t(pos) * num_slabs + y]]);
+                if (peak == top.first) break;
+                places.emplace(peak, pos);
             }
-            taken[best] = 1;
-            dealt[b + best] = chunks[b + i];
-            for (uint32_t y = 0; y < num_slabs; ++y) load[simd_of(best, y)] += cost(i);
+            dealt[b + pos] = chunks[b + i];
+            for (uint32_t y = 0; y < num_slabs; ++y) load[lane[size_t(pos) * num_slabs + y]] += cost(i);
         }
         after = std::max(after, *std::max_element(load.begin(), load.end()));
     }
@@ -316,13 +331,9 @@ int cute_device_layout(int *num_xcds, int *cus_per_xcd, uint64_t *cache_bytes, i
 void cute_hrpb_dev_free(cute_hrpb_dev *d)
 {
     if (!d) return;
-    (void)hipFree(d->dHdr);
-    (void)hipFree(d->dVals);
-    (void)hipFree(d->dRowPtr);
-    (void)hipFree(d->dCols);
-    (void)hipFree(d->dCsrVals);
-    (void)hipFree(d->dQRecs);
-    (void)hipFree(d->dQVals);
+    give_device_memory(d->csrMemory);
+    give_device_memory(d->brickMemory);
+    give_device_memory(d->quadMemory);
     delete d;
 }
 
@@ -336,184 +347,378 @@ namespace {
 
 // ---- building the layouts on the device (kernels: build_kernels.hip.hpp) ----
 
+// Device memory of handles, plans and their set-up.  hipMalloc and hipFree of a megabyte or more cost 25 to 50 us each (a new
+// graph's product, 65 536 nodes: 300 us of 900 went there), so released blocks wait here for the next caller.  Bounded: at
+// most kIdleBytes in kIdleBlocks blocks, none that the last kIdleUses releases have not touched; the rest goes back to the
+// driver, and all of it does when an allocation fails.  Like hipFree, a release waits for the device first, so no kernel of
+// any stream still uses a block that another thread is given; a block stays with its device.
+constexpr uint64_t kIdleBytes = 512ull << 20, kPooledBlock = 1ull << 20, kIdleUses = 64;
+constexpr size_t kIdleBlocks = 32;
+
+class DevicePool {
+    struct Block { void *p; uint64_t bytes; int device; uint64_t used; };
+    std::mutex lock_;
+    std::vector<Block> idle_;
+    std::unordered_map<void *, std::pair<uint64_t, int>> out_;
+    uint64_t idleBytes_ = 0, clock_ = 0;
+
+    void drop(size_t i)
+    {
+        idleBytes_ -= idle_[i].bytes;
+        (void)hipFree(idle_[i].p);
+        idle_.erase(idle_.begin() + std::ptrdiff_t(i));
+    }
+
+public:
+    int take(void **out, uint64_t bytes)
+    {
+        *out = nullptr;
+        if (bytes < kPooledBlock) { HIP_TRY(hipMalloc(out, std::max<uint64_t>(bytes, 16))); return CUTE_OK; }
+        // eight sizes to an octave: matrices of nearly the same size meet in one
+        const uint64_t step = 1ull << (60 - __builtin_clzll(bytes));
+        bytes = (bytes + step - 1) / step * step;
+        int device = 0;
+        HIP_TRY(hipGetDevice(&device));
+        std::lock_guard<std::mutex> g(lock_);
+        for (size_t i = idle_.size(); i-- > 0;)
+            if (idle_[i].bytes == bytes && idle_[i].device == device) {
+                *out = idle_[i].p;
+                idleBytes_ -= bytes;
+                idle_.erase(idle_.begin() + std::ptrdiff_t(i));
+                break;
+            }
+        if (!*out) {
+            hipError_t e = hipMalloc(out, bytes);
+            if (e != hipSuccess && !idle_.empty()) {
+                (void)hipGetLastError();
+                while (!idle_.empty()) drop(idle_.size() - 1);
+                e = hipMalloc(out, bytes);
+            }
+            if (e != hipSuccess) { *out = nullptr; return hip_fail(e, "device memory", __LINE__); }
+        }
+        out_[*out] = {bytes, device};
+        return CUTE_OK;
+    }
+    void give(void *p)
+    {
+        if (!p) return;
+        int device = -1;
+        const bool known = hipGetDevice(&device) == hipSuccess;
+        uint64_t bytes = 0;
+        {
+            std::lock_guard<std::mutex> g(lock_);
+            const auto it = out_.find(p);
+            if (it != out_.end()) {
+                if (known && it->second.second == device) bytes = it->second.first;
+                out_.erase(it);
+            }
+        }
+        if (!bytes || bytes > kIdleBytes / 4u || hipDeviceSynchronize() != hipSuccess) { (void)hipFree(p); return; }
+        std::lock_guard<std::mutex> g(lock_);
+        ++clock_;
+        idle_.push_back({p, bytes, device, clock_});
+        idleBytes_ += bytes;
+        while (idle_.size() > kIdleBlocks || idleBytes_ > kIdleBytes || idle_.front().used + kIdleUses < clock_) drop(0);
+    }
+};
+
+DevicePool &pool()
+{
+    static DevicePool *p = new DevicePool;   // never destroyed: the driver may be gone when a process ends
+    return *p;
+}
+
+void give_device_memory(void *p) { pool().give(p); }
+
 struct DevBuf {                       // device memory that lives as long as a scope
     void *p = nullptr;
     DevBuf() = default;
     DevBuf(const DevBuf &) = delete;
     DevBuf &operator=(const DevBuf &) = delete;
-    ~DevBuf() { if (p) (void)hipFree(p); }
-    int alloc(uint64_t bytes)
-    {
-        HIP_TRY(hipMalloc(&p, std::max<uint64_t>(bytes, 16)));
-        return CUTE_OK;
-    }
+    ~DevBuf() { pool().give(p); }
+    int alloc(uint64_t bytes) { return pool().take(&p, bytes); }
+    void *release() { void *q = p; p = nullptr; return q; }
     template <class T> T *as() const { return static_cast<T *>(p); }
 };
 
-inline dim3 grid_of(uint64_t n) { return dim3(uint32_t((n + cute_build::kThreads - 1) / cute_build::kThreads)); }
+// Several arrays in one allocation: sizes first, then the pointers.
+struct Layout {
+    uint64_t bytes = 0;
+    uint64_t add(uint64_t count, uint64_t size)
+    {
+        const uint64_t at = bytes;
+        bytes += (count * size + 255u) & ~uint64_t(255);
+        return at;
+    }
+    template <class T> static T *at(void *base, uint64_t offset) { return reinterpret_cast<T *>(static_cast<char *>(base) + offset); }
+};
+
+// Pinned host memory through which set-up exchanges its tables with the device: kernels read and write it directly.  A copy
+// call moves up to 16 KB in about 13 us but 64 KB and more in 130 us (the copy engine's start); a kernel reads 64 KB of
+// pinned memory in 3 us and 12 MB in 250.  Allocating and freeing a buffer costs 40 us, so released buffers wait here for the
+// next caller: at most kPinnedBuffers of them and kPinnedBytes in all, anything beyond is freed at once.  A buffer belongs to
+// one caller at a time and comes back only when no kernel uses it any more.
+constexpr size_t kPinnedBuffers = 4;
+constexpr uint64_t kPinnedBytes = 32ull << 20;
+std::mutex g_pinned_lock;
+std::vector<std::pair<void *, uint64_t>> g_pinned;
+
+struct PinnedBuf {
+    void *p = nullptr;
+    uint64_t cap = 0;
+    bool pending = false;             // a kernel that uses it may still run
+    PinnedBuf() = default;
+    PinnedBuf(const PinnedBuf &) = delete;
+    PinnedBuf &operator=(const PinnedBuf &) = delete;
+    ~PinnedBuf()
+    {
+        if (!p) return;
+        if (pending) (void)hipStreamSynchronize(nullptr);
+        {
+            std::lock_guard<std::mutex> g(g_pinned_lock);
+            uint64_t held = cap;
+            for (const auto &b : g_pinned) held += b.second;
+            if (g_pinned.size() < kPinnedBuffers && held <= kPinnedBytes) {
+                g_pinned.emplace_back(p, cap);
+                return;
+            }
+        }
+        (void)hipHostFree(p);
+    }
+    int alloc(uint64_t bytes)
+    {
+        bytes = std::max<uint64_t>(bytes, 64u << 10);
+        {
+            std::lock_guard<std::mutex> g(g_pinned_lock);
+            size_t best = g_pinned.size();
+            for (size_t i = 0; i < g_pinned.size(); ++i)
+                if (g_pinned[i].second >= bytes && (best == g_pinned.size() || g_pinned[i].second < g_pinned[best].second)) best = i;
+            if (best < g_pinned.size()) {
+                p = g_pinned[best].first;
+                cap = g_pinned[best].second;
+                g_pinned.erase(g_pinned.begin() + std::ptrdiff_t(best));
+                return CUTE_OK;
+            }
+        }
+        bytes = (bytes + 0xffffu) & ~uint64_t(0xffff);
+        HIP_TRY(hipHostMalloc(&p, bytes, hipHostMallocPortable | hipHostMallocMapped));
+        cap = bytes;
+        return CUTE_OK;
+    }
+    int wait()
+    {
+        HIP_TRY(hipStreamSynchronize(nullptr));
+        pending = false;
+        return CUTE_OK;
+    }
+    template <class T> T *as(uint64_t offset = 0) const { return Layout::at<T>(p, offset); }
+};
+
+inline dim3 grid_of(uint64_t n) { return dim3(uint32_t(std::max<uint64_t>((n + cute_build::kThreads - 1) / cute_build::kThreads, 1))); }
+// for kernels that walk their range with a stride
+inline dim3 grid_capped(uint64_t n) { return dim3(std::min<uint32_t>(grid_of(n).x, 4096u)); }
 
 int check_launch(const char *what);
 
-// Inclusive prefix sum of n uint32 values, in place, on the default stream.
-int device_scan(uint32_t *data, uint64_t n)
+#define CUTE_BUILD(kernel, grid, ...) CUTE_BUILD_LDS(kernel, grid, 0, __VA_ARGS__)
+#define CUTE_BUILD_LDS(kernel, grid, lds, ...) \
+    hipLaunchKernelGGL(kernel, grid, dim3(cute_build::kThreads), lds, nullptr, __VA_ARGS__)
+
+// The widest column window the panel kernels take on this matrix, and the LDS its bitmap and running counts need.
+inline uint32_t max_span(const cute_hrpb_dev *d) { return std::min(d->K, cute_build::kPanelSpan); }
+inline uint32_t window_lds(const cute_hrpb_dev *d, uint32_t at_least) { return std::max((cute_build::panel_window_words(max_span(d)) + 1u) * 6u, at_least); }
+inline bool panel_is_large(const cute_hrpb_dev *d, uint32_t p) { return d->panelNnz[p] > cute_build::kPanelCap || d->panelSpan[p] > max_span(d); }
+
+// Words of scratch device_scan needs for an array of n values: the block sums of every level.
+inline uint64_t scan_scratch_words(uint64_t n)
 {
-    if (!n) return CUTE_OK;
-    const uint64_t nb = (n + cute_build::kScanBlock - 1) / cute_build::kScanBlock;
-    if (nb > 0x7fffffffull) return CUTE_ERR_SHAPE;
-    if (nb == 1) {
-        hipLaunchKernelGGL(cute_build::scan_block_apply, dim3(1), dim3(cute_build::kThreads), 0, nullptr, data, data, n,
-                           static_cast<const uint32_t *>(nullptr));
-        return check_launch("prefix sum");
-    }
-    DevBuf sums;
-    int rc = sums.alloc(nb * sizeof(uint32_t));
-    if (rc != CUTE_OK) return rc;
-    hipLaunchKernelGGL(cute_build::scan_block_sums, dim3(uint32_t(nb)), dim3(cute_build::kThreads), 0, nullptr, data, n, sums.as<uint32_t>());
-    rc = device_scan(sums.as<uint32_t>(), nb);
-    if (rc != CUTE_OK) return rc;
-    hipLaunchKernelGGL(cute_build::scan_block_apply, dim3(uint32_t(nb)), dim3(cute_build::kThreads), 0, nullptr, data, data, n,
-                       sums.as<const uint32_t>());
-    rc = check_launch("prefix sum");
-    // (the block sums are freed when this scope ends; hipFree waits for the kernels that read them)
-    return rc;
+    uint64_t words = 0;
+    while (n > cute_build::kScanBlock) { n = (n + cute_build::kScanBlock - 1) / cute_build::kScanBlock; words += n; }
+    return words + 1;
 }
 
-// Where every entry of the device CSR copy stands in the (column, row) order of its panel and of its strip,
-// and the running count of distinct columns along both orders.  Checks that rows are sorted, duplicate-free
-// and inside K.  With the two vectors given, also counts active columns per panel and list pairs per strip.
-struct Census {
-    DevBuf rowOf, posP, posS, DP, DS;
+// Inclusive prefix sums of n uint32 values, in place, on the default stream, for `arrays` arrays that stand `pitch` words apart
+// (their scratch `scratch_pitch`).
+void device_scan(uint32_t *data, uint64_t n, uint32_t *scratch, uint32_t arrays = 1, uint64_t pitch = 0, uint64_t scratch_pitch = 0)
+{
+    if (!n) return;
+    const uint64_t nb = (n + cute_build::kScanBlock - 1) / cute_build::kScanBlock;
+    const dim3 grid(uint32_t(nb), arrays);
+    const uint32_t *sums = nullptr;
+    if (nb > 1) {
+        CUTE_BUILD(cute_build::scan_block_sums, grid, data, n, pitch, scratch, scratch_pitch);
+        device_scan(scratch, nb, scratch + nb, arrays, scratch_pitch, scratch_pitch);
+        sums = scratch;
+    }
+    CUTE_BUILD(cute_build::scan_block_apply, grid, data, n, pitch, sums, scratch_pitch);
+}
+
+// The panels that the panel kernels do not take and what their entry-parallel path keeps between its kernels.
+struct LargeWork {
+    std::vector<uint32_t> panel, prefix;
+    DevBuf memory;
+    cute_build::LargePanels L{};
+    uint32_t *posP = nullptr, *posS = nullptr, *DP = nullptr, *DS = nullptr, *scratch = nullptr;
+    cute_build::PanelCensus *res = nullptr;
 };
 
-int device_census(const cute_hrpb_dev *d, Census &c, std::vector<uint32_t> *panelCols, std::vector<uint32_t> *stripPairs,
-                  std::vector<uint32_t> *panelSpan = nullptr)
+// Lists the large panels (panelNnz and panelSpan are known) and numbers their entries.  With `out` given also counts for the planner, into the
+// panels' census records.
+int number_large_panels(const cute_hrpb_dev *d, LargeWork &w, cute_build::PanelCensus *out)
 {
-    const uint32_t nnz = d->nnz, P = d->P;
-    if (panelCols) panelCols->assign(P, 0u);
-    if (stripPairs) stripPairs->assign(size_t(P) * 4u, 0u);
-    if (panelSpan) panelSpan->assign(P, 0u);
-    if (!nnz) return CUTE_OK;
-    const uint64_t bytes = uint64_t(nnz) * sizeof(uint32_t);
-    int rc = c.rowOf.alloc(bytes);
-    if (rc == CUTE_OK) rc = c.posP.alloc(bytes);
-    if (rc == CUTE_OK) rc = c.posS.alloc(bytes);
-    if (rc == CUTE_OK) rc = c.DP.alloc(bytes);
-    if (rc == CUTE_OK) rc = c.DS.alloc(bytes);
-    DevBuf err;
-    if (rc == CUTE_OK) rc = err.alloc(sizeof(int));
+    w.prefix.assign(1, 0u);
+    for (uint32_t p = 0; p < d->P; ++p)
+        if (panel_is_large(d, p)) {
+            w.panel.push_back(p);
+            w.prefix.push_back(w.prefix.back() + d->panelNnz[p]);
+        }
+    const uint32_t count = uint32_t(w.panel.size()), total = w.prefix.back();
+    if (!count) return CUTE_OK;
+    Layout lay;
+    const uint64_t oPanel = lay.add(count, 4), oPrefix = lay.add(count + 1u, 4), oRes = lay.add(count, sizeof(cute_build::PanelCensus));
+    const uint64_t staged = lay.bytes;
+    const uint64_t oPosP = lay.add(total, 4), oPosS = lay.add(total, 4), oDP = lay.add(total, 4), oDS = lay.add(total, 4),
+                   oScratch = lay.add(2u * scan_scratch_words(total), 4);
+    int rc = w.memory.alloc(lay.bytes);
+    PinnedBuf pin;
+    if (rc == CUTE_OK) rc = pin.alloc(staged);
     if (rc != CUTE_OK) return rc;
-    HIP_TRY(hipMemset(err.p, 0, sizeof(int)));
-    hipLaunchKernelGGL(cute_build::row_of_entries, grid_of(nnz), dim3(cute_build::kThreads), 0, nullptr, d->dRowPtr, d->dCols, d->M,
-                       d->K, nnz, c.rowOf.as<uint32_t>(), err.as<int>());
-    int bad = 0;
-    HIP_TRY(hipMemcpy(&bad, err.p, sizeof(int), hipMemcpyDeviceToHost));
-    if (bad & cute_build::kErrRange) return CUTE_ERR_RANGE;
-    if (bad & cute_build::kErrUnsorted) return CUTE_ERR_UNSORTED;
-    hipLaunchKernelGGL(cute_build::entry_positions, grid_of(nnz), dim3(cute_build::kThreads), 0, nullptr, d->dRowPtr, d->dCols,
-                       c.rowOf.as<const uint32_t>(), nnz, c.posP.as<uint32_t>(), c.posS.as<uint32_t>(), c.DP.as<uint32_t>(),
-                       c.DS.as<uint32_t>());
-    rc = check_launch("entry positions");
-    if (rc == CUTE_OK) rc = device_scan(c.DP.as<uint32_t>(), nnz);
-    if (rc == CUTE_OK) rc = device_scan(c.DS.as<uint32_t>(), nnz);
-    if (rc != CUTE_OK || !panelCols || !stripPairs) return rc;
-    DevBuf pc, sp, span;
-    rc = pc.alloc(uint64_t(P) * 4u);
-    if (rc == CUTE_OK) rc = sp.alloc(uint64_t(P) * 16u);
-    if (rc == CUTE_OK) rc = span.alloc(uint64_t(P) * 4u);
-    if (rc != CUTE_OK) return rc;
-    hipLaunchKernelGGL(cute_build::count_columns, grid_of(uint64_t(P) * 4u), dim3(cute_build::kThreads), 0, nullptr, d->dRowPtr, d->dCols,
-                       c.DP.as<const uint32_t>(), c.DS.as<const uint32_t>(), P, pc.as<uint32_t>(), sp.as<uint32_t>(), span.as<uint32_t>());
-    HIP_TRY(hipMemcpy(panelCols->data(), pc.p, uint64_t(P) * 4u, hipMemcpyDeviceToHost));
-    HIP_TRY(hipMemcpy(stripPairs->data(), sp.p, uint64_t(P) * 16u, hipMemcpyDeviceToHost));
-    if (panelSpan) HIP_TRY(hipMemcpy(panelSpan->data(), span.p, uint64_t(P) * 4u, hipMemcpyDeviceToHost));
-    return CUTE_OK;
+    std::memset(pin.p, 0, staged);
+    std::memcpy(pin.as<char>(oPanel), w.panel.data(), count * 4u);
+    std::memcpy(pin.as<char>(oPrefix), w.prefix.data(), (count + 1u) * 4u);
+    void *m = w.memory.p;
+    w.L = {Layout::at<uint32_t>(m, oPanel), Layout::at<uint32_t>(m, oPrefix), count, total};
+    w.posP = Layout::at<uint32_t>(m, oPosP); w.posS = Layout::at<uint32_t>(m, oPosS);
+    w.DP = Layout::at<uint32_t>(m, oDP); w.DS = Layout::at<uint32_t>(m, oDS);
+    w.scratch = Layout::at<uint32_t>(m, oScratch);
+    w.res = Layout::at<cute_build::PanelCensus>(m, oRes);
+    pin.pending = true;
+    CUTE_BUILD(cute_build::copy_words, grid_capped(staged / 4u), pin.as<const uint32_t>(), w.memory.as<uint32_t>(), staged / 4u);
+    CUTE_BUILD(cute_build::large_positions, grid_of(total), w.L, d->dRowPtr, d->dCols, d->dCsrVals, d->K, w.posP, w.posS, w.DP, w.DS,
+               out ? w.res : static_cast<cute_build::PanelCensus *>(nullptr));
+    device_scan(w.DP, total, w.scratch, 2, (oDS - oDP) / 4u, scan_scratch_words(total));
+    if (out) CUTE_BUILD(cute_build::large_counts, grid_of(count), w.L, d->dRowPtr, w.DP, w.DS, w.res, out);
+    rc = check_launch("large panels");
+    return rc == CUTE_OK ? pin.wait() : rc;
 }
 
 // Brick tiles from the device CSR copy: the arrays cute_hrpb_retile makes on the host, word for word.
-int build_bricks_on_device(cute_hrpb_dev *d, const Census &c)
+int build_bricks_on_device(cute_hrpb_dev *d, const LargeWork &w)
 {
     const uint64_t hdr_words = uint64_t(d->nb) * CUTE_TILED_HDR_WORDS, num_vals = uint64_t(d->nnz) + 64u;
-    uint32_t *hdr = nullptr, *brp = nullptr, *pcols = nullptr;
-    float *vals = nullptr;
-    DevBuf hdr_buf, vals_buf, brp_buf, pc_buf;
-    int rc = hdr_buf.alloc(hdr_words * 4u);
-    if (rc == CUTE_OK) rc = vals_buf.alloc(num_vals * 4u);
-    if (rc == CUTE_OK) rc = brp_buf.alloc((uint64_t(d->P) + 1u) * 4u);
-    if (rc == CUTE_OK) rc = pc_buf.alloc(uint64_t(d->P) * 4u);
+    const uint32_t count = uint32_t(w.panel.size());
+    Layout lay, tab;
+    const uint64_t oBrp = tab.add(uint64_t(d->P) + 1u, 4), oUnit = tab.add(count, 4), oPrefix = tab.add(count + 1u, 4), oCols = tab.add(count, 4);
+    const uint64_t oHdr = lay.add(hdr_words, 4), oVals = lay.add(num_vals, 4), oTab = lay.add(tab.bytes, 1);
+    DevBuf mem;
+    PinnedBuf pin;
+    int rc = mem.alloc(lay.bytes);
+    if (rc == CUTE_OK) rc = pin.alloc(tab.bytes);
     if (rc != CUTE_OK) return rc;
-    hdr = hdr_buf.as<uint32_t>(); vals = vals_buf.as<float>(); brp = brp_buf.as<uint32_t>(); pcols = pc_buf.as<uint32_t>();
-    HIP_TRY(hipMemset(hdr, 0, std::max<uint64_t>(hdr_words * 4u, 4u)));
-    HIP_TRY(hipMemset(vals + d->nnz, 0, 64u * sizeof(float)));          // one wavefront of zeros behind the values
-    HIP_TRY(hipMemcpy(brp, d->brp.data(), (uint64_t(d->P) + 1u) * 4u, hipMemcpyHostToDevice));
-    if (d->P) HIP_TRY(hipMemcpy(pcols, d->panelCols.data(), uint64_t(d->P) * 4u, hipMemcpyHostToDevice));
-    if (d->nnz) {
-        hipLaunchKernelGGL(cute_build::brick_scatter, grid_of(d->nnz), dim3(cute_build::kThreads), 0, nullptr, d->dRowPtr, d->dCols,
-                           d->dCsrVals, c.rowOf.as<const uint32_t>(), c.posP.as<const uint32_t>(), c.DP.as<const uint32_t>(), brp,
-                           d->nnz, hdr, vals);
-        hipLaunchKernelGGL(cute_build::brick_finish, grid_of(d->nb), dim3(cute_build::kThreads), 0, nullptr, d->dRowPtr, brp, pcols,
-                           d->P, d->nb, hdr);
-        rc = check_launch("brick tiles");
-        if (rc != CUTE_OK) return rc;
+    auto table = [&](uint64_t o) { return Layout::at<const uint32_t>(mem.p, oTab + o); };
+    uint32_t *hdr = Layout::at<uint32_t>(mem.p, oHdr);
+    float *vals = Layout::at<float>(mem.p, oVals);
+    std::memcpy(pin.p, d->brp.data(), d->brp.size() * 4u);
+    uint32_t *unit = pin.as<uint32_t>(oUnit), *prefix = pin.as<uint32_t>(oPrefix), *cols = pin.as<uint32_t>(oCols);
+    prefix[0] = 0;
+    for (uint32_t k = 0; k < count; ++k) {
+        const uint32_t p = w.panel[k];
+        unit[k] = d->brp[p];
+        prefix[k + 1] = prefix[k] + (d->brp[p + 1] - d->brp[p]);
+        cols[k] = d->panelCols[p];
     }
-    HIP_TRY(hipDeviceSynchronize());
-    d->dHdr = hdr; hdr_buf.p = nullptr;
-    d->dVals = vals; vals_buf.p = nullptr;
+    pin.pending = true;
+    CUTE_BUILD(cute_build::copy_words, grid_capped(tab.bytes / 4u), pin.as<const uint32_t>(), Layout::at<uint32_t>(mem.p, oTab), tab.bytes / 4u);
+    CUTE_BUILD_LDS(cute_build::panel_bricks, dim3(d->P), window_lds(d, (cute_build::kPanelCap + 1u) * 2u), d->dRowPtr, d->dCols, d->dCsrVals, d->P,
+                   d->nnz, max_span(d), table(oBrp), hdr, vals);
+    if (count) {
+        const uint32_t blocks = prefix[count];
+        CUTE_BUILD(cute_build::large_clear, grid_of(uint64_t(blocks) * CUTE_TILED_HDR_WORDS), table(oUnit), table(oPrefix), count, uint32_t(CUTE_TILED_HDR_WORDS), hdr);
+        CUTE_BUILD(cute_build::large_bricks, grid_of(w.L.total), w.L, d->dRowPtr, d->dCols, d->dCsrVals, w.posP, w.DP, table(oUnit), hdr, vals);
+        CUTE_BUILD(cute_build::large_brick_ends, grid_of(blocks), w.L, d->dRowPtr, table(oUnit), table(oPrefix), table(oCols), hdr);
+    }
+    rc = check_launch("brick tiles");
+    if (rc == CUTE_OK) rc = pin.wait();
+    if (rc != CUTE_OK) return rc;
+    d->dHdr = hdr;
+    d->dVals = vals;
+    d->brickMemory = mem.release();
     d->bytes += hdr_words * 4u + num_vals * 4u;
     d->haveBricks = true;
     return CUTE_OK;
 }
 
 // Quad lists (in the layout the census chose) from the device CSR copy: the arrays cute_quad_pack makes.
-int build_quads_on_device(cute_hrpb_dev *d, const Census &c)
+int build_quads_on_device(cute_hrpb_dev *d, const LargeWork &w)
 {
-    const uint64_t G = d->numGroups;
-    const uint32_t U = uint32_t(d->qgp.size() - 1);
+    const uint64_t G = d->numGroups, stored = d->numQuadVals;
     const bool strips = d->quadRows == 4;
-    DevBuf recs_buf, qgp_buf, sp_buf, counts_buf, vals_buf;
-    int rc = recs_buf.alloc(G * CUTE_QUAD_RECORD_WORDS * 4u);
-    if (rc == CUTE_OK) rc = qgp_buf.alloc(d->qgp.size() * 4u);
-    if (rc == CUTE_OK) rc = sp_buf.alloc(d->stripPairs.size() * 4u);
-    if (rc == CUTE_OK) rc = counts_buf.alloc(G * 4u);
+    const uint32_t count = uint32_t(w.panel.size()), per = strips ? 4u : 1u;
+    Layout lay, tab;
+    const uint64_t oGroup = tab.add(d->qgp.size(), 4), oBase = tab.add(uint64_t(d->P) + 1u, 4), oUnit = tab.add(count, 4),
+                   oPrefix = tab.add(count + 1u, 4), oFirst = tab.add(uint64_t(count) * per, 4), oPairs = tab.add(uint64_t(count) * 4u, 4),
+                   oLargeBase = tab.add(count, 4);
+    std::vector<uint32_t> medium;
+    for (uint32_t p = 0; p < d->P; ++p)
+        if (d->panelNnz[p] > cute_build::kPanelSmall && !panel_is_large(d, p)) medium.push_back(p);
+    const uint64_t oMedium = tab.add(medium.size(), 4);
+    const uint64_t oRecs = lay.add(G * CUTE_QUAD_RECORD_WORDS, 4), oVals = lay.add(stored + 64u, 4), oTab = lay.add(tab.bytes, 1);
+    DevBuf mem, counts;
+    PinnedBuf pin;
+    int rc = mem.alloc(lay.bytes);
+    if (rc == CUTE_OK) rc = pin.alloc(tab.bytes);
     if (rc != CUTE_OK) return rc;
-    uint32_t *recs = recs_buf.as<uint32_t>(), *qgp = qgp_buf.as<uint32_t>(), *sp = sp_buf.as<uint32_t>(), *counts = counts_buf.as<uint32_t>();
-    HIP_TRY(hipMemset(recs, 0, std::max<uint64_t>(G * CUTE_QUAD_RECORD_WORDS * 4u, 4u)));
-    HIP_TRY(hipMemcpy(qgp, d->qgp.data(), d->qgp.size() * 4u, hipMemcpyHostToDevice));
-    if (!d->stripPairs.empty()) HIP_TRY(hipMemcpy(sp, d->stripPairs.data(), d->stripPairs.size() * 4u, hipMemcpyHostToDevice));
-    uint32_t stored = 0;
-    if (G) {
-#define CUTE_BUILD_QUADS(S)                                                                                                          \
-    hipLaunchKernelGGL(cute_build::quad_scatter<S>, grid_of(d->nnz), dim3(cute_build::kThreads), 0, nullptr, d->dRowPtr, d->dCols,     \
-                       d->dCsrVals, c.rowOf.as<const uint32_t>(), c.posS.as<const uint32_t>(), c.DS.as<const uint32_t>(), qgp, d->nnz, \
-                       recs);                                                                                                        \
-    hipLaunchKernelGGL(cute_build::quad_groups<S>, grid_of(G), dim3(cute_build::kThreads), 0, nullptr, d->dRowPtr, d->dCols, qgp, U, sp, \
-                       uint32_t(G), recs, counts)
-        if (strips) { CUTE_BUILD_QUADS(true); } else { CUTE_BUILD_QUADS(false); }
+    auto table = [&](uint64_t o) { return Layout::at<const uint32_t>(mem.p, oTab + o); };
+    uint32_t *recs = Layout::at<uint32_t>(mem.p, oRecs);
+    float *packed = Layout::at<float>(mem.p, oVals);
+    std::memcpy(pin.as<char>(oGroup), d->qgp.data(), d->qgp.size() * 4u);
+    if (!medium.empty()) std::memcpy(pin.as<char>(oMedium), medium.data(), medium.size() * 4u);
+    uint32_t *base = pin.as<uint32_t>(oBase), *unit = pin.as<uint32_t>(oUnit), *prefix = pin.as<uint32_t>(oPrefix), *first = pin.as<uint32_t>(oFirst),
+             *pairs = pin.as<uint32_t>(oPairs), *large_base = pin.as<uint32_t>(oLargeBase);
+    base[0] = 0;
+    for (uint32_t p = 0; p < d->P; ++p) base[p + 1] = base[p] + d->panelStored[p];
+    prefix[0] = 0;
+    for (uint32_t k = 0; k < count; ++k) {
+        const uint32_t p = w.panel[k];
+        unit[k] = d->qgp[p * per];
+        prefix[k + 1] = prefix[k] + (d->qgp[(p + 1) * per] - d->qgp[p * per]);
+        for (uint32_t s = 0; s < per; ++s) first[k * per + s] = d->qgp[p * per + s];
+        for (uint32_t s = 0; s < 4u; ++s) pairs[k * 4u + s] = d->stripPairs[p * 4u + s];
+        large_base[k] = base[p];
+    }
+    const uint32_t groups = prefix[count];
+    if (groups) rc = counts.alloc((uint64_t(groups) + scan_scratch_words(groups)) * 4u);
+    if (rc != CUTE_OK) return rc;
+    pin.pending = true;
+    CUTE_BUILD(cute_build::copy_words, grid_capped(tab.bytes / 4u), pin.as<const uint32_t>(), Layout::at<uint32_t>(mem.p, oTab), tab.bytes / 4u);
+    uint32_t *sums = counts.as<uint32_t>();
+#define CUTE_PANEL_QUADS(S, CAP, COUNT, LIST)                                                                                         \
+    CUTE_BUILD_LDS((cute_build::panel_quads<S, CAP>), dim3(COUNT), window_lds(d, CAP * 8u), d->dRowPtr, d->dCols, d->dCsrVals, d->P, d->nnz, \
+                   max_span(d), LIST, table(oGroup), table(oBase), uint32_t(stored), recs, packed)
+#define CUTE_BUILD_QUADS(S)                                                                                                           \
+    CUTE_PANEL_QUADS(S, cute_build::kPanelSmall, d->P, static_cast<const uint32_t *>(nullptr));                                         \
+    if (!medium.empty()) CUTE_PANEL_QUADS(S, cute_build::kPanelCap, uint32_t(medium.size()), table(oMedium));                           \
+    if (count) {                                                                                                                      \
+        CUTE_BUILD(cute_build::large_clear, grid_of(uint64_t(groups) * CUTE_QUAD_RECORD_WORDS), table(oUnit), table(oPrefix), count,    \
+                   uint32_t(CUTE_QUAD_RECORD_WORDS), recs);                                                                           \
+        CUTE_BUILD((cute_build::large_quads<S, false>), grid_of(w.L.total), w.L, d->dRowPtr, d->dCols, d->dCsrVals, w.posS, w.DS,       \
+                   table(oFirst), recs, packed);                                                                                      \
+        CUTE_BUILD(cute_build::large_groups<S>, grid_of(groups), w.L, d->dRowPtr, d->dCols, table(oFirst), table(oPrefix), table(oPairs), recs, sums); \
+        device_scan(sums, groups, sums + groups);                                                                                     \
+        CUTE_BUILD(cute_build::large_first_values, grid_of(groups), table(oUnit), table(oPrefix), table(oLargeBase), count, sums, recs); \
+        CUTE_BUILD((cute_build::large_quads<S, true>), grid_of(w.L.total), w.L, d->dRowPtr, d->dCols, d->dCsrVals, w.posS, w.DS,        \
+                   table(oFirst), recs, packed);                                                                                      \
+    }
+    if (strips) { CUTE_BUILD_QUADS(true) } else { CUTE_BUILD_QUADS(false) }
 #undef CUTE_BUILD_QUADS
-        rc = check_launch("quad lists");
-        if (rc == CUTE_OK) rc = device_scan(counts, G);
-        if (rc != CUTE_OK) return rc;
-        hipLaunchKernelGGL(cute_build::quad_first_values, grid_of(G), dim3(cute_build::kThreads), 0, nullptr, counts, uint32_t(G), recs);
-        HIP_TRY(hipMemcpy(&stored, counts + (G - 1u), sizeof(uint32_t), hipMemcpyDeviceToHost));
-    }
-    rc = vals_buf.alloc((uint64_t(stored) + 64u) * 4u);
+#undef CUTE_PANEL_QUADS
+    rc = check_launch("quad lists");
+    if (rc == CUTE_OK) rc = pin.wait();
     if (rc != CUTE_OK) return rc;
-    float *packed = vals_buf.as<float>();
-    HIP_TRY(hipMemset(packed, 0, (uint64_t(stored) + 64u) * 4u));
-    if (G && d->nnz) {
-        if (strips)
-            hipLaunchKernelGGL(cute_build::quad_values<true>, grid_of(d->nnz), dim3(cute_build::kThreads), 0, nullptr, d->dRowPtr, d->dCsrVals,
-                               c.rowOf.as<const uint32_t>(), c.posS.as<const uint32_t>(), c.DS.as<const uint32_t>(), qgp, d->nnz, recs, packed);
-        else
-            hipLaunchKernelGGL(cute_build::quad_values<false>, grid_of(d->nnz), dim3(cute_build::kThreads), 0, nullptr, d->dRowPtr, d->dCsrVals,
-                               c.rowOf.as<const uint32_t>(), c.posS.as<const uint32_t>(), c.DS.as<const uint32_t>(), qgp, d->nnz, recs, packed);
-        rc = check_launch("quad values");
-        if (rc != CUTE_OK) return rc;
-    }
-    HIP_TRY(hipDeviceSynchronize());
-    d->numQuadVals = stored;
-    d->dQRecs = recs; recs_buf.p = nullptr;
-    d->dQVals = packed; vals_buf.p = nullptr;
-    d->bytes += G * CUTE_QUAD_RECORD_WORDS * 4u + (uint64_t(stored) + 64u) * 4u;
+    d->dQRecs = recs;
+    d->dQVals = packed;
+    d->quadMemory = mem.release();
+    d->bytes += G * CUTE_QUAD_RECORD_WORDS * 4u + (stored + 64u) * 4u;
     d->haveQuads = true;
     return CUTE_OK;
 }
@@ -524,16 +729,17 @@ int ensure_layout(cute_hrpb_dev *d, int which)
 {
     std::lock_guard<std::mutex> guard(d->lock);
     if (which == 1 ? d->haveBricks : d->haveQuads) return CUTE_OK;
-    Census c;
-    int rc = device_census(d, c, nullptr, nullptr);
+    LargeWork w;
+    const int rc = number_large_panels(d, w, nullptr);
     if (rc != CUTE_OK) return rc;
-    return which == 1 ? build_bricks_on_device(d, c) : build_quads_on_device(d, c);
+    return which == 1 ? build_bricks_on_device(d, w) : build_quads_on_device(d, w);
 }
 
 // Group counts of the quad lists from the list length of every strip; picks lockstep lists unless they would
 // be mostly padding (a few very long rows stretch the lists of their panel neighbours): then one list per strip.
-int finish_quad_census(cute_hrpb_dev *d, std::vector<uint32_t> &strip_pairs, int quad_layout)
+int finish_quad_census(cute_hrpb_dev *d, int quad_layout)
 {
+    const std::vector<uint32_t> &strip_pairs = d->stripPairs;
     const uint32_t S = d->M / 4;
     uint64_t pairs = 0, lock_groups = 0;
     for (uint32_t p = 0; p < d->P; ++p) {
@@ -555,7 +761,6 @@ int finish_quad_census(cute_hrpb_dev *d, std::vector<uint32_t> &strip_pairs, int
         d->qgp[u + 1] = uint32_t(groups);
     }
     d->numGroups = groups;
-    d->stripPairs.swap(strip_pairs);
     return CUTE_OK;
 }
 
@@ -579,35 +784,104 @@ int default_layout(const cute_hrpb_dev *d, uint64_t cache_bytes)
     return choose_mfma_shape(slots, bricks, blocks, uint64_t(d->K) + d->M, d->nnz, 128u, 0u, cache_bytes);
 }
 
-// The common tail of both uploads.  d holds the device copy of the CSR arrays, rowPtr is a host copy of the row
-// pointers (checked: ascending from 0 to nnz).  Counts active columns per panel and list pairs per strip on the
-// device, derives the planner's per-panel statistics, and builds the one MFMA layout the planner's default
-// rules would use for this matrix (none when every panel would go to the row kernel).
-int finish_upload(cute_hrpb_dev *d, const uint32_t *rowPtr, int quad_layout, const DeviceContext &c)
+int alloc_csr(cute_hrpb_dev *d)
 {
-    Census cen;
-    std::vector<uint32_t> strip_pairs;
-    int rc = device_census(d, cen, &d->panelCols, &strip_pairs, &d->panelSpan);
+    Layout lay;
+    const uint64_t oRow = lay.add(uint64_t(d->M) + 1u, 4), oCols = lay.add(d->nnz, 4), oVals = lay.add(d->nnz, 4);
+    const int rc = pool().take(&d->csrMemory, lay.bytes);
     if (rc != CUTE_OK) return rc;
-    d->brp.assign(size_t(d->P) + 1, 0u);
-    d->panelNnz.resize(d->P);
-    d->panelMaxRow.resize(d->P);
-    uint64_t blocks = 0;
-    for (uint32_t p = 0; p < d->P; ++p) {
-        d->panelNnz[p] = rowPtr[(p + 1) * CUTE_TM] - rowPtr[p * CUTE_TM];
-        uint32_t longest = 0;
-        for (uint32_t r = p * CUTE_TM; r < (p + 1) * CUTE_TM; ++r) longest = std::max(longest, rowPtr[r + 1] - rowPtr[r]);
-        d->panelMaxRow[p] = longest;
-        blocks += (d->panelCols[p] + CUTE_TK - 1) / CUTE_TK;
-        if (blocks > 0xffffffffull / CUTE_TILED_HDR_WORDS) return CUTE_ERR_SHAPE;
-        d->brp[p + 1] = uint32_t(blocks);
+    d->dRowPtr = Layout::at<uint32_t>(d->csrMemory, oRow);
+    d->dCols = Layout::at<uint32_t>(d->csrMemory, oCols);
+    d->dCsrVals = Layout::at<float>(d->csrMemory, oVals);
+    d->bytes = (uint64_t(d->M) + 1) * 4 + uint64_t(d->nnz) * 8;
+    return CUTE_OK;
+}
+
+// Host arrays to the device through pinned memory, piece by piece: the calling thread fills a piece while a kernel reads
+// the one before.  When the buffer is full the stream is waited for and the buffer used again.
+struct HostToDevice {
+    static constexpr uint64_t kPiece = 1ull << 20;
+    PinnedBuf pin;
+    uint64_t used = 0;
+    int begin(uint64_t bytes) { return pin.alloc(std::min<uint64_t>((bytes + kPiece - 1) / kPiece * kPiece + kPiece, 16ull << 20)); }
+    int copy(void *dst, const void *src, uint64_t bytes)
+    {
+        for (uint64_t at = 0; at < bytes;) {
+            if (used + kPiece > pin.cap) {
+                const int rc = pin.wait();
+                if (rc != CUTE_OK) return rc;
+                used = 0;
+            }
+            const uint64_t n = std::min(kPiece, bytes - at);
+            std::memcpy(pin.as<char>(used), static_cast<const char *>(src) + at, n);
+            pin.pending = true;
+            CUTE_BUILD(cute_build::copy_words, grid_capped(n / 4u), pin.as<const uint32_t>(used), Layout::at<uint32_t>(dst, at), n / 4u);
+            used += (n + 255u) & ~uint64_t(255);
+            at += n;
+        }
+        return CUTE_OK;
     }
-    d->nb = uint32_t(blocks);
-    rc = finish_quad_census(d, strip_pairs, quad_layout);
+};
+
+// The common tail of both uploads.  d's CSR arrays are on their way to the device (default stream).  Checks them, counts what
+// the planner wants to know about every panel, and builds the one MFMA layout the planner's default rules would use for
+// this matrix (none when every panel would go to the row kernel).
+int finish_upload(cute_hrpb_dev *d, int quad_layout, const DeviceContext &c)
+{
+    const uint32_t P = d->P;
+    LargeWork large;
+    {
+        PinnedBuf pin;
+        int rc = pin.alloc(uint64_t(P) * sizeof(cute_build::PanelCensus));
+        if (rc != CUTE_OK) return rc;
+        pin.pending = true;
+        CUTE_BUILD_LDS(cute_build::panel_census, dim3(P), window_lds(d, 0), d->dRowPtr, d->dCols, d->dCsrVals, P, d->K, d->nnz, max_span(d), pin.as<cute_build::PanelCensus>());
+        rc = check_launch("panel census");
+        if (rc == CUTE_OK) rc = pin.wait();
+        if (rc != CUTE_OK) return rc;
+        const cute_build::PanelCensus *r = pin.as<const cute_build::PanelCensus>();
+        uint32_t error = 0;
+        bool any_large = false;
+        d->panelNnz.resize(P);
+        d->panelSpan.resize(P);
+        for (uint32_t p = 0; p < P; ++p) {
+            error |= r[p].error;
+            d->panelNnz[p] = r[p].nnz;
+            d->panelSpan[p] = r[p].span;
+            any_large = any_large || panel_is_large(d, p);
+        }
+        if (!error && any_large) {
+            rc = number_large_panels(d, large, pin.as<cute_build::PanelCensus>());
+            if (rc != CUTE_OK) return rc;
+            for (uint32_t p : large.panel) error |= r[p].error;
+        }
+        if (error & cute_build::kErrRange) return CUTE_ERR_RANGE;
+        if (error & cute_build::kErrUnsorted) return CUTE_ERR_UNSORTED;
+        d->brp.resize(size_t(P) + 1);
+        d->panelCols.resize(P);
+        d->panelMaxRow.resize(P);
+        d->panelStored.resize(P);
+        d->stripPairs.resize(size_t(P) * 4u);
+        uint64_t blocks = 0;
+        d->brp[0] = 0;
+        d->numQuadVals = 0;
+        for (uint32_t p = 0; p < P; ++p) {
+            d->panelCols[p] = r[p].cols;
+            d->panelMaxRow[p] = r[p].maxRow;
+            d->panelStored[p] = r[p].stored;
+            d->numQuadVals += r[p].stored;
+            for (uint32_t s = 0; s < 4u; ++s) d->stripPairs[4u * p + s] = r[p].pairs[s];
+            blocks += (r[p].cols + CUTE_TK - 1) / CUTE_TK;
+            if (blocks > 0xffffffffull / CUTE_TILED_HDR_WORDS) return CUTE_ERR_SHAPE;
+            d->brp[p + 1] = uint32_t(blocks);
+        }
+        d->nb = uint32_t(blocks);
+    }
+    int rc = finish_quad_census(d, quad_layout);
     if (rc != CUTE_OK) return rc;
     const int which = default_layout(d, c.cache_bytes);
-    if (which == 2) rc = build_quads_on_device(d, cen);
-    else if (which == 1) rc = build_bricks_on_device(d, cen);
+    if (which == 2) rc = build_quads_on_device(d, large);
+    else if (which == 1) rc = build_bricks_on_device(d, large);
     return rc;
 }
 
@@ -663,11 +937,15 @@ int cute_hrpb_upload_layout(const cute_hrpb_host *h, int quad_layout, cute_hrpb_
     d->nnz = h->nnz;
     d->P = h->numRowPanels;
     d->numVals = h->nnz;                     // the brick tiles store every entry of the matrix once
-    int rc = upload(&d->dRowPtr, h->rowPtr, uint64_t(h->M) + 1);
-    if (rc == CUTE_OK) rc = upload(&d->dCols, h->cols, h->nnz);
-    if (rc == CUTE_OK) rc = upload(&d->dCsrVals, h->vals, h->nnz);
-    d->bytes = (uint64_t(h->M) + 1) * 4 + uint64_t(h->nnz) * 8;
-    if (rc == CUTE_OK) rc = finish_upload(d, h->rowPtr, quad_layout, c);
+    int rc = alloc_csr(d);
+    {
+        HostToDevice up;
+        if (rc == CUTE_OK) rc = up.begin(d->bytes);
+        if (rc == CUTE_OK) rc = up.copy(d->dRowPtr, h->rowPtr, (uint64_t(h->M) + 1) * 4u);
+        if (rc == CUTE_OK) rc = up.copy(d->dCols, h->cols, uint64_t(h->nnz) * 4u);
+        if (rc == CUTE_OK) rc = up.copy(d->dCsrVals, h->vals, uint64_t(h->nnz) * 4u);
+        if (rc == CUTE_OK) rc = finish_upload(d, quad_layout, c);
+    }
     // the device counted the active columns itself: it must have found the blocks the canonical format has
     if (rc == CUTE_OK && (d->nb != h->numBlocks || std::memcmp(d->brp.data(), h->blockedRowPtr, d->brp.size() * sizeof(uint32_t)) != 0))
         rc = CUTE_ERR_FORMAT;
@@ -678,8 +956,7 @@ int cute_hrpb_upload_layout(const cute_hrpb_host *h, int quad_layout, cute_hrpb_
 
 // The device-side counterpart of HRPB::HRPB + DATASTRUCT (data.cu:80-335, timed at run.cu:17-20) for a CSR
 // matrix that already lives on the device: the handle keeps its own copy of the three arrays (device to
-// device), the layouts are built by kernels, and only per-panel and per-strip counts (and the row pointers,
-// for the planner's per-panel statistics) travel to the host.
+// device), the layouts are built by kernels, and only one 48-byte record per panel travels to the host.
 int cute_hrpb_upload_device_csr(uint32_t M, uint32_t K, uint32_t nnz, const uint32_t *dRowPtr, const uint32_t *dCols,
                                 const float *dVals, int quad_layout, cute_hrpb_dev **out)
 {
@@ -688,25 +965,15 @@ int cute_hrpb_upload_device_csr(uint32_t M, uint32_t K, uint32_t nnz, const uint
     if (M == 0 || K == 0 || M % CUTE_TM || K % CUTE_TK) return CUTE_ERR_SHAPE;
     const DeviceContext &c = context();
     if (c.status != CUTE_OK) return c.status;
-    // the row pointers come to the host first: everything on the device indexes through them
-    std::vector<uint32_t> rowPtr(size_t(M) + 1);
-    HIP_TRY(hipMemcpy(rowPtr.data(), dRowPtr, rowPtr.size() * sizeof(uint32_t), hipMemcpyDeviceToHost));
-    if (rowPtr[0] != 0 || rowPtr[M] != nnz) return CUTE_ERR_RANGE;
-    for (uint32_t r = 0; r < M; ++r)
-        if (rowPtr[r + 1] < rowPtr[r]) return CUTE_ERR_RANGE;
     cute_hrpb_dev *d = new cute_hrpb_dev;
     d->M = M; d->K = K; d->nnz = nnz; d->P = M / CUTE_TM;
     d->numVals = nnz;
-    auto clone = [&](auto **dst, const auto *src, uint64_t count) -> int {
-        HIP_TRY(hipMalloc(reinterpret_cast<void **>(dst), std::max<uint64_t>(count, 1) * 4u));
-        if (count) HIP_TRY(hipMemcpy(*dst, src, count * 4u, hipMemcpyDeviceToDevice));
-        return CUTE_OK;
-    };
-    int rc = clone(&d->dRowPtr, dRowPtr, uint64_t(M) + 1);
-    if (rc == CUTE_OK) rc = clone(&d->dCols, dCols, nnz);
-    if (rc == CUTE_OK) rc = clone(&d->dCsrVals, dVals, nnz);
-    d->bytes = (uint64_t(M) + 1) * 4 + uint64_t(nnz) * 8;
-    if (rc == CUTE_OK) rc = finish_upload(d, rowPtr.data(), quad_layout, c);
+    int rc = alloc_csr(d);
+    if (rc == CUTE_OK) {
+        CUTE_BUILD(cute_build::copy_csr, grid_capped(std::max<uint64_t>(nnz, uint64_t(M) + 1)), dRowPtr, dCols, reinterpret_cast<const uint32_t *>(dVals), M, nnz,
+                   d->dRowPtr, d->dCols, reinterpret_cast<uint32_t *>(d->dCsrVals));
+        rc = finish_upload(d, quad_layout, c);
+    }
     if (rc != CUTE_OK) { cute_hrpb_dev_free(d); return rc; }
     *out = d;
     return CUTE_OK;
@@ -755,13 +1022,9 @@ int cute_hrpb_dev_csr(const cute_hrpb_dev *d, const uint32_t **dRowPtr, const ui
 void cute_spmm_plan_free(cute_spmm_plan *p)
 {
     if (!p) return;
-    (void)hipFree(p->dChunks);
-    (void)hipFree(p->dHeads);
+    give_device_memory(p->memory);
     (void)hipFree(p->dHubRows);
     (void)hipFree(p->dHubRecs);
-    (void)hipFree(p->dFixups);
-    (void)hipFree(p->dPartials);
-    (void)hipFree(p->dRowList);
     delete p;
 }
 
@@ -936,7 +1199,7 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
     // and if the partial tiles of the cut panels then turn out to be more rows than the fast kernels'
     // 24-bit row operand can address, built once more for the pipelined brick kernel, whose stores use
     // 64-bit offsets.
-    uint32_t slab = 0, num_slabs = 0, upp = 1, slots = 0, n_pieces = 0;
+    uint32_t slab = 0, num_slabs = 0, upp_log = 0, slots = 0, n_pieces = 0;
     std::vector<uint4> chunks, fixups;
     for (int attempt = 0;; ++attempt) {
         slab = p->shape == 2 ? 64u : 16u * p->vec * p->ng;   // the quad kernel: one column per lane
@@ -951,22 +1214,41 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
         // of the whole job (and at least 8 blocks), into pieces of about that share.
         // work units along a panel: 16-column blocks for the brick kernel, groups for the quad kernel
         const std::vector<uint32_t> &unit = p->shape == 2 ? d->qgp : d->brp;
-        // units per panel: 4 when the quad lists are kept per 4-row strip
-        upp = (p->shape == 2 && d->quadRows == 4) ? 4u : 1u;
-        const uint32_t num_units = d->P * upp;
+        // units per panel (its logarithm): 4 when the quad lists are kept per 4-row strip
+        upp_log = (p->shape == 2 && d->quadRows == 4) ? 2u : 0u;
+        const uint32_t num_units = d->P << upp_log;
         const uint32_t resident = uint32_t(c.num_cus) * 4u * 8u;   // 4 SIMDs x 8 wavefronts per CU
         slots = t.slots ? t.slots : resident;
-        std::vector<uint32_t> quads;
+        // A chunk of a cut panel carries the 1-based number of its partial tile; the pieces of one panel are
+        // consecutive (panels ascend through the list), and one fixup entry per cut panel adds them up afterwards.
+        chunks.clear();
+        fixups.clear();
+        n_pieces = 0;
+        chunks.reserve((size_t(n_brick) << upp_log) + 64u);
+        auto emit = [&](uint32_t s, uint32_t e, uint32_t pan, bool cut) {
+            const uint32_t len = e - s, cap = t.max_chunk_blocks ? t.max_chunk_blocks : len, step = std::min(cap, len);
+            cut = cut || len > cap;                    // cut further than the partition asked for
+            for (uint32_t cs = s; cs < e; cs += step) {
+                if (cut) {
+                    if (fixups.empty() || fixups.back().x != pan) fixups.push_back(make_uint4(pan, n_pieces, 0u, 0u));
+                    fixups.back().z++;
+                    ++n_pieces;
+                }
+                chunks.push_back(make_uint4(cs, std::min(e, cs + step), pan, cut ? n_pieces : 0u));
+            }
+        };
         if (t.slots) {
-            int64_t n = cute_partition(num_units, unit.data(), num_slabs, slots, nullptr, 0);
+            const int64_t n = cute_partition(num_units, unit.data(), num_slabs, slots, nullptr, 0);
             if (n < 0) { delete p; return int(n); }
-            quads.resize(uint64_t(n) * 4);
+            std::vector<uint32_t> quads(uint64_t(n) * 4);
             cute_partition(num_units, unit.data(), num_slabs, slots, quads.data(), uint64_t(n));
+            for (size_t i = 0; i + 3 < quads.size(); i += 4)
+                if (!to_rows[quads[i + 2] >> upp_log]) emit(quads[i], quads[i + 1], quads[i + 2], quads[i + 3] != 0);
         } else {
             uint64_t work = 0;
             uint64_t busy = 0;
             for (uint32_t q = 0; q < num_units; ++q)
-                if (!to_rows[q / upp] && unit[q + 1] != unit[q]) { work += unit[q + 1] - unit[q]; ++busy; }
+                if (!to_rows[q >> upp_log] && unit[q + 1] != unit[q]) { work += unit[q + 1] - unit[q]; ++busy; }
             const uint64_t mean = busy ? (work + busy - 1) / busy : 1;
             const uint64_t share = (work * num_slabs + resident - 1) / resident;
             // the mean only counts while it is short: a matrix whose few MFMA panels are all very long
@@ -982,60 +1264,37 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
             const uint32_t piece = limit > 2u * target ? uint32_t(4u * share) : target;
             for (uint32_t q = 0; q < num_units; ++q) {
                 const uint32_t s = unit[q], e = unit[q + 1];
-                if (s == e || to_rows[q / upp]) continue;
+                if (s == e || to_rows[q >> upp_log]) continue;
                 const uint32_t nblk = e - s;
                 if (nblk <= limit) {
-                    quads.insert(quads.end(), {s, e, q, 0u});
+                    emit(s, e, q, false);
                     continue;
                 }
                 const uint32_t pieces = (nblk + piece - 1) / piece;
                 const uint32_t step = (nblk + pieces - 1) / pieces;
-                for (uint32_t cs = s; cs < e; cs += step) quads.insert(quads.end(), {cs, std::min(e, cs + step), q, 1u});
-            }
-        }
-        // A chunk of a cut panel carries the 1-based number of its partial tile; the pieces of one panel are
-        // consecutive (panels ascend through the list), and one fixup entry per cut panel adds them up afterwards.
-        chunks.clear();
-        fixups.clear();
-        n_pieces = 0;
-        for (size_t i = 0; i + 3 < quads.size(); i += 4) {
-            const uint32_t s = quads[i], e = quads[i + 1], pan = quads[i + 2];
-            uint32_t cut = quads[i + 3];
-            if (to_rows[pan / upp]) continue;
-            const uint32_t len = e - s;
-            const uint32_t cap = t.max_chunk_blocks ? t.max_chunk_blocks : len;
-            if (len > cap) cut = 1;                    // cut further than the partition asked for
-            const uint32_t step = std::min(cap, len);
-            for (uint32_t cs = s; cs < e; cs += step) {
-                if (cut) {
-                    if (fixups.empty() || fixups.back().x != pan) fixups.push_back(make_uint4(pan, n_pieces, 0u, 0u));
-                    fixups.back().z++;
-                    ++n_pieces;
-                }
-                chunks.push_back(make_uint4(cs, std::min(e, cs + step), pan, cut ? n_pieces : 0u));
+                for (uint32_t cs = s; cs < e; cs += step) emit(cs, std::min(e, cs + step), q, true);
             }
         }
         // a strip without pairs inside an MFMA-routed panel still has to be written (as zeros): an empty chunk
-        if (upp > 1)
+        if (upp_log)
             for (uint32_t q = 0; q < num_units; ++q)
-                if (unit[q] == unit[q + 1] && !to_rows[q / upp]) chunks.push_back(make_uint4(unit[q], unit[q], q, 0u));
+                if (unit[q] == unit[q + 1] && !to_rows[q >> upp_log]) chunks.push_back(make_uint4(unit[q], unit[q], q, 0u));
         const bool lean = p->shape == 2 || p->pipeline == 1;
-        if (!lean || !n_pieces || cute_offsets_fit(d->M, d->K, N, 0, uint64_t(n_pieces) * (CUTE_TM / upp)) == 1) break;
+        if (!lean || !n_pieces || cute_offsets_fit(d->M, d->K, N, 0, uint64_t(n_pieces) * (CUTE_TM >> upp_log)) == 1) break;
         if (attempt || t.mfma_shape == 2 || t.pipeline == 1) { delete p; return CUTE_ERR_SHAPE; }   // the caller forced a fast kernel
         p->shape = 1;
         p->pipeline = 2;
         p->bf16x3 = false;
     }
-    std::vector<uint32_t> row_list;
+    std::vector<uint32_t> row_panels;              // panels of the row kernel
     for (uint32_t q = 0; q < d->P; ++q)
-        if (to_rows[q])
-            for (uint32_t r = 0; r < CUTE_TM; ++r) row_list.push_back(q * CUTE_TM + r);
+        if (to_rows[q]) row_panels.push_back(q);
 
     // Row-kernel blocks per XCD: contiguous ranges of rows (neighbouring rows share B rows, which then stay
     // in one L2), cut where the running work -- nonzeros plus a fixed cost per row -- passes each eighth.
     {
         const uint32_t items_per_block = 256u >> p->rows_logl;             // rows of one 256-thread block (per slab)
-        const uint64_t total_items = uint64_t(row_list.size());
+        const uint64_t total_items = uint64_t(row_panels.size()) * CUTE_TM;
         const uint32_t total_blocks = uint32_t((total_items + items_per_block - 1) / items_per_block);
         uint64_t total_work = 0;
         for (uint32_t q = 0; q < d->P; ++q)
@@ -1092,10 +1351,12 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
                         (uint64_t(longest) * chunks.size() >= 4u * total || fullest * 10u > even * 11u);
     }
     if (longest_first && !chunks.empty()) {
-        std::vector<uint4> sorted(chunks);
-        std::stable_sort(sorted.begin(), sorted.end(), [](const uint4 &a, const uint4 &b) {
-            return __builtin_clz((a.y - a.x) | 1u) < __builtin_clz((b.y - b.x) | 1u);
-        });
+        std::vector<uint4> sorted(chunks.size());
+        size_t place[33] = {};                 // a counting sort by the power of two of the length, longest first, stable
+        auto bucket = [](const uint4 &ck) { return size_t(__builtin_clz((ck.y - ck.x) | 1u)); };
+        for (const uint4 &ck : chunks) ++place[bucket(ck) + 1];
+        for (size_t k = 0; k < 32; ++k) place[k + 1] += place[k];
+        for (const uint4 &ck : chunks) sorted[place[bucket(ck)]++] = ck;
         // work-group g runs on XCD g % 8 and takes the list positions the kernels' XCD mapping gives it: XCD x walks
         // the groups [x * per_xcd, (x + 1) * per_xcd).  Deal the sorted groups round-robin into those ranges.
         const uint32_t wpg = cute_dev::kWavesPerGroup;
@@ -1126,53 +1387,55 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
                                           p->shape == 2 || p->ng == 1 ? 8u : 4u, t.chunk_order == 2) ? 1u : 0u;
     // the layout this plan's MFMA kernel reads, if the upload has not built it
     int rc = chunks.empty() ? int(CUTE_OK) : ensure_layout(d, p->shape);
-    if (rc == CUTE_OK) rc = upload(&p->dChunks, chunks.data(), chunks.size());
     if (rc == CUTE_OK && hub_rows) rc = make_hub_tables(p, d, hub_rows);
-    if (rc == CUTE_OK && p->shape == 2 && !chunks.empty()) {
-        // one 128-byte head per work item: its descriptor and a copy of its first group's record, so that a
-        // wavefront can ask for its first B rows after one scalar fetch instead of two dependent ones; gathered
-        // on the device, where the records are
-        const uint64_t words = uint64_t(chunks.size()) * cute_dev::kQuadHeadWords;
-        if (hipMalloc(reinterpret_cast<void **>(&p->dHeads), words * sizeof(uint32_t)) != hipSuccess) rc = CUTE_ERR_NOMEM;
-        if (rc == CUTE_OK) {
-            hipLaunchKernelGGL(cute_build::quad_heads, grid_of(words), dim3(cute_build::kThreads), 0, nullptr, p->dChunks,
-                               uint32_t(chunks.size()), p->dHubRecs ? p->dHubRecs : d->dQRecs, uint32_t(cute_dev::kQuadHeadWords), p->dHeads);
-            rc = check_launch("quad heads");
-            if (rc == CUTE_OK && hipStreamSynchronize(nullptr) != hipSuccess) rc = CUTE_ERR_HIP;
-        }
-    }
-    if (rc == CUTE_OK) rc = upload(&p->dFixups, fixups.data(), fixups.size());
-    p->unitRows = CUTE_TM / upp;
+    p->unitRows = CUTE_TM >> upp_log;
     // reduce_partials walks a tile along grid.y, a block of sixteen wavefronts taking 16 / G segments of 64 elements, G = 1..16
     // wavefronts to a segment by the number of pieces (see the kernel): the launch gets the blocks its tile with the most
     // pieces needs (the others leave theirs early), not one per segment -- with thousands of cut panels of two or three
     // pieces each the blocks that only start and exit otherwise cost more than the sums
-    if (rc == CUTE_OK && n_pieces && (uint64_t(CUTE_TM / upp) * N + 63u) / 64u > 65535u) rc = CUTE_ERR_SHAPE;
+    if (rc == CUTE_OK && n_pieces && (uint64_t(CUTE_TM >> upp_log) * N + 63u) / 64u > 65535u) rc = CUTE_ERR_SHAPE;
     {
         uint32_t most = 1;
         for (const uint4 &fx : fixups) most = std::max(most, fx.z);
         const uint32_t G = most <= 4 ? 1u : most <= 8 ? 2u : most <= 16 ? 4u : most <= 32 ? 8u : 16u;    // as in reduce_partials
-        const uint32_t segments = (CUTE_TM / upp * N + 63u) / 64u, per_block = uint32_t(cute_dev::kReduceWaves) / G;
+        const uint32_t segments = ((CUTE_TM >> upp_log) * N + 63u) / 64u, per_block = uint32_t(cute_dev::kReduceWaves) / G;
         p->reduceBlocksY = std::max(1u, (segments + per_block - 1u) / per_block);
     }
-    if (rc == CUTE_OK && n_pieces) {
-        // (the fast kernels address the partial tiles like C, with 32-bit byte offsets: checked where the chunks were made)
-        const uint64_t bytes = uint64_t(n_pieces) * p->unitRows * N * sizeof(float);
-        p->partialBytes = bytes;
-        if (hipMalloc(reinterpret_cast<void **>(&p->dPartials), bytes) != hipSuccess) rc = CUTE_ERR_NOMEM;
-    }
-    if (rc == CUTE_OK && !row_list.empty()) {
-        // the list goes up as row indices and is packed with the rows' pointers on the device, where those are
-        uint32_t *rows_only = nullptr;
-        rc = upload(&rows_only, row_list.data(), row_list.size());
-        if (rc == CUTE_OK && hipMalloc(reinterpret_cast<void **>(&p->dRowList), row_list.size() * sizeof(uint4)) != hipSuccess) rc = CUTE_ERR_NOMEM;
+    // (the fast kernels address the partial tiles like C, with 32-bit byte offsets: checked where the chunks were made)
+    p->partialBytes = uint64_t(n_pieces) * p->unitRows * N * sizeof(float);
+    // Every row on the row kernel: no row list needed, which takes one dependent load out of each row's chain.
+    const bool every_row = row_panels.size() == d->P;
+    if (rc == CUTE_OK && (!chunks.empty() || !every_row)) {
+        // The quad kernels get one 128-byte head per work item, its descriptor and a copy of its first group's record, so that
+        // a wavefront can ask for its first B rows after one scalar fetch instead of two dependent ones; heads and row
+        // list are gathered on the device, where the records and the row pointers are.
+        const uint32_t listed = every_row ? 0u : uint32_t(row_panels.size());
+        const bool heads = p->shape == 2;
+        Layout stage, lay;
+        const uint64_t sChunks = stage.add(chunks.size(), sizeof(uint4)), sFixups = stage.add(fixups.size(), sizeof(uint4)), sRows = stage.add(listed, 4);
+        const uint64_t oChunks = lay.add(chunks.size(), heads ? cute_dev::kQuadHeadWords * 4u : sizeof(uint4)), oFixups = lay.add(fixups.size(), sizeof(uint4)),
+                       oRows = lay.add(uint64_t(listed) * CUTE_TM, sizeof(uint4)), oPartials = lay.add(p->partialBytes, 1);
+        PinnedBuf pin;
+        rc = pin.alloc(stage.bytes);
+        if (rc == CUTE_OK && pool().take(&p->memory, lay.bytes) != CUTE_OK) rc = CUTE_ERR_NOMEM;
         if (rc == CUTE_OK) {
-            hipLaunchKernelGGL(cute_build::pack_row_list, grid_of(row_list.size()), dim3(cute_build::kThreads), 0, nullptr, rows_only,
-                               uint32_t(row_list.size()), d->dRowPtr, p->dRowList);
-            rc = check_launch("row list");
-            if (rc == CUTE_OK && hipStreamSynchronize(nullptr) != hipSuccess) rc = CUTE_ERR_HIP;
+            std::memcpy(pin.as<char>(sChunks), chunks.data(), chunks.size() * sizeof(uint4));
+            std::memcpy(pin.as<char>(sFixups), fixups.data(), fixups.size() * sizeof(uint4));
+            if (listed) std::memcpy(pin.as<char>(sRows), row_panels.data(), listed * sizeof(uint32_t));
+            if (heads) p->dHeads = Layout::at<uint32_t>(p->memory, oChunks);
+            else p->dChunks = Layout::at<uint4>(p->memory, oChunks);
+            p->dFixups = Layout::at<uint4>(p->memory, oFixups);
+            p->dRowList = listed ? Layout::at<uint4>(p->memory, oRows) : nullptr;
+            p->dPartials = n_pieces ? Layout::at<float>(p->memory, oPartials) : nullptr;
+            const cute_build::PlanTables T = {pin.as<const uint4>(sChunks), pin.as<const uint4>(sFixups), pin.as<const uint32_t>(sRows),
+                                              uint32_t(chunks.size()), uint32_t(fixups.size()), listed, p->dChunks, p->dHeads, p->dFixups, p->dRowList};
+            const uint64_t items = uint64_t(chunks.size()) * (heads ? cute_dev::kQuadHeadWords : 1) + fixups.size() + uint64_t(listed) * CUTE_TM;
+            pin.pending = true;
+            CUTE_BUILD(cute_build::plan_tables, grid_of(items), T, heads ? (p->dHubRecs ? p->dHubRecs : d->dQRecs) : static_cast<const uint32_t *>(nullptr),
+                       uint32_t(cute_dev::kQuadHeadWords), d->dRowPtr);
+            rc = check_launch("plan tables");
+            if (rc == CUTE_OK) rc = pin.wait();
         }
-        (void)hipFree(rows_only);
     }
     if (rc == CUTE_OK) {
         // cute_spmm_run_static's scratch: its address on this device is looked up here, at set-up, so that the
@@ -1181,7 +1444,7 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
     }
     if (rc != CUTE_OK) { cute_spmm_plan_free(p); return rc; }
     p->numFixups = uint32_t(fixups.size());
-    p->numRows = uint32_t(row_list.size());
+    p->numRows = uint32_t(row_panels.size()) * CUTE_TM;
     p->info.N = N;
     p->info.slabWidth = slab;
     p->info.numSlabs = num_slabs;
@@ -1198,7 +1461,7 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
     p->info.pipeline = uint32_t(p->pipeline);
     // one launch for a mixed plan: the quad kernel with any row shape of 4-float lanes, the rolling brick
     // kernel in the shapes the planner itself picks for N (forced column groups fall back to two launches)
-    const bool rows_fusable = !chunks.empty() && !row_list.empty() && p->rows_vec == 4;
+    const bool rows_fusable = !chunks.empty() && !row_panels.empty() && p->rows_vec == 4;
     const bool brick_default_shape = ng_for_mixed || p->ng == ((p->vec == 4 && N >= 128) ? 2 : 1);
     p->info.partialTileKiB = uint32_t((p->partialBytes + 1023u) / 1024u);
     p->info.fusedLaunch = (rows_fusable && !p->bf16x3 && !p->numHub && (p->shape == 2 || (p->pipeline == 1 && brick_default_shape))) ? 1u : 0u;
@@ -1475,8 +1738,7 @@ int run_with(const cute_spmm_plan *p, const float *dB, float *dC, void *stream, 
         else launch_brick<1, 1>(p, dB, dC, partials, s);
     }
     if (p->numRows && !rows_launched) {
-        // every row: no list needed, which takes one dependent load out of each row's chain
-        launch_rows<true>(p->rows_vec, p->rows_logl, p->numRows == p->d->M ? nullptr : p->dRowList, p->numRows, p->rows_slabs, p->d->dRowPtr, p->d->dCols,
+        launch_rows<true>(p->rows_vec, p->rows_logl, p->dRowList, p->numRows, p->rows_slabs, p->d->dRowPtr, p->d->dCols,
                     p->d->dCsrVals, dB, dC, N, s, &p->rowRanges, p->rowBlocksPerXcd);
     }
     // panels that were cut: add their partial tiles up, in chunk order (no atomics, so a product is
