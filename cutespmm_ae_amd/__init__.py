@@ -281,11 +281,19 @@ class _Owned(np.ndarray):
     _owner = None
 
 
+class _Memory:
+    """Library-owned memory as the array interface describes it; the arrays made of it keep it, and it keeps its owner."""
+
+    def __init__(self, ptr, n, dtype, owner):
+        self.owner = owner
+        self.__array_interface__ = dict(data=(C.cast(ptr, C.c_void_p).value, False), shape=(n,), typestr=np.dtype(dtype).str, version=3)
+
+
 def _view(ptr, n, dtype, owner=None):
     n = int(n)
     if n == 0:
         return np.zeros(0, dtype)
-    a = np.ctypeslib.as_array(ptr, shape=(n,)).view(dtype).view(_Owned)
+    a = np.asarray(_Memory(ptr, n, dtype, owner)).view(_Owned)
     a._owner = owner
     return a
 

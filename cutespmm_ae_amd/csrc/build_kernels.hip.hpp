@@ -32,8 +32,10 @@ constexpr int kThreads = 256;
 constexpr int kScanItems = 8;                               // entries per thread of a scan block
 constexpr uint32_t kScanBlock = kThreads * kScanItems;      // entries per scan block
 
-constexpr uint32_t kPanelCap = 2048;                        // entries of a panel that one work-group holds, eight a thread
-constexpr uint32_t kPanelSmall = kPanelCap / 2;             // list kernel: most panels need half the LDS, twice as many then run at a time
+// Entries of a panel that one work-group holds, eight a thread: 512 threads for up to kPanelCap; the launches over all panels
+// take 256 threads and up to kPanelFirst (list kernel: kPanelList, whose LDS lets six work-groups share a compute unit instead
+// of three, 60 -> 40 us on the graph above), the launches over the few panels between are given their list.
+constexpr uint32_t kPanelCap = 4096, kPanelFirst = 2048, kPanelList = 1024;
 constexpr uint32_t kPanelSpan = 1u << 17;                   // columns of its window: a bitmap of 16 KB and 8 KB of running counts
 
 enum : uint32_t { kErrRange = 1, kErrUnsorted = 2 };
@@ -157,18 +159,20 @@ __device__ __forceinline__ uint32_t row_in_panel(const uint32_t *rp, uint32_t e)
 // ------------------------------------------------------------------------------------------------
 // A panel in LDS.
 // ------------------------------------------------------------------------------------------------
+constexpr uint32_t panel_threads(uint32_t cap) { return cap == kPanelCap ? 512u : 256u; }
 struct Two { uint32_t x, y; };
 template <uint32_t CAP> struct PanelLds {
+    static constexpr uint32_t kBlock = panel_threads(CAP);
     uint32_t rp[17];                         // row starts, from the panel's first entry
     uint32_t lo, hi;                         // first and last column
-    Two waveSum[kThreads / 64];
+    Two waveSum[kBlock / 64];
     uint32_t col[CAP];                       // active columns
     uint32_t rows[CAP];                      // and the rows that hold them: bits 0..15 any entry, bits 16..31 one that is not zero
 };
 
-// The entries t, t + 256, .. of a panel in one thread's registers.
+// The entries t, t + (threads), .. of a panel in one thread's registers.
 template <uint32_t CAP> struct PanelEntries {
-    static constexpr uint32_t kEach = CAP / kThreads;
+    static constexpr uint32_t kEach = CAP / panel_threads(CAP);
     uint32_t active[kEach];                  // index of the entry's column among the panel's active columns
     uint32_t row[kEach];
     float val[kEach];
@@ -187,7 +191,7 @@ template <uint32_t CAP> __device__ __forceinline__ Two block_exclusive(PanelLds<
     Two before = {incl.x - own.x, incl.y - own.y};
     total = {0u, 0u};
 #pragma unroll
-    for (uint32_t w = 0; w < kThreads / 64u; ++w) {
+    for (uint32_t w = 0; w < PanelLds<CAP>::kBlock / 64u; ++w) {
         const Two v = l.waveSum[w];
         if (w < wave) { before.x += v.x; before.y += v.y; }
         total.x += v.x;
@@ -238,18 +242,18 @@ __device__ __forceinline__ uint32_t load_panel(PanelLds<CAP> &l, PanelEntries<CA
     uint32_t lo = ~0u, hi = 0u;
 #pragma unroll
     for (uint32_t k = 0; k < PanelEntries<CAP>::kEach; ++k) {
-        if (k * kThreads >= n) break;
-        const uint32_t i = k * kThreads + t;
+        if (k * PanelLds<CAP>::kBlock >= n) break;
+        const uint32_t i = k * PanelLds<CAP>::kBlock + t;
         if (i >= n) continue;
         e.active[k] = cols[uint64_t(start) + i];             // its column until number_columns
         e.val[k] = vals[uint64_t(start) + i];
     }
-    for (uint32_t w = t; w < panel_window_words(max_span); w += kThreads) window[w] = 0u;
-    for (uint32_t i = t; i < n; i += kThreads) l.rows[i] = 0u;
+    for (uint32_t w = t; w < panel_window_words(max_span); w += PanelLds<CAP>::kBlock) window[w] = 0u;
+    for (uint32_t i = t; i < n; i += PanelLds<CAP>::kBlock) l.rows[i] = 0u;
 #pragma unroll
     for (uint32_t k = 0; k < PanelEntries<CAP>::kEach; ++k) {
-        if (k * kThreads >= n) break;
-        const uint32_t i = k * kThreads + t;
+        if (k * PanelLds<CAP>::kBlock >= n) break;
+        const uint32_t i = k * PanelLds<CAP>::kBlock + t;
         if (i >= n) continue;
         e.row[k] = row_in_panel(l.rp, i);
         const uint32_t c = e.active[k];
@@ -280,11 +284,11 @@ __device__ __forceinline__ uint32_t number_columns(PanelLds<CAP> &l, PanelEntrie
     uint16_t *count = reinterpret_cast<uint16_t *>(window + words);
 #pragma unroll
     for (uint32_t k = 0; k < PanelEntries<CAP>::kEach; ++k) {
-        if (k * kThreads >= n) break;
-        if (k * kThreads + t < n) atomicOr(&window[(e.active[k] - lo) >> 5], 1u << ((e.active[k] - lo) & 31u));
+        if (k * PanelLds<CAP>::kBlock >= n) break;
+        if (k * PanelLds<CAP>::kBlock + t < n) atomicOr(&window[(e.active[k] - lo) >> 5], 1u << ((e.active[k] - lo) & 31u));
     }
     __syncthreads();
-    const uint32_t per = (words + kThreads - 1u) / kThreads, w0 = min(t * per, words), w1 = min(w0 + per, words);
+    const uint32_t per = (words + PanelLds<CAP>::kBlock - 1u) / PanelLds<CAP>::kBlock, w0 = min(t * per, words), w1 = min(w0 + per, words);
     uint32_t own = 0;
     for (uint32_t w = w0; w < w1; ++w) own += uint32_t(__popc(window[w]));
     uint32_t total;
@@ -293,8 +297,8 @@ __device__ __forceinline__ uint32_t number_columns(PanelLds<CAP> &l, PanelEntrie
     __syncthreads();
 #pragma unroll
     for (uint32_t k = 0; k < PanelEntries<CAP>::kEach; ++k) {
-        if (k * kThreads >= n) break;
-        if (k * kThreads + t >= n) continue;
+        if (k * PanelLds<CAP>::kBlock >= n) break;
+        if (k * PanelLds<CAP>::kBlock + t >= n) continue;
         const uint32_t c = e.active[k], w = (c - lo) >> 5;
         const uint32_t a = count[w] + uint32_t(__popc(window[w] & ((1u << ((c - lo) & 31u)) - 1u)));
         e.active[k] = a;
@@ -312,15 +316,17 @@ __device__ __forceinline__ Two strips_of(uint32_t rows)
 }
 __device__ __forceinline__ uint32_t half(const Two &v, uint32_t s) { return ((s & 2u ? v.y : v.x) >> (16u * (s & 1u))) & 0xffffu; }
 
-__global__ __launch_bounds__(kThreads) void panel_census(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols,
+// The panel kernels take every panel of up to CAP entries (list_of = nullptr), or the panels of a list (with CAP = kPanelCap; a
+// second launch over all panels would spend 15 us on work-groups that only leave).
+template <uint32_t CAP>
+__global__ __launch_bounds__(panel_threads(CAP)) void panel_census(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols,
                                                          const float *__restrict__ vals, uint32_t P, uint32_t K, uint32_t nnz, uint32_t max_span,
-                                                         PanelCensus *__restrict__ out)
+                                                         const uint32_t *__restrict__ list_of, PanelCensus *__restrict__ out)
 {
-    constexpr uint32_t CAP = kPanelCap;
     extern __shared__ uint32_t window[];
     __shared__ PanelLds<CAP> l;
     __shared__ PanelCensus res;
-    const uint32_t p = blockIdx.x, t = threadIdx.x;
+    const uint32_t p = list_of ? list_of[blockIdx.x] : blockIdx.x, t = threadIdx.x;
     uint32_t start;
     if (t < 12u) reinterpret_cast<uint32_t *>(&res)[t] = 0u;
     const uint32_t n = panel_rows(l, rowPtr, p, P, nnz, start);
@@ -329,7 +335,7 @@ __global__ __launch_bounds__(kThreads) void panel_census(const uint32_t *__restr
     } else {
         if (t < 16u) atomicMax(&res.maxRow, l.rp[t + 1] - l.rp[t]);
         if (t == 0u) res.nnz = n;
-        if (n > kPanelCap) {
+        if (n > CAP) {
             if (t < 16u && l.rp[t + 1] > l.rp[t]) {
                 atomicMin(&l.lo, cols[uint64_t(start) + l.rp[t]]);
                 atomicMax(&l.hi, cols[uint64_t(start) + l.rp[t + 1] - 1u]);
@@ -343,7 +349,7 @@ __global__ __launch_bounds__(kThreads) void panel_census(const uint32_t *__restr
                 const uint32_t active = number_columns(l, e, window, n);
                 Two pairs = {0u, 0u};
                 uint32_t stored = 0;
-                for (uint32_t a = t; a < active; a += kThreads) {
+                for (uint32_t a = t; a < active; a += PanelLds<CAP>::kBlock) {
                     const Two here = strips_of(l.rows[a]);
                     pairs.x += here.x;
                     pairs.y += here.y;
@@ -368,19 +374,19 @@ __global__ __launch_bounds__(kThreads) void panel_census(const uint32_t *__restr
 
 // Brick tiles of the panels that fit: hdr lines and values (cute_hrpb_retile defines both).  brp: first block of every
 // panel.  Block 0 also writes the wavefront of zeros behind the values.
-__global__ __launch_bounds__(kThreads) void panel_bricks(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols,
+template <uint32_t CAP>
+__global__ __launch_bounds__(panel_threads(CAP)) void panel_bricks(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols,
                                                          const float *__restrict__ vals, uint32_t P, uint32_t nnz, uint32_t max_span,
-                                                         const uint32_t *__restrict__ brp, uint32_t *__restrict__ hdr, float *__restrict__ tile_vals)
+                                                         const uint32_t *__restrict__ list_of, const uint32_t *__restrict__ brp, uint32_t *__restrict__ hdr, float *__restrict__ tile_vals)
 {
-    constexpr uint32_t CAP = kPanelCap;
     extern __shared__ uint32_t window[];
     __shared__ PanelLds<CAP> l;
-    const uint32_t p = blockIdx.x, t = threadIdx.x;
-    if (p == 0u && t < 64u) tile_vals[uint64_t(nnz) + t] = 0.0f;
+    const uint32_t p = list_of ? list_of[blockIdx.x] : blockIdx.x, t = threadIdx.x;
+    if (!list_of && p == 0u && t < 64u) tile_vals[uint64_t(nnz) + t] = 0.0f;
     const uint32_t block0 = brp[p];
     uint32_t start;
     const uint32_t n = panel_rows(l, rowPtr, p, P, nnz, start);
-    if (n == 0u || n > kPanelCap) return;
+    if (n == 0u || n > CAP) return;
     PanelEntries<CAP> e;
     load_panel<false>(l, e, window, cols, vals, start, n, 0u, max_span);
     if (!panel_fits(l, max_span)) return;
@@ -405,7 +411,7 @@ __global__ __launch_bounds__(kThreads) void panel_bricks(const uint32_t *__restr
     }
     __syncthreads();
     const uint32_t slots = ((active + 15u) / 16u) * 16u;
-    for (uint32_t a = t; a < slots; a += kThreads) {          // sixteen lanes are the sixteen columns of one block
+    for (uint32_t a = t; a < slots; a += PanelLds<CAP>::kBlock) {          // sixteen lanes are the sixteen columns of one block
         const uint32_t b = first[min(a, active)];
         const uint32_t mask = a < active ? l.rows[a] & 0xffffu : 0u;
         const uint32_t slot = a & 15u, j = slot >> 2, k = slot & 3u;
@@ -418,8 +424,8 @@ __global__ __launch_bounds__(kThreads) void panel_bricks(const uint32_t *__restr
     }
 #pragma unroll
     for (uint32_t k = 0; k < PanelEntries<CAP>::kEach; ++k) {
-        if (k * kThreads >= n) break;
-        if (k * kThreads + t >= n) continue;
+        if (k * PanelLds<CAP>::kBlock >= n) break;
+        if (k * PanelLds<CAP>::kBlock + t >= n) continue;
         const uint32_t a = e.active[k];
         tile_vals[uint64_t(start) + first[a] + uint32_t(__popc(l.rows[a] & ((1u << e.row[k]) - 1u)))] = e.val[k];
     }
@@ -429,11 +435,9 @@ __global__ __launch_bounds__(kThreads) void panel_bricks(const uint32_t *__restr
 // else four lockstep lists per panel, groups[p].  valBase: first stored value of every panel.  A thread is one
 // (row group, column) pair; the running number of stored values over the pairs of the panel is at once the place of
 // their values and, at a group's first pair, the record's index word.  Block 0 writes the zeros behind the values.
-// list_of: the panels to take (those beyond kPanelSmall: a launch over all panels spends 15 us on work-groups that only leave),
-// nullptr: every panel of up to CAP entries.
 // Dynamic LDS: the window, then (in its place) the list places of every column, four 16-bit numbers each.
 template <bool STRIPS, uint32_t CAP>
-__global__ __launch_bounds__(kThreads) void panel_quads(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols,
+__global__ __launch_bounds__(panel_threads(CAP)) void panel_quads(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols,
                                                         const float *__restrict__ vals, uint32_t P, uint32_t nnz, uint32_t max_span, const uint32_t *__restrict__ list_of,
                                                         const uint32_t *__restrict__ groups, const uint32_t *__restrict__ valBase, uint32_t stored,
                                                         uint32_t *__restrict__ recs, float *__restrict__ packed)
@@ -491,7 +495,7 @@ __global__ __launch_bounds__(kThreads) void panel_quads(const uint32_t *__restri
     }
     const uint32_t slots = total * 16u;
     uint32_t base = 0;
-    for (uint32_t x0 = 0; x0 < slots; x0 += kThreads) {
+    for (uint32_t x0 = 0; x0 < slots; x0 += PanelLds<CAP>::kBlock) {
         const uint32_t x = x0 + t, g = x >> 4, pair = x & 15u;
         const bool live = x < slots;
         const uint32_t s = STRIPS ? (g >= group_before[1] ? 1u : 0u) + (g >= group_before[2] ? 1u : 0u) + (g >= group_before[3] ? 1u : 0u) : pair & 3u;
@@ -522,8 +526,8 @@ __global__ __launch_bounds__(kThreads) void panel_quads(const uint32_t *__restri
     __syncthreads();
 #pragma unroll
     for (uint32_t k = 0; k < PanelEntries<CAP>::kEach; ++k) {
-        if (k * kThreads >= n) break;
-        if (k * kThreads + t >= n || e.val[k] == 0.0f) continue;
+        if (k * PanelLds<CAP>::kBlock >= n) break;
+        if (k * PanelLds<CAP>::kBlock + t >= n || e.val[k] == 0.0f) continue;
         const uint32_t a = e.active[k], s = e.row[k] >> 2, mask = (l.rows[a] >> (16u + 4u * s)) & 15u;
         const uint32_t pr = half(before[a], s);
         packed[uint64_t(value0) + place[pr] + uint32_t(__popc(mask & ((1u << (e.row[k] & 3u)) - 1u)))] = e.val[k];

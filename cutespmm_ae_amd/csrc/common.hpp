@@ -1,11 +1,16 @@
-// Shared host-side helpers of libcutespmm: allocation, a thread pool-less parallel_for,
+// Shared host-side helpers of libcutespmm: allocation, a parallel_for over a pool of threads,
 // and the lane-order <-> canonical bitmap permutation used by the device layout.
 #pragma once
+#include <pthread.h>
+
 #include <algorithm>
+#include <atomic>
+#include <condition_variable>
 #include <cstdint>
 #include <cstdlib>
 #include <cctype>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <thread>
 #include <vector>
@@ -30,7 +35,84 @@ inline unsigned host_threads()
     return std::max(1u, std::min(n, 64u));
 }
 
-// Calls fn(begin, end, thread_index) on contiguous ranges of [0, n).
+// Worker threads that stay between calls: starting and joining 16 threads costs 280 us, handing them work about 20, and the
+// host side of a new matrix is two or three such sections of a few hundred microseconds each.  One job at a time; a second
+// caller (another thread of the program, or a job's own task) starts threads of its own instead.  The workers sleep
+// while there is no job.  A child process after fork has no threads and gets a pool of its own.
+class HostPool {
+    std::mutex job_, m_;
+    std::condition_variable wake_, done_;
+    void (*call_)(void *, unsigned) = nullptr;
+    void *arg_ = nullptr;
+    unsigned next_ = 0, tasks_ = 0, open_ = 0, workers_ = 0;
+
+    void work()
+    {
+        std::unique_lock<std::mutex> l(m_);
+        for (;;) {
+            wake_.wait(l, [this] { return next_ < tasks_; });
+            take(l);
+        }
+    }
+    void take(std::unique_lock<std::mutex> &l)          // the tasks that are left, one after the other
+    {
+        while (next_ < tasks_) {
+            const unsigned i = next_++;
+            l.unlock();
+            call_(arg_, i);
+            l.lock();
+            if (--open_ == 0) done_.notify_one();
+        }
+    }
+
+    static HostPool *&instance()
+    {
+        static HostPool *p = [] {
+            pthread_atfork(nullptr, nullptr, [] { instance() = new HostPool; });
+            return new HostPool;
+        }();
+        return p;
+    }
+
+public:
+    static HostPool &get() { return *instance(); }
+
+    // call(arg, i) for every i < tasks on up to `threads` threads, the caller's among them; false when a job is running.
+    bool run(unsigned tasks, unsigned threads, void (*call)(void *, unsigned), void *arg)
+    {
+        std::unique_lock<std::mutex> job(job_, std::try_to_lock);
+        if (!job.owns_lock()) return false;
+        std::unique_lock<std::mutex> l(m_);
+        for (; workers_ + 1 < threads; ++workers_) std::thread([this] { work(); }).detach();
+        call_ = call; arg_ = arg;
+        next_ = 0; tasks_ = open_ = tasks;
+        for (unsigned i = 1; i < std::min(tasks, threads); ++i) wake_.notify_one();
+        take(l);
+        done_.wait(l, [this] { return open_ == 0; });
+        tasks_ = 0;
+        return true;
+    }
+};
+
+// Calls fn(i) for every i < n; the tasks are handed out as threads become free.
+template <class F>
+inline void parallel_tasks(unsigned n, F fn)
+{
+    const unsigned nt = std::min(host_threads(), n);
+    if (nt > 1) {
+        if (HostPool::get().run(n, nt, [](void *f, unsigned i) { (*static_cast<F *>(f))(i); }, &fn)) return;
+        std::atomic<unsigned> next{0};
+        std::vector<std::thread> th;
+        th.reserve(nt);
+        for (unsigned t = 0; t < nt; ++t)
+            th.emplace_back([&] { for (unsigned i; (i = next.fetch_add(1)) < n;) fn(i); });
+        for (auto &x : th) x.join();
+        return;
+    }
+    for (unsigned i = 0; i < n; ++i) fn(i);
+}
+
+// Calls fn(begin, end, thread_index) on contiguous ranges of [0, n), one per thread.
 template <class F>
 inline void parallel_ranges(uint64_t n, uint64_t min_per_thread, F fn)
 {
@@ -41,13 +123,7 @@ inline void parallel_ranges(uint64_t n, uint64_t min_per_thread, F fn)
         fn(uint64_t(0), n, 0u);
         return;
     }
-    std::vector<std::thread> th;
-    th.reserve(nt);
-    for (unsigned t = 0; t < nt; ++t) {
-        uint64_t b = n * t / nt, e = n * (t + 1) / nt;
-        th.emplace_back([=] { fn(b, e, t); });
-    }
-    for (auto &x : th) x.join();
+    parallel_tasks(nt, [&](unsigned t) { fn(n * t / nt, n * (t + 1) / nt, t); });
 }
 
 // Canonical brick bitmap: bit row*4+k (data.cu:36-38).  Lane order: bit k*16+row, the

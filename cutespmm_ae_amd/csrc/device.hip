@@ -521,12 +521,14 @@ inline dim3 grid_capped(uint64_t n) { return dim3(std::min<uint32_t>(grid_of(n).
 int check_launch(const char *what);
 
 #define CUTE_BUILD(kernel, grid, ...) CUTE_BUILD_LDS(kernel, grid, 0, __VA_ARGS__)
-#define CUTE_BUILD_LDS(kernel, grid, lds, ...) \
-    hipLaunchKernelGGL(kernel, grid, dim3(cute_build::kThreads), lds, nullptr, __VA_ARGS__)
+#define CUTE_BUILD_LDS(kernel, grid, lds, ...) hipLaunchKernelGGL(kernel, grid, dim3(cute_build::kThreads), lds, nullptr, __VA_ARGS__)
+// a panel kernel of the given capacity over `count` panels: all of them, or a list
+#define CUTE_PANELS(kernel, CAP, count, lds, ...) hipLaunchKernelGGL(kernel, dim3(count), dim3(cute_build::panel_threads(CAP)), lds, nullptr, __VA_ARGS__)
 
 // The widest column window the panel kernels take on this matrix, and the LDS its bitmap and running counts need.
 inline uint32_t max_span(const cute_hrpb_dev *d) { return std::min(d->K, cute_build::kPanelSpan); }
 inline uint32_t window_lds(const cute_hrpb_dev *d, uint32_t at_least) { return std::max((cute_build::panel_window_words(max_span(d)) + 1u) * 6u, at_least); }
+constexpr const uint32_t *kAllPanels = nullptr;
 inline bool panel_is_large(const cute_hrpb_dev *d, uint32_t p) { return d->panelNnz[p] > cute_build::kPanelCap || d->panelSpan[p] > max_span(d); }
 
 // Words of scratch device_scan needs for an array of n values: the block sums of every level.
@@ -551,6 +553,15 @@ void device_scan(uint32_t *data, uint64_t n, uint32_t *scratch, uint32_t arrays 
         sums = scratch;
     }
     CUTE_BUILD(cute_build::scan_block_apply, grid, data, n, pitch, sums, scratch_pitch);
+}
+
+// The panels that a launch over all panels leaves out because they hold more than `cap` entries, though a panel kernel takes them.
+std::vector<uint32_t> panels_between(const cute_hrpb_dev *d, uint32_t cap)
+{
+    std::vector<uint32_t> list;
+    for (uint32_t p = 0; p < d->P; ++p)
+        if (d->panelNnz[p] > cap && !panel_is_large(d, p)) list.push_back(p);
+    return list;
 }
 
 // The panels that the panel kernels do not take and what their entry-parallel path keeps between its kernels.
@@ -609,6 +620,8 @@ int build_bricks_on_device(cute_hrpb_dev *d, const LargeWork &w)
     const uint32_t count = uint32_t(w.panel.size());
     Layout lay, tab;
     const uint64_t oBrp = tab.add(uint64_t(d->P) + 1u, 4), oUnit = tab.add(count, 4), oPrefix = tab.add(count + 1u, 4), oCols = tab.add(count, 4);
+    const std::vector<uint32_t> medium = panels_between(d, cute_build::kPanelFirst);
+    const uint64_t oMedium = tab.add(medium.size(), 4);
     const uint64_t oHdr = lay.add(hdr_words, 4), oVals = lay.add(num_vals, 4), oTab = lay.add(tab.bytes, 1);
     DevBuf mem;
     PinnedBuf pin;
@@ -619,6 +632,7 @@ int build_bricks_on_device(cute_hrpb_dev *d, const LargeWork &w)
     uint32_t *hdr = Layout::at<uint32_t>(mem.p, oHdr);
     float *vals = Layout::at<float>(mem.p, oVals);
     std::memcpy(pin.p, d->brp.data(), d->brp.size() * 4u);
+    if (!medium.empty()) std::memcpy(pin.as<char>(oMedium), medium.data(), medium.size() * 4u);
     uint32_t *unit = pin.as<uint32_t>(oUnit), *prefix = pin.as<uint32_t>(oPrefix), *cols = pin.as<uint32_t>(oCols);
     prefix[0] = 0;
     for (uint32_t k = 0; k < count; ++k) {
@@ -629,8 +643,12 @@ int build_bricks_on_device(cute_hrpb_dev *d, const LargeWork &w)
     }
     pin.pending = true;
     CUTE_BUILD(cute_build::copy_words, grid_capped(tab.bytes / 4u), pin.as<const uint32_t>(), Layout::at<uint32_t>(mem.p, oTab), tab.bytes / 4u);
-    CUTE_BUILD_LDS(cute_build::panel_bricks, dim3(d->P), window_lds(d, (cute_build::kPanelCap + 1u) * 2u), d->dRowPtr, d->dCols, d->dCsrVals, d->P,
-                   d->nnz, max_span(d), table(oBrp), hdr, vals);
+    CUTE_PANELS(cute_build::panel_bricks<cute_build::kPanelFirst>, cute_build::kPanelFirst, d->P, window_lds(d, (cute_build::kPanelFirst + 1u) * 2u),
+                d->dRowPtr, d->dCols, d->dCsrVals, d->P, d->nnz, max_span(d), kAllPanels, table(oBrp), hdr, vals);
+    if (!medium.empty())
+        CUTE_PANELS(cute_build::panel_bricks<cute_build::kPanelCap>, cute_build::kPanelCap, uint32_t(medium.size()),
+                    window_lds(d, (cute_build::kPanelCap + 1u) * 2u), d->dRowPtr, d->dCols, d->dCsrVals, d->P, d->nnz, max_span(d), table(oMedium),
+                    table(oBrp), hdr, vals);
     if (count) {
         const uint32_t blocks = prefix[count];
         CUTE_BUILD(cute_build::large_clear, grid_of(uint64_t(blocks) * CUTE_TILED_HDR_WORDS), table(oUnit), table(oPrefix), count, uint32_t(CUTE_TILED_HDR_WORDS), hdr);
@@ -658,9 +676,7 @@ int build_quads_on_device(cute_hrpb_dev *d, const LargeWork &w)
     const uint64_t oGroup = tab.add(d->qgp.size(), 4), oBase = tab.add(uint64_t(d->P) + 1u, 4), oUnit = tab.add(count, 4),
                    oPrefix = tab.add(count + 1u, 4), oFirst = tab.add(uint64_t(count) * per, 4), oPairs = tab.add(uint64_t(count) * 4u, 4),
                    oLargeBase = tab.add(count, 4);
-    std::vector<uint32_t> medium;
-    for (uint32_t p = 0; p < d->P; ++p)
-        if (d->panelNnz[p] > cute_build::kPanelSmall && !panel_is_large(d, p)) medium.push_back(p);
+    const std::vector<uint32_t> medium = panels_between(d, cute_build::kPanelList);
     const uint64_t oMedium = tab.add(medium.size(), 4);
     const uint64_t oRecs = lay.add(G * CUTE_QUAD_RECORD_WORDS, 4), oVals = lay.add(stored + 64u, 4), oTab = lay.add(tab.bytes, 1);
     DevBuf mem, counts;
@@ -693,10 +709,10 @@ int build_quads_on_device(cute_hrpb_dev *d, const LargeWork &w)
     CUTE_BUILD(cute_build::copy_words, grid_capped(tab.bytes / 4u), pin.as<const uint32_t>(), Layout::at<uint32_t>(mem.p, oTab), tab.bytes / 4u);
     uint32_t *sums = counts.as<uint32_t>();
 #define CUTE_PANEL_QUADS(S, CAP, COUNT, LIST)                                                                                         \
-    CUTE_BUILD_LDS((cute_build::panel_quads<S, CAP>), dim3(COUNT), window_lds(d, CAP * 8u), d->dRowPtr, d->dCols, d->dCsrVals, d->P, d->nnz, \
-                   max_span(d), LIST, table(oGroup), table(oBase), uint32_t(stored), recs, packed)
+    CUTE_PANELS((cute_build::panel_quads<S, CAP>), CAP, COUNT, window_lds(d, CAP * 8u), d->dRowPtr, d->dCols, d->dCsrVals, d->P, d->nnz,  \
+                max_span(d), LIST, table(oGroup), table(oBase), uint32_t(stored), recs, packed)
 #define CUTE_BUILD_QUADS(S)                                                                                                           \
-    CUTE_PANEL_QUADS(S, cute_build::kPanelSmall, d->P, static_cast<const uint32_t *>(nullptr));                                         \
+    CUTE_PANEL_QUADS(S, cute_build::kPanelList, d->P, kAllPanels);                                                                      \
     if (!medium.empty()) CUTE_PANEL_QUADS(S, cute_build::kPanelCap, uint32_t(medium.size()), table(oMedium));                           \
     if (count) {                                                                                                                      \
         CUTE_BUILD(cute_build::large_clear, grid_of(uint64_t(groups) * CUTE_QUAD_RECORD_WORDS), table(oUnit), table(oPrefix), count,    \
@@ -797,10 +813,10 @@ int alloc_csr(cute_hrpb_dev *d)
     return CUTE_OK;
 }
 
-// Host arrays to the device through pinned memory, piece by piece: the calling thread fills a piece while a kernel reads
+// Host arrays to the device through pinned memory, piece by piece: the host threads fill a piece while a kernel reads
 // the one before.  When the buffer is full the stream is waited for and the buffer used again.
 struct HostToDevice {
-    static constexpr uint64_t kPiece = 1ull << 20;
+    static constexpr uint64_t kPiece = 2ull << 20;
     PinnedBuf pin;
     uint64_t used = 0;
     int begin(uint64_t bytes) { return pin.alloc(std::min<uint64_t>((bytes + kPiece - 1) / kPiece * kPiece + kPiece, 16ull << 20)); }
@@ -813,7 +829,7 @@ struct HostToDevice {
                 used = 0;
             }
             const uint64_t n = std::min(kPiece, bytes - at);
-            std::memcpy(pin.as<char>(used), static_cast<const char *>(src) + at, n);
+            parallel_ranges(n, 256u << 10, [&](uint64_t b, uint64_t e, unsigned) { std::memcpy(pin.as<char>(used + b), static_cast<const char *>(src) + at + b, e - b); });
             pin.pending = true;
             CUTE_BUILD(cute_build::copy_words, grid_capped(n / 4u), pin.as<const uint32_t>(used), Layout::at<uint32_t>(dst, at), n / 4u);
             used += (n + 255u) & ~uint64_t(255);
@@ -835,24 +851,38 @@ int finish_upload(cute_hrpb_dev *d, int quad_layout, const DeviceContext &c)
         int rc = pin.alloc(uint64_t(P) * sizeof(cute_build::PanelCensus));
         if (rc != CUTE_OK) return rc;
         pin.pending = true;
-        CUTE_BUILD_LDS(cute_build::panel_census, dim3(P), window_lds(d, 0), d->dRowPtr, d->dCols, d->dCsrVals, P, d->K, d->nnz, max_span(d), pin.as<cute_build::PanelCensus>());
+        CUTE_PANELS(cute_build::panel_census<cute_build::kPanelFirst>, cute_build::kPanelFirst, P, window_lds(d, 0), d->dRowPtr, d->dCols,
+                    d->dCsrVals, P, d->K, d->nnz, max_span(d), kAllPanels, pin.as<cute_build::PanelCensus>());
         rc = check_launch("panel census");
         if (rc == CUTE_OK) rc = pin.wait();
         if (rc != CUTE_OK) return rc;
         const cute_build::PanelCensus *r = pin.as<const cute_build::PanelCensus>();
         uint32_t error = 0;
-        bool any_large = false;
+        bool any_large = false, any_medium = false;
         d->panelNnz.resize(P);
         d->panelSpan.resize(P);
         for (uint32_t p = 0; p < P; ++p) {
             error |= r[p].error;
             d->panelNnz[p] = r[p].nnz;
             d->panelSpan[p] = r[p].span;
-            any_large = any_large || panel_is_large(d, p);
+            if (r[p].nnz > cute_build::kPanelFirst || r[p].span > max_span(d)) (panel_is_large(d, p) ? any_large : any_medium) = true;
         }
-        if (!error && any_large) {
-            rc = number_large_panels(d, large, pin.as<cute_build::PanelCensus>());
+        if (!error && (any_medium || any_large)) {
+            const std::vector<uint32_t> medium = panels_between(d, cute_build::kPanelFirst);
+            PinnedBuf list;
+            rc = list.alloc(medium.size() * 4u);
             if (rc != CUTE_OK) return rc;
+            list.pending = true;
+            if (!medium.empty()) {
+                std::memcpy(list.p, medium.data(), medium.size() * 4u);
+                CUTE_PANELS(cute_build::panel_census<cute_build::kPanelCap>, cute_build::kPanelCap, uint32_t(medium.size()), window_lds(d, 0),
+                            d->dRowPtr, d->dCols, d->dCsrVals, P, d->K, d->nnz, max_span(d), list.as<const uint32_t>(), pin.as<cute_build::PanelCensus>());
+                rc = check_launch("panel census");
+            }
+            if (rc == CUTE_OK && any_large) rc = number_large_panels(d, large, pin.as<cute_build::PanelCensus>());
+            if (rc == CUTE_OK) rc = list.wait();
+            if (rc != CUTE_OK) return rc;
+            for (uint32_t p : medium) error |= r[p].error;
             for (uint32_t p : large.panel) error |= r[p].error;
         }
         if (error & cute_build::kErrRange) return CUTE_ERR_RANGE;

@@ -1,4 +1,4 @@
-"""Panels at the edges of the device builders' kinds: a panel that one work-group holds in LDS (up to 1 024 and up to 2 048 entries,
+"""Panels at the edges of the device builders' kinds: a panel that one work-group holds in LDS (up to 1 024, 2 048 or 4 096 entries,
 a column window of up to 131 072), and the entry-parallel path beyond.  Both layouts must equal the host builders word for word,
 and every kind must report the same errors."""
 import numpy as np
@@ -35,7 +35,7 @@ def _panels(rng, K, sizes, spans=None, zeros=True):
 
 
 @pytest.mark.parametrize("quad_layout", [1, 2])
-@pytest.mark.parametrize("sizes", [(1, 0, 16, 255, 256, 257), (1023, 1024, 1025, 0, 3), (2047, 2048, 2049, 5), (0, 6000, 40, 2048, 3000, 0)])
+@pytest.mark.parametrize("sizes", [(1, 0, 16, 255, 256, 257), (1023, 1024, 1025, 0, 3), (2047, 2048, 2049, 5), (4095, 4096, 4097, 8), (0, 9000, 40, 2048, 3000, 0, 4096)])
 def test_entry_counts(cs, torch_cuda, sizes, quad_layout):
     K = 4096
     M, rp, cl, vl = _panels(np.random.default_rng(sum(sizes)), K, sizes)
@@ -54,7 +54,7 @@ def test_column_windows(cs, torch_cuda, quad_layout):
     _check_quads(cs, got, M, rp, cl, vl)
 
 
-@pytest.mark.parametrize("size,K", [(300, 4096), (3000, 4096), (300, 400000)])
+@pytest.mark.parametrize("size,K", [(300, 4096), (3000, 4096), (5000, 4096), (300, 400000)])
 def test_errors_of_every_kind(cs, torch_cuda, size, K):
     M, rp, cl, vl = _panels(np.random.default_rng(9), K, (40, size, 40), None, zeros=False)
     r = int(np.argmax(np.diff(rp[16:33].astype(np.int64)))) + 16          # a row of the middle panel
