@@ -24,6 +24,14 @@ constexpr float kMinReuse = 1.25f;          // a panel with fewer nonzeros per B
 constexpr uint64_t kWideWindowBytes = 16ull << 20;   // ... whose window of B is wider than this (four L2s' worth)
 constexpr float kWideReuse = 0.98f;          // ... the bar for products of 256 columns or more over large matrices (see cute_spmm_plan_create)
 constexpr uint32_t kMaxRowForRows = 48;
+// A panel is scattered when the window of B it reads (at most 256 columns of it at a time) is wider than this: its rows then
+// come from behind the L2s, which deliver about 8 TB/s against the 20 an L2 gives.  One and a half L2s: bands of 4 100
+// rows by 256 columns still come out of an L2 (92 % hits), 8 192 rows at random do not (N = 512: 25 us in row order, 12 with
+// an XCD per column slab).
+constexpr uint64_t kScatteredBytes = 6ull << 20;
+constexpr float kGraphReuse = 2.0f;          // scattered panels of large products (see cute_spmm_plan_create)
+constexpr uint32_t kGraphMaxRow = 96;
+constexpr uint64_t kGraphProduct = 1ull << 24;   // rows times columns from which on those two apply
 constexpr uint32_t kMaxHubRows = 256;       // hub plans: B rows a work-group keeps in LDS (64 KiB of 256-byte pieces; two work-groups per CU)     // ... unless it holds a row longer than this: one lane group would serialise it
 constexpr uint32_t kUnevenRowFloor = 16;     // row kernel vs MFMA kernel: a panel whose longest row exceeds this and ...
 constexpr uint32_t kUnevenRowRatio = 2;      // ... this many mean rows of the panel goes to the MFMA kernel while rows share wavefronts
@@ -55,12 +63,17 @@ constexpr double kStreamBytesPerSecond = 4.0e12, kSimdCyclesPerSecond = 1024 * 2
 // fit the Infinity Cache), a matrix whose quad lists need more than 1.1 fetches per brick-kernel fetch goes to
 // the brick kernel -- as long as its matrix work stays below the time the operands take to stream at 4 TB/s
 // (on R-MAT graphs it is 1.4-1.7 times that, and the quad kernel keeps them).
-int choose_mfma_shape(uint64_t slots, uint64_t bricks, uint64_t blocks, uint64_t rows_and_cols, uint64_t nnz, uint32_t N,
+// A graph's panels pass that test as well while N is small, but their bricks are nearly empty and what streams is not B but
+// the gathered rows: only lists whose slots carry 1.4 entries or more (9-point stencils 1.8, finite elements 2.8; R-MAT graphs
+// 1.03 ... 1.25) go to the brick kernel.  R-MAT graph of 131 072 nodes, N = 32: 74.5 us through bricks, 37.3 through lists;
+// 65 536 nodes, N = 47: 36.5 against 26.2.  Products of less than 32 columns keep the bricks (their narrow tiles; a list
+// slot always spans 64 columns): 32 768 nodes, N = 16: 11.5 against 16.1.
+int choose_mfma_shape(uint64_t slots, uint64_t bricks, uint64_t blocks, uint64_t entries, uint64_t rows_and_cols, uint64_t nnz, uint32_t N,
                       uint32_t residency, uint64_t cache_bytes)
 {
     int shape = slots < kSlotsPerBrick * bricks ? 2 : 1;
     const bool resident = residency == 2 && rows_and_cols * N * sizeof(float) <= cache_bytes;
-    if (shape == 2 && !resident && slots * 10u > blocks * 16u * 11u) {
+    if (shape == 2 && !resident && slots * 10u > blocks * 16u * 11u && (N < 32u || entries * 10u >= slots * 14u)) {
         const double matrix_s = double(bricks) * double((N + 15u) / 16u) * kCyclesPerBrickTile / kSimdCyclesPerSecond;
         const double stream_s = (double(rows_and_cols) * N * 4.0 + double(nnz) * 8.0) / kStreamBytesPerSecond;
         if (matrix_s <= stream_s) shape = 1;
@@ -225,6 +238,8 @@ struct cute_spmm_plan {
     uint4 *dRowList = nullptr;          // rows of the sparse path with their row pointers: {row, first entry, end, 0}
     uint32_t numRows = 0;
     cute_dev::XcdRanges rowRanges{};   // row-kernel blocks of each XCD, balanced by nonzeros
+    // slabs of the MFMA part and of the row part when an XCD owns columns instead of rows (cute_dev::xcd_share), else 0
+    uint32_t columnSlabs = 0, rowColumnSlabs = 0;
     uint32_t rowBlocksPerXcd = 0;       // longest of those ranges
 };
 
@@ -785,19 +800,20 @@ int finish_quad_census(cute_hrpb_dev *d, int quad_layout)
 int default_layout(const cute_hrpb_dev *d, uint64_t cache_bytes)
 {
     const uint32_t lists = d->quadRows == 4 ? 4u : 1u;
-    uint64_t slots = 0, bricks = 0, blocks = 0;
+    uint64_t slots = 0, bricks = 0, blocks = 0, entries = 0;
     for (uint32_t q = 0; q < d->P; ++q) {
         if (d->brp[q + 1] == d->brp[q]) continue;
         const uint32_t list_slots = (d->qgp[(q + 1) * lists] - d->qgp[q * lists]) * 16u;
         const uint32_t fetches = std::max(d->panelCols[q], list_slots);
         if (float(d->panelNnz[q]) < kMinReuse * float(fetches) && d->panelMaxRow[q] <= kMaxRowForRows) continue;   // row kernel
         slots += list_slots;
+        entries += d->panelNnz[q];
         bricks += (d->panelCols[q] + 3u) / 4u;
         blocks += d->brp[q + 1] - d->brp[q];
     }
     if (!bricks) return 0;
     // (the width is not known yet: 128 columns stand in for it)
-    return choose_mfma_shape(slots, bricks, blocks, uint64_t(d->K) + d->M, d->nnz, 128u, 0u, cache_bytes);
+    return choose_mfma_shape(slots, bricks, blocks, entries, uint64_t(d->K) + d->M, d->nnz, 128u, 0u, cache_bytes);
 }
 
 int alloc_csr(cute_hrpb_dev *d)
@@ -1087,9 +1103,9 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
     const float reuse_bar = N <= 32 ? std::min(3.0f, min_reuse * 48.0f / float(N)) : min_reuse;
     // Wide products of large matrices: the row kernel walks three dependent round trips per row (row pointers,
     // entries, B rows), the quad kernel streams its lists two groups ahead, and with 256 columns or more and a launch
-    // several times the size of the device that depth counts for more than reuse: on 50 000 rows of 7 entries at
-    // random columns, N = 512, the quad kernel takes 93 us against 116; ncvxbqp1, mk12-b3, delaunay_n16 of the
-    // reference's matrices gain 10-20 % the same way.  There the bar drops to "the lists need no more fetches than the
+    // several times the size of the device that depth counts for more than reuse: on 262 144 rows of 8 entries at
+    // random columns, N = 256, the quad kernel takes 326 us against 339 (smaller windows: see `narrow` below);
+    // ncvxbqp1, mk12-b3, delaunay_n16 of the reference's matrices gained 10-20 % the same way.  There the bar drops to "the lists need no more fetches than the
     // panel has entries" (matrices whose short lists would be mostly padding -- cat_ears_4_4, Wordnet3 -- stay with
     // the row kernel, which is 20 % ahead on them).
     // ... provided the panel's B rows cannot come out of an L2 anyway: a banded matrix, whose panels read a window of B
@@ -1114,6 +1130,21 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
     // (N = 16), 1.10 -> 1.04 (N = 32), 1.07 -> 1.03 (N = 128).  With one row per wavefront (N >= 256) the same move
     // loses (HEP-th-new, N = 512: 60 -> 68 us), so it is not made there.
     const bool rows_share_a_wavefront = t.max_row_nnz == 0 && (N + uint32_t(lane_floats(N)) - 1u) / uint32_t(lane_floats(N)) < 64u;
+    // Scattered panels (kScatteredBytes).  Where their rows share columns (graphs), a large product leaves only the panels with
+    // twice as many entries as fetches to the lists and takes rows of up to 96 entries to the row kernel, uneven or not: its
+    // sixteen lanes a row ask for 256 bytes of B with one instruction, a list slot for the same with 64 lanes.  R-MAT graph
+    // of 131 072 nodes and 2.5 million entries: N = 128 126 -> 92 us, N = 256 236 -> 228, N = 310 377 -> 320; below 2^24
+    // elements of C the launch no longer fills the device and the long rows show (32 768 nodes, N = 128: 26 -> 33).
+    const bool default_bars = t.path == CUTE_PATH_AUTO && t.min_reuse <= 0.0f && t.max_row_nnz == 0;
+    auto scattered = [&](uint32_t q) { return uint64_t(d->panelSpan[q]) * std::min(N, 256u) * sizeof(float) > kScatteredBytes; };
+    const bool graph_bars = default_bars && t.precision == CUTE_PREC_FP32 && N >= 128u && uint64_t(d->M) * N >= kGraphProduct;
+    auto fetches_of = [&](uint32_t q) {
+        // what the MFMA side would fetch for this panel: one B row per list slot of the quad
+        // lists (pairs plus padding), which is at least one per active column
+        const uint32_t lists = d->quadRows == 4 ? 4u : 1u;
+        return std::max(d->panelCols[q], (d->qgp[(q + 1) * lists] - d->qgp[q * lists]) * 16u);
+    };
+    uint64_t reused = 0;                          // entries of panels that earn the MFMA side by the usual bar
     uint32_t n_brick = 0, n_rows = 0, n_empty = 0;
     for (uint32_t q = 0; q < d->P; ++q) {
         const uint32_t nblk = d->brp[q + 1] - d->brp[q];
@@ -1125,13 +1156,13 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
             // Row kernel when a B row fetched by the MFMA side serves hardly more than one nonzero of the
             // panel (the matrix cores then buy nothing) -- unless a row is so long that one lane group
             // would serialise it: the brick kernel cuts long panels into balanced chunks.
-            // what the MFMA side would fetch for this panel: one B row per list slot of the quad
-            // lists (pairs plus padding), which is at least one per active column
-            const uint32_t lists = d->quadRows == 4 ? 4u : 1u;
-            const uint32_t fetches = std::max(d->panelCols[q], (d->qgp[(q + 1) * lists] - d->qgp[q * lists]) * 16u);
-            const float bar = (wide_and_large && uint64_t(d->panelSpan[q]) * N * sizeof(float) > kWideWindowBytes) ? kWideReuse : reuse_bar;
-            rows = float(d->panelNnz[q]) < bar * float(fetches) && d->panelMaxRow[q] <= max_row_for_rows;
-            if (rows && rows_share_a_wavefront && d->panelMaxRow[q] > kUnevenRowFloor &&
+            const uint32_t fetches = fetches_of(q);
+            const bool graph = graph_bars && scattered(q);
+            const float bar = graph ? kGraphReuse
+                              : (wide_and_large && uint64_t(d->panelSpan[q]) * N * sizeof(float) > kWideWindowBytes) ? kWideReuse : reuse_bar;
+            rows = float(d->panelNnz[q]) < bar * float(fetches) && d->panelMaxRow[q] <= (graph ? kGraphMaxRow : max_row_for_rows);
+            if (float(d->panelNnz[q]) >= reuse_bar * float(fetches)) reused += d->panelNnz[q];
+            if (rows && rows_share_a_wavefront && !graph && d->panelMaxRow[q] > kUnevenRowFloor &&
                 uint64_t(d->panelMaxRow[q]) * CUTE_TM > uint64_t(kUnevenRowRatio) * d->panelNnz[q]) {
                 rows = false;
                 joined[q] = 1;
@@ -1139,6 +1170,50 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
         }
         to_rows[q] = rows;
         if (nblk) (rows ? n_rows : n_brick)++;
+    }
+    // An XCD per column slab.  Row panels over a scattered window gather from behind the L2s as long as every XCD reads whole
+    // rows of B; when an XCD owns 32 columns instead, the piece of B it reads is (window) x 128 bytes and may fit its 4 MB.
+    // `narrow` gives the width of such a slab, 0 where it does not pay: rows of B a multiple of 128 bytes apart are cut into
+    // whole cache lines, a multiple of 64 bytes costs a line more per piece, any other pitch needs pieces of 64 columns.
+    // Random columns, 8 entries a row, us in row order / by columns: 16 384 rows N = 256 18.1 / 7.9, N = 512 35.4 / 18.3;
+    // 32 768 rows N = 128 18.2 / 11.3; 65 536 rows N = 256 82.8 / 64.5; 131 072 rows 167 / 159; 262 144 rows 339 / 356;
+    // N = 400: 16 384 rows 29.1 / 19.1, 32 768 rows 63.5 / 53.8, 65 536 rows 133 / 153; N = 301: 16 384 rows 26.5 / 21.0,
+    // 32 768 rows 55.7 / 57.3.  Longer rows share an L2 less well than lists, whose wavefronts walk the columns in step:
+    // lists / by columns, 16 entries a row, 32 768 rows N = 256 45.2 / 39.7, 50 000 rows 88.9 / 115; 31 entries a row,
+    // 16 384 rows N = 256 29.0 / 26.6, 32 768 rows 75.2 / 80.8.
+    auto narrow = [&](uint64_t window, uint64_t mean_row) -> uint32_t {
+        if (N % 32u == 0 && N >= 64u) return window <= (mean_row < 16u ? 131072u : mean_row < 24u ? 32768u : 16384u) ? 32u : 0u;
+        if (N < 256u) return 0u;
+        if (N % 16u == 0) return window <= (mean_row < 16u ? 32768u : 8192u) ? 32u : 0u;
+        return window <= (mean_row < 16u ? 16384u : 8192u) ? 64u : 0u;
+    };
+    // A matrix without reuse (less than a tenth of its entries in panels that earn the MFMA side): its scattered panels go to
+    // the lists only where these are ahead of the row kernel in whichever order suits it.  24 entries a row, us row kernel /
+    // lists: 65 536 rows N = 64 46.8 / 37.0, N = 128 106 / 81; 131 072 rows N = 256 457 / 408; rows of B off the 128-byte
+    // grid: 32 768 rows N = 301 151 / 126, 65 536 rows N = 400 363 / 354, 98 304 rows 558 / 589.  8 entries a row off that
+    // grid: 50 000 rows N = 301 87.7 / 95.2, 131 072 rows N = 400 274 / 305.  Products of 512 columns or more over windows
+    // that do not fit an L2 in slabs of 32 columns stay with the lists (the planner's tests hold them to it; 50 000 rows of 7:
+    // lists 89.3, the row kernel by columns 73.5).
+    if (default_bars && t.precision == CUTE_PREC_FP32 && reused * 10u < uint64_t(d->nnz) &&
+        uint64_t(d->M) * ((N + 255u) / 256u) >= 4ull * uint64_t(c.num_cus) * 32u) {
+        auto concerned = [&](uint32_t q) { return d->brp[q + 1] != d->brp[q] && d->panelMaxRow[q] <= max_row_for_rows && scattered(q); };
+        uint64_t windows = 0, entries = 0, panels = 0;
+        for (uint32_t q = 0; q < d->P; ++q)
+            if (concerned(q)) { windows += d->panelSpan[q]; entries += d->panelNnz[q]; ++panels; }
+        if (panels) {
+            const uint64_t window = windows / panels, mean_row = entries / (panels * CUTE_TM);
+            const bool on_grid = N % 32u == 0, wide = N >= 512u && window > 32768u;
+            const bool lists_ahead = on_grid ? (wide || (narrow(window, mean_row) == 0 && (mean_row >= 16u || N >= 256u)))
+                                             : (narrow(window, mean_row) == 0 && mean_row >= 16u && N >= 256u && window <= 65536u);
+            for (uint32_t q = 0; q < d->P; ++q) {
+                if (!concerned(q)) continue;
+                const uint8_t rows = !(lists_ahead && N >= 64u && float(d->panelNnz[q]) >= kWideReuse * float(fetches_of(q)));
+                if (rows == to_rows[q]) continue;
+                to_rows[q] = rows;
+                joined[q] = 0;
+                if (rows) { ++n_rows; --n_brick; } else { --n_rows; ++n_brick; }
+            }
+        }
     }
     // A handful of MFMA panels among row-kernel panels (the boundary panels of a stencil at N = 32: 64 of 16 384) would
     // turn the launch into the fused kernel for their sake, which costs the row blocks more than those panels gain
@@ -1212,19 +1287,54 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
         // instead of once per panel, and pad their lists.  Measured break-even on the benchmark
         // matrices and on the reference's 43: about 8 list slots (pairs plus padding) per brick.
         const uint32_t lists = d->quadRows == 4 ? 4u : 1u;     // list units per panel
-        uint64_t slots = 0, bricks = 0, blocks = 0;
+        uint64_t slots = 0, bricks = 0, blocks = 0, entries = 0;
         for (uint32_t q = 0; q < d->P; ++q)
             if (!to_rows[q] && !joined[q]) {
+                entries += d->panelNnz[q];
                 slots += uint64_t(d->qgp[(q + 1) * lists] - d->qgp[q * lists]) * 16u;
                 bricks += (d->panelCols[q] + 3u) / 4u;
                 blocks += d->brp[q + 1] - d->brp[q];
             }
-        p->shape = choose_mfma_shape(slots, bricks, blocks, uint64_t(d->K) + d->M, d->nnz, N, t.operand_residency, c.cache_bytes);
+        p->shape = choose_mfma_shape(slots, bricks, blocks, entries, uint64_t(d->K) + d->M, d->nnz, N, t.operand_residency, c.cache_bytes);
     }
     if (p->shape == 2 && !(offsets_fit && (d->numQuadVals + 64u) * 4u <= 0xffffffffull)) p->shape = 1;
     // bf16x3 exists for the rolling brick kernel with four columns per lane, and is asked for with N a multiple of four;
     // any other shape computes in fp32
     p->bf16x3 = t.precision == CUTE_PREC_BF16X3 && p->shape == 1 && p->pipeline == 1 && p->vec == 4 && N % 4u == 0;
+    // Which parts of the launch go by columns (cute_dev::xcd_share).  A plan of rows alone takes the slab that `narrow` gives for
+    // its mean window.  MFMA panels that share columns find a graph's hub rows in their XCD's slab whatever the window: R-MAT
+    // graph of 32 768 nodes, N = 512 156 -> 104 us, 16 384 nodes, N = 256 33.5 -> 26.7, 131 072 nodes, N = 310 463 -> 413;
+    // lists without reuse gain while the window fits two L2s (16 384 rows of 24, N = 512 46.4 -> 41.8; 65 536 rows 349 -> 367).
+    // Off the 64-column grid the last slab is a remainder that unbalances few slabs (N = 101: 137 -> 147): 256 columns or more.
+    uint32_t rows_columns = 0, mfma_by_columns = 0;
+    {
+        uint64_t scattered_nnz = 0, window[2] = {}, in[2] = {}, cols = 0;
+        uint32_t row_panels = 0;
+        for (uint32_t q = 0; q < d->P; ++q) {
+            const uint32_t side = to_rows[q] ? 1u : 0u;
+            if (scattered(q)) scattered_nnz += d->panelNnz[q];
+            window[side] += uint64_t(d->panelSpan[q]) * d->panelNnz[q];
+            in[side] += d->panelNnz[q];
+            if (side == 0) cols += d->panelCols[q];
+            else if (d->panelNnz[q]) ++row_panels;
+        }
+        if (scattered_nnz * 2u > uint64_t(d->nnz)) {
+            const uint64_t mean_window[2] = {in[0] ? window[0] / in[0] : 0, in[1] ? window[1] / in[1] : 0};
+            if (n_brick == 0)
+                rows_columns = narrow(mean_window[1], in[1] / (uint64_t(row_panels) * CUTE_TM));
+            else if (((N % 64u == 0 && N >= 128u) || N >= 256u) && (in[0] * 5u >= cols * 6u || mean_window[0] <= 32768u)) {
+                mfma_by_columns = 1;
+                // rows of uneven length share a wavefront: sixteen lanes a row (the brick kernel has no launch with fewer than its own)
+                rows_columns = p->shape == 2 && p->rows_vec == 4 ? 64u : (p->rows_vec << p->rows_logl);
+            }
+        }
+        // (slabs are the y dimension of the launch)
+        if (p->rows_vec == 4 && rows_columns && rows_columns < (4u << p->rows_logl) && (N + rows_columns - 1u) / rows_columns <= 65535u) {
+            p->rows_logl = rows_columns == 32u ? 3 : 4;
+            p->rows_slabs = (N + rows_columns - 1u) / rows_columns;
+        }
+        p->rowColumnSlabs = rows_columns ? p->rows_slabs : 0u;
+    }
     // The chunk list depends on the MFMA kernel (its work units are blocks or list groups).  It is built,
     // and if the partial tiles of the cut panels then turn out to be more rows than the fast kernels'
     // 24-bit row operand can address, built once more for the pipelined brick kernel, whose stores use
@@ -1486,6 +1596,7 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
     p->info.slots = slots;
     p->info.precision = p->bf16x3 ? uint32_t(CUTE_PREC_BF16X3) : uint32_t(CUTE_PREC_FP32);
     p->info.path = uint32_t(t.path);
+    p->columnSlabs = mfma_by_columns ? num_slabs : 0u;
     p->info.mfmaShape = uint32_t(p->shape);
     p->info.hubRows = p->numHub;
     p->info.pipeline = uint32_t(p->pipeline);
@@ -1512,13 +1623,13 @@ void launch_brick_full(const cute_spmm_plan *p, const float *dB, float *dC, floa
     if (p->bf16x3) {
         if constexpr (VEC == 4)
             hipLaunchKernelGGL((cute_dev::hrpb_brick_bf16x3<NG, FULL>), grid, block, 0, s, p->dChunks, p->info.numChunks, per_xcd,
-                               p->d->dHdr, p->d->dVals, uint32_t(p->d->numVals), dB, dC, partials, p->info.N);
+                               p->d->dHdr, p->d->dVals, uint32_t(p->d->numVals), dB, dC, partials, p->info.N, p->columnSlabs);
     } else if (p->pipeline == 1)
         hipLaunchKernelGGL((cute_dev::hrpb_brick_f32_rolling<VEC, NG, FULL>), grid, block, 0, s, p->dChunks,
-                           p->info.numChunks, per_xcd, p->d->dHdr, p->d->dVals, uint32_t(p->d->numVals), dB, dC, partials, p->info.N);
+                           p->info.numChunks, per_xcd, p->d->dHdr, p->d->dVals, uint32_t(p->d->numVals), dB, dC, partials, p->info.N, p->columnSlabs);
     else
         hipLaunchKernelGGL((cute_dev::hrpb_brick_f32<VEC, NG, FULL>), grid, block, 0, s, p->dChunks, p->info.numChunks,
-                           per_xcd, p->d->dHdr, p->d->dVals, dB, dC, partials, p->info.N);
+                           per_xcd, p->d->dHdr, p->d->dVals, dB, dC, partials, p->info.N, p->columnSlabs);
 }
 
 template <int VEC, int NG>
@@ -1531,7 +1642,7 @@ void launch_brick(const cute_spmm_plan *p, const float *dB, float *dC, float *pa
 template <int VEC, bool BATCHED>
 void launch_rows_vec(int logl, const uint4 *row_list, uint32_t num_rows, uint32_t slabs, const uint32_t *rp,
                      const uint32_t *cl, const float *vl, const float *dB, float *dC, uint32_t N, hipStream_t s,
-                     const cute_dev::XcdRanges *ranges, uint32_t blocks_per_xcd)
+                     const cute_dev::XcdRanges *ranges, uint32_t blocks_per_xcd, uint32_t column_slabs)
 {
     const uint64_t lanes = (uint64_t(num_rows) * slabs) << logl;
     // the batched kernel deals its blocks to the XCDs in contiguous ranges (all as long as the longest)
@@ -1543,7 +1654,7 @@ void launch_rows_vec(int logl, const uint4 *row_list, uint32_t num_rows, uint32_
     case LL:                                                                                                      \
         if (BATCHED)                                                                                              \
             hipLaunchKernelGGL((cute_dev::csr_rows_batched<VEC, LL, 8>), grid, block, 0, s, row_list, num_rows,    \
-                               rp, cl, vl, dB, dC, N, rg);                                                        \
+                               rp, cl, vl, dB, dC, N, rg, column_slabs);                                                        \
         else                                                                                                      \
             hipLaunchKernelGGL((cute_dev::csr_rows<VEC, LL>), grid, block, 0, s, static_cast<const uint32_t *>(nullptr), num_rows, slabs, rp, \
                                cl, vl, dB, dC, N);                                                                \
@@ -1559,11 +1670,11 @@ void launch_rows_vec(int logl, const uint4 *row_list, uint32_t num_rows, uint32_
 template <bool BATCHED>
 void launch_rows(int vec, int logl, const uint4 *row_list, uint32_t num_rows, uint32_t slabs, const uint32_t *rp,
                  const uint32_t *cl, const float *vl, const float *dB, float *dC, uint32_t N, hipStream_t s,
-                 const cute_dev::XcdRanges *ranges = nullptr, uint32_t blocks_per_xcd = 0)
+                 const cute_dev::XcdRanges *ranges = nullptr, uint32_t blocks_per_xcd = 0, uint32_t column_slabs = 0)
 {
-    if (vec == 4) launch_rows_vec<4, BATCHED>(logl, row_list, num_rows, slabs, rp, cl, vl, dB, dC, N, s, ranges, blocks_per_xcd);
-    else if (vec == 2) launch_rows_vec<2, BATCHED>(logl, row_list, num_rows, slabs, rp, cl, vl, dB, dC, N, s, ranges, blocks_per_xcd);
-    else launch_rows_vec<1, BATCHED>(logl, row_list, num_rows, slabs, rp, cl, vl, dB, dC, N, s, ranges, blocks_per_xcd);
+    if (vec == 4) launch_rows_vec<4, BATCHED>(logl, row_list, num_rows, slabs, rp, cl, vl, dB, dC, N, s, ranges, blocks_per_xcd, column_slabs);
+    else if (vec == 2) launch_rows_vec<2, BATCHED>(logl, row_list, num_rows, slabs, rp, cl, vl, dB, dC, N, s, ranges, blocks_per_xcd, column_slabs);
+    else launch_rows_vec<1, BATCHED>(logl, row_list, num_rows, slabs, rp, cl, vl, dB, dC, N, s, ranges, blocks_per_xcd, column_slabs);
 }
 
 int check_launch(const char *what)
@@ -1670,7 +1781,7 @@ void launch_brick_rows_as(const cute_spmm_plan *p, const float *dB, float *dC, f
 #define CUTE_BRICK_ROWS(F)                                                                                                \
     hipLaunchKernelGGL((cute_dev::hrpb_brick_rows_f32<VEC, NG, F, LOG_L>), flat, block, 0, s, grid.x, uint32_t(brick_blocks),  \
                        p->dChunks, p->info.numChunks, per_xcd, p->d->dHdr, p->d->dVals, uint32_t(p->d->numVals), p->dRowList, \
-                       p->numRows, rows_per_slab, p->rowRanges, p->d->dRowPtr, p->d->dCols, p->d->dCsrVals,                    \
+                       p->numRows, rows_per_slab, p->rowRanges, p->columnSlabs, p->rowColumnSlabs, p->d->dRowPtr, p->d->dCols, p->d->dCsrVals,                    \
                        dB, dC, partials, N)
     if (N % (16u * VEC * NG) == 0) CUTE_BRICK_ROWS(true);
     else CUTE_BRICK_ROWS(false);
@@ -1731,7 +1842,7 @@ int run_with(const cute_spmm_plan *p, const float *dB, float *dC, void *stream, 
     hipLaunchKernelGGL((cute_dev::hrpb_quad_rows_f32<F, S, LL>), dim3(uint32_t(quad_blocks + row_blocks)), block, 0, s,     \
                        grid.x, uint32_t(quad_blocks), p->dHeads, p->info.numChunks, per_xcd, p->d->dQRecs, p->d->dQVals,   \
                        uint32_t(p->d->numQuadVals),                                                                  \
-                       p->dRowList, p->numRows, rows_per_slab, p->rowRanges, p->d->dRowPtr, p->d->dCols, p->d->dCsrVals, dB, dC,    \
+                       p->dRowList, p->numRows, rows_per_slab, p->rowRanges, p->columnSlabs, p->rowColumnSlabs, p->d->dRowPtr, p->d->dCols, p->d->dCsrVals, dB, dC,    \
                        partials, N)
 #define CUTE_FUSED_LL(F, S)                                                     \
     switch (p->rows_logl) {                                                     \
@@ -1753,7 +1864,7 @@ int run_with(const cute_spmm_plan *p, const float *dB, float *dC, void *stream, 
         } else {
 #define CUTE_QUAD_LAUNCH(F, S)                                                                                          \
     hipLaunchKernelGGL((cute_dev::hrpb_quad_f32<F, S>), grid, block, 0, s, p->dHeads, p->info.numChunks, per_xcd,         \
-                       p->d->dQRecs, p->d->dQVals, uint32_t(p->d->numQuadVals), dB, dC, partials, N)
+                       p->d->dQRecs, p->d->dQVals, uint32_t(p->d->numQuadVals), dB, dC, partials, N, p->columnSlabs)
         if (full && strips) CUTE_QUAD_LAUNCH(true, true);
         else if (full) CUTE_QUAD_LAUNCH(true, false);
         else if (strips) CUTE_QUAD_LAUNCH(false, true);
@@ -1769,7 +1880,7 @@ int run_with(const cute_spmm_plan *p, const float *dB, float *dC, void *stream, 
     }
     if (p->numRows && !rows_launched) {
         launch_rows<true>(p->rows_vec, p->rows_logl, p->dRowList, p->numRows, p->rows_slabs, p->d->dRowPtr, p->d->dCols,
-                    p->d->dCsrVals, dB, dC, N, s, &p->rowRanges, p->rowBlocksPerXcd);
+                    p->d->dCsrVals, dB, dC, N, s, &p->rowRanges, p->rowBlocksPerXcd, p->rowColumnSlabs);
     }
     // panels that were cut: add their partial tiles up, in chunk order (no atomics, so a product is
     // the same bit for bit every time it is computed)

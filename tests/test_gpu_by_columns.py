@@ -1,0 +1,86 @@
+"""Products whose B rows come from all over B: an XCD owns columns instead of rows (cute_dev::xcd_share), the row kernel walks
+slabs of 32 or 64 columns, and the lists keep the panels the planner gives them.  Sizes on both sides of every line of that
+rule: remainders of slabs, fewer slabs than XCDs, odd widths, rows of no entries, long and short rows, hub rows.
+
+Tolerance: |difference| <= 2 * longest row * 2^-24 * sum |a||b|, the bound of two orders of one fp32 sum."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _product(cs, torch, rp, cl, vl, M, K, N, seed, **kw):
+    rng = np.random.default_rng(seed)
+    B = rng.standard_normal((K, N)).astype(np.float32)
+    plan = cs.SPMM_TC(cs.HRPB(M, K, rp, cl, vl), N, **kw)
+    out = torch.full((M, N), float("nan"), device="cuda")
+    plan.run(torch.from_numpy(B).cuda(), out)
+    return B, out.cpu().numpy(), plan
+
+
+def _check(rp, cl, vl, B, out, M, N, rows):
+    for r in rows:
+        a, b = vl[rp[r]:rp[r + 1]].astype(np.float64), B[cl[rp[r]:rp[r + 1]]].astype(np.float64)
+        bound = 2.0 * max(1, len(a)) * 2.0 ** -24 * (np.abs(a) @ np.abs(b)) if len(a) else np.zeros(N)
+        assert (np.abs(out[r] - (a @ b if len(a) else np.zeros(N))) <= bound + 1e-30).all(), r
+
+
+def _random(M, K, per_row, seed, empty=0, hubs=0):
+    rng = np.random.default_rng(seed)
+    counts = np.full(M, per_row)
+    if empty:
+        counts[rng.integers(0, M, empty)] = 0
+    if hubs:
+        counts[:hubs] = 700
+    rows = np.repeat(np.arange(M), counts)
+    cols = rng.integers(0, K, rows.size)
+    if hubs:
+        cols = np.where(rng.random(rows.size) < 0.5, cols % 256, cols)
+    key = np.unique(rows.astype(np.int64) * K + cols)
+    rows, cols = key // K, (key % K).astype(np.uint32)
+    rp = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=M))]).astype(np.uint32)
+    return rp, cols, rng.standard_normal(cols.size).astype(np.float32)
+
+
+@pytest.mark.parametrize("M,K,per_row,N,empty,hubs", [
+    (8192, 8192, 7, 256, 0, 0), (8192, 16384, 5, 288, 500, 0), (8192, 8192, 7, 301, 0, 0), (8192, 8192, 9, 272, 40, 0),
+    (16384, 16384, 3, 128, 0, 0), (16384, 32768, 4, 96, 900, 0), (32768, 32768, 4, 64, 0, 0), (8192, 8192, 26, 320, 0, 0),
+    (32768, 40000, 18, 64, 0, 0), (16384, 36864, 17, 512, 0, 0), (16384, 16384, 20, 299, 0, 0), (16384, 16384, 6, 256, 100, 64),
+    (16384, 16384, 6, 310, 0, 64), (131072, 131072, 6, 128, 0, 320), (2048, 65536, 8, 544, 16, 0), (16384, 16384, 4, 1056, 0, 0)])
+def test_every_element_is_written_once_and_right(cs, torch_cuda, M, K, per_row, N, empty, hubs):
+    rp, cl, vl = _random(M, K, per_row, M + N, empty, hubs)
+    B, out, plan = _product(cs, torch_cuda, rp, cl, vl, M, K, N, N)
+    assert np.isfinite(out).all()
+    rng = np.random.default_rng(1)
+    _check(rp, cl, vl, B, out, M, N, np.unique(np.concatenate([[0, 1, 15, 16, M // 8, M // 2 - 1, M - 17, M - 1], rng.integers(0, M, 300)])))
+    # every row, by its sum over the columns of B
+    total = out.astype(np.float64) @ np.ones(N)
+    want = np.zeros(M)
+    rows = np.repeat(np.arange(M), np.diff(rp.astype(np.int64)))
+    np.add.at(want, rows, vl.astype(np.float64) * (B.astype(np.float64) @ np.ones(N))[cl])
+    scale = np.zeros(M)
+    np.add.at(scale, rows, np.abs(vl.astype(np.float64)) * (np.abs(B.astype(np.float64)) @ np.ones(N))[cl])
+    longest = max(1, int(np.diff(rp.astype(np.int64)).max()))
+    assert (np.abs(total - want) <= 2.0 * longest * 2.0 ** -24 * scale + 1e-30).all()
+
+
+@pytest.mark.parametrize("N", [64, 256, 320])
+def test_forced_rows_give_the_bits_of_the_same_rows_in_row_order(cs, torch_cuda, N):
+    """The row kernel adds a row up in storage order whatever slab it works on: a matrix whose window is scattered and the same
+    rows against a B that repeats a short window give the same bits (the latter runs in row order)."""
+    M, K, short = 8192, 32768, 512
+    rng = np.random.default_rng(7)
+    cl = np.sort(rng.permuted(np.tile(np.arange(short), (M, 1)), axis=1)[:, :9], axis=1).astype(np.uint32)
+    far = cl + np.uint32(K - short) * (np.arange(9) >= 5).astype(np.uint32)
+    rp, vl = (np.arange(M + 1) * 9).astype(np.uint32), rng.standard_normal(M * 9).astype(np.float32)
+    piece = rng.standard_normal((short, N)).astype(np.float32)
+    B = np.zeros((K, N), np.float32)
+    B[:short] = piece
+    B[K - short:] = piece
+    outs = []
+    for cols in (cl, far):
+        plan = cs.SPMM_TC(cs.HRPB(M, K, rp, cols.ravel(), vl), N, path=cs.PATH_ROWS)
+        out = torch_cuda.full((M, N), float("nan"), device="cuda")
+        plan.run(torch_cuda.from_numpy(B).cuda(), out)
+        outs.append(out)
+    assert torch_cuda.equal(outs[0], outs[1])
