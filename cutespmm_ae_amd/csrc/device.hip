@@ -24,6 +24,7 @@ constexpr float kMinReuse = 1.25f;          // a panel with fewer nonzeros per B
 constexpr uint64_t kWideWindowBytes = 16ull << 20;   // ... whose window of B is wider than this (four L2s' worth)
 constexpr float kWideReuse = 0.98f;          // ... the bar for products of 256 columns or more over large matrices (see cute_spmm_plan_create)
 constexpr uint32_t kMaxRowForRows = 48;
+constexpr uint32_t kRowBatch = 8;           // entries the row kernel has in flight per row
 // A panel is scattered when the window of B it reads (at most 256 columns of it at a time) is wider than this: its rows then
 // come from behind the L2s, which deliver about 8 TB/s against the 20 an L2 gives.  One and a half L2s: bands of 4 100
 // rows by 256 columns still come out of an L2 (92 % hits), 8 192 rows at random do not (N = 512: 25 us in row order, 12 with
@@ -819,7 +820,8 @@ int default_layout(const cute_hrpb_dev *d, uint64_t cache_bytes)
 int alloc_csr(cute_hrpb_dev *d)
 {
     Layout lay;
-    const uint64_t oRow = lay.add(uint64_t(d->M) + 1u, 4), oCols = lay.add(d->nnz, 4), oVals = lay.add(d->nnz, 4);
+    const uint64_t oRow = lay.add(uint64_t(d->M) + 1u, 4), oCols = lay.add(uint64_t(d->nnz) + kRowBatch, 4),
+                   oVals = lay.add(uint64_t(d->nnz) + kRowBatch, 4);     // the row kernel reads whole batches
     const int rc = pool().take(&d->csrMemory, lay.bytes);
     if (rc != CUTE_OK) return rc;
     d->dRowPtr = Layout::at<uint32_t>(d->csrMemory, oRow);
@@ -1653,7 +1655,7 @@ void launch_rows_vec(int logl, const uint4 *row_list, uint32_t num_rows, uint32_
 #define CUTE_ROWS_CASE(LL)                                                                                        \
     case LL:                                                                                                      \
         if (BATCHED)                                                                                              \
-            hipLaunchKernelGGL((cute_dev::csr_rows_batched<VEC, LL, 8>), grid, block, 0, s, row_list, num_rows,    \
+            hipLaunchKernelGGL((cute_dev::csr_rows_batched<VEC, LL, kRowBatch>), grid, block, 0, s, row_list, num_rows,    \
                                rp, cl, vl, dB, dC, N, rg, column_slabs);                                                        \
         else                                                                                                      \
             hipLaunchKernelGGL((cute_dev::csr_rows<VEC, LL>), grid, block, 0, s, static_cast<const uint32_t *>(nullptr), num_rows, slabs, rp, \
