@@ -1146,7 +1146,7 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
         const uint32_t lists = d->quadRows == 4 ? 4u : 1u;
         return std::max(d->panelCols[q], (d->qgp[(q + 1) * lists] - d->qgp[q * lists]) * 16u);
     };
-    uint64_t reused = 0;                          // entries of panels that earn the MFMA side by the usual bar
+    uint64_t reused = 0;                          // entries of panels that go to the MFMA side by the usual bars: reuse, long or uneven rows
     uint32_t n_brick = 0, n_rows = 0, n_empty = 0;
     for (uint32_t q = 0; q < d->P; ++q) {
         const uint32_t nblk = d->brp[q + 1] - d->brp[q];
@@ -1163,9 +1163,10 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
             const float bar = graph ? kGraphReuse
                               : (wide_and_large && uint64_t(d->panelSpan[q]) * N * sizeof(float) > kWideWindowBytes) ? kWideReuse : reuse_bar;
             rows = float(d->panelNnz[q]) < bar * float(fetches) && d->panelMaxRow[q] <= (graph ? kGraphMaxRow : max_row_for_rows);
-            if (float(d->panelNnz[q]) >= reuse_bar * float(fetches)) reused += d->panelNnz[q];
-            if (rows && rows_share_a_wavefront && !graph && d->panelMaxRow[q] > kUnevenRowFloor &&
-                uint64_t(d->panelMaxRow[q]) * CUTE_TM > uint64_t(kUnevenRowRatio) * d->panelNnz[q]) {
+            const bool uneven = rows_share_a_wavefront && d->panelMaxRow[q] > kUnevenRowFloor &&
+                                uint64_t(d->panelMaxRow[q]) * CUTE_TM > uint64_t(kUnevenRowRatio) * d->panelNnz[q];
+            if (uneven || d->panelMaxRow[q] > max_row_for_rows || float(d->panelNnz[q]) >= reuse_bar * float(fetches)) reused += d->panelNnz[q];
+            if (rows && uneven && !graph) {
                 rows = false;
                 joined[q] = 1;
             }
@@ -1189,7 +1190,7 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
         if (N % 16u == 0) return window <= (mean_row < 16u ? 32768u : 8192u) ? 32u : 0u;
         return window <= (mean_row < 16u ? 16384u : 8192u) ? 64u : 0u;
     };
-    // A matrix without reuse (less than a tenth of its entries in panels that earn the MFMA side): its scattered panels go to
+    // A matrix without reuse or hubs (less than a tenth of its entries in panels for the MFMA side): its scattered panels go to
     // the lists only where these are ahead of the row kernel in whichever order suits it.  24 entries a row, us row kernel /
     // lists: 65 536 rows N = 64 46.8 / 37.0, N = 128 106 / 81; 131 072 rows N = 256 457 / 408; rows of B off the 128-byte
     // grid: 32 768 rows N = 301 151 / 126, 65 536 rows N = 400 363 / 354, 98 304 rows 558 / 589.  8 entries a row off that

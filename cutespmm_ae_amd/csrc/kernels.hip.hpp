@@ -1021,7 +1021,10 @@ __global__ __launch_bounds__(256) void csr_rows(const uint32_t *__restrict__ row
 // row are consumed in batches whose B-row loads are all issued before the first FMA, so a
 // row costs about one memory round trip per batch instead of one per nonzero.  Each C
 // element still accumulates its row in storage order.
-template <int VEC, int LOG_L, int BATCH>
+// AHEAD: the entries of the next round are asked for ahead of this round's B rows (loads return in order), so a row longer than
+// a round waits for one round trip per round, not for two (131 072 rows of 20, N = 64: 93.2 -> 89.4 us).  The fused kernels
+// leave that out where the entries take several registers: their 64 would not do.
+template <int VEC, int LOG_L, int BATCH, bool AHEAD>
 __device__ __forceinline__ void rows_batched_body(uint32_t block_id, uint32_t slab, const uint4 *__restrict__ row_list,
                                                   uint32_t num_rows, const uint32_t *__restrict__ rowPtr,
                                                   const uint32_t *__restrict__ cols, const float *__restrict__ vals,
@@ -1070,9 +1073,7 @@ __device__ __forceinline__ void rows_batched_body(uint32_t block_id, uint32_t sl
     Entries mine, next;
     fetch(s, mine);
     for (uint32_t base = s; base < e; base += ROUND) {
-        // the entries of the next round are asked for ahead of this round's B rows (loads return in order), so a row
-        // longer than a round waits for one round trip per round, not for two
-        fetch(base + ROUND, next);
+        if (AHEAD) fetch(base + ROUND, next);
         const uint32_t cnt = min(ROUND, e - base);
         for (uint32_t q0 = 0; q0 < cnt; q0 += STEP) {
             V b[STEP];
@@ -1090,7 +1091,8 @@ __device__ __forceinline__ void rows_batched_body(uint32_t block_id, uint32_t sl
 #pragma unroll
             for (uint32_t u = 0; u < STEP; ++u) acc += a[u] * b[u];
         }
-        mine = next;
+        if (AHEAD) mine = next;
+        else if (base + ROUND < e) fetch(base + ROUND, mine);
     }
     if (live) store_vec_streaming<VEC>(acc, C + size_t(row) * N + c0);
 }
@@ -1109,7 +1111,7 @@ __global__ __launch_bounds__(256) void csr_rows_batched(const uint4 *__restrict_
     uint32_t block_id, slab = blockIdx.y;
     const uint32_t x = xcd_share(blockIdx.x, slab, column_slabs);
     if (!xcd_range_id(ranges, blockIdx.x, x, block_id)) return;
-    rows_batched_body<VEC, LOG_L, BATCH>(block_id, slab, row_list, num_rows, rowPtr, cols, vals, B, C, N);
+    rows_batched_body<VEC, LOG_L, BATCH, true>(block_id, slab, row_list, num_rows, rowPtr, cols, vals, B, C, N);
 }
 
 // One launch for a plan that uses both the quad kernel and the row kernel: they write disjoint
@@ -1136,7 +1138,7 @@ __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, 8) void hrpb_quad_rows_f
         uint32_t block_id;
         const uint32_t x = xcd_share(bid, slab, row_column_slabs);
         if (!xcd_range_id(row_ranges, bid, x, block_id)) return;
-        rows_batched_body<4, LOG_L, 8>(block_id, slab, row_list, num_rows, rowPtr, cols, vals, B, C, N);
+        rows_batched_body<4, LOG_L, 8, (LOG_L > 3)>(block_id, slab, row_list, num_rows, rowPtr, cols, vals, B, C, N);
     }
 }
 
@@ -1159,7 +1161,7 @@ __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, (NG == 1 ? 8 : 4)) void 
         uint32_t block_id;
         const uint32_t x = xcd_share(bid, slab, row_column_slabs);
         if (!xcd_range_id(row_ranges, bid, x, block_id)) return;
-        rows_batched_body<4, LOG_L, 8>(block_id, slab, row_list, num_rows, rowPtr, cols, vals, B, C, N);
+        rows_batched_body<4, LOG_L, 8, (LOG_L > 3)>(block_id, slab, row_list, num_rows, rowPtr, cols, vals, B, C, N);
     }
 }
 
