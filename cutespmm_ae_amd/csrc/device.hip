@@ -1304,6 +1304,27 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
     // bf16x3 exists for the rolling brick kernel with four columns per lane, and is asked for with N a multiple of four;
     // any other shape computes in fp32
     p->bf16x3 = t.precision == CUTE_PREC_BF16X3 && p->shape == 1 && p->pipeline == 1 && p->vec == 4 && N % 4u == 0;
+    // The brick kernel's slab follows the number of work items as well.  A wavefront walks its panel alone, 32 matrix cycles per
+    // brick and 16 columns, so a launch that leaves SIMDs without a wavefront, or gives some of them one more than the others,
+    // takes (fullest SIMD's wavefronts) x (slab): with T(w) = ceil(items / SIMDs) x w for slabs of 16 w columns, the narrower
+    // slab is taken where T falls.  Narrower pieces of a B row cost more requests per byte, which shows once two or three
+    // wavefronts a SIMD are running: the limits.  Finite-element matrices, us at the slab named, 128 / 64 / 32 / 16 columns:
+    // 24 000 rows N = 128 20.1 / 15.7 / 23.8 / 32.8, N = 256 26.3 / 26.4 (equal T), N = 301 47.0 / 36.4; 2 400 rows N = 128
+    // 19.0 / 13.2 / 10.6 / 10.5, N = 301 19.4 / 13.6 / 13.6 / 11.4; 4 800 rows N = 64 - / 10.7 / 8.1 / 8.5, N = 200
+    // 16.7 / 13.9 / 15.9 / 14.9.  (Odd N gains from single columns a little longer: no other piece of its rows is aligned.)
+    if (p->shape == 1 && p->pipeline == 1 && t.brick_groups == 0 && n_brick) {
+        const uint64_t simds = uint64_t(c.num_cus) * 4u;
+        auto items = [&](uint32_t w) { return uint64_t(n_brick) * ((N + 16u * w - 1u) / (16u * w)); };
+        auto T = [&](uint32_t w) { return (items(w) + simds - 1u) / simds * w; };
+        if (p->ng == 2 && items(4) <= 8u * simds && (T(4) < T(8) || items(8) <= simds)) {
+            p->ng = 1;
+            ng_for_mixed = true;                  // (the fused launch has this shape)
+        }
+        const bool alone = n_rows == 0 && n_empty == 0 && t.precision == CUTE_PREC_FP32;    // no fused launch, no bf16 kernel for less than four
+        if (p->ng == 1 && alone)
+            for (uint32_t w = uint32_t(p->vec) / 2u; w; w /= 2u)
+                if (items(w) <= (w == 1 && N % 2u ? 3u : 2u) * simds && T(w) < T(uint32_t(p->vec))) p->vec = int(w);
+    }
     // Which parts of the launch go by columns (cute_dev::xcd_share).  A plan of rows alone takes the slab that `narrow` gives for
     // its mean window.  MFMA panels that share columns find a graph's hub rows in their XCD's slab whatever the window: R-MAT
     // graph of 32 768 nodes, N = 512 156 -> 104 us, 16 384 nodes, N = 256 33.5 -> 26.7, 131 072 nodes, N = 310 463 -> 413;
