@@ -218,6 +218,7 @@ struct cute_spmm_plan {
     int vec = 4, ng = 1;                // brick kernel shape
     int pipeline = 1;                   // 1: rolling variant, 2: pipelined variant
     int shape = 2;                      // MFMA kernel: 1 16x16x4 bricks, 2 4x4x1 quad lists
+    bool halfLists = false;             // quad kernel on slabs of 32 columns
     bool bf16x3 = false;                // brick kernel on the bf16 matrix pipeline (three products of bf16 hi/lo parts)
     int rows_vec = 4, rows_logl = 6;    // row kernel shape
     uint32_t rows_slabs = 1;
@@ -1190,13 +1191,14 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
         if (N % 16u == 0) return window <= (mean_row < 16u ? 32768u : 8192u) ? 32u : 0u;
         return window <= (mean_row < 16u ? 16384u : 8192u) ? 64u : 0u;
     };
+    bool half_window = false;
     // A matrix without reuse or hubs (less than a tenth of its entries in panels for the MFMA side): its scattered panels go to
     // the lists only where these are ahead of the row kernel in whichever order suits it.  24 entries a row, us row kernel /
     // lists: 65 536 rows N = 64 46.8 / 37.0, N = 128 106 / 81; 131 072 rows N = 256 457 / 408; rows of B off the 128-byte
     // grid: 32 768 rows N = 301 151 / 126, 65 536 rows N = 400 363 / 354, 98 304 rows 558 / 589.  8 entries a row off that
     // grid: 50 000 rows N = 301 87.7 / 95.2, 131 072 rows N = 400 274 / 305.  Products of 512 columns or more over windows
     // that do not fit an L2 in slabs of 32 columns stay with the lists (the planner's tests hold them to it; 50 000 rows of 7:
-    // lists 89.3, the row kernel by columns 73.5).
+    // 32-column lists 80.6, the row kernel by columns 73.5).
     if (default_bars && t.precision == CUTE_PREC_FP32 && reused * 10u < uint64_t(d->nnz) &&
         uint64_t(d->M) * ((N + 255u) / 256u) >= 4ull * uint64_t(c.num_cus) * 32u) {
         auto concerned = [&](uint32_t q) { return d->brp[q + 1] != d->brp[q] && d->panelMaxRow[q] <= max_row_for_rows && scattered(q); };
@@ -1205,6 +1207,11 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
             if (concerned(q)) { windows += d->panelSpan[q]; entries += d->panelNnz[q]; ++panels; }
         if (panels) {
             const uint64_t window = windows / panels, mean_row = entries / (panels * CUTE_TM);
+            // 32-column lists where a 64-column slab of the window outgrows the L2 by more than they do; us 64 / 32 columns:
+            // 16 entries a row, 50 000 rows N = 64 21.2 / 17.9, N = 256 88.9 / 78.0, N = 512 181 / 145; 65 536 rows
+            // N = 128 58.9 / 52.5; 31 entries a row, 32 768 rows N = 256 75.2 / 78.4, N = 512 155 / 135, 65 536 rows
+            // N = 256 205 / 213, 98 304 rows N = 64 82.7 / 76.8; 131 072 rows of 16, N = 256 287 / 301.
+            half_window = N % 32u == 0 && (window > 32768u || N >= 512u) && window <= (N <= 128u ? 98304u : N < 512u ? 57344u : 65536u);
             const bool on_grid = N % 32u == 0, wide = N >= 512u && window > 32768u;
             const bool lists_ahead = on_grid ? (wide || (narrow(window, mean_row) == 0 && (mean_row >= 16u || N >= 256u)))
                                              : (narrow(window, mean_row) == 0 && mean_row >= 16u && N >= 256u && window <= 65536u);
@@ -1330,7 +1337,8 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
     // graph of 32 768 nodes, N = 512 156 -> 104 us, 16 384 nodes, N = 256 33.5 -> 26.7, 131 072 nodes, N = 310 463 -> 413;
     // lists without reuse gain while the window fits two L2s (16 384 rows of 24, N = 512 46.4 -> 41.8; 65 536 rows 349 -> 367).
     // Off the 64-column grid the last slab is a remainder that unbalances few slabs (N = 101: 137 -> 147): 256 columns or more.
-    uint32_t rows_columns = 0, mfma_by_columns = 0;
+    uint32_t rows_columns = 0;
+    bool mfma_by_columns = false;
     {
         uint64_t scattered_nnz = 0, window[2] = {}, in[2] = {}, cols = 0;
         uint32_t row_panels = 0;
@@ -1346,8 +1354,10 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
             const uint64_t mean_window[2] = {in[0] ? window[0] / in[0] : 0, in[1] ? window[1] / in[1] : 0};
             if (n_brick == 0)
                 rows_columns = narrow(mean_window[1], in[1] / (uint64_t(row_panels) * CUTE_TM));
+            else if (half_window && p->shape == 2 && !t.hub_rows && n_rows == 0 && n_empty == 0 && (N + 31u) / 32u <= 65535u)
+                mfma_by_columns = p->halfLists = true;
             else if (((N % 64u == 0 && N >= 128u) || N >= 256u) && (in[0] * 5u >= cols * 6u || mean_window[0] <= 32768u)) {
-                mfma_by_columns = 1;
+                mfma_by_columns = true;
                 // rows of uneven length share a wavefront: sixteen lanes a row (the brick kernel has no launch with fewer than its own)
                 rows_columns = p->shape == 2 && p->rows_vec == 4 ? 64u : (p->rows_vec << p->rows_logl);
             }
@@ -1366,7 +1376,7 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
     uint32_t slab = 0, num_slabs = 0, upp_log = 0, slots = 0, n_pieces = 0;
     std::vector<uint4> chunks, fixups;
     for (int attempt = 0;; ++attempt) {
-        slab = p->shape == 2 ? 64u : 16u * p->vec * p->ng;   // the quad kernel: one column per lane
+        slab = p->shape == 2 ? (p->halfLists ? 32u : 64u) : 16u * p->vec * p->ng;   // the quad kernel: one column per lane (or half of them)
         num_slabs = (N + slab - 1) / slab;
         if (num_slabs > 65535u) { delete p; return CUTE_ERR_ARG; }   // slabs are the y dimension of the launch
 
@@ -1448,7 +1458,7 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
         if (attempt || t.mfma_shape == 2 || t.pipeline == 1) { delete p; return CUTE_ERR_SHAPE; }   // the caller forced a fast kernel
         p->shape = 1;
         p->pipeline = 2;
-        p->bf16x3 = false;
+        p->bf16x3 = p->halfLists = false;
     }
     std::vector<uint32_t> row_panels;              // panels of the row kernel
     for (uint32_t q = 0; q < d->P; ++q)
@@ -1885,6 +1895,13 @@ int run_with(const cute_spmm_plan *p, const float *dB, float *dC, void *stream, 
 #undef CUTE_FUSED_LL
 #undef CUTE_FUSED_LAUNCH
             rows_launched = true;
+        } else if (p->halfLists) {
+            if (strips)
+                hipLaunchKernelGGL(cute_dev::hrpb_quad_half_f32<true>, grid, block, 0, s, p->dHeads, p->info.numChunks, per_xcd, p->d->dQRecs,
+                                   p->d->dQVals, uint32_t(p->d->numQuadVals), dB, dC, partials, N, p->columnSlabs);
+            else
+                hipLaunchKernelGGL(cute_dev::hrpb_quad_half_f32<false>, grid, block, 0, s, p->dHeads, p->info.numChunks, per_xcd, p->d->dQRecs,
+                                   p->d->dQVals, uint32_t(p->d->numQuadVals), dB, dC, partials, N, p->columnSlabs);
         } else {
 #define CUTE_QUAD_LAUNCH(F, S)                                                                                          \
     hipLaunchKernelGGL((cute_dev::hrpb_quad_f32<F, S>), grid, block, 0, s, p->dHeads, p->info.numChunks, per_xcd,         \

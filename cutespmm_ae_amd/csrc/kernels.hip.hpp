@@ -796,6 +796,147 @@ __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, 8) void hrpb_quad_f32(
 }
 
 // ---------------------------------------------------------------------------------------
+// The quad kernel on slabs of 32 columns, for products by columns (xcd_share) whose window of B does not fit the L2s in
+// slabs of 64: what an XCD has to hold is halved, a 128-byte line of every B row.
+//
+// With cbsz = 3 the A block that abid names is broadcast inside each half of the wavefront: lanes 0..31 multiply by pair P,
+// lanes 32..63 by pair P + 8, so eight instructions do the sixteen pairs of a group for 32 columns and the lists are read
+// as they are.  Pairs P and P + 8 belong to the same row group (P & 3); the two halves' sums are added at the end, half a
+// wavefront storing rows 0..7 of the panel and the other rows 8..15.  Same rate per element as the 64-column kernel; two
+// operand sets of eight loads keep half its bytes in flight (four sets were slower: 85.0 against 80.6 us on 50 000 rows of 7
+// random columns, N = 512, where the 64-column kernel takes 90.8).
+// ---------------------------------------------------------------------------------------
+template <int P>
+__device__ __forceinline__ void quad_half_mfma(float a, float b, f32x4 (&acc)[4])
+{
+    acc[P & 3] = __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, acc[P & 3], 3, P, 0);
+}
+
+// the sums of rows r (lo) and r' (hi) over both halves: row r in lanes 0..31, row r' in lanes 32..63
+__device__ __forceinline__ float add_halves(float lo, float hi)
+{
+    const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(lo), __float_as_uint(hi), false, false);
+    return __uint_as_float(s[0]) + __uint_as_float(s[1]);
+}
+
+template <bool STRIPS>
+__global__ __launch_bounds__(kWaveSize *kWavesPerGroup, 8) void hrpb_quad_half_f32(
+    const uint32_t *__restrict__ heads, uint32_t num_chunks, uint32_t groups_per_xcd, const uint32_t *__restrict__ qrecs,
+    const float *__restrict__ qvals, uint32_t zero_index, const float *__restrict__ B, float *__restrict__ C,
+    float *__restrict__ partials, uint32_t N, uint32_t column_slabs)
+{
+    constexpr uint32_t kHalf = kWaveSize / 2;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
+    uint32_t slab = blockIdx.y;
+    const uint32_t share = xcd_share(blockIdx.x, slab, column_slabs);
+    const uint32_t chunk = (share * groups_per_xcd + blockIdx.x / kNumXcd) * kWavesPerGroup + wave;
+    if (chunk >= num_chunks) return;
+    const uint32_t lane = threadIdx.x & (kWaveSize - 1);
+    const uint32_t *head = heads + size_t(chunk) * kQuadHeadWords;
+    uint32_t g = head[0];
+    const uint32_t g_end = head[1], panel = head[2], piece = head[3];
+    uint32_t ca[kQuadRecordWords], cb[kQuadRecordWords];       // as in quad_chunk
+#pragma unroll
+    for (int p = 0; p < kQuadRecordWords; ++p) ca[p] = head[4 + p];
+
+    const uint32_t n = slab * kHalf + (lane & (kHalf - 1));
+    const bool live = n < N;
+    const uint32_t row_pitch = N * 4u;
+    const uint32_t col_off = (live ? n : N - 1u) * 4u;
+    const uint32_t upper = lane >= kHalf ? 0xffffffffu : 0u;
+
+    f32x4 acc[4];
+#pragma unroll
+    for (int rg = 0; rg < 4; ++rg) acc[rg] = f32x4(0.0f);
+
+    if (g < g_end) {
+        float b0[8], b1[8], a0, a1;
+        const uint32_t last = g_end - 1u;
+        auto fetch_cols = [&](uint32_t (&c)[kQuadRecordWords], uint32_t grp) {
+            const uint32_t *src = qrecs + size_t(min(grp, last)) * kQuadRecordWords;
+#pragma unroll
+            for (int p = 0; p < kQuadRecordWords; ++p) c[p] = src[p];
+        };
+        auto fetch_a = [&](const uint32_t (&c)[kQuadRecordWords]) {
+            const uint64_t mask = (uint64_t(c[17]) << 32) | c[16];
+            const uint32_t rank = __builtin_amdgcn_mbcnt_hi(c[17], __builtin_amdgcn_mbcnt_lo(c[16], c[18]));
+            const uint32_t off = (__builtin_amdgcn_inverse_ballot_w64(mask) ? rank : zero_index) * 4u;
+            return *reinterpret_cast<const float *>(reinterpret_cast<const char *>(qvals) + off);
+        };
+        // the row offsets are products of scalars; the upper half adds the difference of its own (modulo 2^32)
+        auto load_b = [&](const uint32_t (&c)[kQuadRecordWords], int p) {
+            const uint32_t lo = c[p] * row_pitch, hi = c[p + 8] * row_pitch;
+            return *reinterpret_cast<const float *>(reinterpret_cast<const char *>(B) + (((hi - lo) & upper) + lo + col_off));
+        };
+        fetch_cols(cb, g + 1);
+        a0 = fetch_a(ca);
+        a1 = fetch_a(cb);
+#pragma unroll
+        for (int p = 0; p < 8; ++p) b0[p] = load_b(ca, p);
+#pragma unroll
+        for (int p = 0; p < 8; ++p) b1[p] = load_b(cb, p);
+#define CUTE_HALF_ROLL(P, A, BSET, COLS)       \
+    quad_half_mfma<P>(A, BSET[P], acc);        \
+    __builtin_amdgcn_sched_barrier(0);         \
+    BSET[P] = load_b(COLS, P);                 \
+    __builtin_amdgcn_sched_barrier(0);
+#define CUTE_HALF_ROLL_REST(A, BSET, COLS)                                                             \
+    CUTE_HALF_ROLL(1, A, BSET, COLS) CUTE_HALF_ROLL(2, A, BSET, COLS) CUTE_HALF_ROLL(3, A, BSET, COLS) \
+    CUTE_HALF_ROLL(4, A, BSET, COLS) CUTE_HALF_ROLL(5, A, BSET, COLS) CUTE_HALF_ROLL(6, A, BSET, COLS) \
+    CUTE_HALF_ROLL(7, A, BSET, COLS)
+#define CUTE_HALF_MFMA8(A, BSET)                                                                                     \
+    quad_half_mfma<0>(A, BSET[0], acc); quad_half_mfma<1>(A, BSET[1], acc); quad_half_mfma<2>(A, BSET[2], acc);      \
+    quad_half_mfma<3>(A, BSET[3], acc); quad_half_mfma<4>(A, BSET[4], acc); quad_half_mfma<5>(A, BSET[5], acc);      \
+    quad_half_mfma<6>(A, BSET[6], acc); quad_half_mfma<7>(A, BSET[7], acc);
+        fetch_cols(ca, g + 2);
+        while (g + 2 < g_end) {              // the pipeline of quad_chunk: groups g, g+1 and g+2 exist
+            const float a0n = fetch_a(ca);
+            __builtin_amdgcn_sched_barrier(0);
+            CUTE_HALF_ROLL(0, a0, b0, ca)
+            fetch_cols(cb, g + 3);
+            __builtin_amdgcn_sched_barrier(0);
+            CUTE_HALF_ROLL_REST(a0, b0, ca)
+            a0 = a0n;
+            const float a1n = fetch_a(cb);
+            __builtin_amdgcn_sched_barrier(0);
+            CUTE_HALF_ROLL(0, a1, b1, cb)
+            fetch_cols(ca, g + 4);
+            __builtin_amdgcn_sched_barrier(0);
+            CUTE_HALF_ROLL_REST(a1, b1, cb)
+            a1 = a1n;
+            g += 2;
+        }
+        CUTE_HALF_MFMA8(a0, b0)
+        if (g + 1 < g_end) { CUTE_HALF_MFMA8(a1, b1) }
+#undef CUTE_HALF_ROLL
+#undef CUTE_HALF_ROLL_REST
+#undef CUTE_HALF_MFMA8
+    }
+    char *out_base = reinterpret_cast<char *>(piece ? partials : C);
+    const uint32_t unit = piece ? piece - 1u : panel;
+    if (STRIPS) {
+        const f32x4 sum = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+        uint32_t off = __umul24(unit * 4u + (upper & 2u), row_pitch) + n * 4u;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const float v = add_halves(sum[i], sum[i + 2]);
+            if (live) __builtin_nontemporal_store(v, reinterpret_cast<float *>(out_base + off));
+            off += row_pitch;
+        }
+    } else {
+        uint32_t off = __umul24(unit * 16u + (upper & 8u), row_pitch) + n * 4u;
+#pragma unroll
+        for (int rg = 0; rg < 2; ++rg)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float v = add_halves(acc[rg][i], acc[rg + 2][i]);
+                if (live) __builtin_nontemporal_store(v, reinterpret_cast<float *>(out_base + off));
+                off += row_pitch;
+            }
+    }
+}
+
+// ---------------------------------------------------------------------------------------
 // The quad kernel with the most referenced B rows staged in LDS (the reference stages the B rows of a block in
 // shared memory for the warps of its thread block, kernel.cu:123-124,143-164; here what is staged is what many
 // work items share: the rows of hub columns).  A work-group of sixteen wavefronts copies, once, the 64-column

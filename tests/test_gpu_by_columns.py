@@ -84,3 +84,24 @@ def test_forced_rows_give_the_bits_of_the_same_rows_in_row_order(cs, torch_cuda,
         plan.run(torch_cuda.from_numpy(B).cuda(), out)
         outs.append(out)
     assert torch_cuda.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("layout", [1, 2])
+@pytest.mark.parametrize("M,K,per_row,N,cut", [(32768, 40000, 20, 64, 0), (32768, 40000, 24, 96, 3), (16384, 49152, 28, 288, 0),
+                                                (16384, 65536, 32, 512, 2), (32768, 90112, 16, 128, 1)])
+def test_lists_on_slabs_of_32_columns(cs, torch_cuda, layout, M, K, per_row, N, cut):
+    """Both kinds of list, whole panels and panels cut into pieces; rows of whole multiples of the list unit fill their slots."""
+    rng = np.random.default_rng(N)
+    cl = np.sort(rng.integers(0, K // per_row, (M, per_row)) + np.arange(per_row) * (K // per_row), axis=1).astype(np.uint32)
+    rp, vl = (np.arange(M + 1) * per_row).astype(np.uint32), rng.standard_normal(M * per_row).astype(np.float32)
+    B = rng.standard_normal((K, N)).astype(np.float32)
+    h = cs.HRPB(M, K, rp, cl.ravel(), vl)
+    h.upload(quad_layout=layout)
+    plan = cs.SPMM_TC(h, N, max_chunk_blocks=cut)
+    out, again = (torch_cuda.full((M, N), float("nan"), device="cuda") for _ in range(2))
+    dB = torch_cuda.from_numpy(B).cuda()
+    plan.run(dB, out)
+    plan.run(dB, again)
+    assert plan.kernel_name == "hrpb_quad_half_f32" and (plan.info["numAtomicChunks"] > 0) == (cut > 0), plan.info
+    assert torch_cuda.equal(out, again)
+    _check(rp, cl.ravel(), vl, B, out.cpu().numpy(), M, N, np.unique(np.concatenate([np.arange(40), np.arange(M - 40, M), rng.integers(0, M, 300)])))
