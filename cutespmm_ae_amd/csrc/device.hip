@@ -1648,7 +1648,7 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
 
 namespace {
 
-template <int VEC, int NG, bool FULL>
+template <int VEC, int NG, bool FULL, bool COLUMNS>
 void launch_brick_full(const cute_spmm_plan *p, const float *dB, float *dC, float *partials, hipStream_t s)
 {
     const uint32_t groups = (p->info.numChunks + cute_dev::kWavesPerGroup - 1) / cute_dev::kWavesPerGroup;
@@ -1656,10 +1656,10 @@ void launch_brick_full(const cute_spmm_plan *p, const float *dB, float *dC, floa
     const dim3 grid(per_xcd * cute_dev::kNumXcd, p->info.numSlabs), block(cute_dev::kWaveSize * cute_dev::kWavesPerGroup);
     if (p->bf16x3) {
         if constexpr (VEC == 4)
-            hipLaunchKernelGGL((cute_dev::hrpb_brick_bf16x3<NG, FULL>), grid, block, 0, s, p->dChunks, p->info.numChunks, per_xcd,
+            hipLaunchKernelGGL((cute_dev::hrpb_brick_bf16x3<NG, FULL, COLUMNS>), grid, block, 0, s, p->dChunks, p->info.numChunks, per_xcd,
                                p->d->dHdr, p->d->dVals, uint32_t(p->d->numVals), dB, dC, partials, p->info.N, p->columnSlabs);
     } else if (p->pipeline == 1)
-        hipLaunchKernelGGL((cute_dev::hrpb_brick_f32_rolling<VEC, NG, FULL>), grid, block, 0, s, p->dChunks,
+        hipLaunchKernelGGL((cute_dev::hrpb_brick_f32_rolling<VEC, NG, FULL, COLUMNS>), grid, block, 0, s, p->dChunks,
                            p->info.numChunks, per_xcd, p->d->dHdr, p->d->dVals, uint32_t(p->d->numVals), dB, dC, partials, p->info.N, p->columnSlabs);
     else
         hipLaunchKernelGGL((cute_dev::hrpb_brick_f32<VEC, NG, FULL>), grid, block, 0, s, p->dChunks, p->info.numChunks,
@@ -1669,8 +1669,11 @@ void launch_brick_full(const cute_spmm_plan *p, const float *dB, float *dC, floa
 template <int VEC, int NG>
 void launch_brick(const cute_spmm_plan *p, const float *dB, float *dC, float *partials, hipStream_t s)
 {
-    if (p->info.N % p->info.slabWidth == 0) launch_brick_full<VEC, NG, true>(p, dB, dC, partials, s);
-    else launch_brick_full<VEC, NG, false>(p, dB, dC, partials, s);
+    const bool full = p->info.N % p->info.slabWidth == 0;
+    if (p->columnSlabs && full) launch_brick_full<VEC, NG, true, true>(p, dB, dC, partials, s);
+    else if (p->columnSlabs) launch_brick_full<VEC, NG, false, true>(p, dB, dC, partials, s);
+    else if (full) launch_brick_full<VEC, NG, true, false>(p, dB, dC, partials, s);
+    else launch_brick_full<VEC, NG, false, false>(p, dB, dC, partials, s);
 }
 
 template <int VEC, bool BATCHED>
@@ -1686,9 +1689,12 @@ void launch_rows_vec(int logl, const uint4 *row_list, uint32_t num_rows, uint32_
     const cute_dev::XcdRanges rg = ranges ? *ranges : cute_dev::XcdRanges{};
 #define CUTE_ROWS_CASE(LL)                                                                                        \
     case LL:                                                                                                      \
-        if (BATCHED)                                                                                              \
-            hipLaunchKernelGGL((cute_dev::csr_rows_batched<VEC, LL, kRowBatch>), grid, block, 0, s, row_list, num_rows,    \
-                               rp, cl, vl, dB, dC, N, rg, column_slabs);                                                        \
+        if (BATCHED && VEC == 4 && LL >= 3 && column_slabs)   /* by columns: 64 columns or more */                \
+            hipLaunchKernelGGL((cute_dev::csr_rows_batched<VEC, LL, kRowBatch, VEC == 4 && LL >= 3>), grid, block, 0, s, row_list, \
+                               num_rows, rp, cl, vl, dB, dC, N, rg, column_slabs);                                \
+        else if (BATCHED)                                                                                         \
+            hipLaunchKernelGGL((cute_dev::csr_rows_batched<VEC, LL, kRowBatch, false>), grid, block, 0, s, row_list, num_rows, \
+                               rp, cl, vl, dB, dC, N, rg, 0u);                                                    \
         else                                                                                                      \
             hipLaunchKernelGGL((cute_dev::csr_rows<VEC, LL>), grid, block, 0, s, static_cast<const uint32_t *>(nullptr), num_rows, slabs, rp, \
                                cl, vl, dB, dC, N);                                                                \
@@ -1812,13 +1818,17 @@ void launch_brick_rows_as(const cute_spmm_plan *p, const float *dB, float *dC, f
     const uint32_t rows_per_slab = p->rowBlocksPerXcd * cute_dev::kNumXcd;
     const uint64_t brick_blocks = uint64_t(grid.x) * grid.y, row_blocks = uint64_t(rows_per_slab) * p->rows_slabs;
     const dim3 flat(uint32_t(brick_blocks + row_blocks)), block(cute_dev::kWaveSize * cute_dev::kWavesPerGroup);
-#define CUTE_BRICK_ROWS(F)                                                                                                \
-    hipLaunchKernelGGL((cute_dev::hrpb_brick_rows_f32<VEC, NG, F, LOG_L>), flat, block, 0, s, grid.x, uint32_t(brick_blocks),  \
+#define CUTE_BRICK_ROWS(F, COLUMNS)                                                                                       \
+    hipLaunchKernelGGL((cute_dev::hrpb_brick_rows_f32<VEC, NG, F, LOG_L, COLUMNS>), flat, block, 0, s, grid.x, uint32_t(brick_blocks),  \
                        p->dChunks, p->info.numChunks, per_xcd, p->d->dHdr, p->d->dVals, uint32_t(p->d->numVals), p->dRowList, \
                        p->numRows, rows_per_slab, p->rowRanges, p->columnSlabs, p->rowColumnSlabs, p->d->dRowPtr, p->d->dCols, p->d->dCsrVals,                    \
                        dB, dC, partials, N)
-    if (N % (16u * VEC * NG) == 0) CUTE_BRICK_ROWS(true);
-    else CUTE_BRICK_ROWS(false);
+    constexpr bool wide = LOG_L >= 5;            // a launch by columns has 128 columns or more
+    const bool full = N % (16u * VEC * NG) == 0;
+    if (wide && p->columnSlabs && full) CUTE_BRICK_ROWS(true, wide);
+    else if (wide && p->columnSlabs) CUTE_BRICK_ROWS(false, wide);
+    else if (full) CUTE_BRICK_ROWS(true, false);
+    else CUTE_BRICK_ROWS(false, false);
 #undef CUTE_BRICK_ROWS
 }
 
@@ -1872,21 +1882,24 @@ int run_with(const cute_spmm_plan *p, const float *dB, float *dC, void *stream, 
         const uint32_t rows_per_slab = p->rowBlocksPerXcd * cute_dev::kNumXcd;
         const uint64_t row_blocks = uint64_t(rows_per_slab) * p->rows_slabs, quad_blocks = uint64_t(grid.x) * grid.y;
         if (p->info.fusedLaunch && quad_blocks + row_blocks < 0x7fffffffull) {
-#define CUTE_FUSED_LAUNCH(F, S, LL)                                                                                       \
-    hipLaunchKernelGGL((cute_dev::hrpb_quad_rows_f32<F, S, LL>), dim3(uint32_t(quad_blocks + row_blocks)), block, 0, s,     \
+#define CUTE_FUSED_LAUNCH(F, S, LL, COLUMNS)                                                                              \
+    hipLaunchKernelGGL((cute_dev::hrpb_quad_rows_f32<F, S, LL, COLUMNS>), dim3(uint32_t(quad_blocks + row_blocks)), block, 0, s,     \
                        grid.x, uint32_t(quad_blocks), p->dHeads, p->info.numChunks, per_xcd, p->d->dQRecs, p->d->dQVals,   \
                        uint32_t(p->d->numQuadVals),                                                                  \
                        p->dRowList, p->numRows, rows_per_slab, p->rowRanges, p->columnSlabs, p->rowColumnSlabs, p->d->dRowPtr, p->d->dCols, p->d->dCsrVals, dB, dC,    \
                        partials, N)
 #define CUTE_FUSED_LL(F, S)                                                     \
     switch (p->rows_logl) {                                                     \
-        case 0: CUTE_FUSED_LAUNCH(F, S, 0); break;                              \
-        case 1: CUTE_FUSED_LAUNCH(F, S, 1); break;                              \
-        case 2: CUTE_FUSED_LAUNCH(F, S, 2); break;                              \
-        case 3: CUTE_FUSED_LAUNCH(F, S, 3); break;                              \
-        case 4: CUTE_FUSED_LAUNCH(F, S, 4); break;                              \
-        case 5: CUTE_FUSED_LAUNCH(F, S, 5); break;                              \
-        default: CUTE_FUSED_LAUNCH(F, S, 6); break;                             \
+        case 0: CUTE_FUSED_LAUNCH(F, S, 0, false); break;                       \
+        case 1: CUTE_FUSED_LAUNCH(F, S, 1, false); break;                       \
+        case 2: CUTE_FUSED_LAUNCH(F, S, 2, false); break;                       \
+        case 3: CUTE_FUSED_LAUNCH(F, S, 3, false); break;                       \
+        case 4:   /* by columns: sixteen lanes a row */                         \
+            if (p->columnSlabs) CUTE_FUSED_LAUNCH(F, S, 4, true);               \
+            else CUTE_FUSED_LAUNCH(F, S, 4, false);                             \
+            break;                             \
+        case 5: CUTE_FUSED_LAUNCH(F, S, 5, false); break;                       \
+        default: CUTE_FUSED_LAUNCH(F, S, 6, false); break;                             \
     }
             if (full && strips) { CUTE_FUSED_LL(true, true) }
             else if (full) { CUTE_FUSED_LL(true, false) }
@@ -1904,12 +1917,16 @@ int run_with(const cute_spmm_plan *p, const float *dB, float *dC, void *stream, 
                                    p->d->dQVals, uint32_t(p->d->numQuadVals), dB, dC, partials, N, p->columnSlabs);
         } else {
 #define CUTE_QUAD_LAUNCH(F, S)                                                                                          \
-    hipLaunchKernelGGL((cute_dev::hrpb_quad_f32<F, S>), grid, block, 0, s, p->dHeads, p->info.numChunks, per_xcd,         \
-                       p->d->dQRecs, p->d->dQVals, uint32_t(p->d->numQuadVals), dB, dC, partials, N, p->columnSlabs)
-        if (full && strips) CUTE_QUAD_LAUNCH(true, true);
-        else if (full) CUTE_QUAD_LAUNCH(true, false);
-        else if (strips) CUTE_QUAD_LAUNCH(false, true);
-        else CUTE_QUAD_LAUNCH(false, false);
+    if (p->columnSlabs)                                                                                                 \
+        hipLaunchKernelGGL((cute_dev::hrpb_quad_f32<F, S, true>), grid, block, 0, s, p->dHeads, p->info.numChunks, per_xcd,  \
+                           p->d->dQRecs, p->d->dQVals, uint32_t(p->d->numQuadVals), dB, dC, partials, N, p->columnSlabs);   \
+    else                                                                                                                \
+        hipLaunchKernelGGL((cute_dev::hrpb_quad_f32<F, S, false>), grid, block, 0, s, p->dHeads, p->info.numChunks, per_xcd, \
+                           p->d->dQRecs, p->d->dQVals, uint32_t(p->d->numQuadVals), dB, dC, partials, N, 0u)
+            if (full && strips) { CUTE_QUAD_LAUNCH(true, true); }
+            else if (full) { CUTE_QUAD_LAUNCH(true, false); }
+            else if (strips) { CUTE_QUAD_LAUNCH(false, true); }
+            else { CUTE_QUAD_LAUNCH(false, false); }
 #undef CUTE_QUAD_LAUNCH
         }
     } else if (p->info.numChunks) {

@@ -89,6 +89,8 @@ __device__ __forceinline__ bool xcd_range_id(const XcdRanges &r, uint32_t bid, u
 // XCD x takes the column_slabs eighths from x * column_slabs on, that is 1/8 of the columns and (almost) all rows of them, and
 // the L2 has to hold those columns only.  The same eighths, only permuted: every (slab, eighth) is still taken once.
 // 16 384 rows of 8 random columns, N = 512: 35.4 us in row order, 18.3 by columns (32-column slabs, 2 MB of B each).
+// The kernels of the default plans are compiled for each order (COLUMNS): deciding at run time put the argument and the
+// division by it in front of a wavefront's first fetch, 0.5 of 13.8 us on the 9-point stencil of 256 x 256 points, N = 128.
 __device__ __forceinline__ uint32_t xcd_share(uint32_t bid, uint32_t &slab, uint32_t column_slabs)
 {
     const uint32_t x = bid % kNumXcd;
@@ -470,14 +472,14 @@ __device__ __forceinline__ void brick_rolling_body(uint32_t block_x, uint32_t bl
     brick_store_lean<VEC, NG, FULL>(it, acc, C, partials, N, lane);
 }
 
-template <int VEC, int NG, bool FULL>
+template <int VEC, int NG, bool FULL, bool COLUMNS>
 __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, (NG == 1 ? 8 : 4)) void hrpb_brick_f32_rolling(
     const uint4 *__restrict__ chunks, uint32_t num_chunks, uint32_t groups_per_xcd, const uint32_t *__restrict__ hdr,
     const float *__restrict__ vals, uint32_t zero_index, const float *__restrict__ B, float *__restrict__ C,
     float *__restrict__ partials, uint32_t N, uint32_t column_slabs)
 {
     brick_rolling_body<VEC, NG, FULL>(blockIdx.x, blockIdx.y, chunks, num_chunks, groups_per_xcd, hdr, vals, zero_index, B, C,
-                                      partials, N, column_slabs);
+                                      partials, N, COLUMNS ? column_slabs : 0u);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -539,7 +541,7 @@ __device__ __forceinline__ void mfma_block_bf16x3(const Bf16Operands<NG> &o, f32
         }
 }
 
-template <int NG, bool FULL>
+template <int NG, bool FULL, bool COLUMNS>
 __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, (NG == 1 ? 6 : 4)) void hrpb_brick_bf16x3(
     const uint4 *__restrict__ chunks, uint32_t num_chunks, uint32_t groups_per_xcd, const uint32_t *__restrict__ hdr,
     const float *__restrict__ vals, uint32_t zero_index, const float *__restrict__ B, float *__restrict__ C,
@@ -547,7 +549,7 @@ __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, (NG == 1 ? 6 : 4)) void 
 {
     constexpr int VEC = 4;
     const uint32_t lane = threadIdx.x & (kWaveSize - 1);
-    const BrickItem it = brick_item<VEC, NG>(chunks, num_chunks, groups_per_xcd, lane, blockIdx.x, blockIdx.y, column_slabs);
+    const BrickItem it = brick_item<VEC, NG>(chunks, num_chunks, groups_per_xcd, lane, blockIdx.x, blockIdx.y, COLUMNS ? column_slabs : 0u);
     if (!it.valid) return;
     const uint32_t end = it.end;
     const uint32_t row_pitch = N * 4u;
@@ -785,14 +787,14 @@ __device__ __forceinline__ void quad_chunk(uint32_t chunk, uint32_t block_y, con
     }
 }
 
-template <bool FULL, bool STRIPS>
+template <bool FULL, bool STRIPS, bool COLUMNS>
 __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, 8) void hrpb_quad_f32(
     const uint32_t *__restrict__ heads, uint32_t num_chunks, uint32_t groups_per_xcd, const uint32_t *__restrict__ qrecs,
     const float *__restrict__ qvals, uint32_t zero_index, const float *__restrict__ B, float *__restrict__ C,
     float *__restrict__ partials, uint32_t N, uint32_t column_slabs)
 {
     quad_body<FULL, STRIPS>(blockIdx.x, blockIdx.y, heads, num_chunks, groups_per_xcd, qrecs, qvals, zero_index, B, C,
-                            partials, N, column_slabs);
+                            partials, N, COLUMNS ? column_slabs : 0u);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1238,7 +1240,7 @@ __device__ __forceinline__ void rows_batched_body(uint32_t block_id, uint32_t sl
     if (live) store_vec_streaming<VEC>(acc, C + size_t(row) * N + c0);
 }
 
-template <int VEC, int LOG_L, int BATCH>
+template <int VEC, int LOG_L, int BATCH, bool COLUMNS>
 __global__ __launch_bounds__(256) void csr_rows_batched(const uint4 *__restrict__ row_list, uint32_t num_rows,
                                                         const uint32_t *__restrict__ rowPtr,
                                                         const uint32_t *__restrict__ cols,
@@ -1250,7 +1252,7 @@ __global__ __launch_bounds__(256) void csr_rows_batched(const uint4 *__restrict_
     // walked slab by slab, each over all rows (y is the slower index of the order in which work-groups start):
     // what the resident rows read of B at one time is then one slab wide, whatever N is.
     uint32_t block_id, slab = blockIdx.y;
-    const uint32_t x = xcd_share(blockIdx.x, slab, column_slabs);
+    const uint32_t x = xcd_share(blockIdx.x, slab, COLUMNS ? column_slabs : 0u);
     if (!xcd_range_id(ranges, blockIdx.x, x, block_id)) return;
     rows_batched_body<VEC, LOG_L, BATCH, true>(block_id, slab, row_list, num_rows, rowPtr, cols, vals, B, C, N);
 }
@@ -1260,7 +1262,7 @@ __global__ __launch_bounds__(256) void csr_rows_batched(const uint4 *__restrict_
 // leave idle.  Blocks [0, quad_blocks) are the quad kernel's 2-D grid flattened (x fastest, so the
 // XCD of a block is still x % 8); the rest are the row kernel's blocks, dealt to the XCDs in
 // contiguous ranges like the row kernel's own launch does.
-template <bool FULL, bool STRIPS, int LOG_L>
+template <bool FULL, bool STRIPS, int LOG_L, bool COLUMNS>
 __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, 8) void hrpb_quad_rows_f32(
     uint32_t quad_blocks_x, uint32_t quad_blocks, const uint32_t *__restrict__ heads, uint32_t num_chunks,
     uint32_t groups_per_xcd, const uint32_t *__restrict__ qrecs, const float *__restrict__ qvals, uint32_t zero_index,
@@ -1271,20 +1273,20 @@ __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, 8) void hrpb_quad_rows_f
     static_assert(kWaveSize * kWavesPerGroup == 256, "both bodies are written for 256-thread blocks");
     if (blockIdx.x < quad_blocks) {
         quad_body<FULL, STRIPS>(blockIdx.x % quad_blocks_x, blockIdx.x / quad_blocks_x, heads, num_chunks, groups_per_xcd,
-                                qrecs, qvals, zero_index, B, C, partials, N, column_slabs);
+                                qrecs, qvals, zero_index, B, C, partials, N, COLUMNS ? column_slabs : 0u);
     } else {   // quad_blocks is a multiple of the XCD count, so the XCD of a row block is (its index) % 8 as well
         const uint32_t rb = blockIdx.x - quad_blocks;
         uint32_t slab = rb / row_blocks_per_slab;      // slab by slab, as in csr_rows_batched
         const uint32_t bid = rb - slab * row_blocks_per_slab;
         uint32_t block_id;
-        const uint32_t x = xcd_share(bid, slab, row_column_slabs);
+        const uint32_t x = xcd_share(bid, slab, COLUMNS ? row_column_slabs : 0u);
         if (!xcd_range_id(row_ranges, bid, x, block_id)) return;
         rows_batched_body<4, LOG_L, 8, (LOG_L > 3)>(block_id, slab, row_list, num_rows, rowPtr, cols, vals, B, C, N);
     }
 }
 
 // The same for a plan that pairs the rolling brick kernel with the row kernel.
-template <int VEC, int NG, bool FULL, int LOG_L>
+template <int VEC, int NG, bool FULL, int LOG_L, bool COLUMNS>
 __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, (NG == 1 ? 8 : 4)) void hrpb_brick_rows_f32(
     uint32_t brick_blocks_x, uint32_t brick_blocks, const uint4 *__restrict__ chunks, uint32_t num_chunks,
     uint32_t groups_per_xcd, const uint32_t *__restrict__ hdr, const float *__restrict__ tile_vals, uint32_t zero_index,
@@ -1294,13 +1296,13 @@ __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, (NG == 1 ? 8 : 4)) void 
 {
     if (blockIdx.x < brick_blocks) {
         brick_rolling_body<VEC, NG, FULL>(blockIdx.x % brick_blocks_x, blockIdx.x / brick_blocks_x, chunks, num_chunks,
-                                          groups_per_xcd, hdr, tile_vals, zero_index, B, C, partials, N, column_slabs);
+                                          groups_per_xcd, hdr, tile_vals, zero_index, B, C, partials, N, COLUMNS ? column_slabs : 0u);
     } else {
         const uint32_t rb = blockIdx.x - brick_blocks;
         uint32_t slab = rb / row_blocks_per_slab;
         const uint32_t bid = rb - slab * row_blocks_per_slab;
         uint32_t block_id;
-        const uint32_t x = xcd_share(bid, slab, row_column_slabs);
+        const uint32_t x = xcd_share(bid, slab, COLUMNS ? row_column_slabs : 0u);
         if (!xcd_range_id(row_ranges, bid, x, block_id)) return;
         rows_batched_body<4, LOG_L, 8, (LOG_L > 3)>(block_id, slab, row_list, num_rows, rowPtr, cols, vals, B, C, N);
     }
