@@ -54,7 +54,9 @@ class HostPool {
             take(l);
         }
     }
-    void take(std::unique_lock<std::mutex> &l)          // the tasks that are left, one after the other
+    // The tasks that are left, one after the other.  noexcept: a task that throws ends the program, as in a thread of its own; the
+    // caller must not leave the frame the other threads work in.
+    void take(std::unique_lock<std::mutex> &l) noexcept
     {
         while (next_ < tasks_) {
             const unsigned i = next_++;
