@@ -372,6 +372,7 @@ struct PanelRange {
     std::vector<uint16_t> rows;       // rows that hold each of them
     std::vector<uint32_t> count;      // active columns of each panel
     uint64_t blocks = 0, words = 0;   // of the range; then where it starts
+    int status = CUTE_OK;             // what is wrong with its first bad row
 };
 
 inline uint32_t record_words(uint32_t nnz_blk)
@@ -409,8 +410,8 @@ extern "C" int cute_hrpb_build(uint32_t M, uint32_t K, const uint32_t *rowPtr, c
     if (M == 0 || K == 0 || M % CUTE_TM || K % CUTE_TK) return CUTE_ERR_SHAPE;
     const uint32_t P = M / CUTE_TM;
     const unsigned tasks = unsigned(std::min<uint64_t>((P + 15u) / 16u, uint64_t(host_threads()) * 4u));
+    const uint32_t nnz = rowPtr[M];
     std::vector<PanelRange> ranges(tasks);
-    std::atomic<int> status{CUTE_OK};
 
     // sweep 1: active columns and their rows, validation, record sizes
     parallel_tasks(tasks, [&](unsigned task) {
@@ -418,8 +419,9 @@ extern "C" int cute_hrpb_build(uint32_t M, uint32_t K, const uint32_t *rowPtr, c
         rg.begin = uint32_t(uint64_t(P) * task / tasks);
         rg.end = uint32_t(uint64_t(P) * (task + 1) / tasks);
         rg.count.reserve(rg.end - rg.begin);
-        const uint32_t first = rowPtr[rg.begin * CUTE_TM], last = rowPtr[rg.end * CUTE_TM];
-        rg.active.reserve(last > first ? (last - first) / 2u + 16u : 16u);
+        // (a hint, bounded because nothing has checked the pointers yet)
+        const uint32_t first = rowPtr[uint64_t(rg.begin) * CUTE_TM], last = rowPtr[uint64_t(rg.end) * CUTE_TM];
+        rg.active.reserve(last > first ? std::min((last - first) / 2u + 16u, 1u << 22) : 16u);
         rg.rows.reserve(rg.active.capacity());
         std::vector<uint64_t> window;                    // all zero between panels
         std::vector<uint32_t> before, sorted;
@@ -427,14 +429,19 @@ extern "C" int cute_hrpb_build(uint32_t M, uint32_t K, const uint32_t *rowPtr, c
             const uint32_t *rp = rowPtr + uint64_t(p) * CUTE_TM;
             uint32_t lo = ~0u, hi = 0u, n = 0;
             for (uint32_t r = 0; r < CUTE_TM; ++r) {
-                const uint32_t s = rp[r], e = rp[r + 1];
-                if (e < s) { status.store(CUTE_ERR_RANGE, std::memory_order_relaxed); return; }
+                // entry by entry up to the first bad one, and never past the last entry of the matrix: a row pointer that is
+                // wrong must not lead outside the arrays
+                const uint32_t s = rp[r], e = rp[r + 1], end = std::min(e, nnz);
+                if (e < s) { rg.status = CUTE_ERR_RANGE; return; }
                 if (e == s) continue;
-                uint32_t prev = cols[s];
-                bool ascending = true;
-                for (uint32_t i = s + 1; i < e; ++i) { ascending &= cols[i] > prev; prev = cols[i]; }
-                if (!ascending) { status.store(CUTE_ERR_UNSORTED, std::memory_order_relaxed); return; }
-                if (prev >= K) { status.store(CUTE_ERR_RANGE, std::memory_order_relaxed); return; }
+                uint32_t prev = 0;
+                for (uint32_t i = s; i < end; ++i) {
+                    const uint32_t c = cols[i];
+                    if (c >= K) { rg.status = CUTE_ERR_RANGE; return; }
+                    if (c <= prev && i > s) { rg.status = CUTE_ERR_UNSORTED; return; }
+                    prev = c;
+                }
+                if (e > nnz) { rg.status = CUTE_ERR_RANGE; return; }
                 lo = std::min(lo, cols[s]);
                 hi = std::max(hi, prev);
                 n += e - s;
@@ -488,7 +495,8 @@ extern "C" int cute_hrpb_build(uint32_t M, uint32_t K, const uint32_t *rowPtr, c
             }
         }
     });
-    if (status != CUTE_OK) return status;
+    for (const PanelRange &rg : ranges)
+        if (rg.status != CUTE_OK) return rg.status;
 
     uint64_t nb64 = 0, words = 0;
     for (PanelRange &rg : ranges) {
@@ -584,7 +592,7 @@ extern "C" int cute_hrpb_build(uint32_t M, uint32_t K, const uint32_t *rowPtr, c
     out->rowPtr = rowPtr;
     out->cols = cols;
     out->vals = vals;
-    out->nnz = rowPtr[M];
+    out->nnz = nnz;
     out->numBricks = uint32_t(bricks.load());
     return CUTE_OK;
 }

@@ -370,6 +370,19 @@ int main(int argc, char **argv)
         EXPECT(cute_csr_sort_rows(&a) == CUTE_ERR_UNSORTED);
     }
 
+    // one row pointer beyond the last entry, inside a panel, at a panel's edge and in the last panel: refused without a read outside
+    for (uint32_t row : {1u, 5u, 16u, 17u, 256u, 511u})
+        for (uint32_t value : {4000000000u, 512u * 3u + 1u}) {
+            const uint32_t M = 512, per_row = 3;
+            std::vector<uint32_t> rp(M + 1), cl(M * per_row);
+            std::vector<float> vl(M * per_row, 1.0f);
+            for (uint32_t r = 0; r <= M; ++r) rp[r] = r * per_row;
+            for (uint32_t i = 0; i < M * per_row; ++i) cl[i] = i;                // ascends over the whole matrix: no row ends the scan
+            rp[row] = value;
+            cute_hrpb_host h{};
+            EXPECT(cute_hrpb_build(M, M * per_row, rp.data(), cl.data(), vl.data(), &h) == CUTE_ERR_RANGE);
+        }
+
     // malformed MatrixMarket files: a status, never a crash
     const char *texts[] = {
         "",
