@@ -51,7 +51,9 @@ class CuteError(RuntimeError):
         self.status = status
         msg = "%s: %s (%d)" % (where, _status_string(status), status)
         if status in (-7, -8, -10):
-            msg += " -- " + _last_hip_error()
+            detail = _last_hip_error()
+            if detail:
+                msg += " -- " + detail
         super().__init__(msg)
 
 
@@ -251,6 +253,8 @@ def load_library():
 
 
 def _status_string(s):
+    if _lib is None and not os.path.exists(LIB_PATH):      # the error being made is that very fact: nothing to ask
+        return "no library"
     try:
         return load_library().cute_status_string(int(s)).decode()
     except Exception:  # library missing: still produce a readable message
@@ -258,6 +262,8 @@ def _status_string(s):
 
 
 def _last_hip_error():
+    if _lib is None and not os.path.exists(LIB_PATH):
+        return ""
     try:
         return load_library().cute_last_hip_error().decode()
     except Exception:
