@@ -40,8 +40,9 @@ inline unsigned host_threads()
 // caller (another thread of the program, or a job's own task) starts threads of its own instead.  The workers sleep
 // while there is no job.  A child process after fork has no threads and gets a pool of its own.
 class HostPool {
-    std::mutex job_, m_;
+    std::mutex m_;
     std::condition_variable wake_, done_;
+    bool running_ = false;               // a job has the pool (a flag: the thread that runs it may come here again, from one of its tasks)
     void (*call_)(void *, unsigned) = nullptr;
     void *arg_ = nullptr;
     unsigned next_ = 0, tasks_ = 0, open_ = 0, workers_ = 0;
@@ -82,16 +83,17 @@ public:
     // call(arg, i) for every i < tasks on up to `threads` threads, the caller's among them; false when a job is running.
     bool run(unsigned tasks, unsigned threads, void (*call)(void *, unsigned), void *arg)
     {
-        std::unique_lock<std::mutex> job(job_, std::try_to_lock);
-        if (!job.owns_lock()) return false;
         std::unique_lock<std::mutex> l(m_);
+        if (running_) return false;
         for (; workers_ + 1 < threads; ++workers_) std::thread([this] { work(); }).detach();
+        running_ = true;
         call_ = call; arg_ = arg;
         next_ = 0; tasks_ = open_ = tasks;
         for (unsigned i = 1; i < std::min(tasks, threads); ++i) wake_.notify_one();
         take(l);
         done_.wait(l, [this] { return open_ == 0; });
         tasks_ = 0;
+        running_ = false;
         return true;
     }
 };

@@ -9,7 +9,7 @@
 #include <string>
 #include <vector>
 
-#include "cutespmm.h"
+#include "../../cutespmm_ae_amd/csrc/common.hpp"
 
 static int g_failures = 0;
 #define EXPECT(cond)                                                                  \
@@ -382,6 +382,21 @@ int main(int argc, char **argv)
             cute_hrpb_host h{};
             EXPECT(cute_hrpb_build(M, M * per_row, rp.data(), cl.data(), vl.data(), &h) == CUTE_ERR_RANGE);
         }
+
+    // sections inside a section's tasks, and from two threads at once: every task runs once, whoever has the pool
+    {
+        std::atomic<int> runs[3][12][5] = {};
+        auto sections = [&](int caller) {
+            cute::parallel_tasks(12u, [&, caller](unsigned i) { cute::parallel_tasks(5u, [&, caller, i](unsigned k) { ++runs[caller][i][k]; }); });
+        };
+        std::thread other([&] { sections(1); });
+        sections(0);
+        other.join();
+        sections(2);
+        for (auto &caller : runs)
+            for (auto &outer : caller)
+                for (auto &n : outer) EXPECT(n == 1);
+    }
 
     // malformed MatrixMarket files: a status, never a crash
     const char *texts[] = {
