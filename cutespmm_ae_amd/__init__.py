@@ -556,7 +556,9 @@ def _launcher():
     with a Stream object (3.0 us), imports and ctypes objects made in each, 4.1 us without, 3.1 of them the launch."""
     import torch
     Tensor, float32 = torch.Tensor, torch.float32
-    raw_stream, device = torch._C._cuda_getCurrentRawStream, torch._C._cuda_getDevice
+    # (these two names of torch are not public; where it lacks them the public ones give the same handle, about 3 us later)
+    device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
+    raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda d: torch.cuda.current_stream(d).cuda_stream)
 
     def address(t):
         if isinstance(t, Tensor) and t.is_cuda and t.dtype is float32 and t.is_contiguous():
