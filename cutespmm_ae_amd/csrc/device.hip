@@ -379,6 +379,15 @@ class DevicePool {
     std::unordered_map<void *, std::pair<uint64_t, int>> out_;
     uint64_t idleBytes_ = 0, clock_ = 0;
 
+    // What hipFree does before it frees, through a block of a page (1.2 us).  Not hipDeviceSynchronize, which breaks a capture
+    // under way on any stream; hipFree is allowed beside a capture in relaxed mode, and a handle may be collected in the middle of one.
+    static bool wait_for_device()
+    {
+        void *page = nullptr;
+        if (hipMalloc(&page, 4096) == hipSuccess) return hipFree(page) == hipSuccess;
+        (void)hipGetLastError();
+        return false;
+    }
     void drop(size_t i)
     {
         idleBytes_ -= idle_[i].bytes;
@@ -430,7 +439,7 @@ public:
                 out_.erase(it);
             }
         }
-        if (!bytes || bytes > kIdleBytes / 4u || hipDeviceSynchronize() != hipSuccess) { (void)hipFree(p); return; }
+        if (!bytes || bytes > kIdleBytes / 4u || !wait_for_device()) { (void)hipFree(p); return; }
         std::lock_guard<std::mutex> g(lock_);
         ++clock_;
         idle_.push_back({p, bytes, device, clock_});

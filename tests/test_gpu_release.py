@@ -1,0 +1,47 @@
+"""Handles and plans released while other work is under way: a stream being captured, kernels still running."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _plan(cs, torch, rows, N):
+    A = cs.gen_matrix(1, 3, rows, 16, 0)
+    csr = [torch.from_numpy(np.array(a) if a.dtype == np.float32 else np.array(a).view(np.int32)).cuda() for a in (A.rowPtr, A.cols, A.vals)]
+    return cs.SPMM_TC(cs.DeviceHRPB(A.M, A.K, *csr), N), torch.randn(A.K, N, device="cuda"), torch.empty(A.M, N, device="cuda")
+
+
+@pytest.mark.parametrize("rows", [512, 65536])        # blocks below and above the size that is kept for the next handle
+def test_release_beside_a_relaxed_capture(cs, torch_cuda, rows):
+    torch = torch_cuda
+    keep, B, C = _plan(cs, torch, 4096, 32)
+    drop, _, _ = _plan(cs, torch, rows, 32)
+    want = keep.run(B, C).clone()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream(), capture_error_mode="relaxed"):
+        keep.run(B, C)
+        del drop
+        keep.run(B, C)
+    for _ in range(3):
+        C.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(C, want)
+        assert torch.equal(keep.run(B, C), want)
+        torch.cuda.synchronize()
+
+
+def test_release_waits_for_running_kernels(cs, torch_cuda):
+    """The block may serve another thread's set-up at once, so a release returns only when every stream is done with it."""
+    torch = torch_cuda
+    plan, B, C = _plan(cs, torch, 65536, 32)
+    side, done = torch.cuda.Stream(), torch.cuda.Event()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(100_000_000)                 # tens of milliseconds
+        plan.run(B, C)
+        done.record()
+    assert not done.query()
+    del plan
+    assert done.query()
