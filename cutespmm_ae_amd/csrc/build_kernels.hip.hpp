@@ -318,6 +318,8 @@ __device__ __forceinline__ uint32_t half(const Two &v, uint32_t s) { return ((s 
 
 // The panel kernels take every panel of up to CAP entries (list_of = nullptr), or the panels of a list (with CAP = kPanelCap; a
 // second launch over all panels would spend 15 us on work-groups that only leave).
+// A launch has at most 2^32 - 1 threads along a dimension of its grid, so all panels are kPanelRow to a row of the grid.
+constexpr uint32_t kPanelRow = 1u << 22;
 template <uint32_t CAP>
 __global__ __launch_bounds__(panel_threads(CAP)) void panel_census(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols,
                                                          const float *__restrict__ vals, uint32_t P, uint32_t K, uint32_t nnz, uint32_t max_span,
@@ -326,7 +328,8 @@ __global__ __launch_bounds__(panel_threads(CAP)) void panel_census(const uint32_
     extern __shared__ uint32_t window[];
     __shared__ PanelLds<CAP> l;
     __shared__ PanelCensus res;
-    const uint32_t p = list_of ? list_of[blockIdx.x] : blockIdx.x, t = threadIdx.x;
+    const uint32_t p = list_of ? list_of[blockIdx.x] : blockIdx.y * gridDim.x + blockIdx.x, t = threadIdx.x;
+    if (p >= P) return;
     uint32_t start;
     if (t < 12u) reinterpret_cast<uint32_t *>(&res)[t] = 0u;
     const uint32_t n = panel_rows(l, rowPtr, p, P, nnz, start);
@@ -381,7 +384,8 @@ __global__ __launch_bounds__(panel_threads(CAP)) void panel_bricks(const uint32_
 {
     extern __shared__ uint32_t window[];
     __shared__ PanelLds<CAP> l;
-    const uint32_t p = list_of ? list_of[blockIdx.x] : blockIdx.x, t = threadIdx.x;
+    const uint32_t p = list_of ? list_of[blockIdx.x] : blockIdx.y * gridDim.x + blockIdx.x, t = threadIdx.x;
+    if (p >= P) return;
     if (!list_of && p == 0u && t < 64u) tile_vals[uint64_t(nnz) + t] = 0.0f;
     const uint32_t block0 = brp[p];
     uint32_t start;
@@ -445,7 +449,8 @@ __global__ __launch_bounds__(panel_threads(CAP)) void panel_quads(const uint32_t
     extern __shared__ uint32_t window[];
     __shared__ PanelLds<CAP> l;
     __shared__ uint16_t list[CAP], place[CAP];    // pair -> active column, and -> its first value from the panel's first
-    const uint32_t p = list_of ? list_of[blockIdx.x] : blockIdx.x, t = threadIdx.x;
+    const uint32_t p = list_of ? list_of[blockIdx.x] : blockIdx.y * gridDim.x + blockIdx.x, t = threadIdx.x;
+    if (p >= P) return;
     if (!list_of && p == 0u && t < 64u) packed[uint64_t(stored) + t] = 0.0f;
     const uint32_t group0 = groups[uint64_t(p) * (STRIPS ? 4u : 1u)], value0 = valBase[p];
     uint32_t start;

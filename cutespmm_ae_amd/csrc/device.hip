@@ -540,6 +540,7 @@ struct PinnedBuf {
     template <class T> T *as(uint64_t offset = 0) const { return Layout::at<T>(p, offset); }
 };
 
+inline dim3 panel_grid(uint32_t n) { return dim3(std::min(n, cute_build::kPanelRow), (n + cute_build::kPanelRow - 1u) / cute_build::kPanelRow); }
 inline dim3 grid_of(uint64_t n) { return dim3(uint32_t(std::max<uint64_t>((n + cute_build::kThreads - 1) / cute_build::kThreads, 1))); }
 // for kernels that walk their range with a stride
 inline dim3 grid_capped(uint64_t n) { return dim3(std::min<uint32_t>(grid_of(n).x, 4096u)); }
@@ -549,7 +550,7 @@ int check_launch(const char *what);
 #define CUTE_BUILD(kernel, grid, ...) CUTE_BUILD_LDS(kernel, grid, 0, __VA_ARGS__)
 #define CUTE_BUILD_LDS(kernel, grid, lds, ...) hipLaunchKernelGGL(kernel, grid, dim3(cute_build::kThreads), lds, nullptr, __VA_ARGS__)
 // a panel kernel of the given capacity over `count` panels: all of them, or a list
-#define CUTE_PANELS(kernel, CAP, count, lds, ...) hipLaunchKernelGGL(kernel, dim3(count), dim3(cute_build::panel_threads(CAP)), lds, nullptr, __VA_ARGS__)
+#define CUTE_PANELS(kernel, CAP, count, lds, ...) hipLaunchKernelGGL(kernel, panel_grid(count), dim3(cute_build::panel_threads(CAP)), lds, nullptr, __VA_ARGS__)
 
 // The widest column window the panel kernels take on this matrix, and the LDS its bitmap and running counts need.
 inline uint32_t max_span(const cute_hrpb_dev *d) { return std::min(d->K, cute_build::kPanelSpan); }

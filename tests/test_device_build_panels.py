@@ -92,3 +92,26 @@ def test_handles_and_plans_come_and_go(cs, orc, torch_cuda):
     torch.cuda.synchronize()
     for k, C in outs:
         assert (C.cpu().numpy() == refs[k]).all()
+
+
+def test_more_panels_than_one_grid_row_holds(cs, torch_cuda):
+    """2^28 rows and a panel: 256 threads a panel are more than 2^32 threads in a row of the grid."""
+    torch = torch_cuda
+    M, K, N = (1 << 28) + 16, 64, 1
+    rng = np.random.default_rng(12)
+    per = 1 << 22                                                          # panels to a row of the grid
+    rows = np.unique(np.concatenate([[0, 15, 16, 16 * per - 1, 16 * per, 32 * per, M - 17, M - 16, M - 1], rng.integers(0, M, 4000)]))
+    counts = rng.integers(1, 9, rows.size)
+    cl = np.concatenate([np.sort(rng.choice(K, c, replace=False)) for c in counts]).astype(np.int32)
+    vl = rng.integers(-4, 5, cl.size).astype(np.float32)
+    starts = torch.from_numpy(np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)).cuda()
+    rp = starts[torch.searchsorted(torch.from_numpy(rows).cuda(), torch.arange(M + 1, device="cuda"))]
+    B = rng.integers(-4, 5, (K, N)).astype(np.float32)
+    C = torch.full((M, N), float("nan"), device="cuda")
+    plan = cs.SPMM_TC(cs.DeviceHRPB(M, K, rp, torch.from_numpy(cl).cuda(), torch.from_numpy(vl).cuda()), N)
+    plan.run(torch.from_numpy(B).cuda(), C)
+    want = np.zeros((rows.size, N))
+    np.add.at(want, np.repeat(np.arange(rows.size), counts), vl[:, None].astype(np.float64) * B[cl])
+    assert torch.equal(C[torch.from_numpy(rows).cuda()].cpu(), torch.from_numpy(want).float())       # whole numbers: exact
+    C[torch.from_numpy(rows).cuda()] = 0.0
+    assert int(torch.count_nonzero(C)) == 0                                # (a NaN counts)
