@@ -364,6 +364,17 @@ namespace {
 
 // ---- building the layouts on the device (kernels: build_kernels.hip.hpp) ----
 
+// Waits for every stream of the device as hipFree does, by freeing a page (1.2 us).  Not hipDeviceSynchronize, which breaks a
+// capture under way on any stream; hipFree is allowed beside a capture in relaxed mode, and a handle may be collected in the
+// middle of one.
+bool wait_for_device()
+{
+    void *page = nullptr;
+    if (hipMalloc(&page, 4096) == hipSuccess) return hipFree(page) == hipSuccess;
+    (void)hipGetLastError();
+    return false;
+}
+
 // Device memory of handles, plans and their set-up.  hipMalloc and hipFree of a megabyte or more cost 25 to 50 us each (a new
 // graph's product, 65 536 nodes: 300 us of 900 went there), so released blocks wait here for the next caller.  Bounded: at
 // most kIdleBytes in kIdleBlocks blocks, none that the last kIdleUses releases have not touched; the rest goes back to the
@@ -379,15 +390,6 @@ class DevicePool {
     std::unordered_map<void *, std::pair<uint64_t, int>> out_;
     uint64_t idleBytes_ = 0, clock_ = 0;
 
-    // What hipFree does before it frees, through a block of a page (1.2 us).  Not hipDeviceSynchronize, which breaks a capture
-    // under way on any stream; hipFree is allowed beside a capture in relaxed mode, and a handle may be collected in the middle of one.
-    static bool wait_for_device()
-    {
-        void *page = nullptr;
-        if (hipMalloc(&page, 4096) == hipSuccess) return hipFree(page) == hipSuccess;
-        (void)hipGetLastError();
-        return false;
-    }
     void drop(size_t i)
     {
         idleBytes_ -= idle_[i].bytes;
@@ -1033,6 +1035,8 @@ int cute_hrpb_upload_device_csr(uint32_t M, uint32_t K, uint32_t nnz, const uint
                    d->dRowPtr, d->dCols, reinterpret_cast<uint32_t *>(d->dCsrVals));
         rc = finish_upload(d, quad_layout, c);
     }
+    // (set-up itself waits for the default stream only; the interface promises the device)
+    if (rc == CUTE_OK && !wait_for_device()) rc = hip_fail(hipErrorUnknown, "waiting for the device", __LINE__);
     if (rc != CUTE_OK) { cute_hrpb_dev_free(d); return rc; }
     *out = d;
     return CUTE_OK;

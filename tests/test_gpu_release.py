@@ -32,6 +32,23 @@ def test_release_beside_a_relaxed_capture(cs, torch_cuda, rows):
         torch.cuda.synchronize()
 
 
+def test_format_from_device_arrays_waits_for_the_device(cs, torch_cuda):
+    """cute_hrpb_upload_device_csr promises it, whatever the construction itself has to wait for."""
+    torch = torch_cuda
+    _plan(cs, torch, 4096, 32)
+    side, done = torch.cuda.Stream(), torch.cuda.Event()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(100_000_000)
+        done.record()
+    rp = torch.arange(0, 513, dtype=torch.int32, device="cuda")
+    cl, vl = torch.zeros(512, dtype=torch.int32, device="cuda"), torch.ones(512, device="cuda")
+    assert not done.query()
+    handle = cs.DeviceHRPB(512, 512, rp, cl, vl)
+    assert done.query()
+    del handle
+
+
 def test_release_waits_for_running_kernels(cs, torch_cuda):
     """The block may serve another thread's set-up at once, so a release returns only when every stream is done with it."""
     torch = torch_cuda
