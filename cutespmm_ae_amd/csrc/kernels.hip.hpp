@@ -1166,7 +1166,8 @@ __global__ __launch_bounds__(256) void csr_rows(const uint32_t *__restrict__ row
 // element still accumulates its row in storage order.
 // AHEAD: the entries of the next round are asked for ahead of this round's B rows (loads return in order), so a row longer than
 // a round waits for one round trip per round, not for two (131 072 rows of 20, N = 64: 93.2 -> 89.4 us).  The fused kernels
-// leave that out where the entries take several registers: their 64 would not do.
+// leave that out where the entries take several registers: their 64 would not do (nor would they for entries that are held
+// from one round to the next in any other way: a register spilled to scratch in four of them).
 template <int VEC, int LOG_L, int BATCH, bool AHEAD>
 __device__ __forceinline__ void rows_batched_body(uint32_t block_id, uint32_t slab, const uint4 *__restrict__ row_list,
                                                   uint32_t num_rows, const uint32_t *__restrict__ rowPtr,
@@ -1214,9 +1215,10 @@ __device__ __forceinline__ void rows_batched_body(uint32_t block_id, uint32_t sl
         }
     };
     Entries mine, next;
-    fetch(s, mine);
+    if (AHEAD) fetch(s, mine);
     for (uint32_t base = s; base < e; base += ROUND) {
         if (AHEAD) fetch(base + ROUND, next);
+        else fetch(base, mine);
         const uint32_t cnt = min(ROUND, e - base);
         for (uint32_t q0 = 0; q0 < cnt; q0 += STEP) {
             V b[STEP];
@@ -1235,7 +1237,6 @@ __device__ __forceinline__ void rows_batched_body(uint32_t block_id, uint32_t sl
             for (uint32_t u = 0; u < STEP; ++u) acc += a[u] * b[u];
         }
         if (AHEAD) mine = next;
-        else if (base + ROUND < e) fetch(base + ROUND, mine);
     }
     if (live) store_vec_streaming<VEC>(acc, C + size_t(row) * N + c0);
 }
