@@ -1167,7 +1167,9 @@ __global__ __launch_bounds__(256) void csr_rows(const uint32_t *__restrict__ row
 // AHEAD: the entries of the next round are asked for ahead of this round's B rows (loads return in order), so a row longer than
 // a round waits for one round trip per round, not for two (131 072 rows of 20, N = 64: 93.2 -> 89.4 us).  The fused kernels
 // leave that out where the entries take several registers: their 64 would not do (nor would they for entries that are held
-// from one round to the next in any other way: a register spilled to scratch in four of them).
+// from one round to the next in any other way: a register spilled to scratch in four of them).  They also leave it out for
+// sixteen lanes a row in row order, where most rows are one round and the lists fill the launch: R-MAT graph of 131 072 nodes,
+// N = 64: 45.5 us with it, 45.0 without; by columns, N = 128: 95.8 and 96.4.
 template <int VEC, int LOG_L, int BATCH, bool AHEAD>
 __device__ __forceinline__ void rows_batched_body(uint32_t block_id, uint32_t slab, const uint4 *__restrict__ row_list,
                                                   uint32_t num_rows, const uint32_t *__restrict__ rowPtr,
@@ -1282,7 +1284,7 @@ __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, 8) void hrpb_quad_rows_f
         uint32_t block_id;
         const uint32_t x = xcd_share(bid, slab, COLUMNS ? row_column_slabs : 0u);
         if (!xcd_range_id(row_ranges, bid, x, block_id)) return;
-        rows_batched_body<4, LOG_L, 8, (LOG_L > 3)>(block_id, slab, row_list, num_rows, rowPtr, cols, vals, B, C, N);
+        rows_batched_body<4, LOG_L, 8, (LOG_L > 4 || COLUMNS)>(block_id, slab, row_list, num_rows, rowPtr, cols, vals, B, C, N);
     }
 }
 
