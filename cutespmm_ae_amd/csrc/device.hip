@@ -169,11 +169,30 @@ int static_scratch(void **out)
     return CUTE_OK;
 }
 
+void drop_idle_device_memory();
+
+// hipMalloc; when there is no memory left, once more without the idle blocks of the pool below.  (An error that is returned is not
+// left behind for the next launch to find.)
+hipError_t device_malloc(void **out, uint64_t bytes)
+{
+    hipError_t e = hipMalloc(out, std::max<uint64_t>(bytes, 16));
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        drop_idle_device_memory();
+        e = hipMalloc(out, std::max<uint64_t>(bytes, 16));
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        *out = nullptr;
+    }
+    return e;
+}
+
 template <class T>
 int upload(T **dst, const T *src, uint64_t count)
 {
     *dst = nullptr;
-    HIP_TRY(hipMalloc(reinterpret_cast<void **>(dst), std::max<uint64_t>(count, 1) * sizeof(T)));
+    HIP_TRY(device_malloc(reinterpret_cast<void **>(dst), count * sizeof(T)));
     if (count) HIP_TRY(hipMemcpy(*dst, src, count * sizeof(T), hipMemcpyHostToDevice));
     return CUTE_OK;
 }
@@ -401,29 +420,24 @@ public:
     int take(void **out, uint64_t bytes)
     {
         *out = nullptr;
-        if (bytes < kPooledBlock) { HIP_TRY(hipMalloc(out, std::max<uint64_t>(bytes, 16))); return CUTE_OK; }
+        if (bytes < kPooledBlock) { HIP_TRY(device_malloc(out, bytes)); return CUTE_OK; }
         // eight sizes to an octave: matrices of nearly the same size meet in one
         const uint64_t step = 1ull << (60 - __builtin_clzll(bytes));
         bytes = (bytes + step - 1) / step * step;
         int device = 0;
         HIP_TRY(hipGetDevice(&device));
-        std::lock_guard<std::mutex> g(lock_);
-        for (size_t i = idle_.size(); i-- > 0;)
-            if (idle_[i].bytes == bytes && idle_[i].device == device) {
-                *out = idle_[i].p;
-                idleBytes_ -= bytes;
-                idle_.erase(idle_.begin() + std::ptrdiff_t(i));
-                break;
-            }
-        if (!*out) {
-            hipError_t e = hipMalloc(out, bytes);
-            if (e != hipSuccess && !idle_.empty()) {
-                (void)hipGetLastError();
-                while (!idle_.empty()) drop(idle_.size() - 1);
-                e = hipMalloc(out, bytes);
-            }
-            if (e != hipSuccess) { *out = nullptr; return hip_fail(e, "device memory", __LINE__); }
+        {
+            std::lock_guard<std::mutex> g(lock_);
+            for (size_t i = idle_.size(); i-- > 0;)
+                if (idle_[i].bytes == bytes && idle_[i].device == device) {
+                    *out = idle_[i].p;
+                    idleBytes_ -= bytes;
+                    idle_.erase(idle_.begin() + std::ptrdiff_t(i));
+                    break;
+                }
         }
+        if (!*out) HIP_TRY(device_malloc(out, bytes));
+        std::lock_guard<std::mutex> g(lock_);
         out_[*out] = {bytes, device};
         return CUTE_OK;
     }
@@ -448,6 +462,11 @@ public:
         idleBytes_ += bytes;
         while (idle_.size() > kIdleBlocks || idleBytes_ > kIdleBytes || idle_.front().used + kIdleUses < clock_) drop(0);
     }
+    void drop_all()
+    {
+        std::lock_guard<std::mutex> g(lock_);
+        while (!idle_.empty()) drop(idle_.size() - 1);
+    }
 };
 
 DevicePool &pool()
@@ -457,6 +476,7 @@ DevicePool &pool()
 }
 
 void give_device_memory(void *p) { pool().give(p); }
+void drop_idle_device_memory() { pool().drop_all(); }
 
 struct DevBuf {                       // device memory that lives as long as a scope
     void *p = nullptr;
@@ -971,7 +991,7 @@ int make_hub_tables(cute_spmm_plan *p, const cute_hrpb_dev *d, uint32_t hub_rows
     HIP_TRY(hipMemcpy(slots.p, slot_of.data(), uint64_t(d->K) * 4u, hipMemcpyHostToDevice));
     rc = upload(&p->dHubRows, order.data(), used);
     if (rc != CUTE_OK) return rc;
-    HIP_TRY(hipMalloc(reinterpret_cast<void **>(&p->dHubRecs), std::max<uint64_t>(G * CUTE_QUAD_RECORD_WORDS * 4u, 16u)));
+    HIP_TRY(device_malloc(reinterpret_cast<void **>(&p->dHubRecs), G * CUTE_QUAD_RECORD_WORDS * 4u));
     hipLaunchKernelGGL(cute_build::mark_hub_columns, grid_of(G * CUTE_QUAD_RECORD_WORDS), dim3(cute_build::kThreads), 0, nullptr,
                        d->dQRecs, G, slots.as<const uint32_t>(), uint32_t(cute_dev::kHubFlag), p->dHubRecs);
     rc = check_launch("hub records");
@@ -1036,7 +1056,10 @@ int cute_hrpb_upload_device_csr(uint32_t M, uint32_t K, uint32_t nnz, const uint
         rc = finish_upload(d, quad_layout, c);
     }
     // (set-up itself waits for the default stream only; the interface promises the device)
-    if (rc == CUTE_OK && !wait_for_device()) rc = hip_fail(hipErrorUnknown, "waiting for the device", __LINE__);
+    if (rc == CUTE_OK && !wait_for_device()) {
+        const hipError_t e = hipDeviceSynchronize();     // (not a page left to free)
+        if (e != hipSuccess) rc = hip_fail(e, "waiting for the device", __LINE__);
+    }
     if (rc != CUTE_OK) { cute_hrpb_dev_free(d); return rc; }
     *out = d;
     return CUTE_OK;
@@ -2178,7 +2201,7 @@ float cute_gpu_csr_spmm(const uint32_t *rowPtr, const uint32_t *cols, const floa
     if (rc == CUTE_OK) rc = upload(&dCl, cols, nnz);
     if (rc == CUTE_OK) rc = upload(&dV, vals, nnz);
     if (rc == CUTE_OK) rc = upload(&dB, hB, uint64_t(k) * n);
-    if (rc == CUTE_OK && hipMalloc(reinterpret_cast<void **>(&dC), uint64_t(m) * n * sizeof(float)) != hipSuccess)
+    if (rc == CUTE_OK && device_malloc(reinterpret_cast<void **>(&dC), uint64_t(m) * n * sizeof(float)) != hipSuccess)
         rc = CUTE_ERR_HIP;
     if (rc == CUTE_OK) rc = csr_launch(alg, dR, dCl, dV, dB, dC, m, n, nullptr);
     if (rc == CUTE_OK && (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess)) rc = CUTE_ERR_HIP;

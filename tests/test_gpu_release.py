@@ -62,3 +62,27 @@ def test_release_waits_for_running_kernels(cs, torch_cuda):
     assert not done.query()
     del plan
     assert done.query()
+
+
+def _free(torch):
+    torch.cuda.synchronize()
+    return torch.cuda.mem_get_info()[0]
+
+
+def test_an_allocation_that_fails_gives_the_kept_blocks_back_first(cs, torch_cuda):
+    """A Blocked-ELL upload of a tebibyte is refused whatever the card holds; the memory kept from freed handles has gone back by
+    then, and the error is not found again by the next product."""
+    import ctypes
+    torch = torch_cuda
+    plan, B, C = _plan(cs, torch, 4096, 32)
+    drop, _, _ = _plan(cs, torch, 524288, 32)                  # 64 MiB of entries
+    del drop
+    before = _free(torch)
+    index, value = np.zeros(1, np.int32), np.zeros(1, np.float32)
+    ell = cs.cute_blocked_ell(1 << 19, 1, 1, 1, 1, index.ctypes.data_as(cs.i32p), value.ctypes.data_as(cs.f32p))
+    handle = ctypes.c_void_p()
+    rc = cs.load_library().cute_blocked_ell_upload(ctypes.byref(ell), ctypes.byref(handle))
+    assert rc == -7 and not handle.value
+    assert _free(torch) - before >= 64 << 20
+    plan.run(B, C)
+    torch.cuda.synchronize()
