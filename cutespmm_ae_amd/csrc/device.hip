@@ -399,7 +399,7 @@ bool wait_for_device()
 // most kIdleBytes in kIdleBlocks blocks, none that the last kIdleUses releases have not touched; the rest goes back to the
 // driver, and all of it does when an allocation fails.  Like hipFree, a release waits for the device first, so no kernel of
 // any stream still uses a block that another thread is given; a block stays with its device.
-constexpr uint64_t kIdleBytes = 512ull << 20, kPooledBlock = 1ull << 20, kIdleUses = 64;
+constexpr uint64_t kIdleBytes = 512ull << 20, kPooledBlock = 1ull << 20, kLargestIdle = kIdleBytes / 4u, kIdleUses = 64;
 constexpr size_t kIdleBlocks = 32;
 
 class DevicePool {
@@ -420,7 +420,8 @@ public:
     int take(void **out, uint64_t bytes)
     {
         *out = nullptr;
-        if (bytes < kPooledBlock) { HIP_TRY(device_malloc(out, bytes)); return CUTE_OK; }
+        // (a block that will not be kept is as large as it was asked for)
+        if (bytes < kPooledBlock || bytes > kLargestIdle) { HIP_TRY(device_malloc(out, bytes)); return CUTE_OK; }
         // eight sizes to an octave: matrices of nearly the same size meet in one
         const uint64_t step = 1ull << (60 - __builtin_clzll(bytes));
         bytes = (bytes + step - 1) / step * step;
@@ -455,7 +456,7 @@ public:
                 out_.erase(it);
             }
         }
-        if (!bytes || bytes > kIdleBytes / 4u || !wait_for_device()) { (void)hipFree(p); return; }
+        if (!bytes || !wait_for_device()) { (void)hipFree(p); return; }
         std::lock_guard<std::mutex> g(lock_);
         ++clock_;
         idle_.push_back({p, bytes, device, clock_});

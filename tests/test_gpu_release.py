@@ -1,4 +1,6 @@
 """Handles and plans released while other work is under way: a stream being captured, kernels still running."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -69,20 +71,39 @@ def _free(torch):
     return torch.cuda.mem_get_info()[0]
 
 
+def _refused(cs):
+    """A Blocked-ELL upload of a tebibyte."""
+    index, value = np.zeros(1, np.int32), np.zeros(1, np.float32)
+    ell = cs.cute_blocked_ell(1 << 19, 1, 1, 1, 1, index.ctypes.data_as(cs.i32p), value.ctypes.data_as(cs.f32p))
+    handle = ctypes.c_void_p()
+    assert cs.load_library().cute_blocked_ell_upload(ctypes.byref(ell), ctypes.byref(handle)) == -7 and not handle.value
+
+
 def test_an_allocation_that_fails_gives_the_kept_blocks_back_first(cs, torch_cuda):
     """A Blocked-ELL upload of a tebibyte is refused whatever the card holds; the memory kept from freed handles has gone back by
     then, and the error is not found again by the next product."""
-    import ctypes
     torch = torch_cuda
     plan, B, C = _plan(cs, torch, 4096, 32)
     drop, _, _ = _plan(cs, torch, 524288, 32)                  # 64 MiB of entries
     del drop
     before = _free(torch)
-    index, value = np.zeros(1, np.int32), np.zeros(1, np.float32)
-    ell = cs.cute_blocked_ell(1 << 19, 1, 1, 1, 1, index.ctypes.data_as(cs.i32p), value.ctypes.data_as(cs.f32p))
-    handle = ctypes.c_void_p()
-    rc = cs.load_library().cute_blocked_ell_upload(ctypes.byref(ell), ctypes.byref(handle))
-    assert rc == -7 and not handle.value
+    _refused(cs)
     assert _free(torch) - before >= 64 << 20
     plan.run(B, C)
     torch.cuda.synchronize()
+
+
+def test_a_block_too_large_to_keep_is_as_large_as_asked_for(cs, torch_cuda):
+    """131 MiB of entries and row pointers, between two of the sizes that kept blocks are rounded to (128 and 144 MiB), and no
+    layout beside them (every panel is the row kernel's)."""
+    torch = torch_cuda
+    M, per = 1040000, 16
+    rp = torch.arange(0, M * per + 1, per, dtype=torch.int32, device="cuda")
+    cl = torch.arange(16 * per, dtype=torch.int32, device="cuda").repeat(M // 16)      # the rows of a panel share no column
+    vl = torch.ones(M * per, device="cuda")
+    _refused(cs)                                       # nothing idle that the construction could take or give back
+    before = _free(torch)
+    handle = cs.DeviceHRPB(M, 16 * per, rp, cl, vl)
+    used, asked = before - _free(torch), handle.device_bytes()
+    del handle
+    assert 130 << 20 <= asked <= 132 << 20 and abs(used - asked) <= 4 << 20, (used, asked)
