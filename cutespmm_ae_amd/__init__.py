@@ -29,7 +29,7 @@ ABI_SYMBOLS = [
     "cute_hrpb_upload", "cute_hrpb_upload_layout", "cute_hrpb_upload_device_csr", "cute_hrpb_dev_layout_sizes",
     "cute_hrpb_dev_read_layouts", "cute_hrpb_dev_free", "cute_hrpb_dev_bytes", "cute_hrpb_dev_csr",
     "cute_spmm_plan_create", "cute_spmm_plan_info", "cute_spmm_plan_free", "cute_spmm_run", "cute_spmm_run_static",
-    "cute_spmm_run_scratch", "cute_spmm_plan_scratch_bytes", "cute_device_layout",
+    "cute_spmm_run_scratch", "cute_spmm_plan_scratch_bytes", "cute_device_layout", "cute_release_idle_memory",
     "cute_csr_spmm_dev", "cute_gpu_csr_spmm", "cute_spmm_time", "cute_csr_spmm_time",
     "cute_device_info",
     "cute_coo_read", "cute_coo_save_mtx", "cute_coo_release", "cute_coo_to_csr", "cute_csr_i32_release",
@@ -208,6 +208,8 @@ def load_library():
     lib.cute_spmm_run_scratch.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_uint64]
     lib.cute_spmm_plan_scratch_bytes.restype = C.c_uint64
     lib.cute_spmm_plan_scratch_bytes.argtypes = [C.c_void_p]
+    lib.cute_release_idle_memory.argtypes = []
+    lib.cute_release_idle_memory.restype = None
     lib.cute_device_layout.argtypes = [C.POINTER(C.c_int), C.POINTER(C.c_int), C.POINTER(C.c_uint64), C.POINTER(C.c_int)]
     lib.cute_csr_spmm_dev.argtypes = [C.c_int, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p,
                                       C.c_uint32, C.c_uint32, C.c_void_p]
@@ -828,6 +830,12 @@ def backward_error(rowPtr, cols, vals, B, C_ref, C_test):
     return float(load_library().cute_backward_error(_ptr(rowPtr, u32p), _ptr(cols, u32p), _ptr(vals, f32p),
                                                     _ptr(B, f32p), _ptr(a, f32p), _ptr(b, f32p),
                                                     len(rowPtr) - 1, B.shape[1]))
+
+
+def release_idle_memory():
+    """Gives back the device and pinned memory the library keeps from freed handles and plans for the next ones (at most 512 and
+    32 MiB); ``torch.cuda.empty_cache()`` does not reach it."""
+    load_library().cute_release_idle_memory()
 
 
 def device_info():

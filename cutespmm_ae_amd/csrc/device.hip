@@ -229,7 +229,7 @@ struct cute_hrpb_dev {
     std::vector<uint32_t> panelStored;  // entries of each panel that are not zero (what the quad lists store)
 };
 
-namespace { void give_device_memory(void *p); }
+namespace { void give_device_memory(void *p); void drop_idle_pinned_memory(); }
 
 struct cute_spmm_plan {
     const cute_hrpb_dev *d = nullptr;
@@ -351,6 +351,12 @@ int cute_device_info(int *num_cus, int *wave_size, char *arch_name, size_t arch_
     if (wave_size) *wave_size = c.wave_size;
     if (arch_name && arch_cap) std::snprintf(arch_name, arch_cap, "%s", c.arch.c_str());
     return CUTE_OK;
+}
+
+void cute_release_idle_memory(void)
+{
+    drop_idle_device_memory();
+    drop_idle_pinned_memory();
 }
 
 int cute_device_layout(int *num_xcds, int *cus_per_xcd, uint64_t *cache_bytes, int *whole_chip)
@@ -562,6 +568,16 @@ struct PinnedBuf {
     }
     template <class T> T *as(uint64_t offset = 0) const { return Layout::at<T>(p, offset); }
 };
+
+void drop_idle_pinned_memory()
+{
+    std::vector<std::pair<void *, uint64_t>> idle;
+    {
+        std::lock_guard<std::mutex> g(g_pinned_lock);
+        idle.swap(g_pinned);
+    }
+    for (const auto &b : idle) (void)hipHostFree(b.first);
+}
 
 inline dim3 panel_grid(uint32_t n) { return dim3(std::min(n, cute_build::kPanelRow), (n + cute_build::kPanelRow - 1u) / cute_build::kPanelRow); }
 inline dim3 grid_of(uint64_t n) { return dim3(uint32_t(std::max<uint64_t>((n + cute_build::kThreads - 1) / cute_build::kThreads, 1))); }

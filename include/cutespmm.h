@@ -539,6 +539,11 @@ int cute_device_info(int *num_cus, int *wave_size, char *arch_name, size_t arch_
  * is the whole chip (the model of where wavefronts land, which orders work items, is used there only).  Stands
  * where spmm.cu:290-690 tabulates resident warps, blocks and SM counts per machine. */
 int cute_device_layout(int *num_xcds, int *cus_per_xcd, uint64_t *cache_bytes, int *whole_chip);
+/* Memory of freed handles and plans stays with the library for the next ones: up to 512 MiB of device memory (blocks of 1 to
+ * 128 MiB, each given back once 64 others have been released after it) and up to 32 MiB of pinned host memory.  An allocation of
+ * the library that fails gives the device memory back by itself; this call gives back both, for the rest of the program (another
+ * allocator, another process).  Handles and plans that exist are untouched.  Like hipFree, not for a stream under capture. */
+void cute_release_idle_memory(void);
 
 #ifdef __cplusplus
 }

@@ -107,3 +107,20 @@ def test_a_block_too_large_to_keep_is_as_large_as_asked_for(cs, torch_cuda):
     used, asked = before - _free(torch), handle.device_bytes()
     del handle
     assert 130 << 20 <= asked <= 132 << 20 and abs(used - asked) <= 4 << 20, (used, asked)
+
+
+def test_idle_memory_is_given_back_on_request(cs, torch_cuda):
+    torch = torch_cuda
+    keep, B, C = _plan(cs, torch, 65536, 32)
+    want = keep.run(B, C).clone()
+    drop, _, _ = _plan(cs, torch, 524288, 32)                  # 64 MiB of entries
+    del drop
+    before = _free(torch)
+    cs.release_idle_memory()
+    freed = _free(torch) - before
+    assert freed >= 64 << 20
+    cs.release_idle_memory()
+    assert torch.equal(keep.run(B, C.zero_()), want)
+    again, B2, C2 = _plan(cs, torch, 65536, 32)
+    again.run(B2, C2)
+    torch.cuda.synchronize()
