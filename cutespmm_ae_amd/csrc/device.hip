@@ -1138,6 +1138,14 @@ int cute_spmm_plan_info(const cute_spmm_plan *p, cute_plan_info *out)
     return CUTE_OK;
 }
 
+int cute_spmm_plan_column_slabs(const cute_spmm_plan *p, uint32_t *mfma, uint32_t *rows)
+{
+    if (!p) return CUTE_ERR_ARG;
+    if (mfma) *mfma = p->info.numChunks ? p->columnSlabs : 0u;
+    if (rows) *rows = p->numRows ? p->rowColumnSlabs : 0u;
+    return CUTE_OK;
+}
+
 // Replaces SPMM_TC's constructor chain (spmm.cu:276-822).  The per-N launch shapes of
 // spmm.cu:11-101 and the occupancy table of spmm.cu:290-690 describe NVIDIA parts; here
 // the shape follows from wave64 MFMA tiles (16 lanes x VEC columns per group) and the slot

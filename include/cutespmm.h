@@ -466,6 +466,9 @@ typedef struct cute_spmm_plan cute_spmm_plan;
 int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *t /* may be NULL */,
                           cute_spmm_plan **out);
 int cute_spmm_plan_info(const cute_spmm_plan *p, cute_plan_info *out);
+/* In which order a plan's work-groups go to the XCDs: 0 by rows (an XCD owns consecutive rows), else by columns (an XCD owns an
+ * eighth of so many column slabs), for the MFMA kernel and for the row kernel of the plan. */
+int cute_spmm_plan_column_slabs(const cute_spmm_plan *p, uint32_t *mfma, uint32_t *rows);
 void cute_spmm_plan_free(cute_spmm_plan *p);
 /* dB [K x N], dC [M x N]: device pointers, row-major, 16-byte aligned.  Asynchronous on
  * `stream` (a hipStream_t, NULL = default stream).  C is fully overwritten: the caller

@@ -18,10 +18,10 @@ def _product(cs, torch, rp, cl, vl, M, K, N, seed, **kw):
     return B, out.cpu().numpy(), plan
 
 
-def _check(rp, cl, vl, B, out, M, N, rows):
+def _check(rp, cl, vl, B, out, M, N, rows, per_product=0.0):
     for r in rows:
         a, b = vl[rp[r]:rp[r + 1]].astype(np.float64), B[cl[rp[r]:rp[r + 1]]].astype(np.float64)
-        bound = 2.0 * max(1, len(a)) * 2.0 ** -24 * (np.abs(a) @ np.abs(b)) if len(a) else np.zeros(N)
+        bound = (2.0 * max(1, len(a)) * 2.0 ** -24 + per_product) * (np.abs(a) @ np.abs(b)) if len(a) else np.zeros(N)
         assert (np.abs(out[r] - (a @ b if len(a) else np.zeros(N))) <= bound + 1e-30).all(), r
 
 
@@ -42,14 +42,17 @@ def _random(M, K, per_row, seed, empty=0, hubs=0):
     return rp, cols, rng.standard_normal(cols.size).astype(np.float32)
 
 
-@pytest.mark.parametrize("M,K,per_row,N,empty,hubs", [
-    (8192, 8192, 7, 256, 0, 0), (8192, 16384, 5, 288, 500, 0), (8192, 8192, 7, 301, 0, 0), (8192, 8192, 9, 272, 40, 0),
-    (16384, 16384, 3, 128, 0, 0), (16384, 32768, 4, 96, 900, 0), (32768, 32768, 4, 64, 0, 0), (8192, 8192, 26, 320, 0, 0),
-    (32768, 40000, 18, 64, 0, 0), (16384, 36864, 17, 512, 0, 0), (16384, 16384, 20, 299, 0, 0), (16384, 16384, 6, 256, 100, 64),
-    (16384, 16384, 6, 310, 0, 64), (131072, 131072, 6, 128, 0, 320), (2048, 65536, 8, 544, 16, 0), (16384, 16384, 4, 1056, 0, 0)])
-def test_every_element_is_written_once_and_right(cs, torch_cuda, M, K, per_row, N, empty, hubs):
+@pytest.mark.parametrize("M,K,per_row,N,empty,hubs,slabs", [
+    (8192, 8192, 7, 256, 0, 0, (0, 8)), (8192, 16384, 5, 288, 500, 0, (0, 9)), (8192, 8192, 7, 301, 0, 0, (0, 5)),
+    (8192, 8192, 9, 272, 40, 0, (0, 9)), (16384, 16384, 3, 128, 0, 0, (0, 4)), (16384, 32768, 4, 96, 900, 0, (0, 3)),
+    (32768, 32768, 4, 64, 0, 0, (0, 2)), (8192, 8192, 26, 320, 0, 0, (0, 10)), (32768, 40000, 18, 64, 0, 0, (2, 0)),
+    (16384, 36864, 17, 512, 0, 0, (16, 0)), (16384, 16384, 20, 299, 0, 0, (5, 0)), (16384, 16384, 6, 256, 100, 64, (4, 4)),
+    (16384, 16384, 6, 310, 0, 64, (5, 0)), (131072, 131072, 6, 128, 0, 320, (2, 2)), (2048, 65536, 8, 544, 16, 0, (0, 17)),
+    (16384, 16384, 4, 1056, 0, 0, (0, 33)), (8192, 2048, 20, 256, 0, 0, (0, 0))])
+def test_every_element_is_written_once_and_right(cs, torch_cuda, M, K, per_row, N, empty, hubs, slabs):
     rp, cl, vl = _random(M, K, per_row, M + N, empty, hubs)
     B, out, plan = _product(cs, torch_cuda, rp, cl, vl, M, K, N, N)
+    assert plan.column_slabs == slabs
     assert np.isfinite(out).all()
     rng = np.random.default_rng(1)
     _check(rp, cl, vl, B, out, M, N, np.unique(np.concatenate([[0, 1, 15, 16, M // 8, M // 2 - 1, M - 17, M - 1], rng.integers(0, M, 300)])))
@@ -82,8 +85,31 @@ def test_forced_rows_give_the_bits_of_the_same_rows_in_row_order(cs, torch_cuda,
         plan = cs.SPMM_TC(cs.HRPB(M, K, rp, cols.ravel(), vl), N, path=cs.PATH_ROWS)
         out = torch_cuda.full((M, N), float("nan"), device="cuda")
         plan.run(torch_cuda.from_numpy(B).cuda(), out)
+        assert (plan.column_slabs[1] > 0) == (cols is far), plan.column_slabs
         outs.append(out)
     assert torch_cuda.equal(outs[0], outs[1])
+
+
+ROLLING, PIPELINED, BF16 = dict(mfma_shape=1), dict(mfma_shape=1, pipeline=2), dict(precision=1)
+
+
+@pytest.mark.parametrize("M,K,per_row,N,hubs,options,kernel,slabs", [
+    (8192, 8192, 20, 256, 0, ROLLING, "hrpb_brick_f32_rolling", (4, 0)), (8192, 8192, 20, 301, 0, ROLLING, "hrpb_brick_f32_rolling", (5, 0)),
+    (8192, 8192, 20, 256, 0, PIPELINED, "hrpb_brick_f32", (2, 0)), (8192, 8192, 20, 515, 0, PIPELINED, "hrpb_brick_f32", (5, 0)),
+    (8192, 16384, 20, 256, 0, BF16, "hrpb_brick_bf16x3", (4, 0)), (8192, 16384, 20, 320, 0, BF16, "hrpb_brick_bf16x3", (5, 0)),
+    (16384, 16384, 6, 256, 64, ROLLING, "hrpb_brick_rows_f32", (4, 1)), (16384, 16384, 6, 260, 64, ROLLING, "hrpb_brick_rows_f32", (5, 2)),
+    (16384, 16384, 6, 301, 64, ROLLING, "hrpb_brick_rows_f32", (5, 2)), (16384, 16384, 6, 260, 64, PIPELINED, "hrpb_brick_f32", (5, 2)),
+    (16384, 16384, 6, 512, 64, BF16, "hrpb_brick_bf16x3", (8, 2)), (8192, 2048, 20, 256, 0, ROLLING, "hrpb_brick_f32_rolling", (0, 0))])
+def test_bricks(cs, torch_cuda, M, K, per_row, N, hubs, options, kernel, slabs):
+    """The brick kernels by columns: alone, beside rows in one launch and in two, whole slabs and remainders, and once in row order;
+    bf16x3 drops at most 2^-15 of each product on top of the bound."""
+    rp, cl, vl = _random(M, K, per_row, M + N, 100 if hubs else 0, hubs)
+    B, out, plan = _product(cs, torch_cuda, rp, cl, vl, M, K, N, N, path=cs.PATH_AUTO if hubs else cs.PATH_BRICK, **options)
+    assert plan.kernel_name == kernel and plan.column_slabs == slabs, (plan.kernel_name, plan.column_slabs, plan.info)
+    assert np.isfinite(out).all()
+    rng = np.random.default_rng(1)
+    rows = np.unique(np.concatenate([np.arange(80), [M // 8, M // 2 - 1], np.arange(M - 40, M), rng.integers(0, M, 400)]))
+    _check(rp, cl, vl, B, out, M, N, rows, 2.0 ** -15 if plan.info["precision"] else 0.0)
 
 
 @pytest.mark.parametrize("layout", [1, 2])
