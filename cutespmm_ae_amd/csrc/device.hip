@@ -1399,6 +1399,11 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
     // graph of 32 768 nodes, N = 512 156 -> 104 us, 16 384 nodes, N = 256 33.5 -> 26.7, 131 072 nodes, N = 310 463 -> 413;
     // lists without reuse gain while the window fits two L2s (16 384 rows of 24, N = 512 46.4 -> 41.8; 65 536 rows 349 -> 367).
     // Off the 64-column grid the last slab is a remainder that unbalances few slabs (N = 101: 137 -> 147): 256 columns or more.
+    // The brick kernels' slabs are up to 128 columns wide, a row kernel's beside them 256, and a remainder unbalances few of those at any
+    // N: at least four times the width, or no remainder.  32 768 rows of 24 at random columns, us in row order / by columns: N = 300 109 / 120
+    // (bf16x3 111 / 122), N = 320 86.2 / 94.5 (83.5 / 96.2); 131 072-node graph, bf16x3, N = 300 337 / 355, and with the rows
+    // beside it in row order, 65 536 nodes, 185 / 189.  In fp32 a graph gains more than that costs (131 072 nodes, N = 257, 472 / 349).
+    auto balanced = [&](uint32_t width) { return N % width == 0 || N >= 4u * width; };
     uint32_t rows_columns = 0;
     bool mfma_by_columns = false;
     {
@@ -1414,14 +1419,18 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
         }
         if (scattered_nnz * 2u > uint64_t(d->nnz)) {
             const uint64_t mean_window[2] = {in[0] ? window[0] / in[0] : 0, in[1] ? window[1] / in[1] : 0};
+            const bool sharing = in[0] * 5u >= cols * 6u;
+            const uint32_t mfma_width = p->shape == 2 ? 64u : 16u * uint32_t(p->vec * p->ng);
             if (n_brick == 0)
                 rows_columns = narrow(mean_window[1], in[1] / (uint64_t(row_panels) * CUTE_TM));
             else if (half_window && p->shape == 2 && !t.hub_rows && n_rows == 0 && n_empty == 0 && (N + 31u) / 32u <= 65535u)
                 mfma_by_columns = p->halfLists = true;
-            else if (((N % 64u == 0 && N >= 128u) || N >= 256u) && (in[0] * 5u >= cols * 6u || mean_window[0] <= 32768u)) {
+            else if (((N % 64u == 0 && N >= 128u) || N >= 256u) &&
+                     (sharing || mean_window[0] <= 32768u) && ((sharing && !p->bf16x3) || balanced(mfma_width))) {
                 mfma_by_columns = true;
                 // rows of uneven length share a wavefront: sixteen lanes a row (the brick kernel has no launch with fewer than its own)
-                rows_columns = p->shape == 2 && p->rows_vec == 4 ? 64u : (p->rows_vec << p->rows_logl);
+                const uint32_t width = p->shape == 2 && p->rows_vec == 4 ? 64u : uint32_t(p->rows_vec << p->rows_logl);
+                rows_columns = p->bf16x3 && !balanced(width) ? 0u : width;
             }
         }
         // (slabs are the y dimension of the launch)

@@ -99,7 +99,12 @@ ROLLING, PIPELINED, BF16 = dict(mfma_shape=1), dict(mfma_shape=1, pipeline=2), d
     (8192, 16384, 20, 256, 0, BF16, "hrpb_brick_bf16x3", (4, 0)), (8192, 16384, 20, 320, 0, BF16, "hrpb_brick_bf16x3", (5, 0)),
     (16384, 16384, 6, 256, 64, ROLLING, "hrpb_brick_rows_f32", (4, 1)), (16384, 16384, 6, 260, 64, ROLLING, "hrpb_brick_rows_f32", (5, 2)),
     (16384, 16384, 6, 301, 64, ROLLING, "hrpb_brick_rows_f32", (5, 2)), (16384, 16384, 6, 260, 64, PIPELINED, "hrpb_brick_f32", (5, 2)),
-    (16384, 16384, 6, 512, 64, BF16, "hrpb_brick_bf16x3", (8, 2)), (8192, 2048, 20, 256, 0, ROLLING, "hrpb_brick_f32_rolling", (0, 0))])
+    (16384, 16384, 6, 512, 64, BF16, "hrpb_brick_bf16x3", (8, 2)), (8192, 2048, 20, 256, 0, ROLLING, "hrpb_brick_f32_rolling", (0, 0)),
+    # two slabs of 128 columns and a remainder: row order, unless an fp32 graph's panels share columns; three whole slabs: by columns
+    (32768, 32768, 24, 300, 0, ROLLING, "hrpb_brick_f32_rolling", (0, 0)), (32768, 32768, 24, 300, 0, BF16, "hrpb_brick_bf16x3", (0, 0)),
+    (32768, 32768, 24, 256, 0, BF16, "hrpb_brick_bf16x3", (2, 0)), (32768, 32768, 24, 640, 0, ROLLING, "hrpb_brick_f32_rolling", (5, 0)),
+    # the rows beside bf16x3 bricks: a slab of 256 columns and a remainder
+    (16384, 16384, 6, 260, 64, BF16, "hrpb_brick_bf16x3", (5, 0))])
 def test_bricks(cs, torch_cuda, M, K, per_row, N, hubs, options, kernel, slabs):
     """The brick kernels by columns: alone, beside rows in one launch and in two, whole slabs and remainders, and once in row order;
     bf16x3 drops at most 2^-15 of each product on top of the bound."""
