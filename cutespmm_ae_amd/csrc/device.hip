@@ -1381,11 +1381,13 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
     // 24 000 rows N = 128 20.1 / 15.7 / 23.8 / 32.8, N = 256 26.3 / 26.4 (equal T), N = 301 47.0 / 36.4; 2 400 rows N = 128
     // 19.0 / 13.2 / 10.6 / 10.5, N = 301 19.4 / 13.6 / 13.6 / 11.4; 4 800 rows N = 64 - / 10.7 / 8.1 / 8.5, N = 200
     // 16.7 / 13.9 / 15.9 / 14.9.  (Odd N gains from single columns a little longer: no other piece of its rows is aligned.)
+    // bf16x3 spends a third of the matrix time, and beside row panels the SIMDs are not idle: where its operands come from HBM
+    // the wide pieces count for more, as above.  131 072-node graph, 10 edges a node, us at 128 / 64 columns: N = 300 225 / 310, 384 227 / 310.
     if (p->shape == 1 && p->pipeline == 1 && t.brick_groups == 0 && n_brick) {
         const uint64_t simds = uint64_t(c.num_cus) * 4u;
         auto items = [&](uint32_t w) { return uint64_t(n_brick) * ((N + 16u * w - 1u) / (16u * w)); };
         auto T = [&](uint32_t w) { return (items(w) + simds - 1u) / simds * w; };
-        if (p->ng == 2 && items(4) <= 8u * simds && (T(4) < T(8) || items(8) <= simds)) {
+        if (p->ng == 2 && items(4) <= 8u * simds && ((T(4) < T(8) && !(p->bf16x3 && n_rows && beyond_cache)) || items(8) <= simds)) {
             p->ng = 1;
             ng_for_mixed = true;                  // (the fused launch has this shape)
         }
