@@ -1200,9 +1200,12 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
     // sixteen lanes a row ask for 256 bytes of B with one instruction, a list slot for the same with 64 lanes.  R-MAT graph
     // of 131 072 nodes and 2.5 million entries: N = 128 126 -> 92 us, N = 256 236 -> 228, N = 310 377 -> 320; below 2^24
     // elements of C the launch no longer fills the device and the long rows show (32 768 nodes, N = 128: 26 -> 33).
+    // Much of that comes from the columns an XCD owns: where the lists stay in row order (below 256 columns, off the grid of 64), graphs of 24
+    // entries a row lose (131 072 nodes, N = 208 235 -> 261, N = 240 263 -> 292; 20 entries a row 208 -> 203, 12 142 -> 134).
     const bool default_bars = t.path == CUTE_PATH_AUTO && t.min_reuse <= 0.0f && t.max_row_nnz == 0;
     auto scattered = [&](uint32_t q) { return uint64_t(d->panelSpan[q]) * std::min(N, 256u) * sizeof(float) > kScatteredBytes; };
-    const bool graph_bars = default_bars && t.precision == CUTE_PREC_FP32 && N >= 128u && uint64_t(d->M) * N >= kGraphProduct;
+    const bool graph_bars = default_bars && t.precision == CUTE_PREC_FP32 && N >= 128u && uint64_t(d->M) * N >= kGraphProduct &&
+                            (N % 64u == 0 || N >= 256u || N % 4u != 0 || uint64_t(d->nnz) < 22ull * d->M);
     auto fetches_of = [&](uint32_t q) {
         // what the MFMA side would fetch for this panel: one B row per list slot of the quad
         // lists (pairs plus padding), which is at least one per active column

@@ -117,6 +117,17 @@ def test_bricks(cs, torch_cuda, M, K, per_row, N, hubs, options, kernel, slabs):
     _check(rp, cl, vl, B, out, M, N, rows, 2.0 ** -15 if plan.info["precision"] else 0.0)
 
 
+def test_a_dense_graph_in_row_order_keeps_its_lists(cs, torch_cuda):
+    """131 072 nodes: the rule that moves panels with little reuse to the row kernel holds for 24 entries a row only by columns."""
+    for per_row, N, many in ((12, 208, False), (12, 256, True), (8, 208, True)):
+        A = cs.gen_matrix(4, 5, 17, per_row, 0)
+        rp, cl, vl = np.array(A.rowPtr), np.array(A.cols), np.array(A.vals)
+        B, out, plan = _product(cs, torch_cuda, rp, cl, vl, A.M, A.K, N, N)
+        assert (plan.info["numRowPanelsSparse"] > 5500) == many, (per_row, N, plan.info)
+        assert np.isfinite(out).all()
+        _check(rp, cl, vl, B, out, A.M, N, np.unique(np.concatenate([np.arange(40), np.random.default_rng(1).integers(0, A.M, 200)])))
+
+
 @pytest.mark.parametrize("layout", [1, 2])
 @pytest.mark.parametrize("M,K,per_row,N,cut", [(32768, 40000, 20, 64, 0), (32768, 40000, 24, 96, 3), (16384, 49152, 28, 288, 0),
                                                 (16384, 65536, 32, 512, 2), (32768, 90112, 16, 128, 1)])
