@@ -1408,6 +1408,9 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
     // N: at least four times the width, or no remainder.  32 768 rows of 24 at random columns, us in row order / by columns: N = 300 109 / 120
     // (bf16x3 111 / 122), N = 320 86.2 / 94.5 (83.5 / 96.2); 131 072-node graph, bf16x3, N = 300 337 / 355, and with the rows
     // beside it in row order, 65 536 nodes, 185 / 189.  In fp32 a graph gains more than that costs (131 072 nodes, N = 257, 472 / 349).
+    // Lists without reuse take a remainder of any size while the window is small (20 000 rows of 20, N = 264: 5 % ahead by columns), and up
+    // to two L2s one that leaves no more than a tenth idle (30 000 rows of 10, us in row order / by columns, N = 257 55.1 / 59.4,
+    // N = 280 26.1 / 27.5 at 4 entries; 24 000 rows of 4, N = 264 19.5 / 20.8; N = 301 equal).
     auto balanced = [&](uint32_t width) { return N % width == 0 || N >= 4u * width; };
     uint32_t rows_columns = 0;
     bool mfma_by_columns = false;
@@ -1431,7 +1434,8 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
             else if (half_window && p->shape == 2 && !t.hub_rows && n_rows == 0 && n_empty == 0 && (N + 31u) / 32u <= 65535u)
                 mfma_by_columns = p->halfLists = true;
             else if (((N % 64u == 0 && N >= 128u) || N >= 256u) &&
-                     (sharing || mean_window[0] <= 32768u) && ((sharing && !p->bf16x3) || balanced(mfma_width))) {
+                     (sharing || mean_window[0] <= 32768u) && ((sharing && !p->bf16x3) || balanced(mfma_width)) &&
+                     (sharing || mean_window[0] <= 20480u || (N + mfma_width - 1u) / mfma_width * mfma_width * 10u <= N * 11u)) {
                 mfma_by_columns = true;
                 // rows of uneven length share a wavefront: sixteen lanes a row (the brick kernel has no launch with fewer than its own)
                 const uint32_t width = p->shape == 2 && p->rows_vec == 4 ? 64u : uint32_t(p->rows_vec << p->rows_logl);

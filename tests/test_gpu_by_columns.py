@@ -95,7 +95,7 @@ ROLLING, PIPELINED, BF16 = dict(mfma_shape=1), dict(mfma_shape=1, pipeline=2), d
 
 @pytest.mark.parametrize("M,K,per_row,N,hubs,options,kernel,slabs", [
     (8192, 8192, 20, 256, 0, ROLLING, "hrpb_brick_f32_rolling", (4, 0)), (8192, 8192, 20, 301, 0, ROLLING, "hrpb_brick_f32_rolling", (5, 0)),
-    (8192, 8192, 20, 256, 0, PIPELINED, "hrpb_brick_f32", (2, 0)), (8192, 8192, 20, 515, 0, PIPELINED, "hrpb_brick_f32", (5, 0)),
+    (8192, 8192, 20, 256, 0, PIPELINED, "hrpb_brick_f32", (2, 0)), (8192, 8192, 20, 600, 0, PIPELINED, "hrpb_brick_f32", (5, 0)),
     (8192, 16384, 20, 256, 0, BF16, "hrpb_brick_bf16x3", (4, 0)), (8192, 16384, 20, 320, 0, BF16, "hrpb_brick_bf16x3", (5, 0)),
     (16384, 16384, 6, 256, 64, ROLLING, "hrpb_brick_rows_f32", (4, 1)), (16384, 16384, 6, 260, 64, ROLLING, "hrpb_brick_rows_f32", (5, 2)),
     (16384, 16384, 6, 301, 64, ROLLING, "hrpb_brick_rows_f32", (5, 2)), (16384, 16384, 6, 260, 64, PIPELINED, "hrpb_brick_f32", (5, 2)),
@@ -115,6 +115,17 @@ def test_bricks(cs, torch_cuda, M, K, per_row, N, hubs, options, kernel, slabs):
     rng = np.random.default_rng(1)
     rows = np.unique(np.concatenate([np.arange(80), [M // 8, M // 2 - 1], np.arange(M - 40, M), rng.integers(0, M, 400)]))
     _check(rp, cl, vl, B, out, M, N, rows, 2.0 ** -15 if plan.info["precision"] else 0.0)
+
+
+@pytest.mark.parametrize("M,per_row,N,kernel,slabs", [(30000, 20, 257, "hrpb_quad_f32", (0, 0)), (30000, 20, 301, "hrpb_quad_f32", (5, 0))])
+def test_lists_or_rows_off_the_grid_of_B(cs, torch_cuda, M, per_row, N, kernel, slabs):
+    """Widths off 128 bytes, both sides of the lines between the lists and the row kernel (its last walk over few columns), and of
+    the remainder that lists by columns take."""
+    rp, cl, vl = _random(M, M, per_row, M + N)
+    B, out, plan = _product(cs, torch_cuda, rp, cl, vl, M, M, N, N)
+    assert (plan.kernel_name, plan.column_slabs) == (kernel, slabs), (plan.kernel_name, plan.column_slabs)
+    assert np.isfinite(out).all()
+    _check(rp, cl, vl, B, out, M, N, np.unique(np.concatenate([np.arange(40), np.arange(M - 40, M), np.random.default_rng(1).integers(0, M, 300)])))
 
 
 def test_a_dense_graph_in_row_order_keeps_its_lists(cs, torch_cuda):
