@@ -1256,6 +1256,19 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
         if (N % 16u == 0) return window <= (mean_row < 16u ? 32768u : 8192u) ? 32u : 0u;
         return window <= (mean_row < 16u ? 16384u : 8192u) ? 64u : 0u;
     };
+    // The row kernel walks 256 columns at a time, and the last walk costs nearly a whole one however few columns are left; lists
+    // pay for pieces of 64.  Off the 128-byte grid of B, lists / row kernel in row order, us, 4 and 10 entries a row:
+    // 20 000 rows N = 264 16.4 / 18.7, 30.1 / 35.8, N = 301 37.1 / 40.3 (10), N = 600 equal; 30 000 rows N = 301 31.5 / 30.1;
+    // 40 000 rows N = 272 32.3 / 37.3, 64.6 / 78.0, N = 301 rows 7 % ahead, N = 432 rows 5 % ahead and 100 / 105, N = 528 60.3 / 64.4,
+    // 124 / 137, N = 600 159 / 147 (10); 65 536 rows N = 272 55.4 / 61.7, 117 / 129, N = 264 3 %, N = 280 equal, N = 528 222 / 233;
+    // 131 072 rows N = 272 116 / 124, N = 264 rows 3 % ahead, N = 528 3 %.
+    auto short_last_slab = [&](uint64_t window, uint64_t mean_row) {
+        const uint32_t last = N % 256u;
+        if (window <= 24576u) return last < 64u;
+        if (window <= 49152u) return (N % 8u == 0 && last <= 48u) || (N % 16u == 0 && mean_row >= 8u);
+        if (window <= 65536u) return N % 8u == 0 && last <= 16u;
+        return N % 16u == 0 && last <= 16u && N < 512u;
+    };
     bool half_window = false;
     // A matrix without reuse or hubs (less than a tenth of its entries in panels for the MFMA side): its scattered panels go to
     // the lists only where these are ahead of the row kernel in whichever order suits it.  24 entries a row, us row kernel /
@@ -1279,7 +1292,8 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
             half_window = N % 32u == 0 && (window > 32768u || N >= 512u) && window <= (N <= 128u ? 98304u : N < 512u ? 57344u : 65536u);
             const bool on_grid = N % 32u == 0, wide = N >= 512u && window > 32768u;
             const bool lists_ahead = on_grid ? (wide || (narrow(window, mean_row) == 0 && (mean_row >= 16u || N >= 256u)))
-                                             : (narrow(window, mean_row) == 0 && mean_row >= 16u && N >= 256u && window <= 65536u);
+                                             : (narrow(window, mean_row) == 0 && N >= 256u &&
+                                                ((mean_row >= 16u && window <= 65536u) || short_last_slab(window, mean_row)));
             for (uint32_t q = 0; q < d->P; ++q) {
                 if (!concerned(q)) continue;
                 const uint8_t rows = !(lists_ahead && N >= 64u && float(d->panelNnz[q]) >= kWideReuse * float(fetches_of(q)));

@@ -117,7 +117,11 @@ def test_bricks(cs, torch_cuda, M, K, per_row, N, hubs, options, kernel, slabs):
     _check(rp, cl, vl, B, out, M, N, rows, 2.0 ** -15 if plan.info["precision"] else 0.0)
 
 
-@pytest.mark.parametrize("M,per_row,N,kernel,slabs", [(30000, 20, 257, "hrpb_quad_f32", (0, 0)), (30000, 20, 301, "hrpb_quad_f32", (5, 0))])
+@pytest.mark.parametrize("M,per_row,N,kernel,slabs", [
+    (20000, 10, 301, "hrpb_quad_f32", (5, 0)), (20000, 10, 600, "csr_rows_batched", (0, 0)), (24000, 4, 264, "hrpb_quad_f32", (0, 0)),
+    (30000, 4, 264, "hrpb_quad_f32", (0, 0)), (30000, 4, 301, "csr_rows_batched", (0, 0)), (30000, 20, 257, "hrpb_quad_f32", (0, 0)),
+    (30000, 20, 301, "hrpb_quad_f32", (5, 0)), (40000, 10, 496, "hrpb_quad_f32", (0, 0)), (40000, 10, 600, "csr_rows_batched", (0, 0)),
+    (65536, 4, 272, "hrpb_quad_f32", (0, 0)), (65536, 4, 296, "csr_rows_batched", (0, 0))])
 def test_lists_or_rows_off_the_grid_of_B(cs, torch_cuda, M, per_row, N, kernel, slabs):
     """Widths off 128 bytes, both sides of the lines between the lists and the row kernel (its last walk over few columns), and of
     the remainder that lists by columns take."""
