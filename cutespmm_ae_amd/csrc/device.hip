@@ -23,7 +23,7 @@ thread_local std::string g_hip_error;
 constexpr float kMinReuse = 1.25f;          // a panel with fewer nonzeros per B row the MFMA side would fetch goes to the row kernel
 constexpr uint64_t kWideWindowBytes = 16ull << 20;   // ... whose window of B is wider than this (four L2s' worth)
 constexpr float kWideReuse = 0.98f;          // ... the bar for products of 256 columns or more over large matrices (see cute_spmm_plan_create)
-constexpr uint32_t kMaxRowForRows = 48;
+constexpr uint32_t kMaxRowForRows = 48;      // ... unless it holds a row longer than this: one lane group would serialise it
 constexpr uint32_t kRowBatch = 8;           // entries the row kernel has in flight per row
 // A panel is scattered when the window of B it reads (at most 256 columns of it at a time) is wider than this: its rows then
 // come from behind the L2s, which deliver about 8 TB/s against the 20 an L2 gives.  One and a half L2s: bands of 4 100
@@ -33,7 +33,7 @@ constexpr uint64_t kScatteredBytes = 6ull << 20;
 constexpr float kGraphReuse = 2.0f;          // scattered panels of large products (see cute_spmm_plan_create)
 constexpr uint32_t kGraphMaxRow = 96;
 constexpr uint64_t kGraphProduct = 1ull << 24;   // rows times columns from which on those two apply
-constexpr uint32_t kMaxHubRows = 256;       // hub plans: B rows a work-group keeps in LDS (64 KiB of 256-byte pieces; two work-groups per CU)     // ... unless it holds a row longer than this: one lane group would serialise it
+constexpr uint32_t kMaxHubRows = 256;       // hub plans: B rows a work-group keeps in LDS (64 KiB of 256-byte pieces; two work-groups per CU)
 constexpr uint32_t kUnevenRowFloor = 16;     // row kernel vs MFMA kernel: a panel whose longest row exceeds this and ...
 constexpr uint32_t kUnevenRowRatio = 2;      // ... this many mean rows of the panel goes to the MFMA kernel while rows share wavefronts
 constexpr float kHybridFill = 0.15f;         // cute_hybrid: a tile goes to the Blocked-ELL part from this fill on (threshold 0)

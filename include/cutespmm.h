@@ -459,9 +459,9 @@ typedef struct cute_plan_info {
 } cute_plan_info;
 
 typedef struct cute_spmm_plan cute_spmm_plan;
-/* Plan creation copies its tables to the device with synchronous copies, gathers the quad kernels' per-item heads
- * with a small kernel on the default stream and waits for it, and -- if the plan is the first to need an MFMA
- * layout the upload did not build -- builds that layout on the device, inside the format handle (which is why the
+/* Plan creation hands its tables to a small kernel on the default stream through pinned host memory and waits for that
+ * stream (a plan without tables, every row on the row kernel, launches nothing), and -- if the plan is the first to need an
+ * MFMA layout the upload did not build -- builds that layout on the device, inside the format handle (which is why the
  * handle is not const; such late builds are serialised by a lock in the handle).  Call it outside stream capture. */
 int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *t /* may be NULL */,
                           cute_spmm_plan **out);
