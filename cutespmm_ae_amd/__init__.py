@@ -28,7 +28,7 @@ ABI_SYMBOLS = [
     "cute_gen_matrix", "cute_gen_dense",
     "cute_hrpb_upload", "cute_hrpb_upload_layout", "cute_hrpb_upload_device_csr", "cute_hrpb_dev_layout_sizes",
     "cute_hrpb_dev_read_layouts", "cute_hrpb_dev_free", "cute_hrpb_dev_bytes", "cute_hrpb_dev_csr",
-    "cute_spmm_plan_create", "cute_spmm_plan_info", "cute_spmm_plan_column_slabs", "cute_spmm_plan_free", "cute_spmm_run", "cute_spmm_run_static",
+    "cute_spmm_plan_create", "cute_spmm_plan_info", "cute_spmm_plan_column_slabs", "cute_spmm_plan_window", "cute_spmm_plan_free", "cute_spmm_run", "cute_spmm_run_static",
     "cute_spmm_run_scratch", "cute_spmm_plan_scratch_bytes", "cute_device_layout", "cute_release_idle_memory",
     "cute_csr_spmm_dev", "cute_gpu_csr_spmm", "cute_spmm_time", "cute_csr_spmm_time",
     "cute_device_info",
@@ -203,6 +203,7 @@ def load_library():
     lib.cute_spmm_plan_create.argtypes = [C.c_void_p, C.c_uint32, C.POINTER(cute_tunables), C.POINTER(C.c_void_p)]
     lib.cute_spmm_plan_info.argtypes = [C.c_void_p, C.POINTER(cute_plan_info)]
     lib.cute_spmm_plan_column_slabs.argtypes = [C.c_void_p, u32p, u32p]
+    lib.cute_spmm_plan_window.argtypes = [C.c_void_p, u32p]
     lib.cute_spmm_plan_free.argtypes = [C.c_void_p]
     lib.cute_spmm_run.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]
     lib.cute_spmm_run_static.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]
@@ -732,6 +733,13 @@ class SPMM_TC:
         mfma, rows = C.c_uint32(), C.c_uint32()
         _check(load_library().cute_spmm_plan_column_slabs(self._plan, C.byref(mfma), C.byref(rows)), "cute_spmm_plan_column_slabs")
         return mfma.value, rows.value
+
+    @property
+    def window_columns(self):
+        """Columns of B that the rows of the plan read from LDS at a time (``csr_rows_window``); 0: they gather from memory."""
+        columns = C.c_uint32()
+        _check(load_library().cute_spmm_plan_window(self._plan, C.byref(columns)), "cute_spmm_plan_window")
+        return columns.value
 
     @property
     def scratch_bytes(self):

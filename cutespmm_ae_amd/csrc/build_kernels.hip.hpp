@@ -28,6 +28,8 @@
 
 namespace cute_build {
 
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
 constexpr int kThreads = 256;
 constexpr int kScanItems = 8;                               // entries per thread of a scan block
 constexpr uint32_t kScanBlock = kThreads * kScanItems;      // entries per scan block
@@ -47,7 +49,8 @@ struct PanelCensus {
     uint32_t pairs[4];         // distinct columns of each 4-row strip
     uint32_t stored;           // entries that are not zero
     uint32_t error;            // kErrRange | kErrUnsorted; the other fields then mean nothing
-    uint32_t pad[2];
+    uint32_t first;            // first column (of a panel with entries)
+    uint32_t pad;
 };
 static_assert(sizeof(PanelCensus) == 48, "written as twelve words");
 
@@ -370,7 +373,10 @@ __global__ __launch_bounds__(panel_threads(CAP)) void panel_census(const uint32_
         }
     }
     __syncthreads();
-    if (t == 0u && n && n != ~0u) res.span = l.hi - l.lo + 1u;
+    if (t == 0u && n && n != ~0u) {
+        res.span = l.hi - l.lo + 1u;
+        res.first = l.lo;
+    }
     __syncthreads();
     if (t < 12u) reinterpret_cast<uint32_t *>(out + p)[t] = reinterpret_cast<const uint32_t *>(&res)[t];
 }
@@ -844,5 +850,80 @@ __global__ __launch_bounds__(kThreads) void mark_hub_columns(const uint32_t *__r
     }
     out[id] = w;
 }
+
+// The entries of csr_rows_window (which describes them): a work-group is a slice.  The slice's part of the CSR arrays is one piece,
+// so it is read, and the quads are written, whole lines at a time by four wavefronts, and one, a row a lane, sorts in between in
+// LDS (a lane that walks its row in global memory touches a line an entry: 33.5 million entries 2 400 us,
+// this way 300).  The order inside a row, (slot +
+// row / 2) mod 8, is a counting sort by the eight bytes of one word: rows of fewer than 256 entries.  `staged`: {first quad, -,
+// quads, -} of every slice, and the tiles' windows, in host memory; slices[] gets the quads that no row of the slice pads besides.
+struct WindowTables {
+    const uint4 *slices;       // staged
+    const uint2 *tiles;
+    uint32_t numTiles;
+    uint4 *dSlices;            // device
+    uint2 *dTiles;
+};
+
+__device__ __forceinline__ uint32_t skewed(uint32_t i) { return i + (i >> 5); }    // rows of 32 entries do not start in one bank
+
+__global__ __launch_bounds__(kThreads) void window_entries(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols, const float *__restrict__ vals,
+                                                     uint32_t M, uint32_t ring_rows, WindowTables T, uint32_t longest, uint2 *__restrict__ slots,
+                                                     f32x4 *__restrict__ out)
+{
+    extern __shared__ uint32_t lds[];
+    const uint32_t slice = blockIdx.x, tid = threadIdx.x, row0 = slice * 64u;
+    for (uint32_t t = slice * kThreads + tid; t < T.numTiles; t += gridDim.x * kThreads) T.dTiles[t] = T.tiles[t];
+    uint32_t *slot_of = lds, *placed = lds + skewed(64u * longest) + 1u;
+    float *val_of = reinterpret_cast<float *>(placed + 32u * longest), *placed_val = val_of + skewed(64u * longest) + 1u;
+    uint16_t *placed_slot = reinterpret_cast<uint16_t *>(placed);
+    uint4 d = T.slices[slice];
+    const uint32_t begin = rowPtr[row0], end = rowPtr[min(row0 + 64u, M)];
+    for (uint32_t base = begin; base < end; base += 8u * kThreads) {
+        uint32_t col[8];
+        float val[8];
+#pragma unroll
+        for (uint32_t u = 0; u < 8u; ++u) {
+            const uint32_t i = base + u * kThreads + tid;
+            if (i < end) { col[u] = cols[i]; val[u] = vals[i]; }
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < 8u; ++u) {
+            const uint32_t i = base + u * kThreads + tid;
+            if (i < end) { slot_of[skewed(i - begin)] = col[u] % ring_rows; val_of[skewed(i - begin)] = val[u]; }
+        }
+    }
+    __syncthreads();
+    if (tid < 64u) {
+        const uint32_t lane = tid, row = row0 + lane, s = rowPtr[min(row, M)], n = rowPtr[min(row + 1u, M)] - s, turn = lane >> 1, first = s - begin;
+        uint64_t place = 0;
+        for (uint32_t i = 0; i < n; ++i) place += 1ull << (8u * ((slot_of[skewed(first + i)] + turn) & 7u));
+        place *= 0x0101010101010100ull;       // where the entries of each of the eight begin
+        auto at = [&](uint32_t k) { return (k / 4u * 64u + lane) * 4u + k % 4u; };
+        for (uint32_t i = 0; i < n; ++i) {
+            const uint32_t slot = slot_of[skewed(first + i)], shift = 8u * ((slot + turn) & 7u), to = at(uint32_t(place >> shift) & 255u);
+            place += 1ull << shift;
+            placed_slot[to] = uint16_t(slot);
+            placed_val[to] = val_of[skewed(first + i)];
+        }
+        for (uint32_t k = n; k < d.z * 4u; ++k) {
+            placed_slot[at(k)] = uint16_t(0xffffu);
+            placed_val[at(k)] = 0.0f;
+        }
+        uint32_t least = n / 4u;
+#pragma unroll
+        for (int step = 1; step < 64; step *= 2) least = min(least, uint32_t(__shfl_xor(int(least), step)));
+        d.y = least;
+        if (lane == 0u) T.dSlices[slice] = d;
+    }
+    __syncthreads();
+    for (uint32_t i = tid; i < d.z * 64u; i += kThreads) {
+        slots[size_t(d.x) * 64u + i] = make_uint2(placed[2u * i], placed[2u * i + 1u]);
+        out[size_t(d.x) * 64u + i] = f32x4{placed_val[4u * i], placed_val[4u * i + 1u], placed_val[4u * i + 2u], placed_val[4u * i + 3u]};
+    }
+}
+
+// LDS of window_entries for rows of up to `longest` entries (a multiple of four).
+inline uint32_t window_entries_lds(uint32_t longest) { return (2u * (64u * longest + 2u * longest + 1u) + 96u * longest) * 4u; }
 
 }  // namespace cute_build

@@ -208,7 +208,7 @@ struct cute_hrpb_dev {
     std::mutex lock;
     bool haveBricks = false, haveQuads = false;
     // one allocation each: the CSR arrays, the brick tiles, the quad lists
-    void *csrMemory = nullptr, *brickMemory = nullptr, *quadMemory = nullptr;
+    void *csrMemory = nullptr, *brickMemory = nullptr, *quadMemory = nullptr, *windowMemory = nullptr;
     uint32_t *dHdr = nullptr;           // brick tiles: one 128-byte header line per block
     float *dVals = nullptr;             // brick tiles: values in lane order, then 64 zeros
     uint32_t *dRowPtr = nullptr, *dCols = nullptr;
@@ -226,6 +226,12 @@ struct cute_hrpb_dev {
     std::vector<uint32_t> panelCols;    // active columns per row panel
     std::vector<uint32_t> panelMaxRow;  // longest row of each panel
     std::vector<uint32_t> panelSpan;    // width of each panel's column window (last column - first column + 1)
+    std::vector<uint32_t> panelFirst;   // ... and its first column
+    // the entries as csr_rows_window reads them (which describes them), built for the first plan that uses that kernel
+    bool haveWindow = false;
+    uint4 *dSlices = nullptr;
+    uint2 *dWindowSlots = nullptr, *dWindowTiles = nullptr;
+    cute_dev::f32x4 *dWindowVals = nullptr;
     std::vector<uint32_t> panelStored;  // entries of each panel that are not zero (what the quad lists store)
 };
 
@@ -262,6 +268,9 @@ struct cute_spmm_plan {
     // slabs of the MFMA part and of the row part when an XCD owns columns instead of rows (cute_dev::xcd_share), else 0
     uint32_t columnSlabs = 0, rowColumnSlabs = 0;
     uint32_t rowBlocksPerXcd = 0;       // longest of those ranges
+    // rows through csr_rows_window: columns of B in its ring (0: not used) and the chains of tiles
+    uint32_t windowColumns = 0, windowChains = 0, windowChainTiles = 0;
+    bool windowWarm = false;
 };
 
 namespace {
@@ -376,6 +385,7 @@ void cute_hrpb_dev_free(cute_hrpb_dev *d)
     give_device_memory(d->csrMemory);
     give_device_memory(d->brickMemory);
     give_device_memory(d->quadMemory);
+    give_device_memory(d->windowMemory);
     delete d;
 }
 
@@ -817,6 +827,84 @@ int ensure_layout(cute_hrpb_dev *d, int which)
     return which == 1 ? build_bricks_on_device(d, w) : build_quads_on_device(d, w);
 }
 
+// What csr_rows_window wants to know of a matrix: of every slice of 64 rows, where its quads begin and how many its longest row takes
+// (one at least), and the column window of every tile, widened so that neither end moves back from one tile to the next.
+struct WindowShape {
+    std::vector<uint4> slices;            // {first quad, -, quads, -}
+    std::vector<uint2> tiles;             // {first column, column behind the last}
+    uint64_t quads = 0;
+    uint32_t longest = 0, widest = 0;
+};
+
+// false: rows or windows that the kernel does not take
+bool window_shape(const cute_hrpb_dev *d, WindowShape &w)
+{
+    constexpr uint32_t per_slice = 64u / CUTE_TM, per_tile = cute_dev::kWindowTile / CUTE_TM;
+    w.slices.resize((size_t(d->P) + per_slice - 1) / per_slice);
+    w.tiles.resize((size_t(d->P) + per_tile - 1) / per_tile);
+    uint32_t end = 0;
+    for (uint32_t p = 0; p < d->P;) {
+        uint2 &tile = w.tiles[p / per_tile];
+        tile.x = d->K;
+        for (const uint32_t last = std::min<uint32_t>(d->P, p + per_tile); p < last;) {
+            uint4 &slice = w.slices[p / per_slice];
+            uint32_t longest = 1;
+            for (const uint32_t upto = std::min<uint32_t>(last, p + per_slice); p < upto; ++p) {
+                longest = std::max(longest, d->panelMaxRow[p]);
+                if (!d->panelNnz[p]) continue;
+                tile.x = std::min(tile.x, d->panelFirst[p]);
+                end = std::max(end, d->panelFirst[p] + d->panelSpan[p]);
+            }
+            if (longest > 64u) return false;
+            w.longest = std::max(w.longest, longest);
+            slice = make_uint4(uint32_t(w.quads), 0u, (longest + 3u) / 4u, 0u);
+            w.quads += (longest + 3u) / 4u;
+        }
+        tile.y = end;
+    }
+    uint32_t first = d->K;
+    for (size_t t = w.tiles.size(); t-- > 0;) {
+        first = std::min(first, w.tiles[t].x);
+        w.tiles[t].x = std::min(first, w.tiles[t].y);
+        w.widest = std::max(w.widest, w.tiles[t].y - w.tiles[t].x);
+    }
+    return w.widest <= cute_dev::kWindowRows<8> && w.quads <= 0xffffffffull;
+}
+
+// The entries csr_rows_window reads, for a ring of `ring_rows` rows (which follows from the widest window, so a handle has one such form).
+int ensure_window(cute_hrpb_dev *d, const WindowShape &w, uint32_t ring_rows)
+{
+    std::lock_guard<std::mutex> guard(d->lock);
+    if (d->haveWindow) return CUTE_OK;
+    Layout lay;
+    const uint64_t oSlices = lay.add(w.slices.size(), sizeof(uint4)), oTiles = lay.add(w.tiles.size(), sizeof(uint2)), staged = lay.bytes;
+    const uint64_t oSlots = lay.add(w.quads * 64u, sizeof(uint2)), oVals = lay.add(w.quads * 64u, 16u);
+    DevBuf mem;
+    PinnedBuf pin;
+    int rc = mem.alloc(lay.bytes);
+    if (rc == CUTE_OK) rc = pin.alloc(staged);
+    if (rc != CUTE_OK) return rc;
+    std::memcpy(pin.as<char>(oSlices), w.slices.data(), w.slices.size() * sizeof(uint4));
+    std::memcpy(pin.as<char>(oTiles), w.tiles.data(), w.tiles.size() * sizeof(uint2));
+    pin.pending = true;
+    const uint32_t longest = (w.longest + 3u) & ~3u;
+    const cute_build::WindowTables T = {pin.as<const uint4>(oSlices), pin.as<const uint2>(oTiles), uint32_t(w.tiles.size()),
+                                        Layout::at<uint4>(mem.p, oSlices), Layout::at<uint2>(mem.p, oTiles)};
+    CUTE_BUILD_LDS(cute_build::window_entries, dim3(uint32_t(w.slices.size())), cute_build::window_entries_lds(longest), d->dRowPtr, d->dCols,
+                   d->dCsrVals, d->M, ring_rows, T, longest, Layout::at<uint2>(mem.p, oSlots), Layout::at<cute_dev::f32x4>(mem.p, oVals));
+    rc = check_launch("window entries");
+    if (rc == CUTE_OK) rc = pin.wait();
+    if (rc != CUTE_OK) return rc;
+    d->dSlices = Layout::at<uint4>(mem.p, oSlices);
+    d->dWindowTiles = Layout::at<uint2>(mem.p, oTiles);
+    d->dWindowSlots = Layout::at<uint2>(mem.p, oSlots);
+    d->dWindowVals = Layout::at<cute_dev::f32x4>(mem.p, oVals);
+    d->windowMemory = mem.release();
+    d->bytes += lay.bytes;
+    d->haveWindow = true;
+    return CUTE_OK;
+}
+
 // Group counts of the quad lists from the list length of every strip; picks lockstep lists unless they would
 // be mostly padding (a few very long rows stretch the lists of their panel neighbours): then one list per strip.
 int finish_quad_census(cute_hrpb_dev *d, int quad_layout)
@@ -929,10 +1017,12 @@ int finish_upload(cute_hrpb_dev *d, int quad_layout, const DeviceContext &c)
         bool any_large = false, any_medium = false;
         d->panelNnz.resize(P);
         d->panelSpan.resize(P);
+        d->panelFirst.resize(P);
         for (uint32_t p = 0; p < P; ++p) {
             error |= r[p].error;
             d->panelNnz[p] = r[p].nnz;
             d->panelSpan[p] = r[p].span;
+            d->panelFirst[p] = r[p].first;
             if (r[p].nnz > cute_build::kPanelFirst || r[p].span > max_span(d)) (panel_is_large(d, p) ? any_large : any_medium) = true;
         }
         if (!error && (any_medium || any_large)) {
@@ -1016,6 +1106,48 @@ int make_hub_tables(cute_spmm_plan *p, const cute_hrpb_dev *d, uint32_t hub_rows
     HIP_TRY(hipDeviceSynchronize());
     p->numHub = used;
     return CUTE_OK;
+}
+
+// Rows of a plan without MFMA panels through csr_rows_window where that is ahead.  Needs the widest window of a tile to fit the ring,
+// rows of up to 64 entries (the LDS of window_entries) and little padding: a lane waits for the longest of 64 rows.  Then both kernels'
+// times are estimated, in us, and the ring has to be ahead by 15 %, of a launch worth the tables.  Fitted on 400 banded matrices drawn
+// over 4 096 ... 640 000 rows, 8 ... 48 entries a row, bands of 64 ... 2 048 and N = 16 ... 600 (rms 18 and 14 % for rings of 8
+// and 16 columns, 15 % for the row kernel): of those it takes, none was more than 2.5 % slower, and over all of them the products take
+// 0.895 of the row kernel's time where the better of the two would take 0.869.  65 536 rows of 32, band of 2 048, us row kernel / ring: N = 32
+// 12.4 / 14.8, N = 256 82.6 / 58.6; 16 rows N = 128 24.4 / 26.2; 262 144 rows of 12, band of 700, N = 128 72.7 / 76.3; 32 768 rows of
+// 24, band of 1 500, N = 128 17.0 / 19.1; band of 200, 65 536 rows of 32, N = 101 39.0 / 25.1; 1 048 576 rows of 32, band of 2 048,
+// N = 256 1 714 / 1 005.
+void plan_window(cute_spmm_plan *p, cute_hrpb_dev *d, uint32_t N, const DeviceContext &c)
+{
+    WindowShape w;
+    if (N < 16u || d->P == 0 || !window_shape(d, w) || w.quads * 256u > uint64_t(d->nnz) + d->nnz / 4u + 4096u) return;
+    const uint32_t W = w.widest <= cute_dev::kWindowRows<16> ? 16u : 8u;
+    const uint32_t n = uint32_t(w.tiles.size()), slabs = (N + W - 1u) / W, cus = uint32_t(c.num_cus) / cute_dev::kNumXcd;
+    const double row = double(w.quads) * 256.0 / double(d->M), bytes = 8.0 * d->M * N + 8.0 * d->nnz, gathers = 4e-6 * double(d->nnz) * N;
+    const bool beyond = uint64_t(d->K + uint64_t(d->M)) * N * sizeof(float) > c.cache_bytes;
+    // a CU holds one work-group at a time: `rounds` of them after each other, each a first window and then its tiles
+    const double first = W == 16u ? 0.8 : 2.0, tile = (W == 16u ? 3.8 + 0.245 * row : 2.6 + 0.143 * row) + (beyond ? (W == 16u ? 2.4 : 1.7) : 0.0);
+    double ring = 0.0;
+    for (uint32_t per_xcd = 1;; ++per_xcd) {
+        const uint32_t chains = per_xcd * cute_dev::kNumXcd, length = (n + chains - 1u) / chains, rounds = (slabs * per_xcd + cus - 1u) / cus;
+        const double time = rounds * (first + length * tile);
+        if (per_xcd == 1 || time < ring) {
+            ring = time;
+            p->windowChains = chains;
+            p->windowChainTiles = length;
+        }
+        if (length == 1u || per_xcd == 64u) break;
+    }
+    const uint32_t walk = uint32_t(p->rows_vec) << p->rows_logl;       // columns a lane group covers, used or not
+    const double covered = double((N + walk - 1u) / walk * walk) / N;
+    const double rows = 3.1 + gathers / 20.0 * (0.29 + 0.40 * covered + (N % 32u ? 0.10 : 0.0)) + bytes * 1e-6 * (0.04 + (beyond ? 0.09 : 0.0));
+    p->windowWarm = beyond;
+#ifdef CUTE_WIN_FORCE
+    if (const char *f = getenv("CUTE_WIN")) { if (f[0] == '0') return; } else
+#endif
+    if (ring * 1.15 > rows || rows - ring < 12.0) return;
+    // (without the memory for a second form of the entries the row kernel takes the rows as ever)
+    if (ensure_window(d, w, W == 16u ? cute_dev::kWindowRows<16> : cute_dev::kWindowRows<8>) == CUTE_OK) p->windowColumns = W;
 }
 
 }  // namespace
@@ -1143,6 +1275,13 @@ int cute_spmm_plan_column_slabs(const cute_spmm_plan *p, uint32_t *mfma, uint32_
     if (!p) return CUTE_ERR_ARG;
     if (mfma) *mfma = p->info.numChunks ? p->columnSlabs : 0u;
     if (rows) *rows = p->numRows ? p->rowColumnSlabs : 0u;
+    return CUTE_OK;
+}
+
+int cute_spmm_plan_window(const cute_spmm_plan *p, uint32_t *columns)
+{
+    if (!p) return CUTE_ERR_ARG;
+    if (columns) *columns = p->windowColumns;
     return CUTE_OK;
 }
 
@@ -1463,6 +1602,7 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
         }
         p->rowColumnSlabs = rows_columns ? p->rows_slabs : 0u;
     }
+    if (n_brick == 0 && default_bars) plan_window(p, d, N, c);
     // The chunk list depends on the MFMA kernel (its work units are blocks or list groups).  It is built,
     // and if the partial tiles of the cut panels then turn out to be more rows than the fast kernels'
     // 24-bit row operand can address, built once more for the pipelined brick kernel, whose stores use
@@ -2030,7 +2170,17 @@ int run_with(const cute_spmm_plan *p, const float *dB, float *dC, void *stream, 
         else if (p->vec == 2) launch_brick<2, 1>(p, dB, dC, partials, s);
         else launch_brick<1, 1>(p, dB, dC, partials, s);
     }
-    if (p->numRows && !rows_launched) {
+    if (p->windowColumns) {
+        const uint32_t slabs = (N + p->windowColumns - 1u) / p->windowColumns;
+        const dim3 grid(p->windowChains * slabs), block(1024);
+#define CUTE_WINDOW_LAUNCH(W, WARM)                                                                                              \
+    hipLaunchKernelGGL((cute_dev::csr_rows_window<W, WARM>), grid, block, 0, s, p->d->dSlices, p->d->dWindowSlots, p->d->dWindowVals, \
+                       p->d->dWindowTiles, (p->d->M + cute_dev::kWindowTile - 1u) / cute_dev::kWindowTile, p->windowChainTiles,   \
+                       p->windowChains, slabs, dB, dC, p->d->M, N)
+        if (p->windowColumns == 16u) { if (p->windowWarm) CUTE_WINDOW_LAUNCH(16, true); else CUTE_WINDOW_LAUNCH(16, false); }
+        else { if (p->windowWarm) CUTE_WINDOW_LAUNCH(8, true); else CUTE_WINDOW_LAUNCH(8, false); }
+#undef CUTE_WINDOW_LAUNCH
+    } else if (p->numRows && !rows_launched) {
         launch_rows<true>(p->rows_vec, p->rows_logl, p->dRowList, p->numRows, p->rows_slabs, p->d->dRowPtr, p->d->dCols,
                     p->d->dCsrVals, dB, dC, N, s, &p->rowRanges, p->rowBlocksPerXcd, p->rowColumnSlabs);
     }

@@ -12,6 +12,7 @@
 //                    only occupied 4-row column pieces cost matrix time.
 //   csr_rows_batched one lane group per CSR row, lanes span N, 8 (col, val) pairs in flight; the kernel
 //                    for panels with too little reuse for the matrix cores.
+//   csr_rows_window  rows whose columns move along with them: their window of B slides through LDS.
 //   hrpb_quad_rows_f32 / hrpb_brick_rows_f32   MFMA work items and sparse rows of a mixed plan in one launch.
 //   reduce_partials  adds up the partial tiles of panels that were cut, in chunk order (no atomics).
 //   blocked_ell_f32  fp32 MFMA over the dense blocks of a Blocked-ELL matrix.
@@ -1258,6 +1259,218 @@ __global__ __launch_bounds__(256) void csr_rows_batched(const uint4 *__restrict_
     const uint32_t x = xcd_share(blockIdx.x, slab, COLUMNS ? column_slabs : 0u);
     if (!xcd_range_id(ranges, blockIdx.x, x, block_id)) return;
     rows_batched_body<VEC, LOG_L, BATCH, true>(block_id, slab, row_list, num_rows, rowPtr, cols, vals, B, C, N);
+}
+
+// Rows whose columns lie in a window that moves along with them (banded matrices, operators in a local numbering): the piece of B
+// they read is kept in LDS, W columns of it for one work-group, as a ring that slides over B, and the gathers are LDS reads.
+// csr_rows_batched gathers through the vector memory path, which returns about 40 bytes a clock and CU (20 TB/s in all) whatever
+// level of the caches answers; LDS returns 128.  A chain is a run of tiles of kWindowTile rows that one work-group of sixteen
+// wavefronts walks, a row a lane, all W columns of it; every row of B enters the ring once a chain.
+//
+// What bounds it: a CU has about 64 lines on their way from the L2 (measured: 59 to 74), and a tile asks for one 128-byte line
+// a row of B (of which W floats are used) and for 6 bytes an entry, once for each slab of W columns.  So W is as wide as the
+// window allows, 8 or 16, an entry is a ring slot of 16 bits beside its value, four entries of a row are fetched at once, and the
+// slabs of a chain run on one XCD at the same time: they ask its L2 for the same entries and lines and fill the same lines of C.
+// Then LDS: 16 bytes a lane, rows at random, so the pieces of a row are read in an order that depends on the lane (the low bits
+// of the address all differ across Q lanes), and the entries of a row stand in the order of (slot + row / 2) mod 8, which lets
+// neighbouring lanes ask for different banks (LDS cycles 98 600 -> 74 900 a CU, 65 536 rows of 32, N = 256: 60.4 -> 56.7 us).
+// Row kernel / this one, us: 1 048 576 rows of 32 entries, band of 2 048 on either side, N = 256 1 720 / 1 007 (34 TB/s of gathers; the
+// operands take 440 at a copy's rate), 262 144 rows 414 / 258, N = 47 and 30 entries 87 / 51; band of 700 (16 columns) 414 / 211.
+// At the first of these 52 % of the time are LDS cycles, 44 % vector instructions, and 59 lines are on their way on average.
+// Tried and slower: B asked for a whole tile ahead (258 -> 276), wavefronts of their own for it (258 -> 292 and more, fewer of
+// them add up), non-temporal loads or stores (+ 10 ... 25 %: the sharing goes).
+constexpr uint32_t kWindowTile = 1024, kWindowBytes = 160u << 10, kWindowPad = 0xffffu;
+template <int W> constexpr uint32_t kWindowRows = kWindowBytes / (W * 4u);     // rows of B in the ring
+
+// x of lane (l ^ XOR) of each four lanes
+template <int XOR> __device__ __forceinline__ f32x4 quad_xor(const f32x4 &v)
+{
+    constexpr int perm = (0 ^ XOR) | (1 ^ XOR) << 2 | (2 ^ XOR) << 4 | (3 ^ XOR) << 6;
+    f32x4 r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float x = v[i];
+        r[i] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), perm, 0xf, 0xf, true));
+    }
+    return r;
+}
+
+// slices[i], 64 rows: {first quad, quads without padding, quads, -}; a quad is four entries of each of the 64 rows, slot and value
+// lane after lane.  tiles[t]: columns [lo, hi) that the rows of tile t and, by lo, of every later tile, by hi, of every earlier one
+// read; hi - lo is at most the ring.  Column c of B stands in slot c mod kWindowRows.
+// WARM: operands from HBM.  The lines of B that the tile after next brings are asked for here, each by one of the work-groups that share
+// them, so that all of them find it in the L2 (262 144 rows, N = 256: 12 entries a row 245 -> 188 us, 32 entries 257 -> 248; from the
+// Infinity Cache, 65 536 rows of 32, 56.6 -> 61.5).
+template <int W, bool WARM>
+__global__ __launch_bounds__(1024) void csr_rows_window(const uint4 *__restrict__ slices, const uint2 *__restrict__ slots, const f32x4 *__restrict__ vals,
+                                                        const uint2 *__restrict__ tiles, uint32_t num_tiles, uint32_t tiles_per_chain,
+                                                        uint32_t num_chains, uint32_t num_slabs, const float *__restrict__ B,
+                                                        float *__restrict__ C, uint32_t M, uint32_t N)
+{
+    constexpr uint32_t Q = W / 4, S = kWindowRows<W>, ROW_LOG = W == 8 ? 5 : 6;    // 16-byte pieces, rows of the ring; bytes of a row
+    constexpr uint32_t STEP = 1024u / Q, AHEAD = kWindowTile / STEP, FIRST = S / STEP;   // rows of B a round; rounds ahead, of the first window
+    constexpr uint32_t HOLD = W == 8 ? 4 : 2;                                      // quads of a row in registers
+    static_assert(W == 8 || W == 16, "a slot and its bytes are packed for these");
+    __shared__ f32x4 ring[S * Q];
+    // the slabs of a chain are neighbours on one XCD
+    const uint32_t local = blockIdx.x / kNumXcd, chain = blockIdx.x % kNumXcd + kNumXcd * (local / num_slabs), slab = local % num_slabs;
+    const uint32_t t0 = chain * tiles_per_chain, t1 = min(t0 + tiles_per_chain, num_tiles);
+    if (chain >= num_chains || t0 >= t1) return;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid / kWaveSize), l = lane % Q;
+    const uint32_t c0 = min(slab * W, N - uint32_t(W));       // the last slab may share columns with the one before: the same bits
+    const float *Bc = B + c0 + l * 4u;
+    const uint32_t r_in = tid / Q;
+    auto load_row = [&](uint32_t r) { return load_vec<4>(Bc + size_t(r) * N); };
+    auto keep_row = [&](uint32_t r, const f32x4 &v) { ring[(r % S) * Q + l] = v; };
+    auto lds_barrier = [] {                                   // (global loads and stores stay under way)
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    };
+    struct Quad {
+        uint2 slot;
+        f32x4 val;
+    };
+    auto fetch = [&](const uint4 &d, uint32_t q) {            // (a slice has a quad at least)
+        const size_t at = (size_t(d.x) + min(q, d.z - 1u)) * kWaveSize + lane;
+        Quad m;
+        m.slot = slots[at];
+        m.val = vals[at];
+        return m;
+    };
+    const uint32_t num_slices = (M + 63u) / 64u;
+    auto slice_of = [&](uint32_t t) { return slices[min(t * (kWindowTile / 64u) + wave, num_slices - 1u)]; };
+    uint4 d = slice_of(t0);
+    Quad held[HOLD];
+    uint32_t have = tiles[t0].x;
+    {
+        f32x4 first[FIRST];
+        const uint32_t hi = tiles[t0].y;
+#pragma unroll
+        for (uint32_t i = 0; i < FIRST; ++i)
+            if (have + i * STEP + r_in < hi) first[i] = load_row(have + i * STEP + r_in);
+#pragma unroll
+        for (uint32_t j = 0; j < HOLD; ++j) held[j] = fetch(d, j);
+#pragma unroll
+        for (uint32_t i = 0; i < FIRST; ++i)
+            if (have + i * STEP + r_in < hi) keep_row(have + i * STEP + r_in, first[i]);
+        have = hi;
+    }
+    lds_barrier();
+    const char *lds = reinterpret_cast<const char *>(ring);
+    // piece j of the lane is piece j ^ l of the row, a lane's pieces differ from its neighbours' in every read
+    auto read = [&](uint32_t slot, f32x4 (&b)[Q]) {
+        const uint32_t at = slot << ROW_LOG | l << 4;
+#pragma unroll
+        for (uint32_t j = 0; j < Q; ++j) b[j] = *reinterpret_cast<const f32x4 *>(lds + (at ^ (j * 16u)));
+    };
+    auto add_quad = [&](const Quad &m, f32x4 (&acc)[Q]) {
+        const uint32_t slot[4] = {m.slot.x & 0xffffu, m.slot.x >> 16, m.slot.y & 0xffffu, m.slot.y >> 16};
+        constexpr int G = 16 / (2 * int(Q));                  // entries whose pieces are on their way together: the registers' share
+#pragma unroll
+        for (int g = 0; g < 4; g += G) {
+            f32x4 b[G][Q];
+#pragma unroll
+            for (int u = 0; u < G; ++u) read(slot[g + u], b[u]);
+#pragma unroll
+            for (int u = 0; u < G; ++u)
+#pragma unroll
+                for (uint32_t j = 0; j < Q; ++j) acc[j] += m.val[g + u] * b[u][j];
+            if (G < 4) __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    auto add_padded = [&](const Quad &m, f32x4 (&acc)[Q]) {   // padding is left out, not multiplied by zero: B may hold what is not finite
+        const uint32_t slot[4] = {m.slot.x & 0xffffu, m.slot.x >> 16, m.slot.y & 0xffffu, m.slot.y >> 16};
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (slot[u] != kWindowPad) {
+                f32x4 b[Q];
+                read(slot[u], b);
+#pragma unroll
+                for (uint32_t j = 0; j < Q; ++j) acc[j] += m.val[u] * b[j];
+            }
+    };
+    const uint32_t lines = WARM ? (N * 4u + 127u) / 128u : 1u;
+    float warm = 0.0f;
+    for (uint32_t t = t0; t < t1; ++t) {
+        // (what lies between two windows is left out)
+        const uint2 coming = t + 1u < t1 ? tiles[t + 1u] : make_uint2(have, have);
+        const uint32_t from = max(have, coming.x), next = coming.y;
+        const uint4 dn = slice_of(min(t + 1u, t1 - 1u));
+        f32x4 acc[Q];
+#pragma unroll
+        for (uint32_t j = 0; j < Q; ++j) acc[j] = f32x4(0.0f);
+        // loads return in order: what is asked for behind the rows of B waits for them, so those come last in a tile, before the
+        // next tile's first entries, and are covered by the HOLD quads at hand
+        uint32_t q = 0;
+        for (; q + HOLD < d.z && q + HOLD <= d.y; q += HOLD) {
+#pragma unroll
+            for (uint32_t j = 0; j < HOLD; ++j) {
+                const Quad now = held[j];
+                held[j] = fetch(d, q + HOLD + j);
+                add_quad(now, acc);
+            }
+        }
+        for (; q + HOLD < d.z; q += HOLD) {
+#pragma unroll
+            for (uint32_t j = 0; j < HOLD; ++j) {
+                const Quad now = held[j];
+                held[j] = fetch(d, q + HOLD + j);
+                if (q + j < d.y) add_quad(now, acc);
+                else add_padded(now, acc);
+            }
+        }
+        f32x4 ahead[AHEAD];
+#pragma unroll
+        for (uint32_t i = 0; i < AHEAD; ++i)
+            if (from + i * STEP + r_in < next) ahead[i] = load_row(from + i * STEP + r_in);
+#pragma unroll
+        for (uint32_t j = 0; j < HOLD; ++j) {
+            const Quad now = held[j];
+            held[j] = fetch(dn, j);
+            if (q + j < d.y) add_quad(now, acc);
+            else if (q + j < d.z) add_padded(now, acc);
+        }
+        d = dn;
+        if (WARM) {
+            asm volatile("" ::"v"(warm));
+            if (t + 2u < t1) {
+                const uint2 later = tiles[t + 2u];
+                const uint32_t line = tid * num_slabs + slab, r = max(next, later.x) + line / lines;
+                if (r < later.y) warm = B[size_t(r) * N + min(line % lines * 32u, N - 1u)];
+            }
+        }
+        // acc[j] is piece j ^ l of the lane's row; after these exchanges y[k] is piece l of row k of the Q lanes, and a store
+        // fills whole pieces of rows
+        f32x4 y[Q];
+        y[0] = acc[0];
+        y[1] = quad_xor<1>(acc[1]);
+        if constexpr (Q == 4) {
+            y[2] = quad_xor<2>(acc[2]);
+            y[3] = quad_xor<3>(acc[3]);
+        }
+#pragma unroll
+        for (uint32_t bit = 1; bit < Q; bit *= 2)
+#pragma unroll
+            for (uint32_t k = 0; k < Q; ++k)
+                if (!(k & bit)) {
+                    const f32x4 a = y[k], b = y[k | bit];
+                    const bool swap = l & bit;
+                    y[k] = swap ? b : a;
+                    y[k | bit] = swap ? a : b;
+                }
+        const uint32_t row = (t * (kWindowTile / 64u) + wave) * 64u + lane - l;
+#pragma unroll
+        for (uint32_t k = 0; k < Q; ++k)      // (through the L2: the slabs beside this one fill the rest of the line)
+            if (row + k < M) *reinterpret_cast<VecInMemory<4>::type *>(C + size_t(row + k) * N + c0 + l * 4u) = y[k];
+        lds_barrier();                        // the rows that leave the window are not read any more
+#pragma unroll
+        for (uint32_t i = 0; i < AHEAD; ++i)
+            if (from + i * STEP + r_in < next) keep_row(from + i * STEP + r_in, ahead[i]);
+        for (uint32_t r = from + kWindowTile + r_in; r < next; r += STEP) keep_row(r, load_row(r));     // a window that jumps
+        have = next;
+        lds_barrier();
+    }
 }
 
 // One launch for a plan that uses both the quad kernel and the row kernel: they write disjoint

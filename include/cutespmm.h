@@ -460,7 +460,7 @@ typedef struct cute_plan_info {
 
 typedef struct cute_spmm_plan cute_spmm_plan;
 /* Plan creation hands its tables to a small kernel on the default stream through pinned host memory and waits for that
- * stream (a plan without tables, every row on the row kernel, launches nothing), and -- if the plan is the first to need an
+ * stream (a plan without tables, every row on the row kernel and not through LDS, launches nothing), and -- if the plan is the first to need an
  * MFMA layout the upload did not build -- builds that layout on the device, inside the format handle (which is why the
  * handle is not const; such late builds are serialised by a lock in the handle).  Call it outside stream capture. */
 int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *t /* may be NULL */,
@@ -469,6 +469,10 @@ int cute_spmm_plan_info(const cute_spmm_plan *p, cute_plan_info *out);
 /* In which order a plan's work-groups go to the XCDs: 0 by rows (an XCD owns consecutive rows), else by columns (an XCD owns an
  * eighth of so many column slabs), for the MFMA kernel and for the row kernel of the plan. */
 int cute_spmm_plan_column_slabs(const cute_spmm_plan *p, uint32_t *mfma, uint32_t *rows);
+/* Columns of B that a plan whose rows all go to the row kernel keeps in LDS at a time (csr_rows_window: rows whose columns lie in a
+ * window that moves along with them), 0: the rows gather from memory.  The first such plan of a handle adds a form of the
+ * entries to it (6 bytes an entry and some padding), as for a late MFMA layout. */
+int cute_spmm_plan_window(const cute_spmm_plan *p, uint32_t *columns);
 void cute_spmm_plan_free(cute_spmm_plan *p);
 /* dB [K x N], dC [M x N]: device pointers, row-major, 16-byte aligned.  Asynchronous on
  * `stream` (a hipStream_t, NULL = default stream).  C is fully overwritten: the caller
