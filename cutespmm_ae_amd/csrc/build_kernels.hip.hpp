@@ -185,17 +185,17 @@ template <uint32_t CAP> struct PanelEntries {
 inline __host__ __device__ uint32_t panel_window_words(uint32_t max_span) { return (max_span + 31u) / 32u; }
 
 // Sum over the threads before this one, and over the whole work-group in `total`, of two words at once.
-template <uint32_t CAP> __device__ __forceinline__ Two block_exclusive(PanelLds<CAP> &l, Two own, Two &total)
+template <uint32_t WAVES> __device__ __forceinline__ Two block_exclusive_over(Two (&waveSum)[WAVES], Two own, Two &total)
 {
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const Two incl = {wave_add(own.x), wave_add(own.y)};
-    if (lane == 63u) l.waveSum[wave] = incl;
+    if (lane == 63u) waveSum[wave] = incl;
     __syncthreads();
     Two before = {incl.x - own.x, incl.y - own.y};
     total = {0u, 0u};
-#pragma unroll
-    for (uint32_t w = 0; w < PanelLds<CAP>::kBlock / 64u; ++w) {
-        const Two v = l.waveSum[w];
+#pragma unroll 8
+    for (uint32_t w = 0; w < WAVES; ++w) {
+        const Two v = waveSum[w];
         if (w < wave) { before.x += v.x; before.y += v.y; }
         total.x += v.x;
         total.y += v.y;
@@ -203,6 +203,7 @@ template <uint32_t CAP> __device__ __forceinline__ Two block_exclusive(PanelLds<
     __syncthreads();
     return before;
 }
+template <uint32_t CAP> __device__ __forceinline__ Two block_exclusive(PanelLds<CAP> &l, Two own, Two &total) { return block_exclusive_over(l.waveSum, own, total); }
 template <uint32_t CAP> __device__ __forceinline__ uint32_t block_exclusive(PanelLds<CAP> &l, uint32_t own, uint32_t &total)
 {
     Two sum;
@@ -542,6 +543,215 @@ __global__ __launch_bounds__(panel_threads(CAP)) void panel_quads(const uint32_t
         const uint32_t a = e.active[k], s = e.row[k] >> 2, mask = (l.rows[a] >> (16u + 4u * s)) & 15u;
         const uint32_t pr = half(before[a], s);
         packed[uint64_t(value0) + place[pr] + uint32_t(__popc(mask & ((1u << (e.row[k] & 3u)) - 1u)))] = e.val[k];
+    }
+}
+
+// ------------------------------------------------------------------------------------------------
+// Panels of more than kPanelCap entries (the hub rows of a graph) whose window the bitmap takes: a work-group of sixteen wavefronts
+// walks the entries instead of holding them, for the census and for the strip lists.  LDS holds the bitmap, its counts and the
+// rows of every active column, and the rest follows from prefix sums over the columns, a thread a run of them.
+// The entry-parallel kernels below need sixteen binary searches an entry, two scans and a launch for each step: MEASURED_BIG
+// ------------------------------------------------------------------------------------------------
+constexpr uint32_t kBigThreads = 1024, kBigEntries = 49152;        // (sums of a panel fit 16 bits)
+
+struct BigLds {
+    uint32_t rp[17], lo, hi;
+    Two waveSum[kBigThreads / 64];
+};
+
+inline __host__ __device__ uint32_t big_window_words(uint32_t window_words) { return window_words + (window_words + 1u) / 2u; }   // bitmap and 16-bit counts
+
+// Row starts, first and last column; returns the entries of the panel.
+__device__ __forceinline__ uint32_t big_rows(BigLds &l, const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols, uint32_t p, uint32_t &start)
+{
+    const uint32_t t = threadIdx.x;
+    start = rowPtr[uint64_t(p) * 16u];
+    if (t < 17u) l.rp[t] = rowPtr[uint64_t(p) * 16u + t] - start;
+    if (t == 0u) { l.lo = ~0u; l.hi = 0u; }
+    __syncthreads();
+    if (t < 16u && l.rp[t + 1] > l.rp[t]) {
+        atomicMin(&l.lo, cols[uint64_t(start) + l.rp[t]]);
+        atomicMax(&l.hi, cols[uint64_t(start) + l.rp[t + 1] - 1u]);
+    }
+    __syncthreads();
+    return l.rp[16];
+}
+
+// Running counts of the bitmap's words; returns how many columns are active.
+__device__ __forceinline__ uint32_t big_counts(Two (&waveSum)[kBigThreads / 64], const uint32_t *window, uint16_t *count, uint32_t words)
+{
+    const uint32_t t = threadIdx.x, per = (words + kBigThreads - 1u) / kBigThreads, w0 = min(t * per, words), w1 = min(w0 + per, words);
+    uint32_t own = 0;
+    for (uint32_t w = w0; w < w1; ++w) own += uint32_t(__popc(window[w]));
+    Two total;
+    uint32_t run = block_exclusive_over(waveSum, {own, 0u}, total).x;
+    for (uint32_t w = w0; w < w1; ++w) { count[w] = uint16_t(run); run += uint32_t(__popc(window[w])); }
+    __syncthreads();
+    return total.x;
+}
+
+__device__ __forceinline__ uint32_t big_number(const uint32_t *window, const uint16_t *count, uint32_t c)      // c: from the window's start
+{
+    return count[c >> 5] + uint32_t(__popc(window[c >> 5] & ((1u << (c & 31u)) - 1u)));
+}
+
+// Completes the census records of the listed panels (panel_census has counted their entries and found their windows).
+__global__ __launch_bounds__(kBigThreads) void big_census(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols, const float *__restrict__ vals,
+                                                          uint32_t K, const uint32_t *__restrict__ list, uint32_t window_words, uint32_t row_words,
+                                                          PanelCensus *__restrict__ out)
+{
+    extern __shared__ uint32_t window[];
+    __shared__ BigLds l;
+    __shared__ uint32_t pairs[4], stored;
+    uint16_t *count = reinterpret_cast<uint16_t *>(window + window_words);
+    uint32_t *rows = window + big_window_words(window_words);      // 16 bits a column
+    const uint32_t p = list[blockIdx.x], t = threadIdx.x;
+    for (uint32_t w = t; w < window_words; w += kBigThreads) window[w] = 0u;
+    for (uint32_t w = t; w < row_words; w += kBigThreads) rows[w] = 0u;
+    if (t < 4u) pairs[t] = 0u;
+    if (t == 4u) stored = 0u;
+    uint32_t start;
+    const uint32_t n = big_rows(l, rowPtr, cols, p, start), lo = l.lo, reach = l.hi - lo, words = reach / 32u + 1u;
+    // (rows that are not sorted: no column outside the window is marked, and the census refuses the matrix)
+    const bool fits = l.hi >= lo && words <= window_words;
+    int range = 0, unsorted = !fits;
+    uint32_t mine = 0;
+#pragma unroll 4
+    for (uint32_t i = t; i < n; i += kBigThreads) {
+        const uint32_t c = cols[uint64_t(start) + i], before = cols[uint64_t(start) + (i ? i - 1u : 0u)];
+        range |= c >= K;
+        unsorted |= i > l.rp[row_in_panel(l.rp, i)] && before >= c;
+        mine += vals[uint64_t(start) + i] != 0.0f ? 1u : 0u;
+        if (fits && c - lo <= reach) atomicOr(&window[(c - lo) >> 5], 1u << ((c - lo) & 31u));
+    }
+    range = __syncthreads_or(range);
+    unsorted = __syncthreads_or(unsorted);
+    if (range || unsorted) {
+        if (t == 0u) out[p].error = (range ? kErrRange : 0u) | (unsorted ? kErrUnsorted : 0u);
+        return;
+    }
+    const uint32_t active = big_counts(l.waveSum, window, count, words);
+#pragma unroll 4
+    for (uint32_t i = t; i < n; i += kBigThreads) {
+        const uint32_t a = big_number(window, count, cols[uint64_t(start) + i] - lo);
+        atomicOr(&rows[a >> 1], 1u << ((a & 1u) * 16u + row_in_panel(l.rp, i)));
+    }
+    __syncthreads();
+    Two own = {0u, 0u};
+    for (uint32_t a = t; a < active; a += kBigThreads) {
+        const Two here = strips_of(reinterpret_cast<const uint16_t *>(rows)[a]);
+        own.x += here.x;
+        own.y += here.y;
+    }
+    own = {wave_add(own.x), wave_add(own.y)};
+    mine = wave_add(mine);
+    if ((t & 63u) == 63u) {
+#pragma unroll
+        for (uint32_t s = 0; s < 4u; ++s) atomicAdd(&pairs[s], half(own, s));
+        atomicAdd(&stored, mine);
+    }
+    __syncthreads();
+    if (t < 4u) out[p].pairs[t] = pairs[t];
+    if (t == 4u) out[p].stored = stored;
+    if (t == 5u) out[p].cols = active;
+}
+
+// Strip lists of the listed panels (panel_quads<true> defines them), a work-group a strip: its entries are one piece of the arrays, its
+// active columns are its pairs.  row_words: a byte a column, the rows that hold it and those whose entry is not zero.
+// (One work-group for all four strips of a panel: 81 us against MEASURED_QUADS.)
+__global__ __launch_bounds__(kBigThreads) void big_quads(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols, const float *__restrict__ vals,
+                                                         const uint32_t *__restrict__ list, uint32_t window_words, uint32_t row_words, uint32_t mask_words,
+                                                         const uint32_t *__restrict__ groups, const uint32_t *__restrict__ valBase,
+                                                         uint32_t *__restrict__ recs, float *__restrict__ packed)
+{
+    extern __shared__ uint32_t window[];
+    __shared__ Two waveSum[kBigThreads / 64];
+    __shared__ uint32_t lo_hi[2];
+    uint16_t *count = reinterpret_cast<uint16_t *>(window + window_words);
+    uint32_t *rows = window + big_window_words(window_words), *masks = rows + row_words;
+    const uint32_t p = list[blockIdx.x / 4u], s = blockIdx.x % 4u, t = threadIdx.x;
+    const uint32_t group0 = groups[uint64_t(p) * 4u + s], num_groups = groups[uint64_t(p) * 4u + s + 1u] - group0;
+    if (num_groups == 0u) return;
+    uint32_t rp[5];                           // the strip's rows
+#pragma unroll
+    for (uint32_t k = 0; k < 5u; ++k) rp[k] = rowPtr[uint64_t(p) * 16u + 4u * s + k];
+    const uint32_t panel = rowPtr[uint64_t(p) * 16u], start = rp[0], end = rp[4];
+    for (uint32_t w = t; w < window_words; w += kBigThreads) window[w] = 0u;
+    for (uint32_t w = t; w < row_words + mask_words; w += kBigThreads) rows[w] = 0u;
+    if (t == 0u) { lo_hi[0] = ~0u; lo_hi[1] = 0u; }
+    __syncthreads();
+    if (t < 4u && rowPtr[uint64_t(p) * 16u + 4u * s + t + 1u] > rowPtr[uint64_t(p) * 16u + 4u * s + t]) {
+        atomicMin(&lo_hi[0], cols[rowPtr[uint64_t(p) * 16u + 4u * s + t]]);
+        atomicMax(&lo_hi[1], cols[rowPtr[uint64_t(p) * 16u + 4u * s + t + 1u] - 1u]);
+    }
+    uint32_t before = 0;                      // values stored for the strips in front of this one
+#pragma unroll 4
+    for (uint32_t i = panel + t; i < start; i += kBigThreads) before += vals[i] != 0.0f ? 1u : 0u;
+    __syncthreads();
+    const uint32_t lo = lo_hi[0], words = (lo_hi[1] - lo) / 32u + 1u;
+#pragma unroll 4
+    for (uint32_t i = start + t; i < end; i += kBigThreads) {
+        const uint32_t c = cols[i] - lo;
+        atomicOr(&window[c >> 5], 1u << (c & 31u));
+    }
+    __syncthreads();
+    const uint32_t active = big_counts(waveSum, window, count, words);
+#pragma unroll 4
+    for (uint32_t i = start + t; i < end; i += kBigThreads) {
+        const uint32_t a = big_number(window, count, cols[i] - lo), r = (i >= rp[1] ? 1u : 0u) + (i >= rp[2] ? 1u : 0u) + (i >= rp[3] ? 1u : 0u);
+        atomicOr(&rows[a >> 2], ((1u << r) | (vals[i] != 0.0f ? 16u << r : 0u)) << (8u * (a & 3u)));
+    }
+    __syncthreads();
+    // this thread's run of columns, and in front of it: the stored values and the entries of every row
+    const uint8_t *row_of = reinterpret_cast<const uint8_t *>(rows);
+    const uint32_t per = (active + kBigThreads - 1u) / kBigThreads, a0 = min(t * per, active), a1 = min(a0 + per, active);
+    Two row = {0u, 0u}, held = {0u, before};
+    for (uint32_t a = a0; a < a1; ++a) {
+        const uint32_t m = row_of[a];
+        row.x += (m & 1u) | (m >> 1 & 1u) << 16;
+        row.y += (m >> 2 & 1u) | (m >> 3 & 1u) << 16;
+        held.x += uint32_t(__popc(m >> 4));
+    }
+    Two all;
+    row = block_exclusive_over(waveSum, row, all);
+    held = block_exclusive_over(waveSum, held, all);
+    uint32_t next[4], value = valBase[p] + all.y + held.x;
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; ++k) next[k] = rp[k] + half(row, k);
+    uint32_t w = 0, bits = 0;
+    if (a0 < a1) {
+        uint32_t top = words - 1u;            // the last word with no more than a0 columns in front of it
+        while (w < top) {
+            const uint32_t mid = (w + top + 1u) >> 1;
+            if (count[mid] <= a0) w = mid;
+            else top = mid - 1u;
+        }
+        bits = window[w];
+        for (uint32_t skip = a0 - count[w]; skip; --skip) bits &= bits - 1u;
+    }
+    for (uint32_t a = a0; a < a1; ++a) {
+        while (!bits) bits = window[++w];
+        const uint32_t c = lo + 32u * w + uint32_t(__ffs(int(bits))) - 1u, m = row_of[a], g = a >> 4, pair = a & 15u, mask = m >> 4;
+        bits &= bits - 1u;
+        float v[4];
+#pragma unroll
+        for (uint32_t k = 0; k < 4u; ++k)
+            if (m >> k & 1u) v[k] = vals[next[k]++];
+        uint32_t *rec = recs + (uint64_t(group0) + g) * CUTE_QUAD_RECORD_WORDS;
+        rec[pair] = c;
+        if (pair == 0u) { rec[18] = value; rec[19] = 0u; }
+        if (mask) atomicOr(&masks[2u * g + (pair >> 3)], mask << (4u * (pair & 7u)));
+#pragma unroll
+        for (uint32_t k = 0; k < 4u; ++k)
+            if (mask >> k & 1u) packed[value++] = v[k];
+        if (a + 1u == active)
+            for (uint32_t x = pair + 1u; x < 16u; ++x) rec[x] = c;           // padding repeats the last column
+    }
+    __syncthreads();
+    for (uint32_t g = t; g < num_groups; g += kBigThreads) {
+        uint32_t *rec = recs + (uint64_t(group0) + g) * CUTE_QUAD_RECORD_WORDS;
+        rec[16] = masks[2u * g];
+        rec[17] = masks[2u * g + 1u];
     }
 }
 

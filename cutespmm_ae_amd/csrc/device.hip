@@ -649,18 +649,52 @@ struct LargeWork {
     cute_build::PanelCensus *res = nullptr;
 };
 
-// Lists the large panels (panelNnz and panelSpan are known) and numbers their entries.  With `out` given also counts for the planner, into the
-// panels' census records.
-int number_large_panels(const cute_hrpb_dev *d, LargeWork &w, cute_build::PanelCensus *out)
+// Lists the large panels (panelNnz and panelSpan are known).
+void list_large_panels(const cute_hrpb_dev *d, LargeWork &w)
 {
+    if (!w.prefix.empty()) return;
     w.prefix.assign(1, 0u);
     for (uint32_t p = 0; p < d->P; ++p)
         if (panel_is_large(d, p)) {
             w.panel.push_back(p);
             w.prefix.push_back(w.prefix.back() + d->panelNnz[p]);
         }
+}
+
+// LDS beside the static part that big_census and big_quads may ask for: a compute unit's, less a little.
+constexpr uint32_t kBigLds = (160u << 10) - 1024u;
+
+// The words big_census wants for the rows of the columns of every large panel; 0: there are some that it does not take.
+uint32_t big_census_rows(const cute_hrpb_dev *d, const LargeWork &w)
+{
+    uint32_t most = 0;
+    for (uint32_t p : w.panel) {
+        if (d->panelNnz[p] > cute_build::kBigEntries || d->panelSpan[p] > max_span(d) || d->panelSpan[p] == 0) return 0;
+        most = std::max(most, std::min(d->panelNnz[p], d->panelSpan[p]));
+    }
+    const uint32_t words = (most + 1u) / 2u;
+    return (cute_build::big_window_words(cute_build::panel_window_words(max_span(d))) + words) * 4u <= kBigLds ? words : 0u;
+}
+
+// The same for big_quads (the census has counted the columns of every strip): a byte a column, and the words of its groups' masks.
+uint32_t big_quad_rows(const cute_hrpb_dev *d, const LargeWork &w, uint32_t &masks)
+{
+    uint32_t most = 0;
+    for (uint32_t p : w.panel) {
+        if (d->panelNnz[p] > cute_build::kBigEntries || d->panelSpan[p] > max_span(d)) return 0;
+        for (uint32_t s = 0; s < 4u; ++s) most = std::max(most, d->stripPairs[4u * p + s]);
+    }
+    masks = (most + 15u) / 16u * 2u;
+    const uint32_t words = (most + 3u) / 4u;
+    return (cute_build::big_window_words(cute_build::panel_window_words(max_span(d))) + words + masks) * 4u <= kBigLds ? words : 0u;
+}
+
+// Numbers the entries of the large panels.  With `out` given also counts for the planner, into the panels' census records.
+int number_large_panels(const cute_hrpb_dev *d, LargeWork &w, cute_build::PanelCensus *out)
+{
+    list_large_panels(d, w);
     const uint32_t count = uint32_t(w.panel.size()), total = w.prefix.back();
-    if (!count) return CUTE_OK;
+    if (!count || w.posP) return CUTE_OK;
     Layout lay;
     const uint64_t oPanel = lay.add(count, 4), oPrefix = lay.add(count + 1u, 4), oRes = lay.add(count, sizeof(cute_build::PanelCensus));
     const uint64_t staged = lay.bytes;
@@ -690,8 +724,10 @@ int number_large_panels(const cute_hrpb_dev *d, LargeWork &w, cute_build::PanelC
 }
 
 // Brick tiles from the device CSR copy: the arrays cute_hrpb_retile makes on the host, word for word.
-int build_bricks_on_device(cute_hrpb_dev *d, const LargeWork &w)
+int build_bricks_on_device(cute_hrpb_dev *d, LargeWork &w)
 {
+    int rc = number_large_panels(d, w, nullptr);
+    if (rc != CUTE_OK) return rc;
     const uint64_t hdr_words = uint64_t(d->nb) * CUTE_TILED_HDR_WORDS, num_vals = uint64_t(d->nnz) + 64u;
     const uint32_t count = uint32_t(w.panel.size());
     Layout lay, tab;
@@ -701,7 +737,7 @@ int build_bricks_on_device(cute_hrpb_dev *d, const LargeWork &w)
     const uint64_t oHdr = lay.add(hdr_words, 4), oVals = lay.add(num_vals, 4), oTab = lay.add(tab.bytes, 1);
     DevBuf mem;
     PinnedBuf pin;
-    int rc = mem.alloc(lay.bytes);
+    rc = mem.alloc(lay.bytes);
     if (rc == CUTE_OK) rc = pin.alloc(tab.bytes);
     if (rc != CUTE_OK) return rc;
     auto table = [&](uint64_t o) { return Layout::at<const uint32_t>(mem.p, oTab + o); };
@@ -743,21 +779,26 @@ int build_bricks_on_device(cute_hrpb_dev *d, const LargeWork &w)
 }
 
 // Quad lists (in the layout the census chose) from the device CSR copy: the arrays cute_quad_pack makes.
-int build_quads_on_device(cute_hrpb_dev *d, const LargeWork &w)
+int build_quads_on_device(cute_hrpb_dev *d, LargeWork &w)
 {
     const uint64_t G = d->numGroups, stored = d->numQuadVals;
     const bool strips = d->quadRows == 4;
-    const uint32_t count = uint32_t(w.panel.size()), per = strips ? 4u : 1u;
+    list_large_panels(d, w);
+    uint32_t big_masks = 0;
+    const uint32_t big_rows = strips ? big_quad_rows(d, w, big_masks) : 0u;      // all large panels through big_quads, or none
+    int rc = big_rows ? int(CUTE_OK) : number_large_panels(d, w, nullptr);
+    if (rc != CUTE_OK) return rc;
+    const uint32_t count = big_rows ? 0u : uint32_t(w.panel.size()), per = strips ? 4u : 1u;
     Layout lay, tab;
     const uint64_t oGroup = tab.add(d->qgp.size(), 4), oBase = tab.add(uint64_t(d->P) + 1u, 4), oUnit = tab.add(count, 4),
                    oPrefix = tab.add(count + 1u, 4), oFirst = tab.add(uint64_t(count) * per, 4), oPairs = tab.add(uint64_t(count) * 4u, 4),
                    oLargeBase = tab.add(count, 4);
     const std::vector<uint32_t> medium = panels_between(d, cute_build::kPanelList);
-    const uint64_t oMedium = tab.add(medium.size(), 4);
+    const uint64_t oMedium = tab.add(medium.size(), 4), oBig = tab.add(w.panel.size(), 4);
     const uint64_t oRecs = lay.add(G * CUTE_QUAD_RECORD_WORDS, 4), oVals = lay.add(stored + 64u, 4), oTab = lay.add(tab.bytes, 1);
     DevBuf mem, counts;
     PinnedBuf pin;
-    int rc = mem.alloc(lay.bytes);
+    rc = mem.alloc(lay.bytes);
     if (rc == CUTE_OK) rc = pin.alloc(tab.bytes);
     if (rc != CUTE_OK) return rc;
     auto table = [&](uint64_t o) { return Layout::at<const uint32_t>(mem.p, oTab + o); };
@@ -765,6 +806,7 @@ int build_quads_on_device(cute_hrpb_dev *d, const LargeWork &w)
     float *packed = Layout::at<float>(mem.p, oVals);
     std::memcpy(pin.as<char>(oGroup), d->qgp.data(), d->qgp.size() * 4u);
     if (!medium.empty()) std::memcpy(pin.as<char>(oMedium), medium.data(), medium.size() * 4u);
+    if (big_rows) std::memcpy(pin.as<char>(oBig), w.panel.data(), w.panel.size() * 4u);
     uint32_t *base = pin.as<uint32_t>(oBase), *unit = pin.as<uint32_t>(oUnit), *prefix = pin.as<uint32_t>(oPrefix), *first = pin.as<uint32_t>(oFirst),
              *pairs = pin.as<uint32_t>(oPairs), *large_base = pin.as<uint32_t>(oLargeBase);
     base[0] = 0;
@@ -801,6 +843,13 @@ int build_quads_on_device(cute_hrpb_dev *d, const LargeWork &w)
         CUTE_BUILD((cute_build::large_quads<S, true>), grid_of(w.L.total), w.L, d->dRowPtr, d->dCols, d->dCsrVals, w.posS, w.DS,        \
                    table(oFirst), recs, packed);                                                                                      \
     }
+    // (the panels that take longest go first)
+    if (big_rows) {
+        const uint32_t words = cute_build::panel_window_words(max_span(d));
+        hipLaunchKernelGGL(cute_build::big_quads, dim3(uint32_t(w.panel.size()) * 4u), dim3(cute_build::kBigThreads),
+                           (cute_build::big_window_words(words) + big_rows + big_masks) * 4u, nullptr, d->dRowPtr, d->dCols, d->dCsrVals, table(oBig), words,
+                           big_rows, big_masks, table(oGroup), table(oBase), recs, packed);
+    }
     if (strips) { CUTE_BUILD_QUADS(true) } else { CUTE_BUILD_QUADS(false) }
 #undef CUTE_BUILD_QUADS
 #undef CUTE_PANEL_QUADS
@@ -822,8 +871,6 @@ int ensure_layout(cute_hrpb_dev *d, int which)
     std::lock_guard<std::mutex> guard(d->lock);
     if (which == 1 ? d->haveBricks : d->haveQuads) return CUTE_OK;
     LargeWork w;
-    const int rc = number_large_panels(d, w, nullptr);
-    if (rc != CUTE_OK) return rc;
     return which == 1 ? build_bricks_on_device(d, w) : build_quads_on_device(d, w);
 }
 
@@ -1027,17 +1074,27 @@ int finish_upload(cute_hrpb_dev *d, int quad_layout, const DeviceContext &c)
         }
         if (!error && (any_medium || any_large)) {
             const std::vector<uint32_t> medium = panels_between(d, cute_build::kPanelFirst);
+            list_large_panels(d, large);
+            const uint32_t big_rows = big_census_rows(d, large);
             PinnedBuf list;
-            rc = list.alloc(medium.size() * 4u);
+            rc = list.alloc((medium.size() + large.panel.size()) * 4u);
             if (rc != CUTE_OK) return rc;
             list.pending = true;
+            if (big_rows) {
+                const uint32_t words = cute_build::panel_window_words(max_span(d));
+                std::memcpy(list.as<uint32_t>() + medium.size(), large.panel.data(), large.panel.size() * 4u);
+                hipLaunchKernelGGL(cute_build::big_census, dim3(uint32_t(large.panel.size())), dim3(cute_build::kBigThreads),
+                                   (cute_build::big_window_words(words) + big_rows) * 4u, nullptr, d->dRowPtr, d->dCols, d->dCsrVals, d->K,
+                                   list.as<const uint32_t>() + medium.size(), words, big_rows, pin.as<cute_build::PanelCensus>());
+                rc = check_launch("panel census");
+            }
             if (!medium.empty()) {
                 std::memcpy(list.p, medium.data(), medium.size() * 4u);
                 CUTE_PANELS(cute_build::panel_census<cute_build::kPanelCap>, cute_build::kPanelCap, uint32_t(medium.size()), window_lds(d, 0),
                             d->dRowPtr, d->dCols, d->dCsrVals, P, d->K, d->nnz, max_span(d), list.as<const uint32_t>(), pin.as<cute_build::PanelCensus>());
-                rc = check_launch("panel census");
+                if (rc == CUTE_OK) rc = check_launch("panel census");
             }
-            if (rc == CUTE_OK && any_large) rc = number_large_panels(d, large, pin.as<cute_build::PanelCensus>());
+            if (rc == CUTE_OK && any_large && !big_rows) rc = number_large_panels(d, large, pin.as<cute_build::PanelCensus>());
             if (rc == CUTE_OK) rc = list.wait();
             if (rc != CUTE_OK) return rc;
             for (uint32_t p : medium) error |= r[p].error;
