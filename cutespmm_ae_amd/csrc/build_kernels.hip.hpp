@@ -550,7 +550,8 @@ __global__ __launch_bounds__(panel_threads(CAP)) void panel_quads(const uint32_t
 // Panels of more than kPanelCap entries (the hub rows of a graph) whose window the bitmap takes: a work-group of sixteen wavefronts
 // walks the entries instead of holding them, for the census and for the strip lists.  LDS holds the bitmap, its counts and the
 // rows of every active column, and the rest follows from prefix sums over the columns, a thread a run of them.
-// The entry-parallel kernels below need sixteen binary searches an entry, two scans and a launch for each step: MEASURED_BIG
+// The entry-parallel kernels below need sixteen binary searches an entry, two scans and a launch for each step: R-MAT graph of 65 536
+// nodes, 449 000 entries in 79 such panels, census 70 -> 38 us, lists 70 -> 34.
 // ------------------------------------------------------------------------------------------------
 constexpr uint32_t kBigThreads = 1024, kBigEntries = 49152;        // (sums of a panel fit 16 bits)
 
@@ -658,7 +659,7 @@ __global__ __launch_bounds__(kBigThreads) void big_census(const uint32_t *__rest
 
 // Strip lists of the listed panels (panel_quads<true> defines them), a work-group a strip: its entries are one piece of the arrays, its
 // active columns are its pairs.  row_words: a byte a column, the rows that hold it and those whose entry is not zero.
-// (One work-group for all four strips of a panel: 81 us against MEASURED_QUADS.)
+// (One work-group for all four strips of a panel: 81 us against 34.)
 __global__ __launch_bounds__(kBigThreads) void big_quads(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols, const float *__restrict__ vals,
                                                          const uint32_t *__restrict__ list, uint32_t window_words, uint32_t row_words, uint32_t mask_words,
                                                          const uint32_t *__restrict__ groups, const uint32_t *__restrict__ valBase,
@@ -1062,11 +1063,11 @@ __global__ __launch_bounds__(kThreads) void mark_hub_columns(const uint32_t *__r
 }
 
 // The entries of csr_rows_window (which describes them): a work-group is a slice.  The slice's part of the CSR arrays is one piece,
-// so it is read, and the quads are written, whole lines at a time by four wavefronts, and one, a row a lane, sorts in between in
-// LDS (a lane that walks its row in global memory touches a line an entry: 33.5 million entries 2 400 us,
-// this way 300).  The order inside a row, (slot +
-// row / 2) mod 8, is a counting sort by the eight bytes of one word: rows of fewer than 256 entries.  `staged`: {first quad, -,
-// quads, -} of every slice, and the tiles' windows, in host memory; slices[] gets the quads that no row of the slice pads besides.
+// so it is read, and the quads are written, whole lines at a time, and four lanes a row sort in between in
+// LDS (a lane that walks its row in global memory touches a line an entry: 33.5 million entries 2 400 us; one lane a row in LDS
+// 300, this way 94, 5 TB/s).  The order inside a row, (slot + row / 2) mod 8, is a counting sort by the eight bytes of one
+// word: rows of fewer than 256 entries.  `staged`: {first quad, -, quads, -} of every slice, and the tiles' windows, in host memory
+// (asked for behind the entries, which would wait for it); slices[] gets the quads that no row of the slice pads besides.
 struct WindowTables {
     const uint4 *slices;       // staged
     const uint2 *tiles;
@@ -1075,20 +1076,22 @@ struct WindowTables {
     uint2 *dTiles;
 };
 
-__device__ __forceinline__ uint32_t skewed(uint32_t i) { return i + (i >> 5); }    // rows of 32 entries do not start in one bank
+// rows of 32 entries do not start in one bank
+__device__ __forceinline__ uint32_t skewed(uint32_t i) { return i + (i >> 5); }
+__device__ __forceinline__ uint32_t skewed_half(uint32_t i) { return i + 2u * (i >> 5); }
 
 __global__ __launch_bounds__(kThreads) void window_entries(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols, const float *__restrict__ vals,
                                                      uint32_t M, uint32_t ring_rows, WindowTables T, uint32_t longest, uint2 *__restrict__ slots,
                                                      f32x4 *__restrict__ out)
 {
+    static_assert(kThreads == 4 * 64, "four lanes a row");
     extern __shared__ uint32_t lds[];
+    __shared__ uint32_t least_of[kThreads / 64];
     const uint32_t slice = blockIdx.x, tid = threadIdx.x, row0 = slice * 64u;
-    for (uint32_t t = slice * kThreads + tid; t < T.numTiles; t += gridDim.x * kThreads) T.dTiles[t] = T.tiles[t];
-    uint32_t *slot_of = lds, *placed = lds + skewed(64u * longest) + 1u;
-    float *val_of = reinterpret_cast<float *>(placed + 32u * longest), *placed_val = val_of + skewed(64u * longest) + 1u;
-    uint16_t *placed_slot = reinterpret_cast<uint16_t *>(placed);
-    uint4 d = T.slices[slice];
-    const uint32_t begin = rowPtr[row0], end = rowPtr[min(row0 + 64u, M)];
+    float *val_of = reinterpret_cast<float *>(lds), *placed_val = val_of + skewed(64u * longest);
+    uint16_t *placed_slot = reinterpret_cast<uint16_t *>(placed_val + 64u * longest), *slot_of = placed_slot + 64u * longest;
+    const uint32_t lane = tid >> 2, part = tid & 3u, row = row0 + lane, begin = rowPtr[row0], end = rowPtr[min(row0 + 64u, M)],
+                   s = rowPtr[min(row, M)], n = rowPtr[min(row + 1u, M)] - s;
     for (uint32_t base = begin; base < end; base += 8u * kThreads) {
         uint32_t col[8];
         float val[8];
@@ -1100,40 +1103,55 @@ __global__ __launch_bounds__(kThreads) void window_entries(const uint32_t *__res
 #pragma unroll
         for (uint32_t u = 0; u < 8u; ++u) {
             const uint32_t i = base + u * kThreads + tid;
-            if (i < end) { slot_of[skewed(i - begin)] = col[u] % ring_rows; val_of[skewed(i - begin)] = val[u]; }
+            if (i < end) { slot_of[skewed_half(i - begin)] = uint16_t(col[u] % ring_rows); val_of[skewed(i - begin)] = val[u]; }
         }
     }
+    uint4 d = T.slices[slice];
+    for (uint32_t t = slice * kThreads + tid; t < T.numTiles; t += gridDim.x * kThreads) T.dTiles[t] = T.tiles[t];
     __syncthreads();
-    if (tid < 64u) {
-        const uint32_t lane = tid, row = row0 + lane, s = rowPtr[min(row, M)], n = rowPtr[min(row + 1u, M)] - s, turn = lane >> 1, first = s - begin;
-        uint64_t place = 0;
-        for (uint32_t i = 0; i < n; ++i) place += 1ull << (8u * ((slot_of[skewed(first + i)] + turn) & 7u));
-        place *= 0x0101010101010100ull;       // where the entries of each of the eight begin
+    {
+        const uint32_t turn = lane >> 1, first = s - begin, per = (n + 3u) / 4u, i0 = min(part * per, n), i1 = min(i0 + per, n);
+        uint64_t mine = 0;
+        for (uint32_t i = i0; i < i1; ++i) mine += 1ull << (8u * ((slot_of[skewed_half(first + i)] + turn) & 7u));
+        uint64_t upto = mine;
+#pragma unroll
+        for (int step = 1; step < 4; step *= 2) {
+            const uint64_t other = __shfl_up(static_cast<unsigned long long>(upto), step, 4);
+            if (part >= uint32_t(step)) upto += other;
+        }
+        // where the entries of each of the eight begin, and this lane's among them
+        const uint64_t all = __shfl(static_cast<unsigned long long>(upto), 3, 4);
+        uint64_t place = all * 0x0101010101010100ull + (upto - mine);
         auto at = [&](uint32_t k) { return (k / 4u * 64u + lane) * 4u + k % 4u; };
-        for (uint32_t i = 0; i < n; ++i) {
-            const uint32_t slot = slot_of[skewed(first + i)], shift = 8u * ((slot + turn) & 7u), to = at(uint32_t(place >> shift) & 255u);
+        for (uint32_t i = i0; i < i1; ++i) {
+            const uint32_t slot = slot_of[skewed_half(first + i)], shift = 8u * ((slot + turn) & 7u), to = at(uint32_t(place >> shift) & 255u);
             place += 1ull << shift;
             placed_slot[to] = uint16_t(slot);
             placed_val[to] = val_of[skewed(first + i)];
         }
-        for (uint32_t k = n; k < d.z * 4u; ++k) {
+        for (uint32_t k = n + part; k < d.z * 4u; k += 4u) {
             placed_slot[at(k)] = uint16_t(0xffffu);
             placed_val[at(k)] = 0.0f;
         }
         uint32_t least = n / 4u;
 #pragma unroll
         for (int step = 1; step < 64; step *= 2) least = min(least, uint32_t(__shfl_xor(int(least), step)));
-        d.y = least;
-        if (lane == 0u) T.dSlices[slice] = d;
+        if ((tid & 63u) == 0u) least_of[tid >> 6] = least;
     }
     __syncthreads();
+    if (tid == 0u) {
+        d.y = min(min(least_of[0], least_of[1]), min(least_of[2], least_of[3]));
+        T.dSlices[slice] = d;
+    }
+    const uint2 *slots_in = reinterpret_cast<const uint2 *>(placed_slot);
+    const f32x4 *vals_in = reinterpret_cast<const f32x4 *>(placed_val);
     for (uint32_t i = tid; i < d.z * 64u; i += kThreads) {
-        slots[size_t(d.x) * 64u + i] = make_uint2(placed[2u * i], placed[2u * i + 1u]);
-        out[size_t(d.x) * 64u + i] = f32x4{placed_val[4u * i], placed_val[4u * i + 1u], placed_val[4u * i + 2u], placed_val[4u * i + 3u]};
+        slots[size_t(d.x) * 64u + i] = slots_in[i];
+        out[size_t(d.x) * 64u + i] = vals_in[i];
     }
 }
 
-// LDS of window_entries for rows of up to `longest` entries (a multiple of four).
-inline uint32_t window_entries_lds(uint32_t longest) { return (2u * (64u * longest + 2u * longest + 1u) + 96u * longest) * 4u; }
+// LDS of window_entries for rows of up to `longest` entries (a multiple of four, so that what is read 16 bytes at a time begins at them).
+inline uint32_t window_entries_lds(uint32_t longest) { return 64u * longest * 12u + 2u * longest * 4u + 4u * longest * 2u; }
 
 }  // namespace cute_build

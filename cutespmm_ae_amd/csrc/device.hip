@@ -227,6 +227,7 @@ struct cute_hrpb_dev {
     std::vector<uint32_t> panelMaxRow;  // longest row of each panel
     std::vector<uint32_t> panelSpan;    // width of each panel's column window (last column - first column + 1)
     std::vector<uint32_t> panelFirst;   // ... and its first column
+    uint32_t widestPanel = 0;           // the largest of panelSpan
     // the entries as csr_rows_window reads them (which describes them), built for the first plan that uses that kernel
     bool haveWindow = false;
     uint4 *dSlices = nullptr;
@@ -1070,6 +1071,7 @@ int finish_upload(cute_hrpb_dev *d, int quad_layout, const DeviceContext &c)
             d->panelNnz[p] = r[p].nnz;
             d->panelSpan[p] = r[p].span;
             d->panelFirst[p] = r[p].first;
+            d->widestPanel = std::max(d->widestPanel, r[p].span);
             if (r[p].nnz > cute_build::kPanelFirst || r[p].span > max_span(d)) (panel_is_large(d, p) ? any_large : any_medium) = true;
         }
         if (!error && (any_medium || any_large)) {
@@ -1167,42 +1169,55 @@ int make_hub_tables(cute_spmm_plan *p, const cute_hrpb_dev *d, uint32_t hub_rows
 
 // Rows of a plan without MFMA panels through csr_rows_window where that is ahead.  Needs the widest window of a tile to fit the ring,
 // rows of up to 64 entries (the LDS of window_entries) and little padding: a lane waits for the longest of 64 rows.  Then both kernels'
-// times are estimated, in us, and the ring has to be ahead by 15 %, of a launch worth the tables.  Fitted on 400 banded matrices drawn
+// times are estimated, in us, and the ring has to be ahead by 15 %.  Fitted on 400 banded matrices drawn
 // over 4 096 ... 640 000 rows, 8 ... 48 entries a row, bands of 64 ... 2 048 and N = 16 ... 600 (rms 18 and 14 % for rings of 8
-// and 16 columns, 15 % for the row kernel): of those it takes, none was more than 2.5 % slower, and over all of them the products take
-// 0.895 of the row kernel's time where the better of the two would take 0.869.  65 536 rows of 32, band of 2 048, us row kernel / ring: N = 32
-// 12.4 / 14.8, N = 256 82.6 / 58.6; 16 rows N = 128 24.4 / 26.2; 262 144 rows of 12, band of 700, N = 128 72.7 / 76.3; 32 768 rows of
-// 24, band of 1 500, N = 128 17.0 / 19.1; band of 200, 65 536 rows of 32, N = 101 39.0 / 25.1; 1 048 576 rows of 32, band of 2 048,
-// N = 256 1 714 / 1 005.
-void plan_window(cute_spmm_plan *p, cute_hrpb_dev *d, uint32_t N, const DeviceContext &c)
+// and 16 columns, 15 % for the row kernel): with a lead of 15 % and 12 us none was more than 2.5 % slower, and over all of them the
+// products take 0.895 of the row kernel's time where the better of the two would take 0.869.  65 536 rows of 32, band of 2 048, us row
+// kernel / ring: N = 32 12.4 / 14.8, N = 256 82.6 / 58.6; 16 rows N = 128 24.4 / 26.2; 262 144 rows of 12, band of 700, N = 128
+// 72.7 / 76.3; 32 768 rows of 24, band of 1 500, N = 128 17.0 / 19.1; band of 200, 65 536 rows of 32, N = 101 39.0 / 25.1; 1 048 576
+// rows of 32, band of 2 048, N = 256 1 714 / 1 005.
+//
+// A plan may be made for one product (a matrix that is new to every step), so the lead has to pay for the second form of the
+// entries as well: plan creation with it takes, in us, 25 longer for 65 536 rows of 32 entries, 32 for 200 000 of 12, 33 for 131 072
+// of 32, 42 for 262 144, 46 for 524 288, 186 for 1 048 576 (format, plan and one product of 65 536 rows, N = 256: 202 / 223; 80 000
+// rows of 30, N = 101: 191 / 212).  A caller that says its product runs in a loop (operand_residency 2) gets the ring without that.
+void plan_window(cute_spmm_plan *p, cute_hrpb_dev *d, uint32_t N, const DeviceContext &c, bool loop)
 {
-    WindowShape w;
-    if (N < 16u || d->P == 0 || !window_shape(d, w) || w.quads * 256u > uint64_t(d->nnz) + d->nnz / 4u + 4096u) return;
-    const uint32_t W = w.widest <= cute_dev::kWindowRows<16> ? 16u : 8u;
-    const uint32_t n = uint32_t(w.tiles.size()), slabs = (N + W - 1u) / W, cus = uint32_t(c.num_cus) / cute_dev::kNumXcd;
-    const double row = double(w.quads) * 256.0 / double(d->M), bytes = 8.0 * d->M * N + 8.0 * d->nnz, gathers = 4e-6 * double(d->nnz) * N;
+    if (N < 16u || d->P == 0) return;
+    const double bytes = 8.0 * d->M * N + 8.0 * d->nnz, gathers = 4e-6 * double(d->nnz) * N;
     const bool beyond = uint64_t(d->K + uint64_t(d->M)) * N * sizeof(float) > c.cache_bytes;
-    // a CU holds one work-group at a time: `rounds` of them after each other, each a first window and then its tiles
-    const double first = W == 16u ? 0.8 : 2.0, tile = (W == 16u ? 3.8 + 0.245 * row : 2.6 + 0.143 * row) + (beyond ? (W == 16u ? 2.4 : 1.7) : 0.0);
-    double ring = 0.0;
-    for (uint32_t per_xcd = 1;; ++per_xcd) {
-        const uint32_t chains = per_xcd * cute_dev::kNumXcd, length = (n + chains - 1u) / chains, rounds = (slabs * per_xcd + cus - 1u) / cus;
-        const double time = rounds * (first + length * tile);
-        if (per_xcd == 1 || time < ring) {
-            ring = time;
-            p->windowChains = chains;
-            p->windowChainTiles = length;
-        }
-        if (length == 1u || per_xcd == 64u) break;
-    }
     const uint32_t walk = uint32_t(p->rows_vec) << p->rows_logl;       // columns a lane group covers, used or not
     const double covered = double((N + walk - 1u) / walk * walk) / N;
     const double rows = 3.1 + gathers / 20.0 * (0.29 + 0.40 * covered + (N % 32u ? 0.10 : 0.0)) + bytes * 1e-6 * (0.04 + (beyond ? 0.09 : 0.0));
+    const double lead = loop ? 12.0 : 15.0 + 2e-3 * d->P + 3e-6 * double(d->nnz);
+    constexpr uint32_t per_tile = cute_dev::kWindowTile / CUTE_TM;
+    const uint32_t n = (d->P + per_tile - 1u) / per_tile, cus = uint32_t(c.num_cus) / cute_dev::kNumXcd;
+    // a CU holds one work-group at a time: `rounds` of them after each other, each a first window and then its tiles
+    auto ring_time = [&](uint32_t W, double row) {
+        const uint32_t slabs = (N + W - 1u) / W;
+        const double first = W == 16u ? 0.8 : 2.0, tile = (W == 16u ? 3.8 + 0.245 * row : 2.6 + 0.143 * row) + (beyond ? (W == 16u ? 2.4 : 1.7) : 0.0);
+        double ring = 0.0;
+        for (uint32_t per_xcd = 1;; ++per_xcd) {
+            const uint32_t chains = per_xcd * cute_dev::kNumXcd, length = (n + chains - 1u) / chains, rounds = (slabs * per_xcd + cus - 1u) / cus;
+            const double time = rounds * (first + length * tile);
+            if (per_xcd == 1 || time < ring) {
+                ring = time;
+                p->windowChains = chains;
+                p->windowChainTiles = length;
+            }
+            if (length <= 1u || per_xcd == 64u) return ring;
+        }
+    };
+    auto ahead = [&](double ring) { return ring * 1.15 <= rows && rows - ring >= lead; };
+    // (what the widest panel and the mean row allow at best, before the panels are looked at)
+    const double mean = double(d->nnz) / double(d->M);
+    if (d->widestPanel > cute_dev::kWindowRows<8> || rows < lead ||
+        !(ahead(ring_time(8, mean)) || (d->widestPanel <= cute_dev::kWindowRows<16> && ahead(ring_time(16, mean))))) return;
+    WindowShape w;
+    if (!window_shape(d, w) || w.quads * 256u > uint64_t(d->nnz) + d->nnz / 4u + 4096u) return;
+    const uint32_t W = w.widest <= cute_dev::kWindowRows<16> ? 16u : 8u;
+    if (!ahead(ring_time(W, double(w.quads) * 256.0 / double(d->M)))) return;
     p->windowWarm = beyond;
-#ifdef CUTE_WIN_FORCE
-    if (const char *f = getenv("CUTE_WIN")) { if (f[0] == '0') return; } else
-#endif
-    if (ring * 1.15 > rows || rows - ring < 12.0) return;
     // (without the memory for a second form of the entries the row kernel takes the rows as ever)
     if (ensure_window(d, w, W == 16u ? cute_dev::kWindowRows<16> : cute_dev::kWindowRows<8>) == CUTE_OK) p->windowColumns = W;
 }
@@ -1659,7 +1674,7 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
         }
         p->rowColumnSlabs = rows_columns ? p->rows_slabs : 0u;
     }
-    if (n_brick == 0 && default_bars) plan_window(p, d, N, c);
+    if (n_brick == 0 && default_bars) plan_window(p, d, N, c, t.operand_residency == 2);
     // The chunk list depends on the MFMA kernel (its work units are blocks or list groups).  It is built,
     // and if the partial tiles of the cut panels then turn out to be more rows than the fast kernels'
     // 24-bit row operand can address, built once more for the pipelined brick kernel, whose stores use

@@ -435,7 +435,8 @@ typedef struct cute_tunables {
                                   fresh data finds its operands in HBM whatever their size; 1 from HBM (a product on data no
                                   cache holds); 2 cache-resident (a tight loop over the same operands that fit the 256 MiB
                                   Infinity Cache together; ignored when they do not).  Chooses between the MFMA kernels
-                                  (and, for 1, keeps two column groups per lane in mixed plans), nothing else. */
+                                  (and, for 1, keeps two column groups per lane in mixed plans); 2 also leaves out what the
+                                  tables of csr_rows_window cost, which the loop pays once (cute_spmm_plan_window). */
     uint32_t hub_rows;         /* > 0 (at most 256): the quad kernel on strip lists runs as persistent work-groups that keep that many
                                   of the most referenced B rows in LDS (graphs with hub vertices); 0: off.  Ignored by other plans
                                   (cute_plan_info.hubRows says how many rows a plan stages) */

@@ -28,7 +28,7 @@ def _band(M, K, counts, reach, seed, start=None):
 def _check(cs, orc, torch, rp, cl, vl, M, K, N, columns, B=None):
     B = np.random.default_rng(N).integers(-8, 9, (K, N)).astype(np.float32) if B is None else B
     h = cs.DeviceHRPB(M, K, *(torch.from_numpy(a.view(np.int32) if a.dtype == np.uint32 else a).cuda() for a in (rp, cl, vl)))
-    plan = cs.SPMM_TC(h, N)
+    plan = cs.SPMM_TC(h, N, operand_residency=2)
     assert plan.window_columns == columns and plan.info["numChunks"] == 0
     C = torch.full((M * N + 64,), 7.5, device="cuda")
     out = C[:M * N].view(M, N)
@@ -82,3 +82,13 @@ def test_rows_of_b_that_are_not_finite(cs, orc, torch_cuda):
     B[::1000] = np.inf
     B[500::1000, ::3] = np.nan
     _check(cs, orc, torch_cuda, rp, cl, vl, M, M, N, 16, B)
+
+
+@pytest.mark.parametrize("M,per_row,reach,N,columns", [(65536, 32, 4097, 256, 0), (80000, 30, 400, 101, 0), (200000, 12, 1400, 256, 0), (1048576, 32, 4097, 256, 8)])
+def test_a_plan_for_one_product(cs, torch_cuda, M, per_row, reach, N, columns):
+    """The lead has to pay for the second form of the entries, unless the caller says that the product runs in a loop."""
+    rp, cl, vl = _band(M, M, per_row, reach, M)
+    h = cs.DeviceHRPB(M, M, *(torch_cuda.from_numpy(a.view(np.int32) if a.dtype == np.uint32 else a).cuda() for a in (rp, cl, vl)))
+    assert cs.SPMM_TC(h, N).window_columns == columns
+    if columns == 0 and M < 200000:
+        assert cs.SPMM_TC(h, N, operand_residency=2).window_columns != 0
