@@ -1183,7 +1183,8 @@ int make_hub_tables(cute_spmm_plan *p, const cute_hrpb_dev *d, uint32_t hub_rows
 // rows of 30, N = 101: 191 / 212).  A caller that says its product runs in a loop (operand_residency 2) gets the ring without that.
 void plan_window(cute_spmm_plan *p, cute_hrpb_dev *d, uint32_t N, const DeviceContext &c, bool loop)
 {
-    if (N < 16u || d->P == 0) return;
+    // (beyond 32 768 columns the 1 024 threads of every slab of up to 512 chains could pass the 2^32 a launch may have)
+    if (N < 16u || N > 32768u || d->P == 0) return;
     const double bytes = 8.0 * d->M * N + 8.0 * d->nnz, gathers = 4e-6 * double(d->nnz) * N;
     const bool beyond = uint64_t(d->K + uint64_t(d->M)) * N * sizeof(float) > c.cache_bytes;
     const uint32_t walk = uint32_t(p->rows_vec) << p->rows_logl;       // columns a lane group covers, used or not
