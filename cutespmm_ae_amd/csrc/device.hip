@@ -5,7 +5,6 @@
 #include <cstdio>
 #include <functional>
 #include <mutex>
-#include <queue>
 #include <string>
 #include <unordered_map>
 
@@ -227,7 +226,7 @@ struct cute_hrpb_dev {
     std::vector<uint32_t> panelMaxRow;  // longest row of each panel
     std::vector<uint32_t> panelSpan;    // width of each panel's column window (last column - first column + 1)
     std::vector<uint32_t> panelFirst;   // ... and its first column
-    uint32_t widestPanel = 0;           // the largest of panelSpan
+    uint32_t widestPanel = 0, longestPanel = 0;         // the largest of panelSpan and of panelNnz
     // the entries as csr_rows_window reads them (which describes them), built for the first plan that uses that kernel
     bool haveWindow = false;
     uint4 *dSlices = nullptr;
@@ -287,62 +286,105 @@ namespace {
 // SIMD it touches lowest (ties: the earliest position, so equal items stay in panel order and keep sharing B
 // rows in the L1).  The new order is used only if the model says it shortens the fullest SIMD by 3 % or more.
 // An item costs its length plus a fixed two units (descriptor, first operands, the store).
+// The positions that meet the same SIMDs in every slab (cus_per_xcd work-groups apart, one wavefront further) are a class, one for every
+// SIMD of the first slab, and a class is as loaded as any of its positions: a heap holds the classes by load and first free
+// position, not the positions.  Nothing is dealt where even a perfect order would not gain the 3 %.  (The host threads take longer to wake than
+// this takes.  One heap of all positions: 400 us of the 510 that a new 9-point matrix of 300 x 300 points took from format to product, N = 64.)
 bool deal_chunks(std::vector<uint4> &chunks, uint32_t num_slabs, uint32_t cus_per_xcd, uint32_t waves_per_simd, bool force)
 {
-    const uint32_t wpg = cute_dev::kWavesPerGroup;
+    constexpr uint32_t wpg = cute_dev::kWavesPerGroup, xcds = cute_dev::kNumXcd;
     if (cus_per_xcd == 0 || wpg != 4) return false;
-    const uint64_t resident = uint64_t(cus_per_xcd) * cute_dev::kNumXcd * 4u * waves_per_simd;
+    const uint64_t resident = uint64_t(cus_per_xcd) * xcds * 4u * waves_per_simd;
     if (uint64_t(chunks.size()) * num_slabs > resident) return false;      // later work-groups go wherever one retires
-    const uint32_t groups = (uint32_t(chunks.size()) + wpg - 1) / wpg;
-    const uint32_t per_xcd = (groups + cute_dev::kNumXcd - 1) / cute_dev::kNumXcd;
-    const size_t span = size_t(per_xcd) * wpg;
-    const uint32_t simds = cus_per_xcd * 4u;
-    auto simd_of = [&](uint32_t pos, uint32_t y) {
-        const uint32_t s = y * per_xcd + pos / wpg;
-        return (s % cus_per_xcd) * 4u + (pos % wpg + s / cus_per_xcd) % 4u;
-    };
-    std::vector<uint32_t> lane(span * num_slabs);            // the SIMDs a position meets, slab by slab
-    for (uint32_t pos = 0; pos < span; ++pos)
-        for (uint32_t y = 0; y < num_slabs; ++y) lane[size_t(pos) * num_slabs + y] = simd_of(pos, y);
-    std::vector<uint4> dealt(chunks);
-    uint64_t before = 0, after = 0;
-    std::vector<uint64_t> load(simds);
-    std::vector<uint32_t> order;
-    // Positions by the load of their fullest SIMD, then by position.  Loads only grow, so an entry's stored load is a lower
-    // bound: one that has grown goes back with its new load, and the first that has not is the position to take.
-    typedef std::pair<uint64_t, uint32_t> Place;
-    std::priority_queue<Place, std::vector<Place>, std::greater<Place>> places;
-    for (uint32_t x = 0; x < cute_dev::kNumXcd; ++x) {
-        const size_t b = std::min(chunks.size(), x * span), e = std::min(chunks.size(), (x + 1) * span);
-        if (e <= b) continue;
-        const uint32_t n = uint32_t(e - b);
-        auto cost = [&](uint32_t i) { return uint64_t(chunks[b + i].y - chunks[b + i].x) + 2u; };
-        std::fill(load.begin(), load.end(), 0);
-        for (uint32_t i = 0; i < n; ++i)
-            for (uint32_t y = 0; y < num_slabs; ++y) load[lane[size_t(i) * num_slabs + y]] += cost(i);
-        before = std::max(before, *std::max_element(load.begin(), load.end()));
-        order.resize(n);
-        for (uint32_t i = 0; i < n; ++i) order[i] = i;
-        std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t c2) { return cost(a) > cost(c2); });
-        std::fill(load.begin(), load.end(), 0);
-        for (uint32_t pos = 0; pos < n; ++pos) places.emplace(uint64_t(0), pos);
-        for (uint32_t i : order) {
-            uint32_t pos;
-            for (;;) {
-                const Place top = places.top();
-                places.pop();
-                pos = top.second;
-                uint64_t peak = 0;
-                for (uint32_t y = 0; y < num_slabs; ++y) peak = std::max(peak, load[lane[size_t(pos) * num_slabs + y]]);
-                if (peak == top.first) break;
-                places.emplace(peak, pos);
-            }
-            dealt[b + pos] = chunks[b + i];
-            for (uint32_t y = 0; y < num_slabs; ++y) load[lane[size_t(pos) * num_slabs + y]] += cost(i);
+    const uint32_t count = uint32_t(chunks.size()), groups = (count + wpg - 1) / wpg;
+    const uint32_t per_xcd = (groups + xcds - 1) / xcds, span = per_xcd * wpg, simds = cus_per_xcd * 4u;
+    std::vector<uint32_t> lane(size_t(simds) * num_slabs);   // the SIMDs a class meets, slab by slab
+    for (uint32_t k = 0; k < simds; ++k)
+        for (uint32_t y = 0; y < num_slabs; ++y) {
+            const uint32_t s = y * per_xcd + k / 4u;
+            lane[size_t(k) * num_slabs + y] = (s % cus_per_xcd) * 4u + (k % 4u + s / cus_per_xcd) % 4u;
         }
-        after = std::max(after, *std::max_element(load.begin(), load.end()));
+    auto cost = [&](uint32_t i) { return uint64_t(chunks[i].y - chunks[i].x) + 2u; };
+    auto begin_of = [&](uint32_t x) { return std::min(count, x * span); };
+    std::vector<uint64_t> load(size_t(simds) * xcds);
+    uint64_t before = 0, bound = 0, longest = 0;
+    for (uint32_t x = 0; x < xcds; ++x) {
+        const uint32_t b = begin_of(x), n = begin_of(x + 1u) - b;
+        uint64_t *const of = load.data() + size_t(x) * simds, total = 0, shortest = ~0ull;
+        for (uint32_t k = 0, cu = 0, turn = 0; k * wpg < n; ++k) {
+            for (uint32_t w = 0; w < std::min(wpg, n - k * wpg); ++w) {
+                const uint64_t c = cost(b + k * wpg + w);
+                const uint32_t *const to = lane.data() + size_t(cu * 4u + (w + turn) % 4u) * num_slabs;
+                for (uint32_t y = 0; y < num_slabs; ++y) of[to[y]] += c;
+                total += c;
+                shortest = std::min(shortest, c);
+                longest = std::max(longest, c);
+            }
+            if (++cu == cus_per_xcd) { cu = 0; ++turn; }
+        }
+        before = std::max(before, *std::max_element(of, of + simds));
+        if (n) bound = std::max({bound, (total * num_slabs + simds - 1u) / simds, (uint64_t(n) * num_slabs + simds - 1u) / simds * shortest});
     }
-    if (!force && after * 100u > before * 97u) return false;
+    bound = std::max(bound, longest);
+    if (!force && bound * 100u > before * 97u) return false;
+
+    std::vector<uint32_t> order(count);                      // of every XCD: longest first, then by position
+    if (longest <= 4096u) {
+        std::vector<uint32_t> place(longest + 1u);
+        for (uint32_t x = 0; x < xcds; ++x) {
+            const uint32_t b = begin_of(x), e = begin_of(x + 1u);
+            std::fill(place.begin(), place.end(), 0u);
+            for (uint32_t i = b; i < e; ++i) ++place[cost(i)];
+            uint32_t at = b;
+            for (size_t k = place.size(); k-- > 0;) { const uint32_t here = place[k]; place[k] = at; at += here; }
+            for (uint32_t i = b; i < e; ++i) order[place[cost(i)]++] = i;
+        }
+    } else {
+        for (uint32_t i = 0; i < count; ++i) order[i] = i;
+        for (uint32_t x = 0; x < xcds; ++x)
+            std::stable_sort(order.begin() + begin_of(x), order.begin() + begin_of(x + 1u), [&](uint32_t i, uint32_t k) { return cost(i) > cost(k); });
+    }
+    struct Class {
+        uint64_t load;                                       // of its fullest SIMD, or what that was
+        uint32_t pos, k;                                     // its first free position; its number
+        bool operator<(const Class &o) const { return load != o.load ? load < o.load : pos < o.pos; }
+    };
+    std::vector<Class> heaps(size_t(simds) * xcds);
+    std::vector<uint4> dealt(chunks);
+    std::fill(load.begin(), load.end(), 0);
+    for (uint32_t x = 0; x < xcds; ++x) {
+        const uint32_t b = begin_of(x), e = begin_of(x + 1u), n = e - b;
+        uint64_t *const of = load.data() + size_t(x) * simds;
+        Class *const heap = heaps.data() + size_t(x) * simds;
+        uint32_t size = std::min(simds, n);
+        for (uint32_t k = 0; k < size; ++k) heap[k] = {0u, k, k};
+        auto peak = [&](uint32_t k) {
+            uint64_t most = 0;
+            for (uint32_t y = 0; y < num_slabs; ++y) most = std::max(most, of[lane[size_t(k) * num_slabs + y]]);
+            return most;
+        };
+        auto sink = [&](const Class c) {                 // c in the place of the first
+            uint32_t at = 0;
+            for (uint32_t child; (child = 2u * at + 1u) < size; at = child) {
+                if (child + 1u < size && heap[child + 1u] < heap[child]) ++child;
+                if (!(heap[child] < c)) break;
+                heap[at] = heap[child];
+            }
+            heap[at] = c;
+        };
+        for (uint32_t o = b; o < e; ++o) {
+            // loads only grow: one that another class has raised goes back with its new load
+            for (uint64_t now; num_slabs > 1u && (now = peak(heap[0].k)) != heap[0].load;) sink({now, heap[0].pos, heap[0].k});
+            Class c = heap[0];
+            dealt[b + c.pos] = chunks[order[o]];
+            for (uint32_t y = 0; y < num_slabs; ++y) of[lane[size_t(c.k) * num_slabs + y]] += cost(order[o]);
+            c.load = peak(c.k);
+            c.pos = (c.pos / 4u + cus_per_xcd) * 4u + (c.pos + 3u) % 4u;
+            if (c.pos < n) sink(c);
+            else if (--size) sink(heap[size]);
+        }
+    }
+    if (!force && *std::max_element(load.begin(), load.end()) * 100u > before * 97u) return false;
     chunks.swap(dealt);
     return true;
 }
@@ -636,7 +678,7 @@ void device_scan(uint32_t *data, uint64_t n, uint32_t *scratch, uint32_t arrays 
 std::vector<uint32_t> panels_between(const cute_hrpb_dev *d, uint32_t cap)
 {
     std::vector<uint32_t> list;
-    for (uint32_t p = 0; p < d->P; ++p)
+    for (uint32_t p = 0; d->longestPanel > cap && p < d->P; ++p)
         if (d->panelNnz[p] > cap && !panel_is_large(d, p)) list.push_back(p);
     return list;
 }
@@ -655,6 +697,7 @@ void list_large_panels(const cute_hrpb_dev *d, LargeWork &w)
 {
     if (!w.prefix.empty()) return;
     w.prefix.assign(1, 0u);
+    if (d->longestPanel <= cute_build::kPanelCap && d->widestPanel <= max_span(d)) return;
     for (uint32_t p = 0; p < d->P; ++p)
         if (panel_is_large(d, p)) {
             w.panel.push_back(p);
@@ -1063,6 +1106,7 @@ int finish_upload(cute_hrpb_dev *d, int quad_layout, const DeviceContext &c)
         const cute_build::PanelCensus *r = pin.as<const cute_build::PanelCensus>();
         uint32_t error = 0;
         bool any_large = false, any_medium = false;
+        uint32_t widest = 0, longest = 0;
         d->panelNnz.resize(P);
         d->panelSpan.resize(P);
         d->panelFirst.resize(P);
@@ -1071,9 +1115,12 @@ int finish_upload(cute_hrpb_dev *d, int quad_layout, const DeviceContext &c)
             d->panelNnz[p] = r[p].nnz;
             d->panelSpan[p] = r[p].span;
             d->panelFirst[p] = r[p].first;
-            d->widestPanel = std::max(d->widestPanel, r[p].span);
+            widest = std::max(widest, r[p].span);
+            longest = std::max(longest, r[p].nnz);
             if (r[p].nnz > cute_build::kPanelFirst || r[p].span > max_span(d)) (panel_is_large(d, p) ? any_large : any_medium) = true;
         }
+        d->widestPanel = widest;
+        d->longestPanel = longest;
         if (!error && (any_medium || any_large)) {
             const std::vector<uint32_t> medium = panels_between(d, cute_build::kPanelFirst);
             list_large_panels(d, large);
