@@ -49,8 +49,7 @@ struct PanelCensus {
     uint32_t pairs[4];         // distinct columns of each 4-row strip
     uint32_t stored;           // entries that are not zero
     uint32_t error;            // kErrRange | kErrUnsorted; the other fields then mean nothing
-    uint32_t first;            // first column (of a panel with entries)
-    uint32_t pad;
+    uint32_t first, end;       // first column, last column + 1; of a panel without entries ~0 and 0
 };
 static_assert(sizeof(PanelCensus) == 48, "written as twelve words");
 
@@ -374,9 +373,12 @@ __global__ __launch_bounds__(panel_threads(CAP)) void panel_census(const uint32_
         }
     }
     __syncthreads();
-    if (t == 0u && n && n != ~0u) {
-        res.span = l.hi - l.lo + 1u;
+    if (t == 0u) {
         res.first = l.lo;
+        if (n && n != ~0u) {
+            res.span = l.hi - l.lo + 1u;
+            res.end = l.hi + 1u;
+        }
     }
     __syncthreads();
     if (t < 12u) reinterpret_cast<uint32_t *>(out + p)[t] = reinterpret_cast<const uint32_t *>(&res)[t];

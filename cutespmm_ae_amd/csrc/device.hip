@@ -24,6 +24,7 @@ constexpr uint64_t kWideWindowBytes = 16ull << 20;   // ... whose window of B is
 constexpr float kWideReuse = 0.98f;          // ... the bar for products of 256 columns or more over large matrices (see cute_spmm_plan_create)
 constexpr uint32_t kMaxRowForRows = 48;      // ... unless it holds a row longer than this: one lane group would serialise it
 constexpr uint32_t kRowBatch = 8;           // entries the row kernel has in flight per row
+constexpr uint32_t kTilePanels = cute_dev::kWindowTile / CUTE_TM;   // panels of a tile of csr_rows_window
 // A panel is scattered when the window of B it reads (at most 256 columns of it at a time) is wider than this: its rows then
 // come from behind the L2s, which deliver about 8 TB/s against the 20 an L2 gives.  One and a half L2s: bands of 4 100
 // rows by 256 columns still come out of an L2 (92 % hits), 8 192 rows at random do not (N = 512: 25 us in row order, 12 with
@@ -225,8 +226,10 @@ struct cute_hrpb_dev {
     std::vector<uint32_t> panelCols;    // active columns per row panel
     std::vector<uint32_t> panelMaxRow;  // longest row of each panel
     std::vector<uint32_t> panelSpan;    // width of each panel's column window (last column - first column + 1)
-    std::vector<uint32_t> panelFirst;   // ... and its first column
-    uint32_t widestPanel = 0, longestPanel = 0;         // the largest of panelSpan and of panelNnz
+    uint32_t longestPanel = 0;          // the largest of panelNnz
+    bool anyLarge = false;              // panels that the panel kernels do not take
+    std::vector<uint2> tileWindow;      // columns [first, end) of every tile of csr_rows_window; a tile without entries: [~0, 0)
+    uint32_t widestTile = 0;            // the widest of these
     // the entries as csr_rows_window reads them (which describes them), built for the first plan that uses that kernel
     bool haveWindow = false;
     uint4 *dSlices = nullptr;
@@ -697,7 +700,7 @@ void list_large_panels(const cute_hrpb_dev *d, LargeWork &w)
 {
     if (!w.prefix.empty()) return;
     w.prefix.assign(1, 0u);
-    if (d->longestPanel <= cute_build::kPanelCap && d->widestPanel <= max_span(d)) return;
+    if (!d->anyLarge) return;
     for (uint32_t p = 0; p < d->P; ++p)
         if (panel_is_large(d, p)) {
             w.panel.push_back(p);
@@ -930,30 +933,20 @@ struct WindowShape {
 // false: rows or windows that the kernel does not take
 bool window_shape(const cute_hrpb_dev *d, WindowShape &w)
 {
-    constexpr uint32_t per_slice = 64u / CUTE_TM, per_tile = cute_dev::kWindowTile / CUTE_TM;
+    constexpr uint32_t per_slice = 64u / CUTE_TM;
     w.slices.resize((size_t(d->P) + per_slice - 1) / per_slice);
-    w.tiles.resize((size_t(d->P) + per_tile - 1) / per_tile);
-    uint32_t end = 0;
+    w.tiles = d->tileWindow;
     for (uint32_t p = 0; p < d->P;) {
-        uint2 &tile = w.tiles[p / per_tile];
-        tile.x = d->K;
-        for (const uint32_t last = std::min<uint32_t>(d->P, p + per_tile); p < last;) {
-            uint4 &slice = w.slices[p / per_slice];
-            uint32_t longest = 1;
-            for (const uint32_t upto = std::min<uint32_t>(last, p + per_slice); p < upto; ++p) {
-                longest = std::max(longest, d->panelMaxRow[p]);
-                if (!d->panelNnz[p]) continue;
-                tile.x = std::min(tile.x, d->panelFirst[p]);
-                end = std::max(end, d->panelFirst[p] + d->panelSpan[p]);
-            }
-            if (longest > 64u) return false;
-            w.longest = std::max(w.longest, longest);
-            slice = make_uint4(uint32_t(w.quads), 0u, (longest + 3u) / 4u, 0u);
-            w.quads += (longest + 3u) / 4u;
-        }
-        tile.y = end;
+        uint4 &slice = w.slices[p / per_slice];
+        uint32_t longest = 1;
+        for (const uint32_t upto = std::min<uint32_t>(d->P, p + per_slice); p < upto; ++p) longest = std::max(longest, d->panelMaxRow[p]);
+        if (longest > 64u) return false;
+        w.longest = std::max(w.longest, longest);
+        slice = make_uint4(uint32_t(w.quads), 0u, (longest + 3u) / 4u, 0u);
+        w.quads += (longest + 3u) / 4u;
     }
-    uint32_t first = d->K;
+    uint32_t first = d->K, end = 0;
+    for (uint2 &tile : w.tiles) tile.y = end = std::max(end, tile.y);
     for (size_t t = w.tiles.size(); t-- > 0;) {
         first = std::min(first, w.tiles[t].x);
         w.tiles[t].x = std::min(first, w.tiles[t].y);
@@ -1095,7 +1088,7 @@ int finish_upload(cute_hrpb_dev *d, int quad_layout, const DeviceContext &c)
     LargeWork large;
     {
         PinnedBuf pin;
-        int rc = pin.alloc(uint64_t(P) * sizeof(cute_build::PanelCensus));
+        int rc = pin.alloc((uint64_t(P) + kTilePanels) * sizeof(cute_build::PanelCensus));      // (the loop below asks for records ahead of it)
         if (rc != CUTE_OK) return rc;
         pin.pending = true;
         CUTE_PANELS(cute_build::panel_census<cute_build::kPanelFirst>, cute_build::kPanelFirst, P, window_lds(d, 0), d->dRowPtr, d->dCols,
@@ -1106,21 +1099,29 @@ int finish_upload(cute_hrpb_dev *d, int quad_layout, const DeviceContext &c)
         const cute_build::PanelCensus *r = pin.as<const cute_build::PanelCensus>();
         uint32_t error = 0;
         bool any_large = false, any_medium = false;
-        uint32_t widest = 0, longest = 0;
+        uint32_t longest = 0;
         d->panelNnz.resize(P);
         d->panelSpan.resize(P);
-        d->panelFirst.resize(P);
-        for (uint32_t p = 0; p < P; ++p) {
-            error |= r[p].error;
-            d->panelNnz[p] = r[p].nnz;
-            d->panelSpan[p] = r[p].span;
-            d->panelFirst[p] = r[p].first;
-            widest = std::max(widest, r[p].span);
-            longest = std::max(longest, r[p].nnz);
-            if (r[p].nnz > cute_build::kPanelFirst || r[p].span > max_span(d)) (panel_is_large(d, p) ? any_large : any_medium) = true;
+        // (a pair for 64 panels, not a word a panel: that cost a small new matrix 1 to 3 % of its way from format to product, 23 616 rows
+        // of 5, N = 8, 63.5 -> 65.3 us)
+        d->tileWindow.resize((size_t(P) + kTilePanels - 1) / kTilePanels);
+        for (uint32_t p = 0; p < P;) {
+            uint2 tile = make_uint2(~0u, 0u), &into = d->tileWindow[p / kTilePanels];
+            for (const uint32_t last = std::min(P, p + kTilePanels); p < last; ++p) {
+                __builtin_prefetch(r + p + kTilePanels);
+                error |= r[p].error;
+                d->panelNnz[p] = r[p].nnz;
+                d->panelSpan[p] = r[p].span;
+                longest = std::max(longest, r[p].nnz);
+                tile.x = std::min(tile.x, r[p].first);
+                tile.y = std::max(tile.y, r[p].end);
+                if (r[p].nnz > cute_build::kPanelFirst || r[p].span > max_span(d)) (panel_is_large(d, p) ? any_large : any_medium) = true;
+            }
+            into = tile;
+            if (tile.y) d->widestTile = std::max(d->widestTile, tile.y - tile.x);
         }
-        d->widestPanel = widest;
         d->longestPanel = longest;
+        d->anyLarge = any_large;
         if (!error && (any_medium || any_large)) {
             const std::vector<uint32_t> medium = panels_between(d, cute_build::kPanelFirst);
             list_large_panels(d, large);
@@ -1238,8 +1239,7 @@ void plan_window(cute_spmm_plan *p, cute_hrpb_dev *d, uint32_t N, const DeviceCo
     const double covered = double((N + walk - 1u) / walk * walk) / N;
     const double rows = 3.1 + gathers / 20.0 * (0.29 + 0.40 * covered + (N % 32u ? 0.10 : 0.0)) + bytes * 1e-6 * (0.04 + (beyond ? 0.09 : 0.0));
     const double lead = loop ? 12.0 : 15.0 + 2e-3 * d->P + 3e-6 * double(d->nnz);
-    constexpr uint32_t per_tile = cute_dev::kWindowTile / CUTE_TM;
-    const uint32_t n = (d->P + per_tile - 1u) / per_tile, cus = uint32_t(c.num_cus) / cute_dev::kNumXcd;
+    const uint32_t n = (d->P + kTilePanels - 1u) / kTilePanels, cus = uint32_t(c.num_cus) / cute_dev::kNumXcd;
     // a CU holds one work-group at a time: `rounds` of them after each other, each a first window and then its tiles
     auto ring_time = [&](uint32_t W, double row) {
         const uint32_t slabs = (N + W - 1u) / W;
@@ -1257,10 +1257,10 @@ void plan_window(cute_spmm_plan *p, cute_hrpb_dev *d, uint32_t N, const DeviceCo
         }
     };
     auto ahead = [&](double ring) { return ring * 1.15 <= rows && rows - ring >= lead; };
-    // (what the widest panel and the mean row allow at best, before the panels are looked at)
+    // (what the widest tile and the mean row allow at best, before the panels are looked at)
     const double mean = double(d->nnz) / double(d->M);
-    if (d->widestPanel > cute_dev::kWindowRows<8> || rows < lead ||
-        !(ahead(ring_time(8, mean)) || (d->widestPanel <= cute_dev::kWindowRows<16> && ahead(ring_time(16, mean))))) return;
+    if (d->widestTile > cute_dev::kWindowRows<8> || rows < lead ||
+        !(ahead(ring_time(8, mean)) || (d->widestTile <= cute_dev::kWindowRows<16> && ahead(ring_time(16, mean))))) return;
     WindowShape w;
     if (!window_shape(d, w) || w.quads * 256u > uint64_t(d->nnz) + d->nnz / 4u + 4096u) return;
     const uint32_t W = w.widest <= cute_dev::kWindowRows<16> ? 16u : 8u;

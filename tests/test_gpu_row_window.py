@@ -71,6 +71,17 @@ def test_windows_that_jump_and_rectangles(cs, orc, torch_cuda, jump, reach):
     _check(cs, orc, torch_cuda, rp, cl, vl, M, K, N, 16)
 
 
+@pytest.mark.parametrize("empty", [[(0, 2048)], [(30 * 1024, 32 * 1024)], [(79 * 1024 - 300, 81920 + 48)], [(0, 16), (1024, 2064), (5000, 9000), (70000, 80000)]])
+def test_tiles_without_entries(cs, orc, torch_cuda, empty):
+    """The windows of tiles come from the census, one pair a tile: none of the rows of a tile, or of its panels at either end, may hold an entry."""
+    M, N = 81920 + 48, 256
+    counts = np.full(M, 40)
+    for a, b in empty:
+        counts[a:b] = 0
+    rp, cl, vl = _band(M, M, counts, 1200, len(empty))
+    _check(cs, orc, torch_cuda, rp, cl, vl, M, M, N, 16)
+
+
 def test_rows_of_b_that_are_not_finite(cs, orc, torch_cuda):
     """An infinity reaches the rows that refer to it and no other: padding is left out, not multiplied by zero."""
     M, N = 65536, 256
