@@ -166,10 +166,10 @@ def plan_kernels(plan):
     if plan.info["numChunks"]:
         kernels.append(plan.kernel_name)
     if (plan.info["numRowPanelsSparse"] or plan.info["numEmptyPanels"]) and not plan.info["fusedLaunch"]:
-        kernels.append("csr_rows_window" if plan.window_columns else "csr_rows_batched")
+        kernels.append("csr_rows_batched" if plan.info["numChunks"] else plan.kernel_name)
     if plan.info["numAtomicChunks"]:
         kernels.append("reduce_partials")
-    return kernels, (plan.kernel_name if plan.info["numChunks"] else kernels[0])
+    return kernels, plan.kernel_name
 
 
 def simple_csr_us(cs, h, dB, dC, nnz, stream):

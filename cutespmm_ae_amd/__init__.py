@@ -700,12 +700,6 @@ class SPMM_TC:
         _check(load_library().cute_spmm_plan_info(self._plan, C.byref(info)), "cute_spmm_plan_info")
         self.info = {k: getattr(info, k) for k, _ in cute_plan_info._fields_ if k != "reserved"}
         self.numRowPanelsSplit = info.numChunks
-        self.kernel_name = ("csr_rows_batched" if info.numChunks == 0 else
-                            "hrpb_quad_hub_f32" if info.hubRows else
-                            ("hrpb_quad_rows_f32" if info.fusedLaunch else "hrpb_quad_half_f32" if info.slabWidth == 32 else "hrpb_quad_f32") if info.mfmaShape == 2 else
-                            "hrpb_brick_rows_f32" if info.fusedLaunch else
-                            "hrpb_brick_bf16x3" if info.precision == PREC_BF16X3 else
-                            "hrpb_brick_f32_rolling" if info.pipeline == 1 else "hrpb_brick_f32")
 
     def _check_shapes(self, MatB, MatC):
         if MatB.shape != self._shapes[0] or MatC.shape != self._shapes[1]:
@@ -740,6 +734,18 @@ class SPMM_TC:
         columns = C.c_uint32()
         _check(load_library().cute_spmm_plan_window(self._plan, C.byref(columns)), "cute_spmm_plan_window")
         return columns.value
+
+    @property
+    def kernel_name(self):
+        """The kernel that does the plan's main work: the MFMA kernel, or the row kernel of a plan without MFMA panels."""
+        info = self.info
+        return (("csr_rows_window" if self.window_columns else "csr_rows_batched") if info["numChunks"] == 0 else
+                "hrpb_quad_hub_f32" if info["hubRows"] else
+                ("hrpb_quad_rows_f32" if info["fusedLaunch"] else "hrpb_quad_half_f32" if info["slabWidth"] == 32 else "hrpb_quad_f32")
+                if info["mfmaShape"] == 2 else
+                "hrpb_brick_rows_f32" if info["fusedLaunch"] else
+                "hrpb_brick_bf16x3" if info["precision"] == PREC_BF16X3 else
+                "hrpb_brick_f32_rolling" if info["pipeline"] == 1 else "hrpb_brick_f32")
 
     @property
     def scratch_bytes(self):

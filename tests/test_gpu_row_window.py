@@ -30,6 +30,7 @@ def _check(cs, orc, torch, rp, cl, vl, M, K, N, columns, B=None):
     h = cs.DeviceHRPB(M, K, *(torch.from_numpy(a.view(np.int32) if a.dtype == np.uint32 else a).cuda() for a in (rp, cl, vl)))
     plan = cs.SPMM_TC(h, N, operand_residency=2)
     assert plan.window_columns == columns and plan.info["numChunks"] == 0
+    assert plan.kernel_name == ("csr_rows_window" if columns else "csr_rows_batched")
     C = torch.full((M * N + 64,), 7.5, device="cuda")
     out = C[:M * N].view(M, N)
     dB = torch.from_numpy(B).cuda()
