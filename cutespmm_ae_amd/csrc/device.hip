@@ -17,6 +17,7 @@ using namespace cute;
 namespace {
 
 thread_local std::string g_hip_error;
+thread_local hipError_t g_hip_status = hipSuccess;      // of the call g_hip_error describes
 
 // The planner's default thresholds (measured on the five benchmark matrices and on the reference's 43).
 constexpr float kMinReuse = 1.25f;          // a panel with fewer nonzeros per B row the MFMA side would fetch goes to the row kernel
@@ -85,8 +86,11 @@ int choose_mfma_shape(uint64_t slots, uint64_t bricks, uint64_t blocks, uint64_t
 // Floats per lane of a B or C row: four wherever a row has four (the kernels need no alignment beyond a float).
 inline int lane_floats(uint32_t N) { return N >= 4u ? 4 : N >= 2u ? 2 : 1; }
 
+// (an error that is returned is not left behind for the next launch to find)
 inline int hip_fail(hipError_t e, const char *what, int line)
 {
+    (void)hipGetLastError();
+    g_hip_status = e;
     g_hip_error = std::string(hipGetErrorString(e)) + " (" + what + ", device.hip:" + std::to_string(line) + ")";
     return CUTE_ERR_HIP;
 }
@@ -171,8 +175,7 @@ int static_scratch(void **out)
 
 void drop_idle_device_memory();
 
-// hipMalloc; when there is no memory left, once more without the idle blocks of the pool below.  (An error that is returned is not
-// left behind for the next launch to find.)
+// hipMalloc; when there is no memory left, once more without the idle blocks of the pool below.
 hipError_t device_malloc(void **out, uint64_t bytes)
 {
     hipError_t e = hipMalloc(out, std::max<uint64_t>(bytes, 16));
@@ -181,10 +184,7 @@ hipError_t device_malloc(void **out, uint64_t bytes)
         drop_idle_device_memory();
         e = hipMalloc(out, std::max<uint64_t>(bytes, 16));
     }
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        *out = nullptr;
-    }
+    if (e != hipSuccess) *out = nullptr;
     return e;
 }
 
@@ -956,6 +956,7 @@ bool window_shape(const cute_hrpb_dev *d, WindowShape &w)
 }
 
 // The entries csr_rows_window reads, for a ring of `ring_rows` rows (which follows from the widest window, so a handle has one such form).
+// CUTE_ERR_NOMEM: there is no memory for them.
 int ensure_window(cute_hrpb_dev *d, const WindowShape &w, uint32_t ring_rows)
 {
     std::lock_guard<std::mutex> guard(d->lock);
@@ -967,7 +968,7 @@ int ensure_window(cute_hrpb_dev *d, const WindowShape &w, uint32_t ring_rows)
     PinnedBuf pin;
     int rc = mem.alloc(lay.bytes);
     if (rc == CUTE_OK) rc = pin.alloc(staged);
-    if (rc != CUTE_OK) return rc;
+    if (rc != CUTE_OK) return g_hip_status == hipErrorOutOfMemory ? int(CUTE_ERR_NOMEM) : rc;
     std::memcpy(pin.as<char>(oSlices), w.slices.data(), w.slices.size() * sizeof(uint4));
     std::memcpy(pin.as<char>(oTiles), w.tiles.data(), w.tiles.size() * sizeof(uint2));
     pin.pending = true;
@@ -1229,10 +1230,10 @@ int make_hub_tables(cute_spmm_plan *p, const cute_hrpb_dev *d, uint32_t hub_rows
 // entries as well: plan creation with it takes, in us, 25 longer for 65 536 rows of 32 entries, 32 for 200 000 of 12, 33 for 131 072
 // of 32, 42 for 262 144, 46 for 524 288, 186 for 1 048 576 (format, plan and one product of 65 536 rows, N = 256: 202 / 223; 80 000
 // rows of 30, N = 101: 191 / 212).  A caller that says its product runs in a loop (operand_residency 2) gets the ring without that.
-void plan_window(cute_spmm_plan *p, cute_hrpb_dev *d, uint32_t N, const DeviceContext &c, bool loop)
+int plan_window(cute_spmm_plan *p, cute_hrpb_dev *d, uint32_t N, const DeviceContext &c, bool loop)
 {
     // (beyond 32 768 columns the 1 024 threads of every slab of up to 512 chains could pass the 2^32 a launch may have)
-    if (N < 16u || N > 32768u || d->P == 0) return;
+    if (N < 16u || N > 32768u || d->P == 0) return CUTE_OK;
     const double bytes = 8.0 * d->M * N + 8.0 * d->nnz, gathers = 4e-6 * double(d->nnz) * N;
     const bool beyond = uint64_t(d->K + uint64_t(d->M)) * N * sizeof(float) > c.cache_bytes;
     const uint32_t walk = uint32_t(p->rows_vec) << p->rows_logl;       // columns a lane group covers, used or not
@@ -1260,14 +1261,17 @@ void plan_window(cute_spmm_plan *p, cute_hrpb_dev *d, uint32_t N, const DeviceCo
     // (what the widest tile and the mean row allow at best, before the panels are looked at)
     const double mean = double(d->nnz) / double(d->M);
     if (d->widestTile > cute_dev::kWindowRows<8> || rows < lead ||
-        !(ahead(ring_time(8, mean)) || (d->widestTile <= cute_dev::kWindowRows<16> && ahead(ring_time(16, mean))))) return;
+        !(ahead(ring_time(8, mean)) || (d->widestTile <= cute_dev::kWindowRows<16> && ahead(ring_time(16, mean))))) return CUTE_OK;
     WindowShape w;
-    if (!window_shape(d, w) || w.quads * 256u > uint64_t(d->nnz) + d->nnz / 4u + 4096u) return;
+    if (!window_shape(d, w) || w.quads * 256u > uint64_t(d->nnz) + d->nnz / 4u + 4096u) return CUTE_OK;
     const uint32_t W = w.widest <= cute_dev::kWindowRows<16> ? 16u : 8u;
-    if (!ahead(ring_time(W, double(w.quads) * 256.0 / double(d->M)))) return;
+    if (!ahead(ring_time(W, double(w.quads) * 256.0 / double(d->M)))) return CUTE_OK;
+    const int rc = ensure_window(d, w, W == 16u ? cute_dev::kWindowRows<16> : cute_dev::kWindowRows<8>);
+    if (rc == CUTE_ERR_NOMEM) return CUTE_OK;       // the row kernel takes the rows, whose sums are then added in the order of the entries
+    if (rc != CUTE_OK) return rc;
+    p->windowColumns = W;
     p->windowWarm = beyond;
-    // (without the memory for a second form of the entries the row kernel takes the rows as ever)
-    if (ensure_window(d, w, W == 16u ? cute_dev::kWindowRows<16> : cute_dev::kWindowRows<8>) == CUTE_OK) p->windowColumns = W;
+    return CUTE_OK;
 }
 
 }  // namespace
@@ -1722,7 +1726,10 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
         }
         p->rowColumnSlabs = rows_columns ? p->rows_slabs : 0u;
     }
-    if (n_brick == 0 && default_bars) plan_window(p, d, N, c, t.operand_residency == 2);
+    if (n_brick == 0 && default_bars) {
+        const int rc = plan_window(p, d, N, c, t.operand_residency == 2);
+        if (rc != CUTE_OK) { delete p; return rc; }
+    }
     // The chunk list depends on the MFMA kernel (its work units are blocks or list groups).  It is built,
     // and if the partial tiles of the cut panels then turn out to be more rows than the fast kernels'
     // 24-bit row operand can address, built once more for the pipelined brick kernel, whose stores use

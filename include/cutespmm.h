@@ -472,13 +472,14 @@ int cute_spmm_plan_info(const cute_spmm_plan *p, cute_plan_info *out);
 int cute_spmm_plan_column_slabs(const cute_spmm_plan *p, uint32_t *mfma, uint32_t *rows);
 /* Columns of B that a plan whose rows all go to the row kernel keeps in LDS at a time (csr_rows_window: rows whose columns lie in a
  * window that moves along with them), 0: the rows gather from memory.  The first such plan of a handle adds a form of the
- * entries to it (6 bytes an entry and some padding), as for a late MFMA layout. */
+ * entries to it (6 bytes an entry and some padding), as for a late MFMA layout.  Where there is no memory for it the rows gather
+ * from memory instead; any other failure is the plan's. */
 int cute_spmm_plan_window(const cute_spmm_plan *p, uint32_t *columns);
 void cute_spmm_plan_free(cute_spmm_plan *p);
 /* dB [K x N], dC [M x N]: device pointers, row-major, 16-byte aligned.  Asynchronous on
  * `stream` (a hipStream_t, NULL = default stream).  C is fully overwritten: the caller
  * need not zero it (the reference requires cudaMemset first, run.cu:43,49).  No atomics are
- * used, so equal inputs give equal bits.  A plan whose panels were cut (numAtomicChunks > 0)
+ * used, so a plan gives equal inputs equal bits; the order in which a row's entries are added is the plan's choice.  A plan whose panels were cut (numAtomicChunks > 0)
  * keeps their partial tiles in a buffer of its own: launches of ONE plan must not overlap in
  * time (same stream, or ordered by events); different plans are independent.
  * B must be finite for the MFMA kernels to give the CSR product: like the reference's kernel
