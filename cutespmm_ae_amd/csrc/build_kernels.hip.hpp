@@ -181,7 +181,7 @@ template <uint32_t CAP> struct PanelEntries {
 };
 
 // Dynamic LDS of the panel kernels: the window's bitmap and the running counts of its words, later reused.
-inline __host__ __device__ uint32_t panel_window_words(uint32_t max_span) { return (max_span + 31u) / 32u; }
+constexpr __host__ __device__ uint32_t panel_window_words(uint32_t max_span) { return (max_span + 31u) / 32u; }
 
 // Sum over the threads before this one, and over the whole work-group in `total`, of two words at once.
 template <uint32_t WAVES> __device__ __forceinline__ Two block_exclusive_over(Two (&waveSum)[WAVES], Two own, Two &total)
@@ -562,7 +562,7 @@ struct BigLds {
     Two waveSum[kBigThreads / 64];
 };
 
-inline __host__ __device__ uint32_t big_window_words(uint32_t window_words) { return window_words + (window_words + 1u) / 2u; }   // bitmap and 16-bit counts
+constexpr __host__ __device__ uint32_t big_window_words(uint32_t window_words) { return window_words + (window_words + 1u) / 2u; }   // bitmap and 16-bit counts
 
 // Row starts, first and last column; returns the entries of the panel.
 __device__ __forceinline__ uint32_t big_rows(BigLds &l, const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols, uint32_t p, uint32_t &start)

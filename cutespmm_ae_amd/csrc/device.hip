@@ -708,10 +708,14 @@ void list_large_panels(const cute_hrpb_dev *d, LargeWork &w)
         }
 }
 
-// LDS beside the static part that big_census and big_quads may ask for: a compute unit's, less a little.
-constexpr uint32_t kBigLds = (160u << 10) - 1024u;
+// The LDS that big_census and big_quads ask for beside their static part (a kilobyte at most) is a compute unit's whatever the matrix: the
+// census keeps 16 bits a column of a panel, the lists a byte a column of a strip and two words a group of sixteen.
+constexpr uint32_t kBigWindow = cute_build::big_window_words(cute_build::panel_window_words(cute_build::kPanelSpan));
+static_assert((kBigWindow + cute_build::kBigEntries / 2u) * 4u + 1024u <= 160u << 10, "big_census");
+static_assert((kBigWindow + cute_build::kBigEntries / 4u + cute_build::kBigEntries / 16u * 2u) * 4u + 1024u <= 160u << 10, "big_quads");
 
-// The words big_census wants for the rows of the columns of every large panel; 0: there are some that it does not take.
+// The words big_census wants for the rows of the columns of every large panel; 0: there are some that it does not take, and then it takes
+// none (nor do the lists): one panel beyond kBigEntries or kPanelSpan sends all large panels of the matrix to the entry-parallel path.
 uint32_t big_census_rows(const cute_hrpb_dev *d, const LargeWork &w)
 {
     uint32_t most = 0;
@@ -719,8 +723,7 @@ uint32_t big_census_rows(const cute_hrpb_dev *d, const LargeWork &w)
         if (d->panelNnz[p] > cute_build::kBigEntries || d->panelSpan[p] > max_span(d) || d->panelSpan[p] == 0) return 0;
         most = std::max(most, std::min(d->panelNnz[p], d->panelSpan[p]));
     }
-    const uint32_t words = (most + 1u) / 2u;
-    return (cute_build::big_window_words(cute_build::panel_window_words(max_span(d))) + words) * 4u <= kBigLds ? words : 0u;
+    return (most + 1u) / 2u;
 }
 
 // The same for big_quads (the census has counted the columns of every strip): a byte a column, and the words of its groups' masks.
@@ -732,8 +735,7 @@ uint32_t big_quad_rows(const cute_hrpb_dev *d, const LargeWork &w, uint32_t &mas
         for (uint32_t s = 0; s < 4u; ++s) most = std::max(most, d->stripPairs[4u * p + s]);
     }
     masks = (most + 15u) / 16u * 2u;
-    const uint32_t words = (most + 3u) / 4u;
-    return (cute_build::big_window_words(cute_build::panel_window_words(max_span(d))) + words + masks) * 4u <= kBigLds ? words : 0u;
+    return (most + 3u) / 4u;
 }
 
 // Numbers the entries of the large panels.  With `out` given also counts for the planner, into the panels' census records.

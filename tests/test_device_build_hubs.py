@@ -1,6 +1,6 @@
-"""Panels of more than 4 096 entries: one work-group walks the entries for the census and for the strip lists up to 49 152 entries in
-a window the bitmap takes, as far as its LDS goes; the others, brick tiles and lockstep lists take the entry-parallel path.  Both
-layouts must equal the host builders word for word."""
+"""Panels of more than 4 096 entries: where none holds more than 49 152 or spans more columns than the bitmap takes, one work-group walks
+the entries of a panel for the census and of a strip for the strip lists; else all of them, and in any case the brick tiles and
+lockstep lists, take the entry-parallel path.  Both layouts must equal the host builders word for word."""
 import numpy as np
 import pytest
 
@@ -16,7 +16,9 @@ pytestmark = pytest.mark.gpu
     ((30000, 5000, 0, 300), None, 65536),
     ((49152, 4097), None, 60000),                          # the most a panel may hold
     ((49153, 8000), None, 60000),                          # one more: the entry-parallel path for both
-    ((40000, 4100), None, 131072),                         # census in LDS, lists beyond it
+    ((40000, 4100), None, 131072),                         # the widest bitmap beside many active columns
+    ((49152, 4097), (131072, 5000), 131072),               # the widest bitmap beside the most entries
+    ((49153, 5000, 6000), None, 60000),                    # one panel too long among others: all of them take the other path
     ((5000, 6000, 7000), (131072, 131071, 1600), 400000),  # windows at the bitmap's edge and narrow ones
     ((5000, 6000), (131073, 9000), 400000)])
 def test_long_panels(cs, torch_cuda, sizes, spans, K, quad_layout):
