@@ -47,7 +47,8 @@ def _check(cs, orc, torch, rp, cl, vl, M, K, N, columns, B=None):
 @pytest.mark.parametrize("M,per_row,reach,N,columns", [
     (65536, 32, 4097, 256, 8), (65536 + 16, 32, 1500, 256, 16), (60 * 1024 - 16, 31, 1000, 301, 16), (61440 + 64, 30, 3000, 203, 8),
     (131072, 45, 700, 33, 16), (260000, 40, 1200, 16, 16), (400000, 40, 4000, 17, 8), (9 * 1024 + 48, 48, 1537, 1000, 16),
-    (65536, 32, 1538, 256, 8), (65536, 32, 4098, 256, 0)])
+    (65536, 32, 1538, 256, 8), (65536, 32, 4098, 256, 0),
+    (163840 + 48, 32, 4097, 301, 8), (200000, 24, 1400, 256, 16)])      # operands of more than 256 MiB, chains of several tiles: B is asked for ahead
 def test_whole_numbers(cs, orc, torch_cuda, M, per_row, reach, N, columns):
     rp, cl, vl = _band(M, M, per_row, reach, M + N)
     _check(cs, orc, torch_cuda, rp, cl, vl, M, M, N, columns)
