@@ -1231,7 +1231,8 @@ int make_hub_tables(cute_spmm_plan *p, const cute_hrpb_dev *d, uint32_t hub_rows
 // A plan may be made for one product (a matrix that is new to every step), so the lead has to pay for the second form of the
 // entries as well: plan creation with it takes, in us, 25 longer for 65 536 rows of 32 entries, 32 for 200 000 of 12, 33 for 131 072
 // of 32, 42 for 262 144, 46 for 524 288, 186 for 1 048 576 (format, plan and one product of 65 536 rows, N = 256: 202 / 223; 80 000
-// rows of 30, N = 101: 191 / 212).  A caller that says its product runs in a loop (operand_residency 2) gets the ring without that.
+// rows of 30, N = 101: 191 / 212).  Nearest to the line of 40 drawn matrices, 73 840 rows of 25, N = 423: 316 / 309, and 357 / 379 on
+// buffers used for the first time.  A caller that says its product runs in a loop (operand_residency 2) gets the ring without that.
 int plan_window(cute_spmm_plan *p, cute_hrpb_dev *d, uint32_t N, const DeviceContext &c, bool loop)
 {
     // (beyond 32 768 columns the 1 024 threads of every slab of up to 512 chains could pass the 2^32 a launch may have)

@@ -433,10 +433,11 @@ typedef struct cute_tunables {
                                   mean: long items first); 1 always in panel order; 2 always dealt; 3 always long items first */
     uint32_t operand_residency; /* where B and C are when a launch starts: 0 unknown -- planned like 1, because a product on
                                   fresh data finds its operands in HBM whatever their size; 1 from HBM (a product on data no
-                                  cache holds); 2 cache-resident (a tight loop over the same operands that fit the 256 MiB
-                                  Infinity Cache together; ignored when they do not).  Chooses between the MFMA kernels
-                                  (and, for 1, keeps two column groups per lane in mixed plans); 2 also leaves out what the
-                                  tables of csr_rows_window cost, which the loop pays once (cute_spmm_plan_window). */
+                                  cache holds); 2 the product runs in a tight loop over the same operands.  Chooses between the
+                                  MFMA kernels, where 2 plans for operands out of the 256 MiB Infinity Cache if they fit it
+                                  together and is planned like 0 if they do not (1 also keeps two column groups per lane in
+                                  mixed plans).  For csr_rows_window 2 leaves out what its tables cost, which the loop pays
+                                  once, whatever the operands' size (cute_spmm_plan_window). */
     uint32_t hub_rows;         /* > 0 (at most 256): the quad kernel on strip lists runs as persistent work-groups that keep that many
                                   of the most referenced B rows in LDS (graphs with hub vertices); 0: off.  Ignored by other plans
                                   (cute_plan_info.hubRows says how many rows a plan stages) */
