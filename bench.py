@@ -167,8 +167,8 @@ def plan_kernels(plan):
         kernels.append(plan.kernel_name)
     if (plan.info["numRowPanelsSparse"] or plan.info["numEmptyPanels"]) and not plan.info["fusedLaunch"]:
         kernels.append("csr_rows_batched" if plan.info["numChunks"] else plan.kernel_name)
-    if plan.info["numAtomicChunks"]:
-        kernels.append("reduce_partials")
+    if plan.info["numAtomicChunks"] and plan.kernel_name in ("hrpb_quad_hub_f32", "hrpb_brick_f32"):
+        kernels.append("reduce_partials")      # (the other kernels' pieces add themselves up)
     return kernels, plan.kernel_name
 
 

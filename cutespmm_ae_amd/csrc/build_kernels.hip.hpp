@@ -1001,8 +1001,9 @@ __global__ __launch_bounds__(kThreads) void large_first_values(const uint32_t *_
 }
 
 // The tables of a plan, from its staged host copy, in one launch: chunk descriptors -- or, for the quad kernels (recs given),
-// one 128-byte head per work item: its descriptor and a copy of its first group's record --, the list of cut panels, and the
-// row kernel's list of a mixed plan, expanded from panels: every row with its row pointers, {row, first entry, end, 0}.
+// one 128-byte head per work item: its descriptor and a copy of its first group's record --, the list of cut panels, the
+// row kernel's list of a mixed plan, expanded from panels: every row with its row pointers, {row, first entry, end, 0}, and what the
+// pieces of cut panels add themselves up with.
 struct PlanTables {
     const uint4 *chunks;       // staged
     const uint4 *fixups;
@@ -1011,6 +1012,9 @@ struct PlanTables {
     uint4 *dChunks;            // device
     uint32_t *dHeads;
     uint4 *dFixups, *dRowList;
+    const uint4 *cut;          // staged: what the pieces of cut panels add themselves up with, and their counters behind it
+    uint4 *dCut;               // device
+    uint64_t numCut, counterWords;
 };
 
 __global__ __launch_bounds__(kThreads) void plan_tables(PlanTables T, const uint32_t *__restrict__ recs, uint32_t head_words,
@@ -1037,7 +1041,11 @@ __global__ __launch_bounds__(kThreads) void plan_tables(PlanTables T, const uint
     if (id < uint64_t(T.numRowPanels) * 16u) {
         const uint32_t r = T.rowPanels[id >> 4] * 16u + uint32_t(id & 15u);
         T.dRowList[id] = make_uint4(r, rowPtr[r], rowPtr[r + 1u], 0u);
+        return;
     }
+    id -= uint64_t(T.numRowPanels) * 16u;
+    if (id < T.numCut) T.dCut[id] = T.cut[id];
+    else if (id - T.numCut < (T.counterWords + 3u) / 4u) T.dCut[id] = make_uint4(0u, 0u, 0u, 0u);      // (an array ends on 256 bytes)
 }
 
 // Hub plans (hrpb_quad_hub_f32): how often every column occurs in the quad records, and a copy of the records in

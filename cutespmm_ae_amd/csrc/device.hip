@@ -257,8 +257,11 @@ struct cute_spmm_plan {
     uint32_t numHub = 0;
     uint32_t *dHubRows = nullptr;       // the hub rows' column ids, slot order
     uint32_t *dHubRecs = nullptr;       // the plan's copy of the quad records, hub columns replaced by their slots
-    // panels (or 4-row strips) cut into several chunks: each chunk stores a partial tile, reduce_partials adds them
+    // panels (or 4-row strips) cut into several chunks: each chunk stores a partial tile, and they are added up by
+    // reduce_partials, or by themselves (store_piece) where the launch has a CutPieces: one set for cute_spmm_run, one for cute_spmm_run_static, because
+    // calls of the two may overlap; cute_spmm_run_scratch, of which any number may, has the reduce_partials launch
     uint4 *dFixups = nullptr;           // {panel or strip, first piece, pieces, -}
+    cute_dev::CutPieces *dCut = nullptr, *dCutStatic = nullptr;
     uint32_t numFixups = 0;
     uint32_t reduceBlocksY = 1;         // blocks of reduce_partials along a tile: enough for the tile with the most pieces
     uint32_t unitRows = CUTE_TM;        // rows of one panel / strip / piece
@@ -1935,7 +1938,7 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
     {
         uint32_t most = 1;
         for (const uint4 &fx : fixups) most = std::max(most, fx.z);
-        const uint32_t G = most <= 4 ? 1u : most <= 8 ? 2u : most <= 16 ? 4u : most <= 32 ? 8u : 16u;    // as in reduce_partials
+        const uint32_t G = cute_dev::reduce_waves(most);
         const uint32_t segments = ((CUTE_TM >> upp_log) * N + 63u) / 64u, per_block = uint32_t(cute_dev::kReduceWaves) / G;
         p->reduceBlocksY = std::max(1u, (segments + per_block - 1u) / per_block);
     }
@@ -1949,10 +1952,15 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
         // list are gathered on the device, where the records and the row pointers are.
         const uint32_t listed = every_row ? 0u : uint32_t(row_panels.size());
         const bool heads = p->shape == 2;
+        uint64_t counters = 0;                     // a unit's eights and the unit, for every slab
+        for (const uint4 &fx : fixups) counters += (fx.z + cute_dev::kPiecesAtOnce - 1u) / cute_dev::kPiecesAtOnce + 1u;
+        const uint64_t counter_words = counters * num_slabs * 2u;
         Layout stage, lay;
-        const uint64_t sChunks = stage.add(chunks.size(), sizeof(uint4)), sFixups = stage.add(fixups.size(), sizeof(uint4)), sRows = stage.add(listed, 4);
+        const uint64_t sChunks = stage.add(chunks.size(), sizeof(uint4)), sFixups = stage.add(fixups.size(), sizeof(uint4)), sRows = stage.add(listed, 4),
+                       sCut = stage.add(n_pieces ? 2u : 0u, sizeof(cute_dev::CutPieces)), sPieces = stage.add(n_pieces, sizeof(uint4));
         const uint64_t oChunks = lay.add(chunks.size(), heads ? cute_dev::kQuadHeadWords * 4u : sizeof(uint4)), oFixups = lay.add(fixups.size(), sizeof(uint4)),
-                       oRows = lay.add(uint64_t(listed) * CUTE_TM, sizeof(uint4)), oPartials = lay.add(p->partialBytes, 1);
+                       oRows = lay.add(uint64_t(listed) * CUTE_TM, sizeof(uint4)), oCut = lay.add(n_pieces ? 2u : 0u, sizeof(cute_dev::CutPieces)), oPieces = lay.add(n_pieces, sizeof(uint4)),
+                       oCounters = lay.add(counter_words, 4), oPartials = lay.add(p->partialBytes, 1);
         PinnedBuf pin;
         rc = pin.alloc(stage.bytes);
         if (rc == CUTE_OK && pool().take(&p->memory, lay.bytes) != CUTE_OK) rc = CUTE_ERR_NOMEM;
@@ -1965,9 +1973,28 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
             p->dFixups = Layout::at<uint4>(p->memory, oFixups);
             p->dRowList = listed ? Layout::at<uint4>(p->memory, oRows) : nullptr;
             p->dPartials = n_pieces ? Layout::at<float>(p->memory, oPartials) : nullptr;
+            if (n_pieces) {
+                uint4 *of_piece = pin.as<uint4>(sPieces);
+                uint32_t counter = 0;
+                for (const uint4 &fx : fixups) {
+                    for (uint32_t k = 0; k < fx.z; ++k) of_piece[fx.y + k] = make_uint4(fx.y, fx.z, counter, fx.x);
+                    counter += (fx.z + cute_dev::kPiecesAtOnce - 1u) / cute_dev::kPiecesAtOnce + 1u;
+                }
+                p->dCut = Layout::at<cute_dev::CutPieces>(p->memory, oCut);
+                p->dCutStatic = p->dCut + 1;
+                uint4 *const dPieces = Layout::at<uint4>(p->memory, oPieces);
+                uint32_t *const dCounters = Layout::at<uint32_t>(p->memory, oCounters);
+                cute_dev::CutPieces *cut = pin.as<cute_dev::CutPieces>(sCut);
+                cut[0] = {dPieces, dCounters, num_slabs};
+                cut[1] = {dPieces, dCounters + counters * num_slabs, num_slabs};
+            }
+            // (the two records, the pieces behind them and the counters behind these are staged and laid out alike)
+            const uint64_t cut_items = n_pieces ? (oCounters - oCut) / sizeof(uint4) : 0u;
             const cute_build::PlanTables T = {pin.as<const uint4>(sChunks), pin.as<const uint4>(sFixups), pin.as<const uint32_t>(sRows),
-                                              uint32_t(chunks.size()), uint32_t(fixups.size()), listed, p->dChunks, p->dHeads, p->dFixups, p->dRowList};
-            const uint64_t items = uint64_t(chunks.size()) * (heads ? cute_dev::kQuadHeadWords : 1) + fixups.size() + uint64_t(listed) * CUTE_TM;
+                                              uint32_t(chunks.size()), uint32_t(fixups.size()), listed, p->dChunks, p->dHeads, p->dFixups, p->dRowList,
+                                              pin.as<const uint4>(sCut), Layout::at<uint4>(p->memory, oCut), cut_items, counter_words};
+            const uint64_t items = uint64_t(chunks.size()) * (heads ? cute_dev::kQuadHeadWords : 1) + fixups.size() + uint64_t(listed) * CUTE_TM + cut_items +
+                                   (counter_words + 3u) / 4u;
             pin.pending = true;
             CUTE_BUILD(cute_build::plan_tables, grid_of(items), T, heads ? (p->dHubRecs ? p->dHubRecs : d->dQRecs) : static_cast<const uint32_t *>(nullptr),
                        uint32_t(cute_dev::kQuadHeadWords), d->dRowPtr);
@@ -2013,7 +2040,7 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
 namespace {
 
 template <int VEC, int NG, bool FULL, bool COLUMNS>
-void launch_brick_full(const cute_spmm_plan *p, const float *dB, float *dC, float *partials, hipStream_t s)
+void launch_brick_full(const cute_spmm_plan *p, const float *dB, float *dC, float *partials, const cute_dev::CutPieces *cut, hipStream_t s)
 {
     const uint32_t groups = (p->info.numChunks + cute_dev::kWavesPerGroup - 1) / cute_dev::kWavesPerGroup;
     const uint32_t per_xcd = (groups + cute_dev::kNumXcd - 1) / cute_dev::kNumXcd;
@@ -2021,23 +2048,23 @@ void launch_brick_full(const cute_spmm_plan *p, const float *dB, float *dC, floa
     if (p->bf16x3) {
         if constexpr (VEC == 4)
             hipLaunchKernelGGL((cute_dev::hrpb_brick_bf16x3<NG, FULL, COLUMNS>), grid, block, 0, s, p->dChunks, p->info.numChunks, per_xcd,
-                               p->d->dHdr, p->d->dVals, uint32_t(p->d->numVals), dB, dC, partials, p->info.N, p->columnSlabs);
+                               p->d->dHdr, p->d->dVals, uint32_t(p->d->numVals), dB, dC, partials, p->info.N, p->columnSlabs, cut);
     } else if (p->pipeline == 1)
         hipLaunchKernelGGL((cute_dev::hrpb_brick_f32_rolling<VEC, NG, FULL, COLUMNS>), grid, block, 0, s, p->dChunks,
-                           p->info.numChunks, per_xcd, p->d->dHdr, p->d->dVals, uint32_t(p->d->numVals), dB, dC, partials, p->info.N, p->columnSlabs);
+                           p->info.numChunks, per_xcd, p->d->dHdr, p->d->dVals, uint32_t(p->d->numVals), dB, dC, partials, p->info.N, p->columnSlabs, cut);
     else
         hipLaunchKernelGGL((cute_dev::hrpb_brick_f32<VEC, NG, FULL>), grid, block, 0, s, p->dChunks, p->info.numChunks,
                            per_xcd, p->d->dHdr, p->d->dVals, dB, dC, partials, p->info.N, p->columnSlabs);
 }
 
 template <int VEC, int NG>
-void launch_brick(const cute_spmm_plan *p, const float *dB, float *dC, float *partials, hipStream_t s)
+void launch_brick(const cute_spmm_plan *p, const float *dB, float *dC, float *partials, const cute_dev::CutPieces *cut, hipStream_t s)
 {
     const bool full = p->info.N % p->info.slabWidth == 0;
-    if (p->columnSlabs && full) launch_brick_full<VEC, NG, true, true>(p, dB, dC, partials, s);
-    else if (p->columnSlabs) launch_brick_full<VEC, NG, false, true>(p, dB, dC, partials, s);
-    else if (full) launch_brick_full<VEC, NG, true, false>(p, dB, dC, partials, s);
-    else launch_brick_full<VEC, NG, false, false>(p, dB, dC, partials, s);
+    if (p->columnSlabs && full) launch_brick_full<VEC, NG, true, true>(p, dB, dC, partials, cut, s);
+    else if (p->columnSlabs) launch_brick_full<VEC, NG, false, true>(p, dB, dC, partials, cut, s);
+    else if (full) launch_brick_full<VEC, NG, true, false>(p, dB, dC, partials, cut, s);
+    else launch_brick_full<VEC, NG, false, false>(p, dB, dC, partials, cut, s);
 }
 
 template <int VEC, bool BATCHED>
@@ -2175,7 +2202,7 @@ namespace {
 // Brick chunks and sparse rows in one launch.  (VEC, NG, lanes per row) follow from N the way the planner
 // picks them; returns false for a combination that is not instantiated (the caller then launches twice).
 template <int VEC, int NG, int LOG_L>
-void launch_brick_rows_as(const cute_spmm_plan *p, const float *dB, float *dC, float *partials, hipStream_t s, const dim3 &grid,
+void launch_brick_rows_as(const cute_spmm_plan *p, const float *dB, float *dC, float *partials, const cute_dev::CutPieces *cut, hipStream_t s, const dim3 &grid,
                           uint32_t per_xcd)
 {
     const uint32_t N = p->info.N;
@@ -2186,7 +2213,7 @@ void launch_brick_rows_as(const cute_spmm_plan *p, const float *dB, float *dC, f
     hipLaunchKernelGGL((cute_dev::hrpb_brick_rows_f32<VEC, NG, F, LOG_L, COLUMNS>), flat, block, 0, s, grid.x, uint32_t(brick_blocks),  \
                        p->dChunks, p->info.numChunks, per_xcd, p->d->dHdr, p->d->dVals, uint32_t(p->d->numVals), p->dRowList, \
                        p->numRows, rows_per_slab, p->rowRanges, p->columnSlabs, p->rowColumnSlabs, p->d->dRowPtr, p->d->dCols, p->d->dCsrVals,                    \
-                       dB, dC, partials, N)
+                       dB, dC, partials, N, cut)
     constexpr bool wide = LOG_L >= 5;            // a launch by columns has 128 columns or more
     const bool full = N % (16u * VEC * NG) == 0;
     if (wide && p->columnSlabs && full) CUTE_BRICK_ROWS(true, wide);
@@ -2196,35 +2223,37 @@ void launch_brick_rows_as(const cute_spmm_plan *p, const float *dB, float *dC, f
 #undef CUTE_BRICK_ROWS
 }
 
-bool launch_brick_rows(const cute_spmm_plan *p, const float *dB, float *dC, float *partials, hipStream_t s)
+bool launch_brick_rows(const cute_spmm_plan *p, const float *dB, float *dC, float *partials, const cute_dev::CutPieces *cut, hipStream_t s)
 {
     const uint32_t groups = (p->info.numChunks + cute_dev::kWavesPerGroup - 1) / cute_dev::kWavesPerGroup;
     const uint32_t per_xcd = (groups + cute_dev::kNumXcd - 1) / cute_dev::kNumXcd;
     const dim3 grid(per_xcd * cute_dev::kNumXcd, p->info.numSlabs);
     if (uint64_t(grid.x) * grid.y + uint64_t(p->rowBlocksPerXcd) * cute_dev::kNumXcd * p->rows_slabs >= 0x7fffffffull) return false;
     const int v = p->vec, g = p->ng, l = p->rows_logl;
-    if (v == 1 && g == 1 && l == 0) launch_brick_rows_as<1, 1, 0>(p, dB, dC, partials, s, grid, per_xcd);
-    else if (v == 1 && g == 1 && l == 1) launch_brick_rows_as<1, 1, 1>(p, dB, dC, partials, s, grid, per_xcd);
-    else if (v == 1 && g == 1 && l == 2) launch_brick_rows_as<1, 1, 2>(p, dB, dC, partials, s, grid, per_xcd);
-    else if (v == 2 && g == 1 && l == 3) launch_brick_rows_as<2, 1, 3>(p, dB, dC, partials, s, grid, per_xcd);
-    else if (v == 4 && g == 1 && l == 4) launch_brick_rows_as<4, 1, 4>(p, dB, dC, partials, s, grid, per_xcd);
-    else if (v == 4 && g == 1 && l == 5) launch_brick_rows_as<4, 1, 5>(p, dB, dC, partials, s, grid, per_xcd);
-    else if (v == 4 && g == 1 && l == 6) launch_brick_rows_as<4, 1, 6>(p, dB, dC, partials, s, grid, per_xcd);
-    else if (v == 4 && g == 2 && l == 5) launch_brick_rows_as<4, 2, 5>(p, dB, dC, partials, s, grid, per_xcd);
-    else if (v == 4 && g == 2 && l == 6) launch_brick_rows_as<4, 2, 6>(p, dB, dC, partials, s, grid, per_xcd);
+    if (v == 1 && g == 1 && l == 0) launch_brick_rows_as<1, 1, 0>(p, dB, dC, partials, cut, s, grid, per_xcd);
+    else if (v == 1 && g == 1 && l == 1) launch_brick_rows_as<1, 1, 1>(p, dB, dC, partials, cut, s, grid, per_xcd);
+    else if (v == 1 && g == 1 && l == 2) launch_brick_rows_as<1, 1, 2>(p, dB, dC, partials, cut, s, grid, per_xcd);
+    else if (v == 2 && g == 1 && l == 3) launch_brick_rows_as<2, 1, 3>(p, dB, dC, partials, cut, s, grid, per_xcd);
+    else if (v == 4 && g == 1 && l == 4) launch_brick_rows_as<4, 1, 4>(p, dB, dC, partials, cut, s, grid, per_xcd);
+    else if (v == 4 && g == 1 && l == 5) launch_brick_rows_as<4, 1, 5>(p, dB, dC, partials, cut, s, grid, per_xcd);
+    else if (v == 4 && g == 1 && l == 6) launch_brick_rows_as<4, 1, 6>(p, dB, dC, partials, cut, s, grid, per_xcd);
+    else if (v == 4 && g == 2 && l == 5) launch_brick_rows_as<4, 2, 5>(p, dB, dC, partials, cut, s, grid, per_xcd);
+    else if (v == 4 && g == 2 && l == 6) launch_brick_rows_as<4, 2, 6>(p, dB, dC, partials, cut, s, grid, per_xcd);
     else return false;
     return true;
 }
 }  // namespace
 
 namespace {
-// The launches of one product; `partials` is where the pieces of cut panels store their tiles.
-int run_with(const cute_spmm_plan *p, const float *dB, float *dC, void *stream, float *partials)
+// The launches of one product; `partials` is where the pieces of cut panels store their tiles, `cut` how they add themselves up
+// (nullptr: reduce_partials does).
+int run_with(const cute_spmm_plan *p, const float *dB, float *dC, void *stream, float *partials, const cute_dev::CutPieces *cut)
 {
     if (!p || !dB || !dC) return CUTE_ERR_ARG;
     if ((reinterpret_cast<uintptr_t>(dB) | reinterpret_cast<uintptr_t>(dC)) & 15u) return CUTE_ERR_ARG;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const uint32_t N = p->info.N;
+    if (p->numHub || (p->shape == 1 && p->pipeline != 1)) cut = nullptr;      // (these kernels leave the tiles to reduce_partials)
     bool rows_launched = false;        // the sparse rows went out together with the MFMA chunks
     if (p->info.numChunks && p->shape == 2 && p->numHub) {
         // persistent work-groups of sixteen wavefronts, two per compute unit, each with the hub rows of its slab in LDS
@@ -2251,7 +2280,7 @@ int run_with(const cute_spmm_plan *p, const float *dB, float *dC, void *stream, 
                        grid.x, uint32_t(quad_blocks), p->dHeads, p->info.numChunks, per_xcd, p->d->dQRecs, p->d->dQVals,   \
                        uint32_t(p->d->numQuadVals),                                                                  \
                        p->dRowList, p->numRows, rows_per_slab, p->rowRanges, p->columnSlabs, p->rowColumnSlabs, p->d->dRowPtr, p->d->dCols, p->d->dCsrVals, dB, dC,    \
-                       partials, N)
+                       partials, N, cut)
 #define CUTE_FUSED_LL(F, S)                                                     \
     switch (p->rows_logl) {                                                     \
         case 0: CUTE_FUSED_LAUNCH(F, S, 0, false); break;                       \
@@ -2275,18 +2304,18 @@ int run_with(const cute_spmm_plan *p, const float *dB, float *dC, void *stream, 
         } else if (p->halfLists) {
             if (strips)
                 hipLaunchKernelGGL(cute_dev::hrpb_quad_half_f32<true>, grid, block, 0, s, p->dHeads, p->info.numChunks, per_xcd, p->d->dQRecs,
-                                   p->d->dQVals, uint32_t(p->d->numQuadVals), dB, dC, partials, N, p->columnSlabs);
+                                   p->d->dQVals, uint32_t(p->d->numQuadVals), dB, dC, partials, N, p->columnSlabs, cut);
             else
                 hipLaunchKernelGGL(cute_dev::hrpb_quad_half_f32<false>, grid, block, 0, s, p->dHeads, p->info.numChunks, per_xcd, p->d->dQRecs,
-                                   p->d->dQVals, uint32_t(p->d->numQuadVals), dB, dC, partials, N, p->columnSlabs);
+                                   p->d->dQVals, uint32_t(p->d->numQuadVals), dB, dC, partials, N, p->columnSlabs, cut);
         } else {
 #define CUTE_QUAD_LAUNCH(F, S)                                                                                          \
     if (p->columnSlabs)                                                                                                 \
         hipLaunchKernelGGL((cute_dev::hrpb_quad_f32<F, S, true>), grid, block, 0, s, p->dHeads, p->info.numChunks, per_xcd,  \
-                           p->d->dQRecs, p->d->dQVals, uint32_t(p->d->numQuadVals), dB, dC, partials, N, p->columnSlabs);   \
+                           p->d->dQRecs, p->d->dQVals, uint32_t(p->d->numQuadVals), dB, dC, partials, N, p->columnSlabs, cut);   \
     else                                                                                                                \
         hipLaunchKernelGGL((cute_dev::hrpb_quad_f32<F, S, false>), grid, block, 0, s, p->dHeads, p->info.numChunks, per_xcd, \
-                           p->d->dQRecs, p->d->dQVals, uint32_t(p->d->numQuadVals), dB, dC, partials, N, 0u)
+                           p->d->dQRecs, p->d->dQVals, uint32_t(p->d->numQuadVals), dB, dC, partials, N, 0u, cut)
             if (full && strips) { CUTE_QUAD_LAUNCH(true, true); }
             else if (full) { CUTE_QUAD_LAUNCH(true, false); }
             else if (strips) { CUTE_QUAD_LAUNCH(false, true); }
@@ -2294,11 +2323,11 @@ int run_with(const cute_spmm_plan *p, const float *dB, float *dC, void *stream, 
 #undef CUTE_QUAD_LAUNCH
         }
     } else if (p->info.numChunks) {
-        if (p->info.fusedLaunch && launch_brick_rows(p, dB, dC, partials, s)) rows_launched = true;
-        else if (p->vec == 4 && p->ng == 2) launch_brick<4, 2>(p, dB, dC, partials, s);
-        else if (p->vec == 4) launch_brick<4, 1>(p, dB, dC, partials, s);
-        else if (p->vec == 2) launch_brick<2, 1>(p, dB, dC, partials, s);
-        else launch_brick<1, 1>(p, dB, dC, partials, s);
+        if (p->info.fusedLaunch && launch_brick_rows(p, dB, dC, partials, cut, s)) rows_launched = true;
+        else if (p->vec == 4 && p->ng == 2) launch_brick<4, 2>(p, dB, dC, partials, cut, s);
+        else if (p->vec == 4) launch_brick<4, 1>(p, dB, dC, partials, cut, s);
+        else if (p->vec == 2) launch_brick<2, 1>(p, dB, dC, partials, cut, s);
+        else launch_brick<1, 1>(p, dB, dC, partials, cut, s);
     }
     if (p->windowColumns) {
         const uint32_t slabs = (N + p->windowColumns - 1u) / p->windowColumns;
@@ -2314,9 +2343,7 @@ int run_with(const cute_spmm_plan *p, const float *dB, float *dC, void *stream, 
         launch_rows<true>(p->rows_vec, p->rows_logl, p->dRowList, p->numRows, p->rows_slabs, p->d->dRowPtr, p->d->dCols,
                     p->d->dCsrVals, dB, dC, N, s, &p->rowRanges, p->rowBlocksPerXcd, p->rowColumnSlabs);
     }
-    // panels that were cut: add their partial tiles up, in chunk order (no atomics, so a product is
-    // the same bit for bit every time it is computed)
-    if (p->numFixups)
+    if (p->numFixups && !cut)
         hipLaunchKernelGGL(cute_dev::reduce_partials, dim3(p->numFixups, p->reduceBlocksY),
                            dim3(cute_dev::kWaveSize * cute_dev::kReduceWaves), 0, s, p->dFixups, p->numFixups, p->unitRows,
                            partials, dC, N);
@@ -2331,7 +2358,7 @@ extern "C" {
 int cute_spmm_run(cute_spmm_plan *p, const float *dB, float *dC, void *stream)
 {
     if (!p) return CUTE_ERR_ARG;
-    return run_with(p, dB, dC, stream, p->dPartials);
+    return run_with(p, dB, dC, stream, p->dPartials, p->dCut);
 }
 
 // The same launches with the partial tiles in the library's static device array instead of the plan's
@@ -2344,7 +2371,7 @@ int cute_spmm_run_static(cute_spmm_plan *p, const float *dB, float *dC, void *st
                       std::to_string(uint64_t(CUTE_STATIC_SCRATCH_BYTES));
         return CUTE_ERR_SCRATCH;
     }
-    return run_with(p, dB, dC, stream, static_cast<float *>(p->staticScratch));   // the address was fetched when the plan was made
+    return run_with(p, dB, dC, stream, static_cast<float *>(p->staticScratch), p->dCutStatic);   // the address was fetched when the plan was made
 }
 
 uint64_t cute_spmm_plan_scratch_bytes(const cute_spmm_plan *p) { return p ? p->partialBytes : 0; }
@@ -2362,7 +2389,7 @@ int cute_spmm_run_scratch(cute_spmm_plan *p, const float *dB, float *dC, void *s
             return CUTE_ERR_SCRATCH;
         }
     }
-    return run_with(p, dB, dC, stream, static_cast<float *>(scratch));
+    return run_with(p, dB, dC, stream, static_cast<float *>(scratch), nullptr);
 }
 
 int cute_csr_spmm_dev(int alg, const uint32_t *dRowPtr, const uint32_t *dCols, const float *dVals, const float *dB,

@@ -14,7 +14,7 @@
 //                    for panels with too little reuse for the matrix cores.
 //   csr_rows_window  rows whose columns move along with them: their window of B slides through LDS.
 //   hrpb_quad_rows_f32 / hrpb_brick_rows_f32   MFMA work items and sparse rows of a mixed plan in one launch.
-//   reduce_partials  adds up the partial tiles of panels that were cut, in chunk order (no atomics).
+//   reduce_partials  adds up the partial tiles of panels that were cut, where their pieces do not do it themselves (store_piece).
 //   blocked_ell_f32  fp32 MFMA over the dense blocks of a Blocked-ELL matrix.
 //   csr_rows / csr_thread_per_element / csr_wave_scalar   the simple CSR comparison kernels.
 #pragma once
@@ -170,14 +170,14 @@ __device__ __forceinline__ void mfma_block(const BlockOperands<VEC, NG> &o, f32x
 
 // chunks[i] = {first block, end block, row panel, piece}.  piece = 0: the chunk is its panel's only one and
 // stores the C tile; piece = k > 0: the panel is cut, and this chunk stores its partial tile as "panel" k-1
-// of the partials matrix (same row pitch as C), which reduce_partials adds up afterwards.  A work item is (chunk, slab);
+// of the partials matrix (same row pitch as C); store_piece says who adds them up.  A work item is (chunk, slab);
 // slab s covers columns [s*16*VEC*NG, (s+1)*16*VEC*NG).  Lane L = 16*g + j owns, inside
 // column group ng, the VEC consecutive columns starting at s*slab + ng*16*VEC + j*VEC;
 // MFMA tile v of that group therefore holds the columns {.. + j*VEC + v}, and after the
 // MFMA lane L holds rows 4g..4g+3 of exactly those VEC columns -> one vector store per row.
 // FULL: N is a multiple of the slab width, so no column guard is compiled in.
 struct BrickItem {
-    uint32_t start, end, panel, piece, col0;
+    uint32_t start, end, panel, piece, col0, slab;
     bool valid;
 };
 
@@ -199,8 +199,118 @@ __device__ __forceinline__ BrickItem brick_item(const uint4 *__restrict__ chunks
     it.end = __builtin_amdgcn_readfirstlane(ck.y);
     it.panel = __builtin_amdgcn_readfirstlane(ck.z);
     it.piece = __builtin_amdgcn_readfirstlane(ck.w);
+    it.slab = block_y;
     it.col0 = block_y * (16u * VEC * NG) + (lane & 15u) * VEC;
     return it;
+}
+
+// ---------------------------------------------------------------------------------------
+// Panels (or 4-row strips) that the planner cut: every piece stores its partial tile, and the pieces are added up in an order
+// that depends on their number alone -- eight consecutive pieces one after the other, then the sums of these eights one after
+// the other -- so the same product gives the same bits every time, whoever does the adding.
+//
+// Inside the launch (a CutPieces given) the pieces of an eight count themselves in behind their tiles, the one that comes last adds
+// the eight up, and of those, where there are several eights, the last one adds the sums up.  Nobody waits for anybody, and a
+// counter returns to zero by itself (atomicInc wraps), so the next launch finds it as this one did.  What a piece stores for
+// others, and what it reads of theirs, passes by the XCD's own L2 (agent-scope accesses): counting in then needs the stores to have
+// arrived, not the write-back of everything the L2 holds that a device-wide release is on this part (which made counting in 1.1 to 5.5
+// times slower than a second launch).
+// With a second launch (reduce_partials), as calls whose scratch comes without counters and kernels that are no plan's default have it, and
+// without, us: R-MAT graph of 131 072 nodes, N = 64 45.0 / 44.0; 65 536 nodes, N = 47 26.6 / 23.9.
+// ---------------------------------------------------------------------------------------
+constexpr uint32_t kPiecesAtOnce = 8;
+
+struct CutPieces {             // in device memory: an argument more would be in registers from a wavefront's start
+    const uint4 *of_piece;     // {first piece of the unit, pieces, first counter, unit}
+    uint32_t *counters;        // an eight's counters, then one for the eights; a word for each slab
+    uint64_t slabs;
+};
+
+__device__ __forceinline__ void store_shared(float *p, float x) { __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ float load_shared(const float *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+// The lane, without a register that holds it: what the end of a piece needs is not kept through its main loop.
+__device__ __forceinline__ uint32_t lane_again() { return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
+
+// Counts the wavefront in; true for the last of `members`.
+__device__ __forceinline__ bool last_to_arrive(uint32_t *counter, uint32_t members)
+{
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");          // what this wavefront stored has arrived
+    uint32_t before = 0;
+    if (lane_again() == 0u) before = atomicInc(counter, members - 1u);
+    const bool last = __builtin_amdgcn_readfirstlane(before) == members - 1u;
+    asm volatile("" ::: "memory");
+    return last;
+}
+
+// sum (of `count` values so far), then value(0) .. value(n - 1) one after the other; n is up to kPiecesAtOnce
+template <class Value> __device__ __forceinline__ float add_pieces(float sum, bool none_so_far, uint32_t n, Value value)
+{
+    float v[kPiecesAtOnce];
+#pragma unroll
+    for (uint32_t k = 0; k < kPiecesAtOnce; ++k) v[k] = value(min(k, n - 1u));
+#pragma unroll
+    for (uint32_t k = 0; k < kPiecesAtOnce; ++k) {
+        const float next = k == 0u && none_so_far ? v[0] : sum + v[k];
+        sum = k < n ? next : sum;
+    }
+    return sum;
+}
+
+// A lane's part of the tile of a piece: E elements, at(unit, e) the byte offset of element e of tile (or panel, or strip) `unit`.
+// Near the last column two lanes, or two elements of one, hold the same sum: owned(e) is true for one of them.  (The sums of an eight
+// stand where its first tile does, so a place that was read again after it was written would count twice.)
+template <int E, class At, class Owned>
+__device__ __forceinline__ void store_piece(const CutPieces *__restrict__ cut, uint32_t piece, uint32_t slab, const float (&mine)[E], At at, Owned owned,
+                                            float *__restrict__ partials, float *__restrict__ C)
+{
+    char *const tiles = reinterpret_cast<char *>(partials);
+    auto element = [&](uint32_t tile, int e) { return reinterpret_cast<float *>(tiles + at(tile, e)); };
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        if (owned(e)) store_shared(element(piece - 1u, e), mine[e]);
+        if (e % 4 == 3) __builtin_amdgcn_sched_barrier(0);     // (or the addresses of all of them take registers first)
+    }
+    if (!cut) return;
+    const uint4 of = cut->of_piece[piece - 1u];
+    uint32_t *const counters = cut->counters + slab;
+    const uint32_t slabs = uint32_t(cut->slabs);
+    const uint32_t first = __builtin_amdgcn_readfirstlane(of.x), pieces = __builtin_amdgcn_readfirstlane(of.y),
+                   counter = __builtin_amdgcn_readfirstlane(of.z), unit = __builtin_amdgcn_readfirstlane(of.w);
+    const uint32_t eights = (pieces + kPiecesAtOnce - 1u) / kPiecesAtOnce, eight = (piece - 1u - first) / kPiecesAtOnce,
+                   tile0 = first + eight * kPiecesAtOnce, members = min(kPiecesAtOnce, pieces - eight * kPiecesAtOnce);
+    if (!last_to_arrive(counters + size_t(counter + eight) * slabs, members)) return;
+    // (one loop for every E, a few elements a turn: the tile is not held in registers again)
+    constexpr int kTurn = E <= 4 ? E : 2;
+    auto to_c = [&](int e, float x) { __builtin_nontemporal_store(x, reinterpret_cast<float *>(reinterpret_cast<char *>(C) + at(unit, e))); };
+#pragma unroll 1
+    for (int e0 = 0; e0 < E; e0 += kTurn) {
+        float sum[kTurn];
+#pragma unroll
+        for (int e = 0; e < kTurn; ++e) sum[e] = add_pieces(0.0f, true, members, [&](uint32_t k) { return load_shared(element(tile0 + k, e0 + e)); });
+#pragma unroll
+        for (int e = 0; e < kTurn; ++e)
+            if (owned(e0 + e)) {
+                if (eights == 1u) to_c(e0 + e, sum[e]);
+                else store_shared(element(tile0, e0 + e), sum[e]);
+            }
+    }
+    if (eights == 1u || !last_to_arrive(counters + size_t(counter + eights) * slabs, eights)) return;
+#pragma unroll 1
+    for (int e0 = 0; e0 < E; e0 += kTurn) {
+        float sum[kTurn];
+#pragma unroll
+        for (int e = 0; e < kTurn; ++e) sum[e] = 0.0f;
+#pragma unroll 1
+        for (uint32_t base = 0; base < eights; base += kPiecesAtOnce)
+#pragma unroll
+            for (int e = 0; e < kTurn; ++e)
+                sum[e] = add_pieces(sum[e], base == 0u, min(kPiecesAtOnce, eights - base),
+                                    [&](uint32_t k) { return load_shared(element(first + (base + k) * kPiecesAtOnce, e0 + e)); });
+#pragma unroll
+        for (int e = 0; e < kTurn; ++e)
+            if (owned(e0 + e)) to_c(e0 + e, sum[e]);
+    }
 }
 
 template <int VEC, int NG, bool FULL>
@@ -368,14 +478,29 @@ __device__ __forceinline__ void load_brick_lean(typename Vec<VEC>::type (&b_out)
     }
 }
 
+template <int VEC, int NG, bool FULL>
+__device__ __forceinline__ void brick_store_piece(const BrickItem &it, const f32x4 (&acc)[NG][VEC], float *__restrict__ C,
+                                                  float *__restrict__ partials, uint32_t N, const CutPieces *__restrict__ cut)
+{
+    const uint32_t lane = lane_again(), col0 = it.slab * (16u * VEC * NG) + (lane & 15u) * VEC;
+    float mine[NG * 4 * VEC];
+#pragma unroll
+    for (int e = 0; e < NG * 4 * VEC; ++e) mine[e] = acc[e / (4 * VEC)][e % VEC][e / VEC % 4];
+    auto first_of = [&](int e) { return col0 + uint32_t(e / (4 * VEC)) * 16u * VEC; };
+    auto column = [&](int e) { return (FULL ? first_of(e) : first_column<VEC>(first_of(e), N)) + uint32_t(e % VEC); };
+    auto at = [&](uint32_t unit, int e) { return __umul24(unit * 16u + (lane >> 4) * 4u + uint32_t(e / VEC % 4), N * 4u) + column(e) * 4u; };
+    store_piece(cut, it.piece, it.slab, mine, at, [&](int e) { return FULL || column(e) >= first_of(e); }, partials, C);
+}
+
 // C tile of one item, addressed like the loads: 32-bit byte offsets from a scalar base.
 template <int VEC, int NG, bool FULL>
 __device__ __forceinline__ void brick_store_lean(const BrickItem &it, const f32x4 (&acc)[NG][VEC], float *__restrict__ C,
-                                                 float *__restrict__ partials, uint32_t N, uint32_t lane)
+                                                 float *__restrict__ partials, uint32_t N, uint32_t lane, const CutPieces *__restrict__ cut)
 {
     typedef typename Vec<VEC>::type V;
-    char *out_base = reinterpret_cast<char *>(it.piece ? partials : C);
-    const uint32_t row0 = (it.piece ? it.piece - 1u : it.panel) * 16u + (lane >> 4) * 4u;
+    if (it.piece) return brick_store_piece<VEC, NG, FULL>(it, acc, C, partials, N, cut);
+    char *out_base = reinterpret_cast<char *>(C);
+    const uint32_t row0 = it.panel * 16u + (lane >> 4) * 4u;
 #pragma unroll
     for (int ng = 0; ng < NG; ++ng) {
         const uint32_t c = it.col0 + uint32_t(ng) * 16u * VEC;
@@ -402,7 +527,7 @@ __device__ __forceinline__ void brick_rolling_body(uint32_t block_x, uint32_t bl
                                                    uint32_t num_chunks, uint32_t groups_per_xcd,
                                                    const uint32_t *__restrict__ hdr, const float *__restrict__ vals,
                                                    uint32_t zero_index, const float *__restrict__ B, float *__restrict__ C,
-                                                   float *__restrict__ partials, uint32_t N, uint32_t column_slabs)
+                                                   float *__restrict__ partials, uint32_t N, uint32_t column_slabs, const CutPieces *__restrict__ cut)
 {
     typedef typename Vec<VEC>::type V;
     const uint32_t lane = threadIdx.x & (kWaveSize - 1);
@@ -470,17 +595,17 @@ __device__ __forceinline__ void brick_rolling_body(uint32_t block_x, uint32_t bl
                     acc[ng][v] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], vec_get<VEC>(b[j][ng], v), acc[ng][v], 0, 0, 0);
         }
     }
-    brick_store_lean<VEC, NG, FULL>(it, acc, C, partials, N, lane);
+    brick_store_lean<VEC, NG, FULL>(it, acc, C, partials, N, lane, cut);
 }
 
 template <int VEC, int NG, bool FULL, bool COLUMNS>
 __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, (NG == 1 ? 8 : 4)) void hrpb_brick_f32_rolling(
     const uint4 *__restrict__ chunks, uint32_t num_chunks, uint32_t groups_per_xcd, const uint32_t *__restrict__ hdr,
     const float *__restrict__ vals, uint32_t zero_index, const float *__restrict__ B, float *__restrict__ C,
-    float *__restrict__ partials, uint32_t N, uint32_t column_slabs)
+    float *__restrict__ partials, uint32_t N, uint32_t column_slabs, const CutPieces *__restrict__ cut)
 {
     brick_rolling_body<VEC, NG, FULL>(blockIdx.x, blockIdx.y, chunks, num_chunks, groups_per_xcd, hdr, vals, zero_index, B, C,
-                                      partials, N, COLUMNS ? column_slabs : 0u);
+                                      partials, N, COLUMNS ? column_slabs : 0u, cut);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -546,7 +671,7 @@ template <int NG, bool FULL, bool COLUMNS>
 __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, (NG == 1 ? 6 : 4)) void hrpb_brick_bf16x3(
     const uint4 *__restrict__ chunks, uint32_t num_chunks, uint32_t groups_per_xcd, const uint32_t *__restrict__ hdr,
     const float *__restrict__ vals, uint32_t zero_index, const float *__restrict__ B, float *__restrict__ C,
-    float *__restrict__ partials, uint32_t N, uint32_t column_slabs)
+    float *__restrict__ partials, uint32_t N, uint32_t column_slabs, const CutPieces *__restrict__ cut)
 {
     constexpr int VEC = 4;
     const uint32_t lane = threadIdx.x & (kWaveSize - 1);
@@ -592,7 +717,7 @@ __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, (NG == 1 ? 6 : 4)) void 
         split_block<NG>(o, a, b);
         mfma_block_bf16x3<NG>(o, acc);
     }
-    brick_store_lean<VEC, NG, FULL>(it, acc, C, partials, N, lane);
+    brick_store_lean<VEC, NG, FULL>(it, acc, C, partials, N, lane, cut);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -638,27 +763,27 @@ template <bool FULL, bool STRIPS, bool HUB>
 __device__ __forceinline__ void quad_chunk(uint32_t chunk, uint32_t block_y, const uint32_t *__restrict__ heads,
                                            const uint32_t *__restrict__ qrecs, const float *__restrict__ qvals, uint32_t zero_index,
                                            const float *__restrict__ B, float *__restrict__ C, float *__restrict__ partials,
-                                           uint32_t N, const float *hub);
+                                           uint32_t N, const CutPieces *__restrict__ cut, const float *hub);
 
 template <bool FULL, bool STRIPS>
 __device__ __forceinline__ void quad_body(uint32_t block_x, uint32_t block_y, const uint32_t *__restrict__ heads,
                                           uint32_t num_chunks, uint32_t groups_per_xcd, const uint32_t *__restrict__ qrecs,
                                           const float *__restrict__ qvals, uint32_t zero_index,
                                           const float *__restrict__ B, float *__restrict__ C,
-                                          float *__restrict__ partials, uint32_t N, uint32_t column_slabs)
+                                          float *__restrict__ partials, uint32_t N, uint32_t column_slabs, const CutPieces *__restrict__ cut)
 {
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
     const uint32_t x = xcd_share(block_x, block_y, column_slabs);
     const uint32_t chunk = (x * groups_per_xcd + block_x / kNumXcd) * kWavesPerGroup + wave;
     if (chunk >= num_chunks) return;
-    quad_chunk<FULL, STRIPS, false>(chunk, block_y, heads, qrecs, qvals, zero_index, B, C, partials, N, nullptr);
+    quad_chunk<FULL, STRIPS, false>(chunk, block_y, heads, qrecs, qvals, zero_index, B, C, partials, N, cut, nullptr);
 }
 
 template <bool FULL, bool STRIPS, bool HUB>
 __device__ __forceinline__ void quad_chunk(uint32_t chunk, uint32_t block_y, const uint32_t *__restrict__ heads,
                                            const uint32_t *__restrict__ qrecs, const float *__restrict__ qvals, uint32_t zero_index,
                                            const float *__restrict__ B, float *__restrict__ C, float *__restrict__ partials,
-                                           uint32_t N, const float *hub)
+                                           uint32_t N, const CutPieces *__restrict__ cut, const float *hub)
 {
     const uint32_t lane = threadIdx.x & (kWaveSize - 1);
     // One entry of kQuadHeadWords per chunk: its descriptor and, behind it, the record of its first group, so
@@ -760,22 +885,29 @@ __device__ __forceinline__ void quad_chunk(uint32_t chunk, uint32_t block_y, con
 #undef CUTE_QUAD_ROLL_REST
 #undef CUTE_QUAD_MFMA16
     }
-    if (live) {
-        // a cut panel's chunk stores its tile into the partials matrix instead (rows (piece-1)*16.., same pitch)
-        char *out_base = reinterpret_cast<char *>(piece ? partials : C);
-        const uint32_t out_unit = piece ? piece - 1u : panel;
+    if (piece) {              // (the partials matrix: rows (piece-1)*16.., same pitch as C)
+        constexpr int E = STRIPS ? 4 : 16;
+        float mine[E];
+        const f32x4 sum = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+#pragma unroll
+        for (int e = 0; e < E; ++e) mine[e] = STRIPS ? sum[e] : acc[e / 4][e % 4];
+        const uint32_t column = block_y * kWaveSize + lane_again(), offset = min(column, N - 1u) * 4u;
+        auto at = [&](uint32_t unit, int e) { return __umul24(unit * uint32_t(E) + uint32_t(e), N * 4u) + offset; };
+        store_piece(cut, piece, block_y, mine, at, [&](int) { return FULL || column < N; }, partials, C);
+    } else if (live) {
+        char *out_base = reinterpret_cast<char *>(C);
         if (STRIPS) {
             // all 16 pairs of a group belong to one 4-row strip; the four accumulators only break
             // the dependency chain and are summed here
             const f32x4 sum = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-            uint32_t off = __umul24(out_unit * 4u, row_pitch) + n * 4u;
+            uint32_t off = __umul24(panel * 4u, row_pitch) + n * 4u;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 __builtin_nontemporal_store(sum[i], reinterpret_cast<float *>(out_base + off));
                 off += row_pitch;
             }
         } else {
-            uint32_t off = __umul24(out_unit * 16u, row_pitch) + n * 4u;
+            uint32_t off = __umul24(panel * 16u, row_pitch) + n * 4u;
 #pragma unroll
             for (int rg = 0; rg < 4; ++rg)
 #pragma unroll
@@ -792,10 +924,10 @@ template <bool FULL, bool STRIPS, bool COLUMNS>
 __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, 8) void hrpb_quad_f32(
     const uint32_t *__restrict__ heads, uint32_t num_chunks, uint32_t groups_per_xcd, const uint32_t *__restrict__ qrecs,
     const float *__restrict__ qvals, uint32_t zero_index, const float *__restrict__ B, float *__restrict__ C,
-    float *__restrict__ partials, uint32_t N, uint32_t column_slabs)
+    float *__restrict__ partials, uint32_t N, uint32_t column_slabs, const CutPieces *__restrict__ cut)
 {
     quad_body<FULL, STRIPS>(blockIdx.x, blockIdx.y, heads, num_chunks, groups_per_xcd, qrecs, qvals, zero_index, B, C,
-                            partials, N, COLUMNS ? column_slabs : 0u);
+                            partials, N, COLUMNS ? column_slabs : 0u, cut);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -826,7 +958,7 @@ template <bool STRIPS>
 __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, 8) void hrpb_quad_half_f32(
     const uint32_t *__restrict__ heads, uint32_t num_chunks, uint32_t groups_per_xcd, const uint32_t *__restrict__ qrecs,
     const float *__restrict__ qvals, uint32_t zero_index, const float *__restrict__ B, float *__restrict__ C,
-    float *__restrict__ partials, uint32_t N, uint32_t column_slabs)
+    float *__restrict__ partials, uint32_t N, uint32_t column_slabs, const CutPieces *__restrict__ cut)
 {
     constexpr uint32_t kHalf = kWaveSize / 2;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
@@ -915,28 +1047,18 @@ __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, 8) void hrpb_quad_half_f
 #undef CUTE_HALF_ROLL_REST
 #undef CUTE_HALF_MFMA8
     }
-    char *out_base = reinterpret_cast<char *>(piece ? partials : C);
-    const uint32_t unit = piece ? piece - 1u : panel;
-    if (STRIPS) {
-        const f32x4 sum = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-        uint32_t off = __umul24(unit * 4u + (upper & 2u), row_pitch) + n * 4u;
+    // the lane's rows of the tile: rows `half` and up, for the halves' sums of rows i and i + E
+    constexpr int E = STRIPS ? 2 : 8;
+    const uint32_t first_row = upper & uint32_t(E);
+    const f32x4 sum = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+    float mine[E];
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const float v = add_halves(sum[i], sum[i + 2]);
-            if (live) __builtin_nontemporal_store(v, reinterpret_cast<float *>(out_base + off));
-            off += row_pitch;
-        }
-    } else {
-        uint32_t off = __umul24(unit * 16u + (upper & 8u), row_pitch) + n * 4u;
+    for (int e = 0; e < E; ++e) mine[e] = STRIPS ? add_halves(sum[e], sum[(e + 2) % 4]) : add_halves(acc[e / 4][e % 4], acc[(e / 4 + 2) % 4][e % 4]);
+    auto at = [&](uint32_t unit, int e) { return __umul24(unit * uint32_t(2 * E) + first_row + uint32_t(e), row_pitch) + col_off; };
+    if (piece) store_piece(cut, piece, slab, mine, at, [&](int) { return live; }, partials, C);
+    else if (live)
 #pragma unroll
-        for (int rg = 0; rg < 2; ++rg)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float v = add_halves(acc[rg][i], acc[rg + 2][i]);
-                if (live) __builtin_nontemporal_store(v, reinterpret_cast<float *>(out_base + off));
-                off += row_pitch;
-            }
-    }
+        for (int e = 0; e < E; ++e) __builtin_nontemporal_store(mine[e], reinterpret_cast<float *>(reinterpret_cast<char *>(C) + at(panel, e)));
 }
 
 // ---------------------------------------------------------------------------------------
@@ -966,7 +1088,7 @@ __global__ __launch_bounds__(kWaveSize *kHubWaves) void hrpb_quad_hub_f32(
     // consecutive chunks of the list (longest first) go to different work-groups
     const uint32_t stride = gridDim.x * kHubWaves;
     for (uint32_t chunk = wave * gridDim.x + blockIdx.x; chunk < num_chunks; chunk += stride)
-        quad_chunk<FULL, true, true>(chunk, blockIdx.y, heads, qrecs, qvals, zero_index, B, C, partials, N, hub);
+        quad_chunk<FULL, true, true>(chunk, blockIdx.y, heads, qrecs, qvals, zero_index, B, C, partials, N, nullptr, hub);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1074,15 +1196,14 @@ __global__ __launch_bounds__(256) void blocked_ell_f32(const int32_t *__restrict
     }
 }
 
-// Adds up the partial tiles of the panels (16 rows) or strips (4 rows) that were cut into several chunks:
-// fixups[i] = {panel or strip, first piece, number of pieces, -}; piece k is rows [k*rows, (k+1)*rows) of the
+// Adds up the partial tiles of the panels (16 rows) or strips (4 rows) that were cut into several chunks, for calls whose pieces do
+// not do it themselves: fixups[i] = {panel or strip, first piece, number of pieces, -}; piece k is rows [k*rows, (k+1)*rows) of the
 // partials matrix, whose row pitch is N like C's.  A block of sixteen wavefronts works on tile i in segments
-// of 64 elements.  With few pieces every wavefront takes a segment of its own; with many, G = 2..16
-// wavefronts share a segment, wavefront g adding the pieces g, g+G, g+2G, ... (independent loads, four at a
-// time), and their sums are then added in wavefront order.  G depends on the piece count alone and every
-// order is fixed, so the result does not depend on which chunk finished first: the same product gives the
-// same bits every time.  The launch has one block per (tile, segment); blocks past the last segment group exit.
+// of 64 elements.  With up to eight pieces every wavefront takes a segment of its own; with more, G = 2..16 wavefronts share a
+// segment, each an eight of the pieces, and the sums are added in order: store_piece's order, hence its bits.
+// The launch has one block per (tile, segment); blocks past the last segment group exit.
 constexpr int kReduceWaves = 16;
+constexpr __host__ __device__ uint32_t reduce_waves(uint32_t pieces) { return pieces <= 8u ? 1u : pieces <= 16u ? 2u : pieces <= 32u ? 4u : pieces <= 64u ? 8u : 16u; }
 
 __global__ __launch_bounds__(kWaveSize *kReduceWaves) void reduce_partials(const uint4 *__restrict__ fixups, uint32_t count,
                                                                            uint32_t rows, const float *__restrict__ partials,
@@ -1093,8 +1214,8 @@ __global__ __launch_bounds__(kWaveSize *kReduceWaves) void reduce_partials(const
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
     if (blockIdx.x >= count) return;
     const uint4 fx = fixups[blockIdx.x];
-    const uint32_t pieces = __builtin_amdgcn_readfirstlane(fx.z);
-    const uint32_t G = pieces <= 4 ? 1u : pieces <= 8 ? 2u : pieces <= 16 ? 4u : pieces <= 32 ? 8u : 16u;
+    const uint32_t pieces = __builtin_amdgcn_readfirstlane(fx.z), eights = (pieces + kPiecesAtOnce - 1u) / kPiecesAtOnce;
+    const uint32_t G = reduce_waves(pieces);
     const uint32_t segs_per_block = kReduceWaves / G;
     const uint32_t tile = rows * N;
     if (blockIdx.y * segs_per_block * kWaveSize >= tile) return;      // whole block: nothing left of this tile
@@ -1102,22 +1223,20 @@ __global__ __launch_bounds__(kWaveSize *kReduceWaves) void reduce_partials(const
     const uint32_t e = seg * kWaveSize + lane;
     const bool valid = e < tile;
     const float *src = partials + size_t(fx.y) * tile + (valid ? e : 0u);
-    float sum = 0.0f;
-    uint32_t k = g;
-    for (; k < pieces; k += 4u * G) {          // four loads in flight; a piece past the end counts as zero
-        const float p0 = src[size_t(k) * tile];
-        const float p1 = k + G < pieces ? src[size_t(k + G) * tile] : 0.0f;
-        const float p2 = k + 2u * G < pieces ? src[size_t(k + 2u * G) * tile] : 0.0f;
-        const float p3 = k + 3u * G < pieces ? src[size_t(k + 3u * G) * tile] : 0.0f;
-        sum = (((sum + p0) + p1) + p2) + p3;
-    }
-    if (G > 1) {
+    float total = 0.0f;
+    for (uint32_t base = 0; base < eights; base += G) {               // (a block works on one unit: the rounds are the same for all of it)
+        const uint32_t eight = base + g, piece0 = eight * kPiecesAtOnce;
+        float sum = 0.0f;
+        if (eight < eights)
+            sum = add_pieces(0.0f, true, min(kPiecesAtOnce, pieces - piece0), [&](uint32_t k) { return src[size_t(piece0 + k) * tile]; });
+        if (G == 1u) { total = sum; break; }
         sums[wave][lane] = sum;
         __syncthreads();
-        if (g != 0) return;
-        for (uint32_t w = 1; w < G; ++w) sum += sums[wave + w][lane];
+        if (g == 0u)
+            for (uint32_t w = 0; w < min(G, eights - base); ++w) total = base + w == 0u ? sums[wave][lane] : total + sums[wave + w][lane];
+        __syncthreads();
     }
-    if (valid) __builtin_nontemporal_store(sum, C + size_t(fx.x) * tile + e);
+    if (valid && g == 0u) __builtin_nontemporal_store(total, C + size_t(fx.x) * tile + e);
 }
 
 // One group of L = 1<<LOG_L lanes per row; lane t of the group owns VEC consecutive columns
@@ -1484,12 +1603,12 @@ __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, 8) void hrpb_quad_rows_f
     uint32_t groups_per_xcd, const uint32_t *__restrict__ qrecs, const float *__restrict__ qvals, uint32_t zero_index,
     const uint4 *__restrict__ row_list, uint32_t num_rows, uint32_t row_blocks_per_slab, XcdRanges row_ranges, uint32_t column_slabs, uint32_t row_column_slabs,
     const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols, const float *__restrict__ vals,
-    const float *__restrict__ B, float *__restrict__ C, float *__restrict__ partials, uint32_t N)
+    const float *__restrict__ B, float *__restrict__ C, float *__restrict__ partials, uint32_t N, const CutPieces *__restrict__ cut)
 {
     static_assert(kWaveSize * kWavesPerGroup == 256, "both bodies are written for 256-thread blocks");
     if (blockIdx.x < quad_blocks) {
         quad_body<FULL, STRIPS>(blockIdx.x % quad_blocks_x, blockIdx.x / quad_blocks_x, heads, num_chunks, groups_per_xcd,
-                                qrecs, qvals, zero_index, B, C, partials, N, COLUMNS ? column_slabs : 0u);
+                                qrecs, qvals, zero_index, B, C, partials, N, COLUMNS ? column_slabs : 0u, cut);
     } else {   // quad_blocks is a multiple of the XCD count, so the XCD of a row block is (its index) % 8 as well
         const uint32_t rb = blockIdx.x - quad_blocks;
         uint32_t slab = rb / row_blocks_per_slab;      // slab by slab, as in csr_rows_batched
@@ -1508,11 +1627,11 @@ __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, (NG == 1 ? 8 : 4)) void 
     uint32_t groups_per_xcd, const uint32_t *__restrict__ hdr, const float *__restrict__ tile_vals, uint32_t zero_index,
     const uint4 *__restrict__ row_list, uint32_t num_rows, uint32_t row_blocks_per_slab, XcdRanges row_ranges, uint32_t column_slabs, uint32_t row_column_slabs,
     const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols, const float *__restrict__ vals,
-    const float *__restrict__ B, float *__restrict__ C, float *__restrict__ partials, uint32_t N)
+    const float *__restrict__ B, float *__restrict__ C, float *__restrict__ partials, uint32_t N, const CutPieces *__restrict__ cut)
 {
     if (blockIdx.x < brick_blocks) {
         brick_rolling_body<VEC, NG, FULL>(blockIdx.x % brick_blocks_x, blockIdx.x / brick_blocks_x, chunks, num_chunks,
-                                          groups_per_xcd, hdr, tile_vals, zero_index, B, C, partials, N, COLUMNS ? column_slabs : 0u);
+                                          groups_per_xcd, hdr, tile_vals, zero_index, B, C, partials, N, COLUMNS ? column_slabs : 0u, cut);
     } else {
         const uint32_t rb = blockIdx.x - brick_blocks;
         uint32_t slab = rb / row_blocks_per_slab;

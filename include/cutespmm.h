@@ -448,7 +448,7 @@ typedef struct cute_plan_info {
     uint32_t slabWidth;        /* columns of C per work item                              */
     uint32_t numSlabs;
     uint32_t numChunks;        /* MFMA-kernel work items along the panel axis             */
-    uint32_t numAtomicChunks;  /* of which are pieces of cut panels (partial tiles, added up by a second kernel; the name dates from atomics) */
+    uint32_t numAtomicChunks;  /* of which are pieces of cut panels (partial tiles, added up in a fixed order; the name dates from atomics) */
     uint32_t numBrickPanels, numRowPanelsSparse, numEmptyPanels;
     uint32_t slots;
     uint32_t precision, path;
@@ -479,8 +479,8 @@ int cute_spmm_plan_window(const cute_spmm_plan *p, uint32_t *columns);
 void cute_spmm_plan_free(cute_spmm_plan *p);
 /* dB [K x N], dC [M x N]: device pointers, row-major, 16-byte aligned.  Asynchronous on
  * `stream` (a hipStream_t, NULL = default stream).  C is fully overwritten: the caller
- * need not zero it (the reference requires cudaMemset first, run.cu:43,49).  No atomics are
- * used, so a plan gives equal inputs equal bits; the order in which a row's entries are added is the plan's choice.  A plan whose panels were cut (numAtomicChunks > 0)
+ * need not zero it (the reference requires cudaMemset first, run.cu:43,49).  Nothing is added up in the
+ * order of arrival, so a plan gives equal inputs equal bits; the order in which a row's entries are added is the plan's choice.  A plan whose panels were cut (numAtomicChunks > 0)
  * keeps their partial tiles in a buffer of its own: launches of ONE plan must not overlap in
  * time (same stream, or ordered by events); different plans are independent.
  * B must be finite for the MFMA kernels to give the CSR product: like the reference's kernel
@@ -500,7 +500,7 @@ int cute_spmm_run(cute_spmm_plan *p, const float *dB, float *dC, void *stream);
  * (cute_plan_info.partialTileKiB) exceed the array gives CUTE_ERR_SCRATCH, and cute_last_hip_error()
  * then names both sizes.  Every call on a GPU shares that GPU's array: calls that may overlap in time
  * on one GPU -- of any plans -- race; order them (one stream, or events).  Nothing in the array has to
- * start at zero: every piece overwrites its whole tile before the adding kernel reads it. */
+ * start at zero: every piece overwrites its whole tile before it is read. */
 #define CUTE_STATIC_SCRATCH_BYTES (32u << 20)
 int cute_spmm_run_static(cute_spmm_plan *p, const float *dB, float *dC, void *stream);
 
