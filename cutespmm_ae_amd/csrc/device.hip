@@ -1736,8 +1736,8 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
         const int rc = plan_window(p, d, N, c, t.operand_residency == 2);
         if (rc != CUTE_OK) { delete p; return rc; }
     }
-    // The chunk list depends on the MFMA kernel (its work units are blocks or list groups).  It is built,
-    // and if the partial tiles of the cut panels then turn out to be more rows than the fast kernels'
+    // The chunk list depends on the MFMA kernel (its work units are blocks or list groups).  It is built, once more with fewer
+    // cuts if these need more scratch than there is, and if the partial tiles of the cut panels then turn out to be more rows than the fast kernels'
     // 24-bit row operand can address, built once more for the pipelined brick kernel, whose stores use
     // 64-bit offsets.
     uint32_t slab = 0, num_slabs = 0, upp_log = 0, slots = 0, n_pieces = 0;
@@ -1797,12 +1797,19 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
             const uint32_t target = uint32_t(std::max<uint64_t>(std::max<uint64_t>(share, std::min<uint64_t>(mean, 16)), 8));
             // A launch that keeps every wavefront slot busy runs at the rate the memory system gathers B rows, and a
             // work item then advances about five times slower than one that runs alone (measured on the R-MAT
-            // benchmark matrix: 0.39 us per list group alone, 1.7 us per group and slot under load).  So an item up to
-            // six shares long still ends with the launch, and cutting it finer only adds partial tiles: such a launch
-            // cuts at six shares, into pieces of four.  A launch that does not fill the device is bound by its longest
-            // item instead and keeps the finer cut (twice the target, pieces of one target).
-            const uint32_t limit = uint32_t(std::max<uint64_t>(2u * uint64_t(target), 6u * share));
-            const uint32_t piece = limit > 2u * target ? uint32_t(4u * share) : target;
+            // benchmark matrix: 0.39 us per list group alone, 1.7 us per group and slot under load).  So an item of several
+            // shares still ends with the launch, and cutting it finer only adds partial tiles: lists are cut at four shares, into
+            // pieces of two.  R-MAT graphs, nodes (log 2) / edges / N, us cut at six shares into fours, at four into twos, at three into twos,
+            // at two into ones: 17/10/64 45.3, 43.2, 44.3, 46.7; 16/10/47 23.9, 21.6, 21.4, 22.9; 15/10/64 18.3, 17.2, 18.7, 18.5;
+            // 15/6/100 26.6, 19.4, 18.9, 18.5; 16/6/128 35.4, 29.4, 29.3, 34.3; 14/10/200 29.3, 23.4, 23.5, 24.7; 16/12/256 115, 95.6, 95.7,
+            // 95.2; 17/10/128 90.1, 89.8, 89.9, 94.0.  (Before the pieces added themselves up, six and four were the best.)
+            // A graph's bricks, which it has below 32 columns, are bound by their matrix work and are cut like a launch that does not fill the device
+            // and is bound by its longest item: at twice the target, into pieces of one (17/10/16 51.0, 39.2, 39.2, 30.3; 16/8/16 19.7, 18.2,
+            // 18.1, 18.1).  Wider bricks keep six shares and four: bf16x3 loses (16/10/128 85.4, 88.0, 88.2, 102), in fp32 they are
+            // those of even panels.  So do plans whose finer cut's tiles would not fit cute_spmm_run_static's scratch.
+            const bool finer = attempt == 0 && (p->shape == 2 || N < 32u);
+            const uint32_t limit = uint32_t(std::max<uint64_t>(2u * uint64_t(target), (finer ? (p->shape == 2 ? 4u : 0u) : 6u) * share));
+            const uint32_t piece = limit > 2u * target ? uint32_t((finer ? 2u : 4u) * share) : target;
             for (uint32_t q = 0; q < num_units; ++q) {
                 const uint32_t s = unit[q], e = unit[q + 1];
                 if (s == e || to_rows[q >> upp_log]) continue;
@@ -1821,8 +1828,12 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
             for (uint32_t q = 0; q < num_units; ++q)
                 if (unit[q] == unit[q + 1] && !to_rows[q >> upp_log]) chunks.push_back(make_uint4(unit[q], unit[q], q, 0u));
         const bool lean = p->shape == 2 || p->pipeline == 1;
-        if (!lean || !n_pieces || cute_offsets_fit(d->M, d->K, N, 0, uint64_t(n_pieces) * (CUTE_TM >> upp_log)) == 1) break;
-        if (attempt || t.mfma_shape == 2 || t.pipeline == 1) { delete p; return CUTE_ERR_SHAPE; }   // the caller forced a fast kernel
+        const uint64_t tile_rows = uint64_t(n_pieces) * (CUTE_TM >> upp_log);
+        const bool fits = !lean || !n_pieces || cute_offsets_fit(d->M, d->K, N, 0, tile_rows) == 1;
+        if (attempt == 0 && (!fits || tile_rows * N * sizeof(float) > uint64_t(CUTE_STATIC_SCRATCH_BYTES))) continue;
+        if (fits) break;
+        if (attempt == 2 || t.mfma_shape == 2 || t.pipeline == 1) { delete p; return CUTE_ERR_SHAPE; }   // the caller forced a fast kernel
+        attempt = 1;
         p->shape = 1;
         p->pipeline = 2;
         p->bf16x3 = p->halfLists = false;
