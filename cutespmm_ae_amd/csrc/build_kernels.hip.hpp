@@ -15,9 +15,9 @@
 // and no global atomic is needed.  About six LDS operations an entry; ranking it by binary searches over the panel's other rows
 // takes 50 to 100 (LDS merges of the rows, measured: census 57, strip lists 52 us on the graph below, 44 and 40 on the
 // finite-element matrix).
-// R-MAT graph of 65 536 nodes, 1.24 million entries: census 28 us, strip lists 40, where the entry-parallel kernels
-// over the whole matrix took 226 and 64; finite-element matrix of 24 000 rows, 1.44 million entries: census 13, brick tiles
-// 15 (before: 166 and 37).  What bounds it is latency: a dozen dependent steps a panel, four to six work-groups a compute unit.
+// R-MAT graph of 65 536 nodes, 1.24 million entries: strip lists 40 us, where the entry-parallel kernels
+// over the whole matrix took 64; finite-element matrix of 24 000 rows, 1.44 million entries: brick tiles
+// 15 (before: 37).  The census (panel_census) numbers nothing.  What bounds it is latency: a dozen dependent steps a panel, four to six work-groups a compute unit.
 // Other panels (hub rows of a graph, windows too wide for the bitmap) take the entry-parallel path at the end, where an entry's
 // position is a sum of binary searches over the panel's rows in global memory; both write the same words.
 #pragma once
@@ -234,14 +234,13 @@ template <uint32_t CAP> __device__ __forceinline__ uint32_t panel_rows(PanelLds<
 
 template <uint32_t CAP> __device__ __forceinline__ bool panel_fits(const PanelLds<CAP> &l, uint32_t max_span) { return l.hi - l.lo < max_span; }
 
-// Loads the entries of a panel of up to CAP of them, finds its column window and clears the LDS that numbers it (while the
-// loads are on their way).  CHECK: returns the error bits of the panel, every thread the same.
-template <bool CHECK, uint32_t CAP>
-__device__ __forceinline__ uint32_t load_panel(PanelLds<CAP> &l, PanelEntries<CAP> &e, uint32_t *window, const uint32_t *__restrict__ cols,
-                                               const float *__restrict__ vals, uint32_t start, uint32_t n, uint32_t K, uint32_t max_span)
+// Loads the entries of a panel of up to CAP of them (the census has checked them), finds its column window and clears the LDS that
+// numbers it while the loads are on their way.
+template <uint32_t CAP>
+__device__ __forceinline__ void load_panel(PanelLds<CAP> &l, PanelEntries<CAP> &e, uint32_t *window, const uint32_t *__restrict__ cols,
+                                           const float *__restrict__ vals, uint32_t start, uint32_t n, uint32_t max_span)
 {
     const uint32_t t = threadIdx.x;
-    int range = 0, unsorted = 0;
     uint32_t lo = ~0u, hi = 0u;
 #pragma unroll
     for (uint32_t k = 0; k < PanelEntries<CAP>::kEach; ++k) {
@@ -262,21 +261,11 @@ __device__ __forceinline__ uint32_t load_panel(PanelLds<CAP> &l, PanelEntries<CA
         const uint32_t c = e.active[k];
         lo = min(lo, c);
         hi = max(hi, c);
-        if (CHECK) {
-            range |= c >= K;
-            unsorted |= i > l.rp[e.row[k]] && cols[uint64_t(start) + i - 1u] >= c;
-        }
     }
     lo = wave_scan<~0u>(lo, [](uint32_t a, uint32_t b) { return min(a, b); });
     hi = wave_scan<0u>(hi, [](uint32_t a, uint32_t b) { return max(a, b); });
     if ((t & 63u) == 63u) { atomicMin(&l.lo, lo); atomicMax(&l.hi, hi); }
-    if (!CHECK) {
-        __syncthreads();
-        return 0u;
-    }
-    if (!__syncthreads_or(range | unsorted)) return 0u;
-    range = __syncthreads_or(range);
-    return (range ? kErrRange : 0u) | (__syncthreads_or(unsorted) ? kErrUnsorted : 0u);
+    __syncthreads();
 }
 
 // Numbers the active columns and fills l.col and l.rows; returns how many there are.
@@ -323,62 +312,181 @@ __device__ __forceinline__ uint32_t half(const Two &v, uint32_t s) { return ((s 
 // second launch over all panels would spend 15 us on work-groups that only leave).
 // A launch has at most 2^32 - 1 threads along a dimension of its grid, so all panels are kPanelRow to a row of the grid.
 constexpr uint32_t kPanelRow = 1u << 22;
-template <uint32_t CAP>
-__global__ __launch_bounds__(panel_threads(CAP)) void panel_census(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols,
+
+// Counts every panel for the planner and checks its rows.  A strip's pairs are the entries that find their column's bit clear in the
+// strip's bitmap of the panel's window, the panel's active columns those that find it clear in the panel's: nothing is numbered and no bitmap
+// is read through.  The bitmaps of four strips at a time where the window leaves room for them, else of two strips or of one.
+// Panels of more entries than the registers hold, up to kBigEntries, are walked strip after strip.
+// A chain of memory and LDS round trips a panel bounds this -- row starts, entries, window, bits -- so what counts is how many work-groups a compute unit
+// holds, hence the choice of census_words.  Numbering the columns in the
+// census as the builders below do took twice the steps and a second launch, with a wait for the first, for panels of more than 2 048 entries.
+// us, then (both launches) / now: R-MAT graph of 65 536 nodes 68 / 36.5; finite-element matrix of 24 000 rows 22.7 / 12.5; 9-point stencil of
+// 128 x 128 points 7.3 / 6.2; 65 536 rows of 32 in a band of 500, format to product, 156 / 147; 131 072 rows of 8 at random columns 280 / 219.
+// Dynamic LDS: lds_words, two bitmaps of max_span columns at least.
+constexpr uint32_t kBigEntries = 49152;
+constexpr uint32_t kCensusEach = 8;                          // entries a thread has on their way
+// Three bitmaps up to 65 536 columns (24 KB a work-group), then two (32 KB).  Four of 65 536 columns and their sums by reading them through took
+// 50 000 rows of 16 at random columns 22.3 us (16.0 now), 65 536 rows in a band of 500 26.9 (17.8 now), R-MAT graph of 131 072 nodes and 4
+// edges a node 109 (68 now).
+constexpr uint32_t census_words(uint32_t max_span) { return panel_window_words(max_span) * (max_span <= 65536u ? 3u : 2u); }
+
+__global__ __launch_bounds__(kThreads, 7) void panel_census(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols,
                                                          const float *__restrict__ vals, uint32_t P, uint32_t K, uint32_t nnz, uint32_t max_span,
-                                                         const uint32_t *__restrict__ list_of, PanelCensus *__restrict__ out)
+                                                         uint32_t lds_words, PanelCensus *__restrict__ out)
 {
-    extern __shared__ uint32_t window[];
-    __shared__ PanelLds<CAP> l;
+    extern __shared__ uint32_t bits[];
     __shared__ PanelCensus res;
-    const uint32_t p = list_of ? list_of[blockIdx.x] : blockIdx.y * gridDim.x + blockIdx.x, t = threadIdx.x;
+    __shared__ uint32_t lo_hi[2];
+    constexpr uint32_t kQuarter = kThreads / 4u;             // threads of a strip
+    const uint32_t p = blockIdx.y * gridDim.x + blockIdx.x, t = threadIdx.x;
     if (p >= P) return;
-    uint32_t start;
-    if (t < 12u) reinterpret_cast<uint32_t *>(&res)[t] = 0u;
-    const uint32_t n = panel_rows(l, rowPtr, p, P, nnz, start);
-    if (n == ~0u) {
-        if (t == 0u) res.error = kErrRange;
-    } else {
-        if (t < 16u) atomicMax(&res.maxRow, l.rp[t + 1] - l.rp[t]);
-        if (t == 0u) res.nnz = n;
-        if (n > CAP) {
-            if (t < 16u && l.rp[t + 1] > l.rp[t]) {
-                atomicMin(&l.lo, cols[uint64_t(start) + l.rp[t]]);
-                atomicMax(&l.hi, cols[uint64_t(start) + l.rp[t + 1] - 1u]);
-            }
-        } else if (n) {
-            PanelEntries<CAP> e;
-            const uint32_t err = load_panel<true>(l, e, window, cols, vals, start, n, K, max_span);
-            if (err) {
-                if (t == 0u) res.error = err;
-            } else if (panel_fits(l, max_span)) {
-                const uint32_t active = number_columns(l, e, window, n);
-                Two pairs = {0u, 0u};
-                uint32_t stored = 0;
-                for (uint32_t a = t; a < active; a += PanelLds<CAP>::kBlock) {
-                    const Two here = strips_of(l.rows[a]);
-                    pairs.x += here.x;
-                    pairs.y += here.y;
-                    stored += uint32_t(__popc(l.rows[a] >> 16));
-                }
-                pairs = {wave_add(pairs.x), wave_add(pairs.y)};
-                stored = wave_add(stored);
-                if ((t & 63u) == 63u) {
+    // the row pointers are the work-group's (scalar registers); every panel checks its own, so together they check all of them before
+    // anything is indexed through them
+    uint32_t rp[17];
 #pragma unroll
-                    for (uint32_t s = 0; s < 4u; ++s) atomicAdd(&res.pairs[s], half(pairs, s));
-                    atomicAdd(&res.stored, stored);
+    for (uint32_t k = 0; k < 17u; ++k) rp[k] = rowPtr[uint64_t(p) * 16u + k];
+    const uint32_t start = rp[0];
+    bool bad = rp[16] > nnz || (p == P - 1u && rp[16] != nnz) || (p == 0u && start != 0u);
+#pragma unroll
+    for (uint32_t k = 0; k < 16u; ++k) bad = bad || rp[k] > rp[k + 1u];
+#pragma unroll
+    for (uint32_t k = 0; k < 17u; ++k) rp[k] -= start;
+    // row starts of a strip, and the end of its last row
+    auto at_row = [&](uint32_t s, uint32_t k) { return s == 0u ? rp[k] : s == 1u ? rp[4u + k] : s == 2u ? rp[8u + k] : rp[12u + k]; };
+    const uint32_t n = bad ? 0u : rp[16];
+    if (t < 12u) reinterpret_cast<uint32_t *>(&res)[t] = 0u;
+    if (n) {
+        const uint32_t *const c = cols + start;
+        const float *const v = vals + start;
+        uint32_t range = 0, unsorted = 0, stored = 0, pairs = 0, active = 0, lo = 0, reach = 0, words = 0, longest = 0;
+        uint32_t at_once = 4;                                // strips whose bitmaps are in LDS at one time
+        bool fits = false;
+        struct Entries { uint32_t col[kCensusEach], before[kCensusEach]; float val[kCensusEach]; };
+        // entries i0 + k * step below `end`; the thread's own is `mine` further
+        auto fetch = [&](Entries &e, uint32_t i0, uint32_t mine, uint32_t step, uint32_t end) {
+#pragma unroll
+            for (uint32_t k = 0; k < kCensusEach; ++k) {
+                if (i0 + k * step >= end) break;
+                const uint32_t i = min(i0 + mine + k * step, n - 1u);
+                e.col[k] = c[i];
+                e.before[k] = c[i ? i - 1u : 0u];
+                e.val[k] = v[i];
+            }
+        };
+        auto window = [&] {                                  // and LDS cleared for it
+            if (t < 64u) {
+                uint32_t low = ~0u, high = 0u, row = 0u;
+                if (t < 16u) {
+                    const uint32_t b = rowPtr[uint64_t(p) * 16u + t], e = rowPtr[uint64_t(p) * 16u + t + 1u];
+                    if (e > b) { low = cols[b]; high = cols[e - 1u]; row = e - b; }
                 }
-                if (t == 0u) res.cols = active;
+                low = wave_scan<~0u>(low, [](uint32_t a, uint32_t b) { return min(a, b); });
+                high = wave_scan<0u>(high, [](uint32_t a, uint32_t b) { return max(a, b); });
+                longest = wave_scan<0u>(row, [](uint32_t a, uint32_t b) { return max(a, b); });
+                if (t == 63u) { lo_hi[0] = low; lo_hi[1] = high; }
+            }
+            __syncthreads();
+            // (rows that are not sorted may lie outside the window: they are not marked, and the census refuses the matrix)
+            lo = lo_hi[0];
+            reach = lo_hi[1] - lo;
+            words = reach / 32u + 1u;
+            fits = lo_hi[1] >= lo && reach < max_span;
+            at_once = !fits || 5u * words <= lds_words ? 4u : 3u * words <= lds_words ? 2u : 1u;
+            if (fits)                                        // (the panel's bitmap first)
+                for (uint32_t w = t; w < (at_once + 1u) * words; w += kThreads) bits[w] = 0u;
+            __syncthreads();
+        };
+        // mark(word, bit) for every column
+        auto take = [&](const Entries &e, uint32_t i0, uint32_t mine, uint32_t step, uint32_t s, auto mark) {
+            const uint32_t r0 = at_row(s, 0), r1 = at_row(s, 1), r2 = at_row(s, 2), r3 = at_row(s, 3), end = at_row(s, 4);
+#pragma unroll
+            for (uint32_t k = 0; k < kCensusEach; ++k) {
+                if (i0 + k * step >= end) break;
+                const uint32_t i = i0 + mine + k * step;
+                if (i >= end) continue;
+                range |= e.col[k] >= K ? 1u : 0u;
+                unsorted |= i != r0 && i != r1 && i != r2 && i != r3 && e.before[k] >= e.col[k] ? 1u : 0u;
+                stored += e.val[k] != 0.0f ? 1u : 0u;
+                const uint32_t at = e.col[k] - lo;
+                if (fits && at <= reach) mark(at >> 5, 1u << (at & 31u));
+            }
+        };
+        auto add_pairs = [&](uint32_t s) {
+            pairs = wave_add(pairs);
+            if ((t & 63u) == 63u) atomicAdd(&res.pairs[s], pairs);
+            pairs = 0;
+        };
+        bool held = n <= 4u * kCensusEach * kQuarter;
+#pragma unroll
+        for (uint32_t s = 0; s < 4u; ++s) held = held && rp[4u * s + 4u] - rp[4u * s] <= kCensusEach * kQuarter;
+        if (held) {
+            // every strip has at most kCensusEach entries for each thread of its quarter of the work-group: asked for before the window is known
+            const uint32_t strip = __builtin_amdgcn_readfirstlane(t / kQuarter), mine = t % kQuarter, from = at_row(strip, 0), end = at_row(strip, 4);
+            Entries e;
+            fetch(e, from, mine, kQuarter, end);
+            window();
+#pragma unroll 1
+            for (uint32_t s = 0; s < 4u; s += at_once) {
+                uint32_t *const marked = bits + (strip - s + 1u) * words;
+                if (strip - s < at_once)
+                    take(e, from, mine, kQuarter, strip, [&](uint32_t w, uint32_t bit) {
+                        pairs += atomicOr(&marked[w], bit) & bit ? 0u : 1u;
+                        active += atomicOr(&bits[w], bit) & bit ? 0u : 1u;
+                    });
+                if (s + at_once == 4u || !fits) continue;
+                __syncthreads();
+                if (strip - s < at_once)                     // the next strips' bits begin clear
+#pragma unroll
+                    for (uint32_t k = 0; k < kCensusEach; ++k) {
+                        if (from + k * kQuarter >= end) break;
+                        if (e.col[k] - lo <= reach) marked[(e.col[k] - lo) >> 5] = 0u;
+                    }
+                __syncthreads();
+            }
+            add_pairs(strip);
+        } else {
+            window();
+            if (n <= kBigEntries) {
+                // (so many entries that their strip's bitmap is soon read through)
+#pragma unroll 1
+                for (uint32_t s = 0; s < 4u; ++s) {
+#pragma unroll 1
+                    for (uint32_t i0 = at_row(s, 0); i0 < at_row(s, 4); i0 += kCensusEach * kThreads) {
+                        Entries e;
+                        fetch(e, i0, t, kThreads, at_row(s, 4));
+                        take(e, i0, t, kThreads, s, [&](uint32_t w, uint32_t bit) { atomicOr(&bits[words + w], bit); });
+                    }
+                    __syncthreads();
+                    if (fits)
+                        for (uint32_t w = t; w < words; w += kThreads) {          // (a thread's words are its own from strip to strip)
+                            const uint32_t b = bits[words + w], all = bits[w] | b;
+                            pairs += uint32_t(__popc(b));
+                            if (s == 3u) active += uint32_t(__popc(all));
+                            bits[w] = all;
+                            bits[words + w] = 0u;
+                        }
+                    add_pairs(s);
+                    __syncthreads();
+                }
             }
         }
-    }
-    __syncthreads();
-    if (t == 0u) {
-        res.first = l.lo;
-        if (n && n != ~0u) {
-            res.span = l.hi - l.lo + 1u;
-            res.end = l.hi + 1u;
+        if (range | unsorted) atomicOr(&res.error, (range ? uint32_t(kErrRange) : 0u) | (unsorted ? uint32_t(kErrUnsorted) : 0u));
+        active = wave_add(active);
+        stored = wave_add(stored);
+        if ((t & 63u) == 63u) {
+            atomicAdd(&res.cols, active);
+            atomicAdd(&res.stored, stored);
         }
+        if (t == 63u) {                                      // (its wavefront's `longest` is in its last lane)
+            res.nnz = n;
+            res.maxRow = longest;
+            res.first = lo;
+            res.span = reach + 1u;
+            res.end = lo + reach + 1u;
+        }
+    } else if (t == 0u) {
+        res.first = ~0u;
+        res.error = bad ? uint32_t(kErrRange) : 0u;
     }
     __syncthreads();
     if (t < 12u) reinterpret_cast<uint32_t *>(out + p)[t] = reinterpret_cast<const uint32_t *>(&res)[t];
@@ -401,7 +509,7 @@ __global__ __launch_bounds__(panel_threads(CAP)) void panel_bricks(const uint32_
     const uint32_t n = panel_rows(l, rowPtr, p, P, nnz, start);
     if (n == 0u || n > CAP) return;
     PanelEntries<CAP> e;
-    load_panel<false>(l, e, window, cols, vals, start, n, 0u, max_span);
+    load_panel(l, e, window, cols, vals, start, n, max_span);
     if (!panel_fits(l, max_span)) return;
     const uint32_t active = number_columns(l, e, window, n);
     uint16_t *first = reinterpret_cast<uint16_t *>(window);   // position of every active column's first entry, and n behind the last
@@ -466,7 +574,7 @@ __global__ __launch_bounds__(panel_threads(CAP)) void panel_quads(const uint32_t
     const uint32_t n = panel_rows(l, rowPtr, p, P, nnz, start);
     if (n == 0u || n > CAP) return;
     PanelEntries<CAP> e;
-    load_panel<false>(l, e, window, cols, vals, start, n, 0u, max_span);
+    load_panel(l, e, window, cols, vals, start, n, max_span);
     if (!panel_fits(l, max_span)) return;
     const uint32_t active = number_columns(l, e, window, n);
     Two *before = reinterpret_cast<Two *>(window);            // pairs in front of an active column's, in each strip's list
@@ -550,35 +658,14 @@ __global__ __launch_bounds__(panel_threads(CAP)) void panel_quads(const uint32_t
 
 // ------------------------------------------------------------------------------------------------
 // Panels of more than kPanelCap entries (the hub rows of a graph) whose window the bitmap takes: a work-group of sixteen wavefronts
-// walks the entries instead of holding them, for the census and for the strip lists.  LDS holds the bitmap, its counts and the
+// walks the entries of a strip instead of holding them, for the strip lists.  LDS holds the bitmap, its counts and the
 // rows of every active column, and the rest follows from prefix sums over the columns, a thread a run of them.
 // The entry-parallel kernels below need sixteen binary searches an entry, two scans and a launch for each step: R-MAT graph of 65 536
-// nodes, 449 000 entries in 79 such panels, census 70 -> 38 us, lists 70 -> 34.
+// nodes, 449 000 entries in 79 such panels, lists 70 -> 34 us.
 // ------------------------------------------------------------------------------------------------
-constexpr uint32_t kBigThreads = 1024, kBigEntries = 49152;        // (sums of a panel fit 16 bits)
-
-struct BigLds {
-    uint32_t rp[17], lo, hi;
-    Two waveSum[kBigThreads / 64];
-};
+constexpr uint32_t kBigThreads = 1024;        // (with kBigEntries the sums of a panel fit 16 bits)
 
 constexpr __host__ __device__ uint32_t big_window_words(uint32_t window_words) { return window_words + (window_words + 1u) / 2u; }   // bitmap and 16-bit counts
-
-// Row starts, first and last column; returns the entries of the panel.
-__device__ __forceinline__ uint32_t big_rows(BigLds &l, const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols, uint32_t p, uint32_t &start)
-{
-    const uint32_t t = threadIdx.x;
-    start = rowPtr[uint64_t(p) * 16u];
-    if (t < 17u) l.rp[t] = rowPtr[uint64_t(p) * 16u + t] - start;
-    if (t == 0u) { l.lo = ~0u; l.hi = 0u; }
-    __syncthreads();
-    if (t < 16u && l.rp[t + 1] > l.rp[t]) {
-        atomicMin(&l.lo, cols[uint64_t(start) + l.rp[t]]);
-        atomicMax(&l.hi, cols[uint64_t(start) + l.rp[t + 1] - 1u]);
-    }
-    __syncthreads();
-    return l.rp[16];
-}
 
 // Running counts of the bitmap's words; returns how many columns are active.
 __device__ __forceinline__ uint32_t big_counts(Two (&waveSum)[kBigThreads / 64], const uint32_t *window, uint16_t *count, uint32_t words)
@@ -596,67 +683,6 @@ __device__ __forceinline__ uint32_t big_counts(Two (&waveSum)[kBigThreads / 64],
 __device__ __forceinline__ uint32_t big_number(const uint32_t *window, const uint16_t *count, uint32_t c)      // c: from the window's start
 {
     return count[c >> 5] + uint32_t(__popc(window[c >> 5] & ((1u << (c & 31u)) - 1u)));
-}
-
-// Completes the census records of the listed panels (panel_census has counted their entries and found their windows).
-__global__ __launch_bounds__(kBigThreads) void big_census(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols, const float *__restrict__ vals,
-                                                          uint32_t K, const uint32_t *__restrict__ list, uint32_t window_words, uint32_t row_words,
-                                                          PanelCensus *__restrict__ out)
-{
-    extern __shared__ uint32_t window[];
-    __shared__ BigLds l;
-    __shared__ uint32_t pairs[4], stored;
-    uint16_t *count = reinterpret_cast<uint16_t *>(window + window_words);
-    uint32_t *rows = window + big_window_words(window_words);      // 16 bits a column
-    const uint32_t p = list[blockIdx.x], t = threadIdx.x;
-    for (uint32_t w = t; w < window_words; w += kBigThreads) window[w] = 0u;
-    for (uint32_t w = t; w < row_words; w += kBigThreads) rows[w] = 0u;
-    if (t < 4u) pairs[t] = 0u;
-    if (t == 4u) stored = 0u;
-    uint32_t start;
-    const uint32_t n = big_rows(l, rowPtr, cols, p, start), lo = l.lo, reach = l.hi - lo, words = reach / 32u + 1u;
-    // (rows that are not sorted: no column outside the window is marked, and the census refuses the matrix)
-    const bool fits = l.hi >= lo && words <= window_words;
-    int range = 0, unsorted = !fits;
-    uint32_t mine = 0;
-#pragma unroll 4
-    for (uint32_t i = t; i < n; i += kBigThreads) {
-        const uint32_t c = cols[uint64_t(start) + i], before = cols[uint64_t(start) + (i ? i - 1u : 0u)];
-        range |= c >= K;
-        unsorted |= i > l.rp[row_in_panel(l.rp, i)] && before >= c;
-        mine += vals[uint64_t(start) + i] != 0.0f ? 1u : 0u;
-        if (fits && c - lo <= reach) atomicOr(&window[(c - lo) >> 5], 1u << ((c - lo) & 31u));
-    }
-    range = __syncthreads_or(range);
-    unsorted = __syncthreads_or(unsorted);
-    if (range || unsorted) {
-        if (t == 0u) out[p].error = (range ? kErrRange : 0u) | (unsorted ? kErrUnsorted : 0u);
-        return;
-    }
-    const uint32_t active = big_counts(l.waveSum, window, count, words);
-#pragma unroll 4
-    for (uint32_t i = t; i < n; i += kBigThreads) {
-        const uint32_t a = big_number(window, count, cols[uint64_t(start) + i] - lo);
-        atomicOr(&rows[a >> 1], 1u << ((a & 1u) * 16u + row_in_panel(l.rp, i)));
-    }
-    __syncthreads();
-    Two own = {0u, 0u};
-    for (uint32_t a = t; a < active; a += kBigThreads) {
-        const Two here = strips_of(reinterpret_cast<const uint16_t *>(rows)[a]);
-        own.x += here.x;
-        own.y += here.y;
-    }
-    own = {wave_add(own.x), wave_add(own.y)};
-    mine = wave_add(mine);
-    if ((t & 63u) == 63u) {
-#pragma unroll
-        for (uint32_t s = 0; s < 4u; ++s) atomicAdd(&pairs[s], half(own, s));
-        atomicAdd(&stored, mine);
-    }
-    __syncthreads();
-    if (t < 4u) out[p].pairs[t] = pairs[t];
-    if (t == 4u) out[p].stored = stored;
-    if (t == 5u) out[p].cols = active;
 }
 
 // Strip lists of the listed panels (panel_quads<true> defines them), a work-group a strip: its entries are one piece of the arrays, its

@@ -711,25 +711,14 @@ void list_large_panels(const cute_hrpb_dev *d, LargeWork &w)
         }
 }
 
-// The LDS that big_census and big_quads ask for beside their static part (a kilobyte at most) is a compute unit's whatever the matrix: the
-// census keeps 16 bits a column of a panel, the lists a byte a column of a strip and two words a group of sixteen.
+// The LDS that big_quads asks for beside its static part (a kilobyte at most) is a compute unit's whatever the matrix: a byte a column of a
+// strip and two words a group of sixteen.
 constexpr uint32_t kBigWindow = cute_build::big_window_words(cute_build::panel_window_words(cute_build::kPanelSpan));
-static_assert((kBigWindow + cute_build::kBigEntries / 2u) * 4u + 1024u <= 160u << 10, "big_census");
 static_assert((kBigWindow + cute_build::kBigEntries / 4u + cute_build::kBigEntries / 16u * 2u) * 4u + 1024u <= 160u << 10, "big_quads");
 
-// The words big_census wants for the rows of the columns of every large panel; 0: there are some that it does not take, and then it takes
-// none (nor do the lists): one panel beyond kBigEntries or kPanelSpan sends all large panels of the matrix to the entry-parallel path.
-uint32_t big_census_rows(const cute_hrpb_dev *d, const LargeWork &w)
-{
-    uint32_t most = 0;
-    for (uint32_t p : w.panel) {
-        if (d->panelNnz[p] > cute_build::kBigEntries || d->panelSpan[p] > max_span(d) || d->panelSpan[p] == 0) return 0;
-        most = std::max(most, std::min(d->panelNnz[p], d->panelSpan[p]));
-    }
-    return (most + 1u) / 2u;
-}
-
-// The same for big_quads (the census has counted the columns of every strip): a byte a column, and the words of its groups' masks.
+// The LDS words big_quads wants for the rows of the columns of every large panel's strips (the census has counted them), a byte a column,
+// and for the masks of their groups; 0: there are panels that it does not take, and then it takes none.  One panel beyond kBigEntries
+// or kPanelSpan sends all large panels of the matrix to the entry-parallel path.
 uint32_t big_quad_rows(const cute_hrpb_dev *d, const LargeWork &w, uint32_t &masks)
 {
     uint32_t most = 0;
@@ -1097,14 +1086,14 @@ int finish_upload(cute_hrpb_dev *d, int quad_layout, const DeviceContext &c)
         int rc = pin.alloc((uint64_t(P) + kTilePanels) * sizeof(cute_build::PanelCensus));      // (the loop below asks for records ahead of it)
         if (rc != CUTE_OK) return rc;
         pin.pending = true;
-        CUTE_PANELS(cute_build::panel_census<cute_build::kPanelFirst>, cute_build::kPanelFirst, P, window_lds(d, 0), d->dRowPtr, d->dCols,
-                    d->dCsrVals, P, d->K, d->nnz, max_span(d), kAllPanels, pin.as<cute_build::PanelCensus>());
+        CUTE_BUILD_LDS(cute_build::panel_census, panel_grid(P), cute_build::census_words(max_span(d)) * 4u, d->dRowPtr, d->dCols, d->dCsrVals, P, d->K,
+                       d->nnz, max_span(d), cute_build::census_words(max_span(d)), pin.as<cute_build::PanelCensus>());
         rc = check_launch("panel census");
         if (rc == CUTE_OK) rc = pin.wait();
         if (rc != CUTE_OK) return rc;
         const cute_build::PanelCensus *r = pin.as<const cute_build::PanelCensus>();
         uint32_t error = 0;
-        bool any_large = false, any_medium = false;
+        bool any_large = false, any_left = false;      // panels for the lists' entry-parallel or long kernels; panels the census leaves to number_large_panels
         uint32_t longest = 0;
         d->panelNnz.resize(P);
         d->panelSpan.resize(P);
@@ -1121,39 +1110,19 @@ int finish_upload(cute_hrpb_dev *d, int quad_layout, const DeviceContext &c)
                 longest = std::max(longest, r[p].nnz);
                 tile.x = std::min(tile.x, r[p].first);
                 tile.y = std::max(tile.y, r[p].end);
-                if (r[p].nnz > cute_build::kPanelFirst || r[p].span > max_span(d)) (panel_is_large(d, p) ? any_large : any_medium) = true;
+                if (panel_is_large(d, p)) {
+                    any_large = true;
+                    any_left = any_left || r[p].nnz > cute_build::kBigEntries || r[p].span > max_span(d);
+                }
             }
             into = tile;
             if (tile.y) d->widestTile = std::max(d->widestTile, tile.y - tile.x);
         }
         d->longestPanel = longest;
         d->anyLarge = any_large;
-        if (!error && (any_medium || any_large)) {
-            const std::vector<uint32_t> medium = panels_between(d, cute_build::kPanelFirst);
-            list_large_panels(d, large);
-            const uint32_t big_rows = big_census_rows(d, large);
-            PinnedBuf list;
-            rc = list.alloc((medium.size() + large.panel.size()) * 4u);
+        if (!error && any_left) {
+            rc = number_large_panels(d, large, pin.as<cute_build::PanelCensus>());
             if (rc != CUTE_OK) return rc;
-            list.pending = true;
-            if (big_rows) {
-                const uint32_t words = cute_build::panel_window_words(max_span(d));
-                std::memcpy(list.as<uint32_t>() + medium.size(), large.panel.data(), large.panel.size() * 4u);
-                hipLaunchKernelGGL(cute_build::big_census, dim3(uint32_t(large.panel.size())), dim3(cute_build::kBigThreads),
-                                   (cute_build::big_window_words(words) + big_rows) * 4u, nullptr, d->dRowPtr, d->dCols, d->dCsrVals, d->K,
-                                   list.as<const uint32_t>() + medium.size(), words, big_rows, pin.as<cute_build::PanelCensus>());
-                rc = check_launch("panel census");
-            }
-            if (!medium.empty()) {
-                std::memcpy(list.p, medium.data(), medium.size() * 4u);
-                CUTE_PANELS(cute_build::panel_census<cute_build::kPanelCap>, cute_build::kPanelCap, uint32_t(medium.size()), window_lds(d, 0),
-                            d->dRowPtr, d->dCols, d->dCsrVals, P, d->K, d->nnz, max_span(d), list.as<const uint32_t>(), pin.as<cute_build::PanelCensus>());
-                if (rc == CUTE_OK) rc = check_launch("panel census");
-            }
-            if (rc == CUTE_OK && any_large && !big_rows) rc = number_large_panels(d, large, pin.as<cute_build::PanelCensus>());
-            if (rc == CUTE_OK) rc = list.wait();
-            if (rc != CUTE_OK) return rc;
-            for (uint32_t p : medium) error |= r[p].error;
             for (uint32_t p : large.panel) error |= r[p].error;
         }
         if (error & cute_build::kErrRange) return CUTE_ERR_RANGE;
