@@ -132,19 +132,10 @@ __global__ __launch_bounds__(kThreads) void scan_block_apply(uint32_t *data, uin
         if (base + i < n) data[base + i] = offset + v[i];
 }
 
-// The three CSR arrays into the handle's own memory: from the caller's device arrays, or from pinned host memory.
+// From pinned host memory into device memory.
 __global__ __launch_bounds__(kThreads) void copy_words(const uint32_t *__restrict__ src, uint32_t *__restrict__ dst, uint64_t n)
 {
     for (uint64_t i = global_id(); i < n; i += uint64_t(gridDim.x) * kThreads) dst[i] = src[i];
-}
-
-__global__ __launch_bounds__(kThreads) void copy_csr(const uint32_t *__restrict__ srcRowPtr, const uint32_t *__restrict__ srcCols,
-                                                     const uint32_t *__restrict__ srcVals, uint32_t M, uint32_t nnz,
-                                                     uint32_t *__restrict__ rowPtr, uint32_t *__restrict__ cols, uint32_t *__restrict__ vals)
-{
-    const uint64_t stride = uint64_t(gridDim.x) * kThreads;
-    for (uint64_t i = global_id(); i < nnz; i += stride) { cols[i] = srcCols[i]; vals[i] = srcVals[i]; }
-    for (uint64_t i = global_id(); i <= M; i += stride) rowPtr[i] = srcRowPtr[i];
 }
 
 __device__ __forceinline__ uint32_t row_in_panel(const uint32_t *rp, uint32_t e)
@@ -322,6 +313,8 @@ constexpr uint32_t kPanelRow = 1u << 22;
 // census as the builders below do took twice the steps and a second launch, with a wait for the first, for panels of more than 2 048 entries.
 // us, then (both launches) / now: R-MAT graph of 65 536 nodes 68 / 36.5; finite-element matrix of 24 000 rows 22.7 / 12.5; 9-point stencil of
 // 128 x 128 points 7.3 / 6.2; 65 536 rows of 32 in a band of 500, format to product, 156 / 147; 131 072 rows of 8 at random columns 280 / 219.
+// COPY: the arrays are the caller's and are copied to `to` as well.  With a launch of its own for that, format to product took, us: stencil of
+// 128 x 128 points, N = 32 78.6 (75.6 now), 65 536 rows of 32 in a band 147 (138 now), 50 000 rows of 16 at random columns 178 (173 now).
 // Dynamic LDS: lds_words, two bitmaps of max_span columns at least.
 constexpr uint32_t kBigEntries = 49152;
 constexpr uint32_t kCensusEach = 8;                          // entries a thread has on their way
@@ -330,9 +323,15 @@ constexpr uint32_t kCensusEach = 8;                          // entries a thread
 // edges a node 109 (68 now).
 constexpr uint32_t census_words(uint32_t max_span) { return panel_window_words(max_span) * (max_span <= 65536u ? 3u : 2u); }
 
+struct CsrCopy {
+    uint32_t *rowPtr, *cols;
+    float *vals;
+};
+
+template <bool COPY>
 __global__ __launch_bounds__(kThreads, 7) void panel_census(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols,
                                                          const float *__restrict__ vals, uint32_t P, uint32_t K, uint32_t nnz, uint32_t max_span,
-                                                         uint32_t lds_words, PanelCensus *__restrict__ out)
+                                                         uint32_t lds_words, uint32_t share, CsrCopy to, PanelCensus *__restrict__ out)
 {
     extern __shared__ uint32_t bits[];
     __shared__ PanelCensus res;
@@ -355,6 +354,7 @@ __global__ __launch_bounds__(kThreads, 7) void panel_census(const uint32_t *__re
     auto at_row = [&](uint32_t s, uint32_t k) { return s == 0u ? rp[k] : s == 1u ? rp[4u + k] : s == 2u ? rp[8u + k] : rp[12u + k]; };
     const uint32_t n = bad ? 0u : rp[16];
     if (t < 12u) reinterpret_cast<uint32_t *>(&res)[t] = 0u;
+    if (COPY && t < (p == P - 1u ? 17u : 16u)) to.rowPtr[uint64_t(p) * 16u + t] = rowPtr[uint64_t(p) * 16u + t];
     if (n) {
         const uint32_t *const c = cols + start;
         const float *const v = vals + start;
@@ -487,6 +487,11 @@ __global__ __launch_bounds__(kThreads, 7) void panel_census(const uint32_t *__re
     } else if (t == 0u) {
         res.first = ~0u;
         res.error = bad ? uint32_t(kErrRange) : 0u;
+    }
+    if (COPY) {                                              // the same share for every work-group (beside the rest its own entries would take registers)
+        const uint64_t upto = min(uint64_t(nnz), (p + uint64_t(1)) * share);
+#pragma unroll 4
+        for (uint64_t i = p * uint64_t(share) + t; i < upto; i += kThreads) { to.cols[i] = cols[i]; to.vals[i] = vals[i]; }
     }
     __syncthreads();
     if (t < 12u) reinterpret_cast<uint32_t *>(out + p)[t] = reinterpret_cast<const uint32_t *>(&res)[t];

@@ -1074,10 +1074,11 @@ struct HostToDevice {
     }
 };
 
-// The common tail of both uploads.  d's CSR arrays are on their way to the device (default stream).  Checks them, counts what
+// The common tail of both uploads.  The CSR arrays are on their way to the device (default stream): to d's own, or they are the caller's and
+// the census copies them.  Checks them, counts what
 // the planner wants to know about every panel, and builds the one MFMA layout the planner's default rules would use for
 // this matrix (none when every panel would go to the row kernel).
-int finish_upload(cute_hrpb_dev *d, int quad_layout, const DeviceContext &c)
+int finish_upload(cute_hrpb_dev *d, int quad_layout, const DeviceContext &c, const uint32_t *rowPtr, const uint32_t *cols, const float *vals)
 {
     const uint32_t P = d->P;
     LargeWork large;
@@ -1086,8 +1087,14 @@ int finish_upload(cute_hrpb_dev *d, int quad_layout, const DeviceContext &c)
         int rc = pin.alloc((uint64_t(P) + kTilePanels) * sizeof(cute_build::PanelCensus));      // (the loop below asks for records ahead of it)
         if (rc != CUTE_OK) return rc;
         pin.pending = true;
-        CUTE_BUILD_LDS(cute_build::panel_census, panel_grid(P), cute_build::census_words(max_span(d)) * 4u, d->dRowPtr, d->dCols, d->dCsrVals, P, d->K,
-                       d->nnz, max_span(d), cute_build::census_words(max_span(d)), pin.as<cute_build::PanelCensus>());
+        const uint32_t lds_words = cute_build::census_words(max_span(d)), share = uint32_t((uint64_t(d->nnz) + P - 1u) / P);
+        const cute_build::CsrCopy to = {d->dRowPtr, d->dCols, d->dCsrVals};
+        if (rowPtr == d->dRowPtr)
+            CUTE_BUILD_LDS(cute_build::panel_census<false>, panel_grid(P), lds_words * 4u, rowPtr, cols, vals, P, d->K, d->nnz, max_span(d), lds_words, share, to,
+                           pin.as<cute_build::PanelCensus>());
+        else
+            CUTE_BUILD_LDS(cute_build::panel_census<true>, panel_grid(P), lds_words * 4u, rowPtr, cols, vals, P, d->K, d->nnz, max_span(d), lds_words, share, to,
+                           pin.as<cute_build::PanelCensus>());
         rc = check_launch("panel census");
         if (rc == CUTE_OK) rc = pin.wait();
         if (rc != CUTE_OK) return rc;
@@ -1273,7 +1280,7 @@ int cute_hrpb_upload_layout(const cute_hrpb_host *h, int quad_layout, cute_hrpb_
         if (rc == CUTE_OK) rc = up.copy(d->dRowPtr, h->rowPtr, (uint64_t(h->M) + 1) * 4u);
         if (rc == CUTE_OK) rc = up.copy(d->dCols, h->cols, uint64_t(h->nnz) * 4u);
         if (rc == CUTE_OK) rc = up.copy(d->dCsrVals, h->vals, uint64_t(h->nnz) * 4u);
-        if (rc == CUTE_OK) rc = finish_upload(d, quad_layout, c);
+        if (rc == CUTE_OK) rc = finish_upload(d, quad_layout, c, d->dRowPtr, d->dCols, d->dCsrVals);
     }
     // the device counted the active columns itself: it must have found the blocks the canonical format has
     if (rc == CUTE_OK && (d->nb != h->numBlocks || std::memcmp(d->brp.data(), h->blockedRowPtr, d->brp.size() * sizeof(uint32_t)) != 0))
@@ -1298,11 +1305,7 @@ int cute_hrpb_upload_device_csr(uint32_t M, uint32_t K, uint32_t nnz, const uint
     d->M = M; d->K = K; d->nnz = nnz; d->P = M / CUTE_TM;
     d->numVals = nnz;
     int rc = alloc_csr(d);
-    if (rc == CUTE_OK) {
-        CUTE_BUILD(cute_build::copy_csr, grid_capped(std::max<uint64_t>(nnz, uint64_t(M) + 1)), dRowPtr, dCols, reinterpret_cast<const uint32_t *>(dVals), M, nnz,
-                   d->dRowPtr, d->dCols, reinterpret_cast<uint32_t *>(d->dCsrVals));
-        rc = finish_upload(d, quad_layout, c);
-    }
+    if (rc == CUTE_OK) rc = finish_upload(d, quad_layout, c, dRowPtr, dCols, dVals);
     // (set-up itself waits for the default stream only; the interface promises the device)
     if (rc == CUTE_OK && !wait_for_device()) {
         const hipError_t e = hipDeviceSynchronize();     // (not a page left to free)
