@@ -712,21 +712,21 @@ void list_large_panels(const cute_hrpb_dev *d, LargeWork &w)
 }
 
 // The LDS that big_quads asks for beside its static part (a kilobyte at most) is a compute unit's whatever the matrix: a byte a column of a
-// strip and two words a group of sixteen.
+// strip and three words for every 64 columns.
 constexpr uint32_t kBigWindow = cute_build::big_window_words(cute_build::panel_window_words(cute_build::kPanelSpan));
-static_assert((kBigWindow + cute_build::kBigEntries / 4u + cute_build::kBigEntries / 16u * 2u) * 4u + 1024u <= 160u << 10, "big_quads");
+static_assert((kBigWindow + cute_build::kBigEntries / 4u + cute_build::kBigEntries / 64u * 3u) * 4u + 1024u <= 160u << 10, "big_quads");
 
 // The LDS words big_quads wants for the rows of the columns of every large panel's strips (the census has counted them), a byte a column,
-// and for the masks of their groups; 0: there are panels that it does not take, and then it takes none.  One panel beyond kBigEntries
+// and for its steps of 64 columns; 0: there are panels that it does not take, and then it takes none.  One panel beyond kBigEntries
 // or kPanelSpan sends all large panels of the matrix to the entry-parallel path.
-uint32_t big_quad_rows(const cute_hrpb_dev *d, const LargeWork &w, uint32_t &masks)
+uint32_t big_quad_rows(const cute_hrpb_dev *d, const LargeWork &w, uint32_t &steps)
 {
     uint32_t most = 0;
     for (uint32_t p : w.panel) {
         if (d->panelNnz[p] > cute_build::kBigEntries || d->panelSpan[p] > max_span(d)) return 0;
         for (uint32_t s = 0; s < 4u; ++s) most = std::max(most, d->stripPairs[4u * p + s]);
     }
-    masks = (most + 15u) / 16u * 2u;
+    steps = (most + 63u) / 64u * 3u;
     return (most + 3u) / 4u;
 }
 
@@ -825,8 +825,8 @@ int build_quads_on_device(cute_hrpb_dev *d, LargeWork &w)
     const uint64_t G = d->numGroups, stored = d->numQuadVals;
     const bool strips = d->quadRows == 4;
     list_large_panels(d, w);
-    uint32_t big_masks = 0;
-    const uint32_t big_rows = strips ? big_quad_rows(d, w, big_masks) : 0u;      // all large panels through big_quads, or none
+    uint32_t big_steps = 0;
+    const uint32_t big_rows = strips ? big_quad_rows(d, w, big_steps) : 0u;      // all large panels through big_quads, or none
     int rc = big_rows ? int(CUTE_OK) : number_large_panels(d, w, nullptr);
     if (rc != CUTE_OK) return rc;
     const uint32_t count = big_rows ? 0u : uint32_t(w.panel.size()), per = strips ? 4u : 1u;
@@ -888,8 +888,8 @@ int build_quads_on_device(cute_hrpb_dev *d, LargeWork &w)
     if (big_rows) {
         const uint32_t words = cute_build::panel_window_words(max_span(d));
         hipLaunchKernelGGL(cute_build::big_quads, dim3(uint32_t(w.panel.size()) * 4u), dim3(cute_build::kBigThreads),
-                           (cute_build::big_window_words(words) + big_rows + big_masks) * 4u, nullptr, d->dRowPtr, d->dCols, d->dCsrVals, table(oBig), words,
-                           big_rows, big_masks, table(oGroup), table(oBase), recs, packed);
+                           (cute_build::big_window_words(words) + big_rows + big_steps) * 4u, nullptr, d->dRowPtr, d->dCols, d->dCsrVals, table(oBig), words,
+                           big_rows, table(oGroup), table(oBase), recs, packed);
     }
     if (strips) { CUTE_BUILD_QUADS(true) } else { CUTE_BUILD_QUADS(false) }
 #undef CUTE_BUILD_QUADS
