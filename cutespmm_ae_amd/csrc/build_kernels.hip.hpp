@@ -36,11 +36,13 @@ constexpr uint32_t kScanBlock = kThreads * kScanItems;      // entries per scan 
 
 // Entries of a panel that one work-group holds, eight a thread: 512 threads for up to kPanelCap; the launches over all panels
 // take 256 threads and up to kPanelFirst (list kernel: kPanelList, whose LDS lets six work-groups share a compute unit instead
-// of three, 60 -> 40 us on the graph above), the launches over the few panels between are given their list.
+// of three, 60 -> 40 us on the graph above), panels between have a launch that is given their list, or, for the strip lists, a
+// work-group a strip.
 constexpr uint32_t kPanelCap = 4096, kPanelFirst = 2048, kPanelList = 1024;
 constexpr uint32_t kPanelSpan = 1u << 17;                   // columns of its window: a bitmap of 16 KB and 8 KB of running counts
 
-enum : uint32_t { kErrRange = 1, kErrUnsorted = 2 };
+enum : uint32_t { kErrRange = 1, kErrUnsorted = 2, kAnyError = kErrRange | kErrUnsorted };
+constexpr uint32_t kLongStrip = 16;                         // << strip, beside the errors: the strip has more than kPanelList entries
 
 // What the planner wants to know about a panel; one 48-byte record each, written to host memory.
 struct PanelCensus {
@@ -48,7 +50,7 @@ struct PanelCensus {
     uint32_t cols, span;       // distinct (active) columns, last column - first column + 1
     uint32_t pairs[4];         // distinct columns of each 4-row strip
     uint32_t stored;           // entries that are not zero
-    uint32_t error;            // kErrRange | kErrUnsorted; the other fields then mean nothing
+    uint32_t error;            // kErrRange | kErrUnsorted, with either of which the other fields mean nothing; kLongStrip
     uint32_t first, end;       // first column, last column + 1; of a panel without entries ~0 and 0
 };
 static_assert(sizeof(PanelCensus) == 48, "written as twelve words");
@@ -148,6 +150,13 @@ __global__ __launch_bounds__(kThreads) void copy_words(const uint32_t *__restric
     for (uint64_t i = global_id(); i < n; i += uint64_t(gridDim.x) * kThreads) dst[i] = src[i];
 }
 
+// table[i] by a vector load: the table may stand in host memory, 1.5 us away, and what waits for a scalar load waits for LDS as well.
+__device__ __forceinline__ uint32_t table_word(const uint32_t *__restrict__ table, uint32_t i)
+{
+    asm volatile("" : "+v"(i));
+    return table[i];
+}
+
 __device__ __forceinline__ uint32_t row_in_panel(const uint32_t *rp, uint32_t e)
 {
     uint32_t lo = 0, hi = 15u;                               // the row r with rp[r] <= e < rp[r+1]
@@ -231,6 +240,27 @@ template <uint32_t CAP> __device__ __forceinline__ uint32_t panel_rows(PanelLds<
     bad = __syncthreads_or(bad);
     start = s;
     return bad ? ~0u : l.rp[16];
+}
+
+// The same for one strip: the other rows are empty.
+template <uint32_t CAP> __device__ __forceinline__ uint32_t strip_rows(PanelLds<CAP> &l, const uint32_t *__restrict__ rowPtr, uint32_t p, uint32_t strip, uint32_t &start)
+{
+    const uint32_t t = threadIdx.x, s = rowPtr[uint64_t(p) * 16u + 4u * strip];
+    if (t < 17u) l.rp[t] = rowPtr[uint64_t(p) * 16u + min(max(t, 4u * strip), 4u * strip + 4u)] - s;
+    if (t == 0u) { l.lo = ~0u; l.hi = 0u; }
+    __syncthreads();
+    start = s;
+    return l.rp[16];
+}
+
+// How many of the entries [begin, end) are not zero; every thread of the work-group has the answer.
+template <uint32_t CAP> __device__ __forceinline__ uint32_t values_in(PanelLds<CAP> &l, const float *__restrict__ vals, uint32_t begin, uint32_t end)
+{
+    uint32_t own = 0, total;
+#pragma unroll 8
+    for (uint32_t i = begin + threadIdx.x; i < end; i += PanelLds<CAP>::kBlock) own += vals[i] != 0.0f ? 1u : 0u;
+    block_exclusive(l, own, total);
+    return total;
 }
 
 template <uint32_t CAP> __device__ __forceinline__ bool panel_fits(const PanelLds<CAP> &l, uint32_t max_span) { return l.hi - l.lo < max_span; }
@@ -456,6 +486,7 @@ __global__ __launch_bounds__(kThreads, 7) void panel_census(const uint32_t *__re
             add_pairs(strip);
         } else {
             window();
+            if (t < 4u && at_row(t, 4) - at_row(t, 0) > kPanelList) atomicOr(&res.error, kLongStrip << t);
             if (n <= kBigEntries) {
                 // (so many entries that their strip's bitmap is soon read through)
 #pragma unroll 1
@@ -519,13 +550,13 @@ __global__ __launch_bounds__(panel_threads(CAP)) void panel_bricks(const uint32_
     const uint32_t p = list_of ? list_of[blockIdx.x] : blockIdx.y * gridDim.x + blockIdx.x, t = threadIdx.x;
     if (p >= P) return;
     if (!list_of && p == 0u && t < 64u) tile_vals[uint64_t(nnz) + t] = 0.0f;
-    const uint32_t block0 = brp[p];
     uint32_t start;
     const uint32_t n = panel_rows(l, rowPtr, p, P, nnz, start);
     if (n == 0u || n > CAP) return;
     PanelEntries<CAP> e;
     load_panel(l, e, window, cols, vals, start, n, max_span);
     if (!panel_fits(l, max_span)) return;
+    const uint32_t block_word = table_word(brp, p);
     const uint32_t active = number_columns(l, e, window, n);
     uint16_t *first = reinterpret_cast<uint16_t *>(window);   // position of every active column's first entry, and n behind the last
     {
@@ -546,7 +577,7 @@ __global__ __launch_bounds__(panel_threads(CAP)) void panel_bricks(const uint32_
         if (t == 0u && active == CAP) first[CAP] = uint16_t(n);
     }
     __syncthreads();
-    const uint32_t slots = ((active + 15u) / 16u) * 16u;
+    const uint32_t slots = ((active + 15u) / 16u) * 16u, block0 = __builtin_amdgcn_readfirstlane(block_word);
     for (uint32_t a = t; a < slots; a += PanelLds<CAP>::kBlock) {          // sixteen lanes are the sixteen columns of one block
         const uint32_t b = first[min(a, active)];
         const uint32_t mask = a < active ? l.rows[a] & 0xffffu : 0u;
@@ -572,25 +603,40 @@ __global__ __launch_bounds__(panel_threads(CAP)) void panel_bricks(const uint32_
 // (row group, column) pair; the running number of stored values over the pairs of the panel is at once the place of
 // their values and, at a group's first pair, the record's index word.  Block 0 writes the zeros behind the values.
 // Dynamic LDS: the window, then (in its place) the list places of every column, four 16-bit numbers each.
+// The first `listed` work-groups of STRIPS take a strip each of panels of more than CAP entries (4 panel + strip, kHasZeros), which have no
+// launch of their own: three launches one after the other took 27 + 25 + 18 us (big_quads, panels of up to 1 024, of up to 4 096 entries) on the
+// graph above, now big_quads runs beside this one on a second stream, 36 us from first to last; format to product 346 -> 322.  Without
+// STRIPS `listed` says that `list` names the panels.
+constexpr uint32_t kHasZeros = 1u << 31;
 template <bool STRIPS, uint32_t CAP>
 __global__ __launch_bounds__(panel_threads(CAP)) void panel_quads(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols,
-                                                        const float *__restrict__ vals, uint32_t P, uint32_t nnz, uint32_t max_span, const uint32_t *__restrict__ list_of,
+                                                        const float *__restrict__ vals, uint32_t P, uint32_t nnz, uint32_t max_span,
+                                                        const uint32_t *__restrict__ list_of, uint32_t listed,
                                                         const uint32_t *__restrict__ groups, const uint32_t *__restrict__ valBase, uint32_t stored,
                                                         uint32_t *__restrict__ recs, float *__restrict__ packed)
 {
     extern __shared__ uint32_t window[];
     __shared__ PanelLds<CAP> l;
     __shared__ uint16_t list[CAP], place[CAP];    // pair -> active column, and -> its first value from the panel's first
-    const uint32_t p = list_of ? list_of[blockIdx.x] : blockIdx.y * gridDim.x + blockIdx.x, t = threadIdx.x;
-    if (p >= P) return;
-    if (!list_of && p == 0u && t < 64u) packed[uint64_t(stored) + t] = 0.0f;
-    const uint32_t group0 = groups[uint64_t(p) * (STRIPS ? 4u : 1u)], value0 = valBase[p];
+    const uint32_t id = blockIdx.y * gridDim.x + blockIdx.x, t = threadIdx.x;
+    const bool one_strip = STRIPS && id < listed;
+    const uint32_t word = id < listed ? list_of[id] : 0u, strip = one_strip ? word & 3u : 0u;
+    const uint32_t p = one_strip ? (word & ~kHasZeros) >> 2 : STRIPS ? id - listed : listed ? word : id;
+    if (p >= P || (!STRIPS && listed && id >= listed)) return;
+    if (p == 0u && t < 64u && (STRIPS ? !one_strip : !listed)) packed[uint64_t(stored) + t] = 0.0f;
     uint32_t start;
-    const uint32_t n = panel_rows(l, rowPtr, p, P, nnz, start);
+    const uint32_t n = one_strip ? strip_rows(l, rowPtr, p, strip, start) : panel_rows(l, rowPtr, p, P, nnz, start);
     if (n == 0u || n > CAP) return;
     PanelEntries<CAP> e;
     load_panel(l, e, window, cols, vals, start, n, max_span);
     if (!panel_fits(l, max_span)) return;
+    const uint32_t group_word = table_word(groups, p * (STRIPS ? 4u : 1u) + strip), value_word = table_word(valBase, p);
+    // values of the strips in front
+    uint32_t front = 0;
+    if (one_strip && strip) {
+        const uint32_t panel = rowPtr[uint64_t(p) * 16u];
+        front = word & kHasZeros ? values_in(l, vals, panel, start) : start - panel;
+    }
     const uint32_t active = number_columns(l, e, window, n);
     Two *before = reinterpret_cast<Two *>(window);            // pairs in front of an active column's, in each strip's list
     Two lens;
@@ -630,7 +676,7 @@ __global__ __launch_bounds__(panel_threads(CAP)) void panel_quads(const uint32_t
         group_before[s] = total;
         total = STRIPS ? total + (len[s] + 15u) / 16u : max(total, (len[s] + 3u) / 4u);
     }
-    const uint32_t slots = total * 16u;
+    const uint32_t slots = total * 16u, group0 = __builtin_amdgcn_readfirstlane(group_word), value0 = __builtin_amdgcn_readfirstlane(value_word + front);
     uint32_t base = 0;
     for (uint32_t x0 = 0; x0 < slots; x0 += PanelLds<CAP>::kBlock) {
         const uint32_t x = x0 + t, g = x >> 4, pair = x & 15u;
@@ -669,7 +715,7 @@ __global__ __launch_bounds__(panel_threads(CAP)) void panel_quads(const uint32_t
 }
 
 // ------------------------------------------------------------------------------------------------
-// Panels of more than kPanelCap entries (the hub rows of a graph) whose window the bitmap takes: a work-group of sixteen wavefronts
+// Strips of more than kPanelList entries (the hub rows of a graph) whose panel's window the bitmap takes: a work-group of sixteen wavefronts
 // walks the entries of a strip instead of holding them, for the strip lists.  LDS holds the bitmap, its counts and the
 // rows of every active column, and the rest follows from prefix sums over the columns, a thread a run of them.
 // The entry-parallel kernels below need sixteen binary searches an entry, two scans and a launch for each step: R-MAT graph of 65 536
@@ -697,7 +743,7 @@ __device__ __forceinline__ uint32_t big_number(const uint32_t *window, const uin
     return count[c >> 5] + uint32_t(__popc(window[c >> 5] & ((1u << (c & 31u)) - 1u)));
 }
 
-// Strip lists of the listed panels (panel_quads<true> defines them), a work-group a strip: its entries are one piece of the arrays, its
+// The listed strips of more than kPanelList entries (panel_quads<true> defines the lists), a work-group each: a strip's entries are one piece of the arrays, its
 // active columns are its pairs.  row_words: a byte a column, the rows that hold it and those whose entry is not zero; step_words: three
 // words for every 64 columns.  (One work-group for all four strips of a panel: 81 us against 34.)
 // A wavefront takes 64 columns of the list at a time: where their entries stand in each row, and where their values go, is the sum of what
@@ -714,7 +760,7 @@ __global__ __launch_bounds__(kBigThreads) void big_quads(const uint32_t *__restr
     __shared__ uint32_t lo_hi[2], front;      // front: values stored for the strips in front of this one
     uint16_t *count = reinterpret_cast<uint16_t *>(window + window_words);
     uint32_t *rows = window + big_window_words(window_words), *steps = rows + row_words;
-    const uint32_t p = list[blockIdx.x / 4u], s = blockIdx.x % 4u, t = threadIdx.x, lane = t & 63u;
+    const uint32_t word = list[blockIdx.x], p = (word & ~kHasZeros) >> 2, s = word & 3u, t = threadIdx.x, lane = t & 63u;
     const uint32_t group0 = groups[uint64_t(p) * 4u + s], num_groups = groups[uint64_t(p) * 4u + s + 1u] - group0;
     if (num_groups == 0u) return;
     uint32_t rp[5];                           // the strip's rows
@@ -724,14 +770,14 @@ __global__ __launch_bounds__(kBigThreads) void big_quads(const uint32_t *__restr
     uint32_t *const strip_recs = recs + uint64_t(group0) * CUTE_QUAD_RECORD_WORDS;
     for (uint32_t w = t; w < window_words; w += kBigThreads) window[w] = 0u;
     for (uint32_t w = t; w < row_words; w += kBigThreads) rows[w] = 0u;
-    if (t == 0u) { lo_hi[0] = ~0u; lo_hi[1] = 0u; front = 0u; }
+    if (t == 0u) { lo_hi[0] = ~0u; lo_hi[1] = 0u; front = word & kHasZeros ? 0u : start - panel; }
     __syncthreads();
     if (t < 4u && rowPtr[uint64_t(p) * 16u + 4u * s + t + 1u] > rowPtr[uint64_t(p) * 16u + 4u * s + t]) {
         atomicMin(&lo_hi[0], cols[rowPtr[uint64_t(p) * 16u + 4u * s + t]]);
         atomicMax(&lo_hi[1], cols[rowPtr[uint64_t(p) * 16u + 4u * s + t + 1u] - 1u]);
     }
     uint32_t before = 0;
-    for (uint32_t i0 = panel; i0 < start; i0 += 16u * kBigThreads) {          // (sixteen loads on their way, whatever is left)
+    for (uint32_t i0 = word & kHasZeros ? panel : start; i0 < start; i0 += 16u * kBigThreads) {          // (sixteen loads on their way, whatever is left)
         float v[16];
 #pragma unroll
         for (uint32_t k = 0; k < 16u; ++k) {

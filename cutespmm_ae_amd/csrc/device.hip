@@ -235,6 +235,7 @@ struct cute_hrpb_dev {
     uint4 *dSlices = nullptr;
     uint2 *dWindowSlots = nullptr, *dWindowTiles = nullptr;
     cute_dev::f32x4 *dWindowVals = nullptr;
+    std::vector<uint32_t> longStrips;   // 4 panel + strip of every strip of more than kPanelList entries, ascending
     std::vector<uint32_t> panelStored;  // entries of each panel that are not zero (what the quad lists store)
 };
 
@@ -638,6 +639,38 @@ void drop_idle_pinned_memory()
     for (const auto &b : idle) (void)hipHostFree(b.first);
 }
 
+// A stream beside the default one for set-up kernels that need nothing from those on the default stream: one per device and process, non-blocking
+// (what its kernels read is complete when they are launched), at the default priority.  Whoever has launched on it waits for it before it returns.
+class SideStream {
+    hipStream_t used_ = nullptr;
+
+public:
+    SideStream() = default;
+    SideStream(const SideStream &) = delete;
+    SideStream &operator=(const SideStream &) = delete;
+    ~SideStream() { (void)wait(); }
+    // the default stream where there is none
+    hipStream_t get()
+    {
+        static std::mutex lock;
+        static hipStream_t streams[kMaxDevices];
+        int dev = -1;
+        if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return nullptr;
+        std::lock_guard<std::mutex> g(lock);
+        if (!streams[dev] && hipStreamCreateWithFlags(&streams[dev], hipStreamNonBlocking) != hipSuccess) {
+            (void)hipGetLastError();
+            streams[dev] = nullptr;
+        }
+        return used_ = streams[dev];
+    }
+    int wait()
+    {
+        const hipError_t e = used_ ? hipStreamSynchronize(used_) : hipSuccess;
+        used_ = nullptr;
+        return e == hipSuccess ? int(CUTE_OK) : hip_fail(e, "waiting for the side stream", __LINE__);
+    }
+};
+
 inline dim3 panel_grid(uint32_t n) { return dim3(std::min(n, cute_build::kPanelRow), (n + cute_build::kPanelRow - 1u) / cute_build::kPanelRow); }
 inline dim3 grid_of(uint64_t n) { return dim3(uint32_t(std::max<uint64_t>((n + cute_build::kThreads - 1) / cute_build::kThreads, 1))); }
 // for kernels that walk their range with a stride
@@ -648,7 +681,8 @@ int check_launch(const char *what);
 #define CUTE_BUILD(kernel, grid, ...) CUTE_BUILD_LDS(kernel, grid, 0, __VA_ARGS__)
 #define CUTE_BUILD_LDS(kernel, grid, lds, ...) hipLaunchKernelGGL(kernel, grid, dim3(cute_build::kThreads), lds, nullptr, __VA_ARGS__)
 // a panel kernel of the given capacity over `count` panels: all of them, or a list
-#define CUTE_PANELS(kernel, CAP, count, lds, ...) hipLaunchKernelGGL(kernel, panel_grid(count), dim3(cute_build::panel_threads(CAP)), lds, nullptr, __VA_ARGS__)
+#define CUTE_PANELS(kernel, CAP, count, lds, stream, ...) \
+    hipLaunchKernelGGL(kernel, panel_grid(count), dim3(cute_build::panel_threads(CAP)), lds, stream, __VA_ARGS__)
 
 // The widest column window the panel kernels take on this matrix, and the LDS its bitmap and running counts need.
 inline uint32_t max_span(const cute_hrpb_dev *d) { return std::min(d->K, cute_build::kPanelSpan); }
@@ -716,18 +750,38 @@ void list_large_panels(const cute_hrpb_dev *d, LargeWork &w)
 constexpr uint32_t kBigWindow = cute_build::big_window_words(cute_build::panel_window_words(cute_build::kPanelSpan));
 static_assert((kBigWindow + cute_build::kBigEntries / 4u + cute_build::kBigEntries / 64u * 3u) * 4u + 1024u <= 160u << 10, "big_quads");
 
-// The LDS words big_quads wants for the rows of the columns of every large panel's strips (the census has counted them), a byte a column,
-// and for its steps of 64 columns; 0: there are panels that it does not take, and then it takes none.  One panel beyond kBigEntries
-// or kPanelSpan sends all large panels of the matrix to the entry-parallel path.
-uint32_t big_quad_rows(const cute_hrpb_dev *d, const LargeWork &w, uint32_t &steps)
+// Does big_quads take every large panel?  One panel beyond kBigEntries or kPanelSpan sends all large panels of the matrix to the entry-parallel path.
+bool big_takes_all(const cute_hrpb_dev *d, const LargeWork &w)
 {
-    uint32_t most = 0;
-    for (uint32_t p : w.panel) {
-        if (d->panelNnz[p] > cute_build::kBigEntries || d->panelSpan[p] > max_span(d)) return 0;
-        for (uint32_t s = 0; s < 4u; ++s) most = std::max(most, d->stripPairs[4u * p + s]);
+    for (uint32_t p : w.panel)
+        if (d->panelNnz[p] > cute_build::kBigEntries || d->panelSpan[p] > max_span(d)) return false;
+    return true;
+}
+
+// The strips that panel_quads<true> takes beside whole panels (of up to kPanelList entries) and the longer ones, for big_quads: those of
+// every panel of more than kPanelList entries, but of large panels only where big_quads takes them all.
+struct StripLists {
+    std::vector<uint32_t> strips, big;        // 4 panel + strip, cute_build::kHasZeros where the panel has entries of value zero
+    uint32_t bigRows = 0, bigSteps = 0;       // LDS words of big_quads: a byte a column of the longest strip, and its steps of 64 columns
+};
+
+StripLists list_strips(const cute_hrpb_dev *d, bool with_large)
+{
+    StripLists l;
+    auto next = d->longStrips.begin();
+    for (uint32_t p = 0; d->longestPanel > cute_build::kPanelList && p < d->P; ++p) {
+        if (d->panelNnz[p] <= cute_build::kPanelList || (!with_large && panel_is_large(d, p))) continue;
+        const uint32_t zeros = d->panelStored[p] != d->panelNnz[p] ? cute_build::kHasZeros : 0u;
+        for (uint32_t u = 4u * p; u < 4u * p + 4u; ++u) {
+            if (!d->stripPairs[u]) continue;
+            while (next != d->longStrips.end() && *next < u) ++next;
+            if (next == d->longStrips.end() || *next != u) { l.strips.push_back(u | zeros); continue; }
+            l.big.push_back(u | zeros);
+            l.bigRows = std::max(l.bigRows, (d->stripPairs[u] + 3u) / 4u);
+            l.bigSteps = std::max(l.bigSteps, (d->stripPairs[u] + 63u) / 64u * 3u);
+        }
     }
-    steps = (most + 63u) / 64u * 3u;
-    return (most + 3u) / 4u;
+    return l;
 }
 
 // Numbers the entries of the large panels.  With `out` given also counts for the planner, into the panels' census records.
@@ -764,6 +818,12 @@ int number_large_panels(const cute_hrpb_dev *d, LargeWork &w, cute_build::PanelC
     return rc == CUTE_OK ? pin.wait() : rc;
 }
 
+// Up to this many panels the layout builders read their tables where the host wrote them: no copy_words launch in front of them (4 us and the
+// gap behind it), for a read of 1.5 us a work-group that waits for nothing until the panel's columns are numbered.  Format to product, copied / in
+// place: 9-point stencils of 64 x 64 points 77.6 / 75.7, 300 x 300 (5 625 panels) 217 / 215, 500 x 500 (15 625 panels, whose reads
+// add up) 486 / 492 us.  Nothing stands between the launches then, and those for longer panels go to the side stream.
+constexpr uint32_t kTablesInPlace = 8192;
+
 // Brick tiles from the device CSR copy: the arrays cute_hrpb_retile makes on the host, word for word.
 int build_bricks_on_device(cute_hrpb_dev *d, LargeWork &w)
 {
@@ -781,7 +841,9 @@ int build_bricks_on_device(cute_hrpb_dev *d, LargeWork &w)
     rc = mem.alloc(lay.bytes);
     if (rc == CUTE_OK) rc = pin.alloc(tab.bytes);
     if (rc != CUTE_OK) return rc;
-    auto table = [&](uint64_t o) { return Layout::at<const uint32_t>(mem.p, oTab + o); };
+    const bool in_place = !count && d->P <= kTablesInPlace;
+    auto table = [&](uint64_t o) { return in_place ? pin.as<const uint32_t>(o) : Layout::at<const uint32_t>(mem.p, oTab + o); };
+    SideStream side;
     uint32_t *hdr = Layout::at<uint32_t>(mem.p, oHdr);
     float *vals = Layout::at<float>(mem.p, oVals);
     std::memcpy(pin.p, d->brp.data(), d->brp.size() * 4u);
@@ -795,12 +857,13 @@ int build_bricks_on_device(cute_hrpb_dev *d, LargeWork &w)
         cols[k] = d->panelCols[p];
     }
     pin.pending = true;
-    CUTE_BUILD(cute_build::copy_words, grid_capped(tab.bytes / 4u), pin.as<const uint32_t>(), Layout::at<uint32_t>(mem.p, oTab), tab.bytes / 4u);
-    CUTE_PANELS(cute_build::panel_bricks<cute_build::kPanelFirst>, cute_build::kPanelFirst, d->P, window_lds(d, (cute_build::kPanelFirst + 1u) * 2u),
+    if (!in_place)
+        CUTE_BUILD(cute_build::copy_words, grid_capped(tab.bytes / 4u), pin.as<const uint32_t>(), Layout::at<uint32_t>(mem.p, oTab), tab.bytes / 4u);
+    CUTE_PANELS(cute_build::panel_bricks<cute_build::kPanelFirst>, cute_build::kPanelFirst, d->P, window_lds(d, (cute_build::kPanelFirst + 1u) * 2u), nullptr,
                 d->dRowPtr, d->dCols, d->dCsrVals, d->P, d->nnz, max_span(d), kAllPanels, table(oBrp), hdr, vals);
     if (!medium.empty())
         CUTE_PANELS(cute_build::panel_bricks<cute_build::kPanelCap>, cute_build::kPanelCap, uint32_t(medium.size()),
-                    window_lds(d, (cute_build::kPanelCap + 1u) * 2u), d->dRowPtr, d->dCols, d->dCsrVals, d->P, d->nnz, max_span(d), table(oMedium),
+                    window_lds(d, (cute_build::kPanelCap + 1u) * 2u), in_place ? side.get() : nullptr, d->dRowPtr, d->dCols, d->dCsrVals, d->P, d->nnz, max_span(d), table(oMedium),
                     table(oBrp), hdr, vals);
     if (count) {
         const uint32_t blocks = prefix[count];
@@ -810,6 +873,7 @@ int build_bricks_on_device(cute_hrpb_dev *d, LargeWork &w)
     }
     rc = check_launch("brick tiles");
     if (rc == CUTE_OK) rc = pin.wait();
+    if (rc == CUTE_OK) rc = side.wait();
     if (rc != CUTE_OK) return rc;
     d->dHdr = hdr;
     d->dVals = vals;
@@ -825,29 +889,31 @@ int build_quads_on_device(cute_hrpb_dev *d, LargeWork &w)
     const uint64_t G = d->numGroups, stored = d->numQuadVals;
     const bool strips = d->quadRows == 4;
     list_large_panels(d, w);
-    uint32_t big_steps = 0;
-    const uint32_t big_rows = strips ? big_quad_rows(d, w, big_steps) : 0u;      // all large panels through big_quads, or none
-    int rc = big_rows ? int(CUTE_OK) : number_large_panels(d, w, nullptr);
+    const bool with_large = strips && big_takes_all(d, w);
+    const StripLists lists = strips ? list_strips(d, with_large) : StripLists();
+    int rc = with_large ? int(CUTE_OK) : number_large_panels(d, w, nullptr);
     if (rc != CUTE_OK) return rc;
-    const uint32_t count = big_rows ? 0u : uint32_t(w.panel.size()), per = strips ? 4u : 1u;
+    const uint32_t count = with_large ? 0u : uint32_t(w.panel.size()), per = strips ? 4u : 1u;
     Layout lay, tab;
     const uint64_t oGroup = tab.add(d->qgp.size(), 4), oBase = tab.add(uint64_t(d->P) + 1u, 4), oUnit = tab.add(count, 4),
                    oPrefix = tab.add(count + 1u, 4), oFirst = tab.add(uint64_t(count) * per, 4), oPairs = tab.add(uint64_t(count) * 4u, 4),
                    oLargeBase = tab.add(count, 4);
-    const std::vector<uint32_t> medium = panels_between(d, cute_build::kPanelList);
-    const uint64_t oMedium = tab.add(medium.size(), 4), oBig = tab.add(w.panel.size(), 4);
+    const std::vector<uint32_t> medium = strips ? lists.strips : panels_between(d, cute_build::kPanelList);
+    const uint64_t oMedium = tab.add(medium.size(), 4), oBig = tab.add(lists.big.size(), 4);
     const uint64_t oRecs = lay.add(G * CUTE_QUAD_RECORD_WORDS, 4), oVals = lay.add(stored + 64u, 4), oTab = lay.add(tab.bytes, 1);
     DevBuf mem, counts;
     PinnedBuf pin;
     rc = mem.alloc(lay.bytes);
     if (rc == CUTE_OK) rc = pin.alloc(tab.bytes);
     if (rc != CUTE_OK) return rc;
-    auto table = [&](uint64_t o) { return Layout::at<const uint32_t>(mem.p, oTab + o); };
+    const bool in_place = !count && d->P <= kTablesInPlace;
+    auto table = [&](uint64_t o) { return in_place ? pin.as<const uint32_t>(o) : Layout::at<const uint32_t>(mem.p, oTab + o); };
+    SideStream side;
     uint32_t *recs = Layout::at<uint32_t>(mem.p, oRecs);
     float *packed = Layout::at<float>(mem.p, oVals);
     std::memcpy(pin.as<char>(oGroup), d->qgp.data(), d->qgp.size() * 4u);
     if (!medium.empty()) std::memcpy(pin.as<char>(oMedium), medium.data(), medium.size() * 4u);
-    if (big_rows) std::memcpy(pin.as<char>(oBig), w.panel.data(), w.panel.size() * 4u);
+    if (!lists.big.empty()) std::memcpy(pin.as<char>(oBig), lists.big.data(), lists.big.size() * 4u);
     uint32_t *base = pin.as<uint32_t>(oBase), *unit = pin.as<uint32_t>(oUnit), *prefix = pin.as<uint32_t>(oPrefix), *first = pin.as<uint32_t>(oFirst),
              *pairs = pin.as<uint32_t>(oPairs), *large_base = pin.as<uint32_t>(oLargeBase);
     base[0] = 0;
@@ -865,14 +931,17 @@ int build_quads_on_device(cute_hrpb_dev *d, LargeWork &w)
     if (groups) rc = counts.alloc((uint64_t(groups) + scan_scratch_words(groups)) * 4u);
     if (rc != CUTE_OK) return rc;
     pin.pending = true;
-    CUTE_BUILD(cute_build::copy_words, grid_capped(tab.bytes / 4u), pin.as<const uint32_t>(), Layout::at<uint32_t>(mem.p, oTab), tab.bytes / 4u);
+    if (!in_place)
+        CUTE_BUILD(cute_build::copy_words, grid_capped(tab.bytes / 4u), pin.as<const uint32_t>(), Layout::at<uint32_t>(mem.p, oTab), tab.bytes / 4u);
     uint32_t *sums = counts.as<uint32_t>();
-#define CUTE_PANEL_QUADS(S, CAP, COUNT, LIST)                                                                                         \
-    CUTE_PANELS((cute_build::panel_quads<S, CAP>), CAP, COUNT, window_lds(d, CAP * 8u), d->dRowPtr, d->dCols, d->dCsrVals, d->P, d->nnz,  \
-                max_span(d), LIST, table(oGroup), table(oBase), uint32_t(stored), recs, packed)
+    const uint32_t listed = uint32_t(medium.size());
+#define CUTE_PANEL_QUADS(S, CAP, COUNT, LIST, LISTED, STREAM)                                                                         \
+    CUTE_PANELS((cute_build::panel_quads<S, CAP>), CAP, COUNT, window_lds(d, CAP * 8u), STREAM, d->dRowPtr, d->dCols, d->dCsrVals, d->P, d->nnz,  \
+                max_span(d), LIST, LISTED, table(oGroup), table(oBase), uint32_t(stored), recs, packed)
 #define CUTE_BUILD_QUADS(S)                                                                                                           \
-    CUTE_PANEL_QUADS(S, cute_build::kPanelList, d->P, kAllPanels);                                                                      \
-    if (!medium.empty()) CUTE_PANEL_QUADS(S, cute_build::kPanelCap, uint32_t(medium.size()), table(oMedium));                           \
+    CUTE_PANEL_QUADS(S, cute_build::kPanelList, (S) ? d->P + listed : d->P, (S) ? table(oMedium) : kAllPanels, (S) ? listed : 0u, nullptr); \
+    if constexpr (!(S))                                                                                                               \
+        if (listed) CUTE_PANEL_QUADS(S, cute_build::kPanelCap, listed, table(oMedium), listed, in_place ? side.get() : nullptr);        \
     if (count) {                                                                                                                      \
         CUTE_BUILD(cute_build::large_clear, grid_of(uint64_t(groups) * CUTE_QUAD_RECORD_WORDS), table(oUnit), table(oPrefix), count,    \
                    uint32_t(CUTE_QUAD_RECORD_WORDS), recs);                                                                           \
@@ -884,18 +953,19 @@ int build_quads_on_device(cute_hrpb_dev *d, LargeWork &w)
         CUTE_BUILD((cute_build::large_quads<S, true>), grid_of(w.L.total), w.L, d->dRowPtr, d->dCols, d->dCsrVals, w.posS, w.DS,        \
                    table(oFirst), recs, packed);                                                                                      \
     }
-    // (the panels that take longest go first)
-    if (big_rows) {
+    // (the strips that take longest go first)
+    if (!lists.big.empty()) {
         const uint32_t words = cute_build::panel_window_words(max_span(d));
-        hipLaunchKernelGGL(cute_build::big_quads, dim3(uint32_t(w.panel.size()) * 4u), dim3(cute_build::kBigThreads),
-                           (cute_build::big_window_words(words) + big_rows + big_steps) * 4u, nullptr, d->dRowPtr, d->dCols, d->dCsrVals, table(oBig), words,
-                           big_rows, table(oGroup), table(oBase), recs, packed);
+        hipLaunchKernelGGL(cute_build::big_quads, dim3(uint32_t(lists.big.size())), dim3(cute_build::kBigThreads),
+                           (cute_build::big_window_words(words) + lists.bigRows + lists.bigSteps) * 4u, in_place ? side.get() : nullptr, d->dRowPtr, d->dCols, d->dCsrVals,
+                           table(oBig), words, lists.bigRows, table(oGroup), table(oBase), recs, packed);
     }
     if (strips) { CUTE_BUILD_QUADS(true) } else { CUTE_BUILD_QUADS(false) }
 #undef CUTE_BUILD_QUADS
 #undef CUTE_PANEL_QUADS
     rc = check_launch("quad lists");
     if (rc == CUTE_OK) rc = pin.wait();
+    if (rc == CUTE_OK) rc = side.wait();
     if (rc != CUTE_OK) return rc;
     d->dQRecs = recs;
     d->dQVals = packed;
@@ -1111,7 +1181,11 @@ int finish_upload(cute_hrpb_dev *d, int quad_layout, const DeviceContext &c, con
             uint2 tile = make_uint2(~0u, 0u), &into = d->tileWindow[p / kTilePanels];
             for (const uint32_t last = std::min(P, p + kTilePanels); p < last; ++p) {
                 __builtin_prefetch(r + p + kTilePanels);
-                error |= r[p].error;
+                const uint32_t flags = r[p].error;
+                error |= flags & cute_build::kAnyError;
+                if (flags >= cute_build::kLongStrip)
+                    for (uint32_t s = 0; s < 4u; ++s)
+                        if (flags & (cute_build::kLongStrip << s)) d->longStrips.push_back(4u * p + s);
                 d->panelNnz[p] = r[p].nnz;
                 d->panelSpan[p] = r[p].span;
                 longest = std::max(longest, r[p].nnz);
@@ -1130,7 +1204,7 @@ int finish_upload(cute_hrpb_dev *d, int quad_layout, const DeviceContext &c, con
         if (!error && any_left) {
             rc = number_large_panels(d, large, pin.as<cute_build::PanelCensus>());
             if (rc != CUTE_OK) return rc;
-            for (uint32_t p : large.panel) error |= r[p].error;
+            for (uint32_t p : large.panel) error |= r[p].error & cute_build::kAnyError;
         }
         if (error & cute_build::kErrRange) return CUTE_ERR_RANGE;
         if (error & cute_build::kErrUnsorted) return CUTE_ERR_UNSORTED;

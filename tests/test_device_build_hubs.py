@@ -1,6 +1,6 @@
 """Panels of more than 4 096 entries: where none holds more than 49 152 or spans more columns than the bitmap takes, one work-group walks
 the entries of a panel for the census and of a strip for the strip lists; else all of them, and in any case the brick tiles and
-lockstep lists, take the entry-parallel path.  Both layouts must equal the host builders word for word."""
+lockstep lists, take the entry-parallel path.  Strips of panels of more than 1 024 go by their own length.  Both layouts must equal the host builders word for word."""
 import numpy as np
 import pytest
 
@@ -26,6 +26,25 @@ def test_long_panels(cs, torch_cuda, sizes, spans, K, quad_layout):
     got = _both_layouts(cs, torch_cuda, M, K, rp, cl, vl, quad_layout).layouts()
     _check_bricks(cs, got, M, K, rp, cl, vl)
     _check_quads(cs, got, M, rp, cl, vl)
+
+
+@pytest.mark.parametrize("zeros", [False, True])
+@pytest.mark.parametrize("strips", [(1023, 2, 0, 0), (0, 1024, 1, 0), (1, 1025, 0, 1024), (1024, 1024, 1024, 1024), (0, 0, 900, 125), (1025, 1, 1026, 1023), (1500, 40, 0, 3000)])
+def test_strips_of_panels_beyond_one_work_group(cs, torch_cuda, strips, zeros):
+    """Panels of more than 1 024 entries: a strip of up to as many is a work-group's beside the small panels, a longer one big_quads'."""
+    rng = np.random.default_rng(sum(strips))
+    K, rows = 8192, [np.sort(rng.choice(8192, 5, replace=False)) for _ in range(16)]
+    for n in strips:
+        a = n // 3
+        rows += [np.sort(rng.choice(K, k, replace=False)) for k in (a, 0, n - a - a // 2, a // 2)]
+    rows += rows[:16]
+    rp = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.uint32)
+    cl = np.concatenate(rows).astype(np.uint32)
+    vl = rng.standard_normal(cl.size).astype(np.float32)
+    if zeros:
+        vl[rng.random(cl.size) < 0.3] = 0.0
+    got = _both_layouts(cs, torch_cuda, 48, K, rp, cl, vl, 2).layouts()
+    _check_quads(cs, got, 48, rp, cl, vl)
 
 
 def test_rows_alone_and_products(cs, orc, torch_cuda):
