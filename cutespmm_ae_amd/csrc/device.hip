@@ -282,6 +282,17 @@ struct cute_spmm_plan {
 
 namespace {
 
+// Work items of a plan: every one is written before it is read, so making room for them writes nothing.
+template <class T> struct Unset : std::allocator<T> {
+    template <class U> struct rebind { using other = Unset<U>; };
+    template <class U, class... A> void construct(U *at, A &&...a)
+    {
+        if constexpr (sizeof...(A) == 0) ::new (static_cast<void *>(at)) U;
+        else ::new (static_cast<void *>(at)) U(std::forward<A>(a)...);
+    }
+};
+using WorkItems = std::vector<uint4, Unset<uint4>>;
+
 // Deals the MFMA work items to the SIMDs by length.  When a launch fits on the device at once, nothing balances
 // it afterwards: every wavefront is placed when the launch starts, and a SIMD that was handed three long panels
 // keeps the whole launch waiting.  Where the work-groups land is regular (observed with the hardware id
@@ -297,7 +308,7 @@ namespace {
 // SIMD of the first slab, and a class is as loaded as any of its positions: a heap holds the classes by load and first free
 // position, not the positions.  Nothing is dealt where even a perfect order would not gain the 3 %.  (The host threads take longer to wake than
 // this takes.  One heap of all positions: 400 us of the 510 that a new 9-point matrix of 300 x 300 points took from format to product, N = 64.)
-bool deal_chunks(std::vector<uint4> &chunks, uint32_t num_slabs, uint32_t cus_per_xcd, uint32_t waves_per_simd, bool force)
+bool deal_chunks(WorkItems &chunks, uint32_t num_slabs, uint32_t cus_per_xcd, uint32_t waves_per_simd, bool force)
 {
     constexpr uint32_t wpg = cute_dev::kWavesPerGroup, xcds = cute_dev::kNumXcd;
     if (cus_per_xcd == 0 || wpg != 4) return false;
@@ -357,7 +368,7 @@ bool deal_chunks(std::vector<uint4> &chunks, uint32_t num_slabs, uint32_t cus_pe
         bool operator<(const Class &o) const { return load != o.load ? load < o.load : pos < o.pos; }
     };
     std::vector<Class> heaps(size_t(simds) * xcds);
-    std::vector<uint4> dealt(chunks);
+    WorkItems dealt(count);
     std::fill(load.begin(), load.end(), 0);
     for (uint32_t x = 0; x < xcds; ++x) {
         const uint32_t b = begin_of(x), e = begin_of(x + 1u), n = e - b;
@@ -1058,28 +1069,29 @@ int ensure_window(cute_hrpb_dev *d, const WindowShape &w, uint32_t ring_rows)
 // be mostly padding (a few very long rows stretch the lists of their panel neighbours): then one list per strip.
 int finish_quad_census(cute_hrpb_dev *d, int quad_layout)
 {
-    const std::vector<uint32_t> &strip_pairs = d->stripPairs;
-    const uint32_t S = d->M / 4;
-    uint64_t pairs = 0, lock_groups = 0;
-    for (uint32_t p = 0; p < d->P; ++p) {
-        uint32_t longest = 0;
-        for (uint32_t l = 0; l < 4; ++l) { longest = std::max(longest, strip_pairs[4 * p + l]); pairs += strip_pairs[4 * p + l]; }
-        lock_groups += (longest + 3) / 4;
+    const uint32_t *const pairs_of = d->stripPairs.data(), P = d->P;
+    uint64_t pairs = 0, lock_groups = 0, strip_groups = 0;
+    for (uint32_t p = 0; p < P; ++p) {
+        const uint32_t a = pairs_of[4 * p], b = pairs_of[4 * p + 1], c = pairs_of[4 * p + 2], e = pairs_of[4 * p + 3];
+        pairs += uint64_t(a) + b + c + e;
+        lock_groups += (std::max(std::max(a, b), std::max(c, e)) + 3) / 4;
+        strip_groups += uint64_t((a + 15) / 16) + (b + 15) / 16 + (c + 15) / 16 + (e + 15) / 16;
     }
     if (quad_layout == 0) quad_layout = (lock_groups && double(pairs) < 0.6 * 16.0 * double(lock_groups)) ? 2 : 1;
-    d->quadRows = quad_layout == 2 ? 4u : CUTE_TM;
+    const bool strips = quad_layout == 2;
+    d->quadRows = strips ? 4u : CUTE_TM;
     d->quadPairs = pairs;
-    const uint32_t per_unit = d->quadRows / 4, U = S / per_unit;
-    d->qgp.assign(size_t(U) + 1, 0u);
-    uint64_t groups = 0;
-    for (uint32_t u = 0; u < U; ++u) {
-        uint32_t longest = 0;
-        for (uint32_t l = 0; l < per_unit; ++l) longest = std::max(longest, strip_pairs[u * per_unit + l]);
-        groups += per_unit == 4 ? (longest + 3) / 4 : (longest + 15) / 16;
-        if (groups > 0xffffffffull / 64) return CUTE_ERR_SHAPE;
-        d->qgp[u + 1] = uint32_t(groups);
+    d->numGroups = strips ? strip_groups : lock_groups;
+    if (d->numGroups > 0xffffffffull / 64) return CUTE_ERR_SHAPE;
+    d->qgp.resize((strips ? size_t(P) * 4u : size_t(P)) + 1);
+    uint32_t *const qgp = d->qgp.data(), groups = 0;
+    qgp[0] = 0;
+    for (uint32_t p = 0; p < P; ++p) {
+        const uint32_t *const of = pairs_of + 4 * size_t(p);
+        if (!strips) qgp[p + 1] = groups += (std::max(std::max(of[0], of[1]), std::max(of[2], of[3])) + 3) / 4;
+        else
+            for (uint32_t l = 0; l < 4u; ++l) qgp[4 * size_t(p) + l + 1] = groups += (of[l] + 15) / 16;
     }
-    d->numGroups = groups;
     return CUTE_OK;
 }
 
@@ -1496,11 +1508,14 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
 
     cute_spmm_plan *p = new cute_spmm_plan;
     p->d = d;
+    // (in locals: what is stored to a byte array could be a member of d)
+    const uint32_t P = d->P, *const brp = d->brp.data(), *const qgp = d->qgp.data(), *const panelCols = d->panelCols.data(), *const panelNnz = d->panelNnz.data(),
+                   *const panelMaxRow = d->panelMaxRow.data(), *const panelSpan = d->panelSpan.data();
     // classify panels
-    std::vector<uint8_t> to_rows(d->P, 0);
+    std::vector<uint8_t> to_rows(P, 0);
     // panels that go to the MFMA kernel for another reason than their reuse (below); the choice of the MFMA shape is
     // made on the panels that earned it
-    std::vector<uint8_t> joined(d->P, 0);
+    std::vector<uint8_t> joined(P, 0);
     // The row kernel gives a row N / VEC lanes; up to N = 128 several rows share a wavefront, which then takes as long
     // as its longest row.  A panel whose longest row is more than twice its mean row (and longer than two batches of
     // eight entries) keeps its wavefronts waiting for that one row, and the MFMA kernel, which walks the panel's
@@ -1518,19 +1533,19 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
     // Much of that comes from the columns an XCD owns: where the lists stay in row order (below 256 columns, off the grid of 64), graphs of 24
     // entries a row lose (131 072 nodes, N = 208 235 -> 261, N = 240 263 -> 292; 20 entries a row 208 -> 203, 12 142 -> 134).
     const bool default_bars = t.path == CUTE_PATH_AUTO && t.min_reuse <= 0.0f && t.max_row_nnz == 0;
-    auto scattered = [&](uint32_t q) { return uint64_t(d->panelSpan[q]) * std::min(N, 256u) * sizeof(float) > kScatteredBytes; };
+    auto scattered = [&](uint32_t q) { return uint64_t(panelSpan[q]) * std::min(N, 256u) * sizeof(float) > kScatteredBytes; };
     const bool graph_bars = default_bars && t.precision == CUTE_PREC_FP32 && N >= 128u && uint64_t(d->M) * N >= kGraphProduct &&
                             (N % 64u == 0 || N >= 256u || N % 4u != 0 || uint64_t(d->nnz) < 22ull * d->M);
     auto fetches_of = [&](uint32_t q) {
         // what the MFMA side would fetch for this panel: one B row per list slot of the quad
         // lists (pairs plus padding), which is at least one per active column
         const uint32_t lists = d->quadRows == 4 ? 4u : 1u;
-        return std::max(d->panelCols[q], (d->qgp[(q + 1) * lists] - d->qgp[q * lists]) * 16u);
+        return std::max(panelCols[q], (qgp[(q + 1) * lists] - qgp[q * lists]) * 16u);
     };
     uint64_t reused = 0;                          // entries of panels that go to the MFMA side by the usual bars: reuse, long or uneven rows
     uint32_t n_brick = 0, n_rows = 0, n_empty = 0;
-    for (uint32_t q = 0; q < d->P; ++q) {
-        const uint32_t nblk = d->brp[q + 1] - d->brp[q];
+    for (uint32_t q = 0; q < P; ++q) {
+        const uint32_t nblk = brp[q + 1] - brp[q];
         bool rows;
         if (nblk == 0) { rows = true; n_empty++; }
         else if (t.path == CUTE_PATH_BRICK) rows = false;
@@ -1542,11 +1557,11 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
             const uint32_t fetches = fetches_of(q);
             const bool graph = graph_bars && scattered(q);
             const float bar = graph ? kGraphReuse
-                              : (wide_and_large && uint64_t(d->panelSpan[q]) * N * sizeof(float) > kWideWindowBytes) ? kWideReuse : reuse_bar;
-            rows = float(d->panelNnz[q]) < bar * float(fetches) && d->panelMaxRow[q] <= (graph ? kGraphMaxRow : max_row_for_rows);
-            const bool uneven = rows_share_a_wavefront && d->panelMaxRow[q] > kUnevenRowFloor &&
-                                uint64_t(d->panelMaxRow[q]) * CUTE_TM > uint64_t(kUnevenRowRatio) * d->panelNnz[q];
-            if (uneven || d->panelMaxRow[q] > max_row_for_rows || float(d->panelNnz[q]) >= reuse_bar * float(fetches)) reused += d->panelNnz[q];
+                              : (wide_and_large && uint64_t(panelSpan[q]) * N * sizeof(float) > kWideWindowBytes) ? kWideReuse : reuse_bar;
+            rows = float(panelNnz[q]) < bar * float(fetches) && panelMaxRow[q] <= (graph ? kGraphMaxRow : max_row_for_rows);
+            const bool uneven = rows_share_a_wavefront && panelMaxRow[q] > kUnevenRowFloor &&
+                                uint64_t(panelMaxRow[q]) * CUTE_TM > uint64_t(kUnevenRowRatio) * panelNnz[q];
+            if (uneven || panelMaxRow[q] > max_row_for_rows || float(panelNnz[q]) >= reuse_bar * float(fetches)) reused += panelNnz[q];
             if (rows && uneven && !graph) {
                 rows = false;
                 joined[q] = 1;
@@ -1594,10 +1609,10 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
     // 32-column lists 80.6, the row kernel by columns 73.5).
     if (default_bars && t.precision == CUTE_PREC_FP32 && reused * 10u < uint64_t(d->nnz) &&
         uint64_t(d->M) * ((N + 255u) / 256u) >= 4ull * uint64_t(c.num_cus) * 32u) {
-        auto concerned = [&](uint32_t q) { return d->brp[q + 1] != d->brp[q] && d->panelMaxRow[q] <= max_row_for_rows && scattered(q); };
+        auto concerned = [&](uint32_t q) { return brp[q + 1] != brp[q] && panelMaxRow[q] <= max_row_for_rows && scattered(q); };
         uint64_t windows = 0, entries = 0, panels = 0;
-        for (uint32_t q = 0; q < d->P; ++q)
-            if (concerned(q)) { windows += d->panelSpan[q]; entries += d->panelNnz[q]; ++panels; }
+        for (uint32_t q = 0; q < P; ++q)
+            if (concerned(q)) { windows += panelSpan[q]; entries += panelNnz[q]; ++panels; }
         if (panels) {
             const uint64_t window = windows / panels, mean_row = entries / (panels * CUTE_TM);
             // 32-column lists where a 64-column slab of the window outgrows the L2 by more than they do; us 64 / 32 columns:
@@ -1609,9 +1624,9 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
             const bool lists_ahead = on_grid ? (wide || (narrow(window, mean_row) == 0 && (mean_row >= 16u || N >= 256u)))
                                              : (narrow(window, mean_row) == 0 && N >= 256u &&
                                                 ((mean_row >= 16u && window <= 65536u) || short_last_slab(window, mean_row)));
-            for (uint32_t q = 0; q < d->P; ++q) {
+            for (uint32_t q = 0; q < P; ++q) {
                 if (!concerned(q)) continue;
-                const uint8_t rows = !(lists_ahead && N >= 64u && float(d->panelNnz[q]) >= kWideReuse * float(fetches_of(q)));
+                const uint8_t rows = !(lists_ahead && N >= 64u && float(panelNnz[q]) >= kWideReuse * float(fetches_of(q)));
                 if (rows == to_rows[q]) continue;
                 to_rows[q] = rows;
                 joined[q] = 0;
@@ -1630,18 +1645,18 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
     if (t.path == CUTE_PATH_AUTO && n_brick && n_rows) {
         uint64_t nnz_mfma = 0;
         bool movable = true;
-        for (uint32_t q = 0; q < d->P; ++q)
+        for (uint32_t q = 0; q < P; ++q)
             if (!to_rows[q]) {
-                nnz_mfma += d->panelNnz[q];
-                movable = movable && d->panelMaxRow[q] <= max_row_for_rows;
+                nnz_mfma += panelNnz[q];
+                movable = movable && panelMaxRow[q] <= max_row_for_rows;
             }
         if (movable && nnz_mfma * 50u < uint64_t(d->nnz)) {
             std::fill(to_rows.begin(), to_rows.end(), uint8_t(1));
             n_rows += n_brick;
             n_brick = 0;
         } else if ((uint64_t(d->nnz) - nnz_mfma) * 50u < uint64_t(d->nnz)) {
-            for (uint32_t q = 0; q < d->P; ++q)
-                if (to_rows[q] && d->brp[q + 1] != d->brp[q]) { to_rows[q] = 0; joined[q] = 1; }   // (empty panels stay: the row kernel zeroes their rows)
+            for (uint32_t q = 0; q < P; ++q)
+                if (to_rows[q] && brp[q + 1] != brp[q]) { to_rows[q] = 0; joined[q] = 1; }   // (empty panels stay: the row kernel zeroes their rows)
             n_brick += n_rows;
             n_rows = 0;
         }
@@ -1692,12 +1707,12 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
         // matrices and on the reference's 43: about 8 list slots (pairs plus padding) per brick.
         const uint32_t lists = d->quadRows == 4 ? 4u : 1u;     // list units per panel
         uint64_t slots = 0, bricks = 0, blocks = 0, entries = 0;
-        for (uint32_t q = 0; q < d->P; ++q)
+        for (uint32_t q = 0; q < P; ++q)
             if (!to_rows[q] && !joined[q]) {
-                entries += d->panelNnz[q];
-                slots += uint64_t(d->qgp[(q + 1) * lists] - d->qgp[q * lists]) * 16u;
-                bricks += (d->panelCols[q] + 3u) / 4u;
-                blocks += d->brp[q + 1] - d->brp[q];
+                entries += panelNnz[q];
+                slots += uint64_t(qgp[(q + 1) * lists] - qgp[q * lists]) * 16u;
+                bricks += (panelCols[q] + 3u) / 4u;
+                blocks += brp[q + 1] - brp[q];
             }
         p->shape = choose_mfma_shape(slots, bricks, blocks, entries, uint64_t(d->K) + d->M, d->nnz, N, t.operand_residency, c.cache_bytes);
     }
@@ -1746,13 +1761,13 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
     {
         uint64_t scattered_nnz = 0, window[2] = {}, in[2] = {}, cols = 0;
         uint32_t row_panels = 0;
-        for (uint32_t q = 0; q < d->P; ++q) {
+        for (uint32_t q = 0; q < P; ++q) {
             const uint32_t side = to_rows[q] ? 1u : 0u;
-            if (scattered(q)) scattered_nnz += d->panelNnz[q];
-            window[side] += uint64_t(d->panelSpan[q]) * d->panelNnz[q];
-            in[side] += d->panelNnz[q];
-            if (side == 0) cols += d->panelCols[q];
-            else if (d->panelNnz[q]) ++row_panels;
+            if (scattered(q)) scattered_nnz += panelNnz[q];
+            window[side] += uint64_t(panelSpan[q]) * panelNnz[q];
+            in[side] += panelNnz[q];
+            if (side == 0) cols += panelCols[q];
+            else if (panelNnz[q]) ++row_panels;
         }
         if (scattered_nnz * 2u > uint64_t(d->nnz)) {
             const uint64_t mean_window[2] = {in[0] ? window[0] / in[0] : 0, in[1] ? window[1] / in[1] : 0};
@@ -1787,7 +1802,10 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
     // 24-bit row operand can address, built once more for the pipelined brick kernel, whose stores use
     // 64-bit offsets.
     uint32_t slab = 0, num_slabs = 0, upp_log = 0, slots = 0, n_pieces = 0;
-    std::vector<uint4> chunks, fixups;
+    WorkItems chunks;
+    std::vector<uint4> fixups;
+    uint64_t total_units = 0;          // of all work items, and of the longest
+    uint32_t longest_item = 0;
     for (int attempt = 0;; ++attempt) {
         slab = p->shape == 2 ? (p->halfLists ? 32u : 64u) : 16u * p->vec * p->ng;   // the quad kernel: one column per lane (or half of them)
         num_slabs = (N + slab - 1) / slab;
@@ -1800,17 +1818,18 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
         // outliers: a panel is split when it is more than twice as long as the per-item share
         // of the whole job (and at least 8 blocks), into pieces of about that share.
         // work units along a panel: 16-column blocks for the brick kernel, groups for the quad kernel
-        const std::vector<uint32_t> &unit = p->shape == 2 ? d->qgp : d->brp;
+        const uint32_t *const unit = p->shape == 2 ? qgp : brp;
         // units per panel (its logarithm): 4 when the quad lists are kept per 4-row strip
         upp_log = (p->shape == 2 && d->quadRows == 4) ? 2u : 0u;
-        const uint32_t num_units = d->P << upp_log;
+        const uint32_t num_units = P << upp_log;
         const uint32_t resident = uint32_t(c.num_cus) * 4u * 8u;   // 4 SIMDs x 8 wavefronts per CU
         slots = t.slots ? t.slots : resident;
         // A chunk of a cut panel carries the 1-based number of its partial tile; the pieces of one panel are
         // consecutive (panels ascend through the list), and one fixup entry per cut panel adds them up afterwards.
         chunks.clear();
         fixups.clear();
-        n_pieces = 0;
+        n_pieces = longest_item = 0;
+        total_units = 0;
         chunks.reserve((size_t(n_brick) << upp_log) + 64u);
         auto emit = [&](uint32_t s, uint32_t e, uint32_t pan, bool cut) {
             const uint32_t len = e - s, cap = t.max_chunk_blocks ? t.max_chunk_blocks : len, step = std::min(cap, len);
@@ -1823,19 +1842,24 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
                 }
                 chunks.push_back(make_uint4(cs, std::min(e, cs + step), pan, cut ? n_pieces : 0u));
             }
+            total_units += len;
+            longest_item = std::max(longest_item, step);
         };
         if (t.slots) {
-            const int64_t n = cute_partition(num_units, unit.data(), num_slabs, slots, nullptr, 0);
+            const int64_t n = cute_partition(num_units, unit, num_slabs, slots, nullptr, 0);
             if (n < 0) { delete p; return int(n); }
             std::vector<uint32_t> quads(uint64_t(n) * 4);
-            cute_partition(num_units, unit.data(), num_slabs, slots, quads.data(), uint64_t(n));
+            cute_partition(num_units, unit, num_slabs, slots, quads.data(), uint64_t(n));
             for (size_t i = 0; i + 3 < quads.size(); i += 4)
                 if (!to_rows[quads[i + 2] >> upp_log]) emit(quads[i], quads[i + 1], quads[i + 2], quads[i + 3] != 0);
-        } else {
+        } else if (n_brick) {
             uint64_t work = 0;
             uint64_t busy = 0;
-            for (uint32_t q = 0; q < num_units; ++q)
-                if (!to_rows[q >> upp_log] && unit[q + 1] != unit[q]) { work += unit[q + 1] - unit[q]; ++busy; }
+            for (uint32_t q = 0; q < P; ++q) {
+                if (to_rows[q]) continue;
+                work += unit[(q + 1) << upp_log] - unit[q << upp_log];
+                for (uint32_t u = q << upp_log; u < (q + 1) << upp_log; ++u) busy += unit[u + 1] != unit[u];
+            }
             const uint64_t mean = busy ? (work + busy - 1) / busy : 1;
             const uint64_t share = (work * num_slabs + resident - 1) / resident;
             // the mean only counts while it is short: a matrix whose few MFMA panels are all very long
@@ -1856,21 +1880,32 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
             const bool finer = attempt == 0 && (p->shape == 2 || N < 32u);
             const uint32_t limit = uint32_t(std::max<uint64_t>(2u * uint64_t(target), (finer ? (p->shape == 2 ? 4u : 0u) : 6u) * share));
             const uint32_t piece = limit > 2u * target ? uint32_t((finer ? 2u : 4u) * share) : target;
+            chunks.resize(std::max<size_t>(chunks.capacity(), 64u));
+            size_t at = 0;
             for (uint32_t q = 0; q < num_units; ++q) {
-                const uint32_t s = unit[q], e = unit[q + 1];
-                if (s == e || to_rows[q >> upp_log]) continue;
-                const uint32_t nblk = e - s;
-                if (nblk <= limit) {
-                    emit(s, e, q, false);
+                if (to_rows[q >> upp_log]) { q |= (1u << upp_log) - 1u; continue; }
+                const uint32_t s = unit[q], e = unit[q + 1], nblk = e - s;
+                if (nblk == 0) continue;
+                if (nblk <= limit && !t.max_chunk_blocks) {
+                    if (at == chunks.size()) chunks.resize(at + at / 2u);
+                    chunks[at++] = make_uint4(s, e, q, 0u);
+                    longest_item = std::max(longest_item, nblk);
+                    total_units += nblk;
                     continue;
                 }
-                const uint32_t pieces = (nblk + piece - 1) / piece;
-                const uint32_t step = (nblk + pieces - 1) / pieces;
-                for (uint32_t cs = s; cs < e; cs += step) emit(cs, std::min(e, cs + step), q, true);
+                chunks.resize(at);
+                if (nblk <= limit) emit(s, e, q, false);
+                else {
+                    const uint32_t pieces = (nblk + piece - 1) / piece, step = (nblk + pieces - 1) / pieces;
+                    for (uint32_t cs = s; cs < e; cs += step) emit(cs, std::min(e, cs + step), q, true);
+                }
+                at = chunks.size();
+                chunks.resize(std::max(chunks.capacity(), at + 64u));
             }
+            chunks.resize(at);
         }
         // a strip without pairs inside an MFMA-routed panel still has to be written (as zeros): an empty chunk
-        if (upp_log)
+        if (upp_log && n_brick)
             for (uint32_t q = 0; q < num_units; ++q)
                 if (unit[q] == unit[q + 1] && !to_rows[q >> upp_log]) chunks.push_back(make_uint4(unit[q], unit[q], q, 0u));
         const bool lean = p->shape == 2 || p->pipeline == 1;
@@ -1884,27 +1919,35 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
         p->pipeline = 2;
         p->bf16x3 = p->halfLists = false;
     }
-    std::vector<uint32_t> row_panels;              // panels of the row kernel
-    for (uint32_t q = 0; q < d->P; ++q)
-        if (to_rows[q]) row_panels.push_back(q);
+    uint32_t num_row_panels = 0;
+    for (uint32_t q = 0; q < P; ++q) num_row_panels += to_rows[q];
+    // Every row on the row kernel: no row list needed, which takes one dependent load out of each row's chain.
+    const bool every_row = num_row_panels == P;
+    std::vector<uint32_t> row_panels;              // panels of the row kernel, unless it has them all
+    if (!every_row && num_row_panels) {
+        row_panels.reserve(num_row_panels);
+        for (uint32_t q = 0; q < P; ++q)
+            if (to_rows[q]) row_panels.push_back(q);
+    }
 
     // Row-kernel blocks per XCD: contiguous ranges of rows (neighbouring rows share B rows, which then stay
     // in one L2), cut where the running work -- nonzeros plus a fixed cost per row -- passes each eighth.
     {
         const uint32_t items_per_block = 256u >> p->rows_logl;             // rows of one 256-thread block (per slab)
-        const uint64_t total_items = uint64_t(row_panels.size()) * CUTE_TM;
+        const uint64_t total_items = uint64_t(num_row_panels) * CUTE_TM;
         const uint32_t total_blocks = uint32_t((total_items + items_per_block - 1) / items_per_block);
         uint64_t total_work = 0;
-        for (uint32_t q = 0; q < d->P; ++q)
-            if (to_rows[q]) total_work += d->panelNnz[q] + 4u * CUTE_TM;
+        for (uint32_t q = 0; q < P; ++q) total_work += to_rows[q] ? panelNnz[q] + uint64_t(4u * CUTE_TM) : 0u;
         uint64_t work = 0, items = 0;
         uint32_t x = 1;
         p->rowRanges.first[0] = 0;
-        for (uint32_t q = 0; q < d->P && x < cute_dev::kNumXcd; ++q) {
+        auto share = [&] { return (total_work * x + cute_dev::kNumXcd - 1u) / cute_dev::kNumXcd; };      // where range x begins
+        uint64_t next = share();
+        for (uint32_t q = 0; q < P && num_row_panels && x < cute_dev::kNumXcd; ++q) {
             if (!to_rows[q]) continue;
-            work += d->panelNnz[q] + 4u * CUTE_TM;
+            work += panelNnz[q] + uint64_t(4u * CUTE_TM);
             items += uint64_t(CUTE_TM);
-            while (x < cute_dev::kNumXcd && work * cute_dev::kNumXcd >= total_work * x)
+            for (; x < cute_dev::kNumXcd && work >= next; next = share())
                 p->rowRanges.first[x++] = uint32_t(std::min<uint64_t>(total_blocks, (items + items_per_block - 1) / items_per_block));
         }
         while (x <= cute_dev::kNumXcd) p->rowRanges.first[x++] = total_blocks;
@@ -1933,51 +1976,51 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
     bool longest_first = t.chunk_order == 3 && !hub_rows;
     if (t.chunk_order == 0 && !chunks.empty() && !hub_rows) {
         const uint64_t resident = uint64_t(c.num_cus) * 4u * ((p->shape == 2 || p->ng == 1) ? 8u : 4u);
-        uint64_t total = 0;
-        uint32_t longest = 0;
-        for (const uint4 &ck : chunks) { total += ck.y - ck.x; longest = std::max(longest, ck.y - ck.x); }
-        const uint32_t groups = (uint32_t(chunks.size()) + cute_dev::kWavesPerGroup - 1) / cute_dev::kWavesPerGroup;
-        const size_t span = size_t((groups + cute_dev::kNumXcd - 1) / cute_dev::kNumXcd) * cute_dev::kWavesPerGroup;
-        uint64_t fullest = 0;
-        for (uint32_t x = 0; x < cute_dev::kNumXcd; ++x) {
-            uint64_t work = 0;
-            for (size_t i = std::min(chunks.size(), x * span); i < std::min(chunks.size(), (x + 1) * span); ++i) work += chunks[i].y - chunks[i].x + 2u;
-            fullest = std::max(fullest, work);
+        longest_first = uint64_t(chunks.size()) * num_slabs > resident;
+        if (longest_first && uint64_t(longest_item) * chunks.size() < 4u * total_units) {
+            const uint32_t groups = (uint32_t(chunks.size()) + cute_dev::kWavesPerGroup - 1) / cute_dev::kWavesPerGroup;
+            const size_t span = size_t((groups + cute_dev::kNumXcd - 1) / cute_dev::kNumXcd) * cute_dev::kWavesPerGroup;
+            uint64_t fullest = 0;
+            for (uint32_t x = 0; x < cute_dev::kNumXcd; ++x) {
+                uint64_t work = 0;
+                for (size_t i = std::min(chunks.size(), x * span); i < std::min(chunks.size(), (x + 1) * span); ++i) work += chunks[i].y - chunks[i].x + 2u;
+                fullest = std::max(fullest, work);
+            }
+            const uint64_t even = (total_units + 2u * chunks.size() + cute_dev::kNumXcd - 1) / cute_dev::kNumXcd;
+            longest_first = fullest * 10u > even * 11u;
         }
-        const uint64_t even = (total + 2u * chunks.size() + cute_dev::kNumXcd - 1) / cute_dev::kNumXcd;
-        longest_first = uint64_t(chunks.size()) * num_slabs > resident &&
-                        (uint64_t(longest) * chunks.size() >= 4u * total || fullest * 10u > even * 11u);
     }
     if (longest_first && !chunks.empty()) {
-        std::vector<uint4> sorted(chunks.size());
         size_t place[33] = {};                 // a counting sort by the power of two of the length, longest first, stable
         auto bucket = [](const uint4 &ck) { return size_t(__builtin_clz((ck.y - ck.x) | 1u)); };
         for (const uint4 &ck : chunks) ++place[bucket(ck) + 1];
         for (size_t k = 0; k < 32; ++k) place[k + 1] += place[k];
-        for (const uint4 &ck : chunks) sorted[place[bucket(ck)]++] = ck;
         // work-group g runs on XCD g % 8 and takes the list positions the kernels' XCD mapping gives it: XCD x walks
-        // the groups [x * per_xcd, (x + 1) * per_xcd).  Deal the sorted groups round-robin into those ranges.
+        // the groups [x * per_xcd, (x + 1) * per_xcd).  The sorted groups go round-robin into those ranges.
         const uint32_t wpg = cute_dev::kWavesPerGroup;
-        const uint32_t groups = (uint32_t(sorted.size()) + wpg - 1) / wpg;
+        const uint32_t groups = (uint32_t(chunks.size()) + wpg - 1) / wpg;
         const uint32_t per_xcd = (groups + cute_dev::kNumXcd - 1) / cute_dev::kNumXcd;
         uint32_t fill[cute_dev::kNumXcd] = {}, cap[cute_dev::kNumXcd];
         for (uint32_t x = 0; x < cute_dev::kNumXcd; ++x)
             cap[x] = uint32_t(std::min<uint64_t>(per_xcd, groups > x * per_xcd ? groups - x * per_xcd : 0));
         // the last group may be short: it must stay the last one of the list
-        const bool ragged = sorted.size() % wpg != 0;
+        const bool ragged = chunks.size() % wpg != 0;
         uint32_t last_xcd = 0;
         for (uint32_t x = 0; x < cute_dev::kNumXcd; ++x) if (cap[x]) last_xcd = x;
         if (ragged) cap[last_xcd]--;
+        std::vector<uint32_t> to(groups);      // where the sorted groups go
         for (uint32_t k = 0; k < groups - (ragged ? 1u : 0u); ++k) {
             uint32_t x = k % cute_dev::kNumXcd;
             while (fill[x] == cap[x]) x = (x + 1) % cute_dev::kNumXcd;
-            const size_t dst = (size_t(x) * per_xcd + fill[x]++) * wpg;
-            for (uint32_t w = 0; w < wpg; ++w) chunks[dst + w] = sorted[size_t(k) * wpg + w];
+            to[k] = x * per_xcd + fill[x]++;
         }
-        if (ragged) {
-            const size_t dst = (size_t(last_xcd) * per_xcd + cap[last_xcd]) * wpg, src = size_t(groups - 1) * wpg;
-            for (size_t w = 0; src + w < sorted.size(); ++w) chunks[dst + w] = sorted[src + w];
+        if (ragged) to[groups - 1u] = last_xcd * per_xcd + cap[last_xcd];
+        WorkItems dealt(chunks.size());
+        for (const uint4 &ck : chunks) {
+            const size_t i = place[bucket(ck)]++;
+            dealt[size_t(to[i / wpg]) * wpg + i % wpg] = ck;
         }
+        chunks.swap(dealt);
         p->info.dealtChunks = 2;
     } else
     if (t.chunk_order != 1 && !hub_rows && c.whole_chip && (p->shape == 2 || p->pipeline == 1) && !chunks.empty())
@@ -2001,8 +2044,6 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
     }
     // (the fast kernels address the partial tiles like C, with 32-bit byte offsets: checked where the chunks were made)
     p->partialBytes = uint64_t(n_pieces) * p->unitRows * N * sizeof(float);
-    // Every row on the row kernel: no row list needed, which takes one dependent load out of each row's chain.
-    const bool every_row = row_panels.size() == d->P;
     if (rc == CUTE_OK && (!chunks.empty() || !every_row)) {
         // The quad kernels get one 128-byte head per work item, its descriptor and a copy of its first group's record, so that
         // a wavefront can ask for its first B rows after one scalar fetch instead of two dependent ones; heads and row
@@ -2066,7 +2107,7 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
     }
     if (rc != CUTE_OK) { cute_spmm_plan_free(p); return rc; }
     p->numFixups = uint32_t(fixups.size());
-    p->numRows = uint32_t(row_panels.size()) * CUTE_TM;
+    p->numRows = num_row_panels * CUTE_TM;
     p->info.N = N;
     p->info.slabWidth = slab;
     p->info.numSlabs = num_slabs;
@@ -2084,7 +2125,7 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
     p->info.pipeline = uint32_t(p->pipeline);
     // one launch for a mixed plan: the quad kernel with any row shape of 4-float lanes, the rolling brick
     // kernel in the shapes the planner itself picks for N (forced column groups fall back to two launches)
-    const bool rows_fusable = !chunks.empty() && !row_panels.empty() && p->rows_vec == 4;
+    const bool rows_fusable = !chunks.empty() && num_row_panels && p->rows_vec == 4;
     const bool brick_default_shape = ng_for_mixed || p->ng == ((p->vec == 4 && N >= 128) ? 2 : 1);
     p->info.partialTileKiB = uint32_t((p->partialBytes + 1023u) / 1024u);
     p->info.fusedLaunch = (rows_fusable && !p->bf16x3 && !p->numHub && (p->shape == 2 || (p->pipeline == 1 && brick_default_shape))) ? 1u : 0u;
