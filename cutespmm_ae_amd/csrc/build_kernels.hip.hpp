@@ -363,22 +363,29 @@ constexpr uint32_t kCensusEach = 8;                          // entries a thread
 // edges a node 109 (68 now).
 constexpr uint32_t census_words(uint32_t max_span) { return panel_window_words(max_span) * (max_span <= 65536u ? 3u : 2u); }
 
+// Of panel_census_waves: a hash table of kWaveEntries entries for each wavefront where five bitmaps of the widest window need more.
+constexpr uint32_t kWaveEntries = 512, kWaveMean = 512, kWaveFront = 1024;      // up to kWaveFront panels: one in front each
+constexpr uint32_t wave_census_words(uint32_t max_span)
+{
+    const uint32_t maps = 5u * panel_window_words(max_span), table = 2u * kWaveEntries, all = census_words(max_span);
+    const uint32_t four = 4u * (maps < table ? maps : table);
+    return all > four ? (all + 3u) / 4u * 4u : four;
+}
+
 struct CsrCopy {
     uint32_t *rowPtr, *cols;
     float *vals;
 };
 
+// Panel p by a whole work-group; `res` and `lo_hi` are shared.  With COPY the work-group also copies the panel's row pointers and its share of
+// the entries, the same for every work-group (beside the rest its own entries would take registers).
 template <bool COPY>
-__global__ __launch_bounds__(kThreads, 7) void panel_census(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols,
-                                                         const float *__restrict__ vals, uint32_t P, uint32_t K, uint32_t nnz, uint32_t max_span,
-                                                         uint32_t lds_words, uint32_t share, CsrCopy to, PanelCensus *__restrict__ out)
+__device__ __forceinline__ void census_by_group(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols, const float *__restrict__ vals, uint32_t p,
+                                                uint32_t P, uint32_t K, uint32_t nnz, uint32_t max_span, uint32_t lds_words, uint32_t share, const CsrCopy &to,
+                                                uint32_t *bits, PanelCensus &res, uint32_t (&lo_hi)[2])
 {
-    extern __shared__ uint32_t bits[];
-    __shared__ PanelCensus res;
-    __shared__ uint32_t lo_hi[2];
     constexpr uint32_t kQuarter = kThreads / 4u;             // threads of a strip
-    const uint32_t p = blockIdx.y * gridDim.x + blockIdx.x, t = threadIdx.x;
-    if (p >= P) return;
+    const uint32_t t = threadIdx.x;
     // the row pointers are the work-group's (scalar registers); every panel checks its own, so together they check all of them before
     // anything is indexed through them
     uint32_t rp[17];
@@ -529,13 +536,172 @@ __global__ __launch_bounds__(kThreads, 7) void panel_census(const uint32_t *__re
         res.first = ~0u;
         res.error = bad ? uint32_t(kErrRange) : 0u;
     }
-    if (COPY) {                                              // the same share for every work-group (beside the rest its own entries would take registers)
+    if (COPY) {
         const uint64_t upto = min(uint64_t(nnz), (p + uint64_t(1)) * share);
 #pragma unroll 4
         for (uint64_t i = p * uint64_t(share) + t; i < upto; i += kThreads) { to.cols[i] = cols[i]; to.vals[i] = vals[i]; }
     }
     __syncthreads();
+}
+
+template <bool COPY>
+__global__ __launch_bounds__(kThreads, 7) void panel_census(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols,
+                                                         const float *__restrict__ vals, uint32_t P, uint32_t K, uint32_t nnz, uint32_t max_span,
+                                                         uint32_t lds_words, uint32_t share, CsrCopy to, PanelCensus *__restrict__ out)
+{
+    extern __shared__ uint32_t bits[];
+    __shared__ PanelCensus res;
+    __shared__ uint32_t lo_hi[2];
+    const uint32_t p = blockIdx.y * gridDim.x + blockIdx.x, t = threadIdx.x;
+    if (p >= P) return;
+    census_by_group<COPY>(rowPtr, cols, vals, p, P, K, nnz, max_span, lds_words, share, to, bits, res, lo_hi);
     if (t < 12u) reinterpret_cast<uint32_t *>(out + p)[t] = reinterpret_cast<const uint32_t *>(&res)[t];
+}
+
+// The same where panels are short (up to kWaveMean entries on average): a wavefront a panel and no barrier.  A panel of up to kWaveEntries entries
+// stays in the wavefront's registers; columns are told apart by five bitmaps of its window or, where these do not fit the wavefront's share of the
+// LDS, in a hash table of twice the entries (column from the window's start, plus one, and a bit a strip).  The first `front` work-groups take
+// the longer panels, one after the other, and mostly find none: of one panel each, or of the same fours of panels, which come from four quarters of
+// the matrix, `skew` panels apart, because a graph's long panels stand together at its beginning and at the quarters.  Those are copied by the
+// work-group that has them among its wavefronts' panels, not by the one that counts them.
+// A work-group a panel takes as long for these as for others, its chain of round trips: us, that way / this way, 131 072 rows of 12 at random columns
+// 54.4 / 24.6; 9-point stencils of 300 x 300 points 23.2 / 16.2, 128 x 128 6.8 / 5.5; 65 536 rows of 32 in a band 18.7 / 17.5; R-MAT graph of 65 536
+// nodes, bound by its longest panel, 39.1 / 40.3.  (Longer panels after the wavefronts' own: graph 49.  Up to 1 024 entries a wavefront: 16.1 for the
+// stencil of 300 x 300.)
+template <bool COPY>
+__global__ __launch_bounds__(kThreads, 6) void panel_census_waves(const uint32_t *__restrict__ rowPtr, const uint32_t *__restrict__ cols,
+                                                               const float *__restrict__ vals, uint32_t P, uint32_t K, uint32_t nnz, uint32_t max_span,
+                                                               uint32_t lds_words, uint32_t quarter, uint32_t skew, uint32_t front, CsrCopy to, PanelCensus *__restrict__ out)
+{
+    extern __shared__ uint32_t bits[];
+    __shared__ PanelCensus res;
+    __shared__ uint32_t lo_hi[2], starts_of[4][kWaveEntries / 32u];
+    const uint32_t id = blockIdx.y * gridDim.x + blockIdx.x, t = threadIdx.x, lane = t & 63u, wave = __builtin_amdgcn_readfirstlane(t / 64u);
+    if (id >= front + quarter) return;
+    const uint32_t group = id < front ? id : id - front;
+    auto panel_of = [&](uint32_t w) {
+        const uint32_t x = group + w * skew;
+        return w * quarter + (x >= quarter ? x - quarter : x);
+    };
+    if (id < front) {
+        const bool one = front != quarter;
+        uint32_t entries[4];
+#pragma unroll
+        for (uint32_t w = 0; w < 4u; ++w) {
+            const uint32_t q = one ? (w ? P : id) : panel_of(w), in = min(q, P - 1u);
+            entries[w] = q < P ? rowPtr[uint64_t(in) * 16u + 16u] - rowPtr[uint64_t(in) * 16u] : 0u;
+        }
+#pragma unroll 1
+        for (uint32_t w = 0; w < 4u; ++w) {
+            if ((w == 0u ? entries[0] : w == 1u ? entries[1] : w == 2u ? entries[2] : entries[3]) <= kWaveEntries) continue;
+            const uint32_t q = one ? id : panel_of(w);
+            census_by_group<false>(rowPtr, cols, vals, q, P, K, nnz, max_span, lds_words, 0u, to, bits, res, lo_hi);
+            if (t < 12u) reinterpret_cast<uint32_t *>(out + q)[t] = reinterpret_cast<const uint32_t *>(&res)[t];
+            __syncthreads();
+        }
+        return;
+    }
+    const uint32_t p = panel_of(wave);
+    if (p < P) {
+        const uint32_t own = rowPtr[uint64_t(p) * 16u + min(lane, 16u)];
+        const uint32_t next = uint32_t(__builtin_amdgcn_update_dpp(0, int(own), 0x130, 0xf, 0xf, true));      // wave_shl:1, the next lane's
+        auto row_start = [&](int r) { return uint32_t(__builtin_amdgcn_readlane(int(own), r)); };
+        const uint32_t start = row_start(0), stop = row_start(16);
+        if (COPY && lane < (p == P - 1u ? 17u : 16u)) to.rowPtr[uint64_t(p) * 16u + lane] = own;
+        const bool bad = stop > nnz || (p == P - 1u && stop != nnz) || (p == 0u && start != 0u) || __ballot(lane < 16u && own > next) != 0u;
+        const uint32_t n = bad ? 0u : stop - start;
+        if (stop - start <= kWaveEntries) {
+            uint32_t word = lane == 10u ? ~0u : lane == 9u && bad ? uint32_t(kErrRange) : 0u;       // the record, a word a lane
+            if (n) {
+                constexpr uint32_t kEach = kWaveEntries / 64u;
+                const uint32_t *const c = cols + start;
+                const float *const v = vals + start;
+                uint32_t col[kEach];
+                float val[kEach];
+#pragma unroll
+                for (uint32_t k = 0; k < kEach; ++k) {
+                    if (k * 64u >= n) break;
+                    col[k] = c[min(k * 64u + lane, n - 1u)];
+                    val[k] = v[min(k * 64u + lane, n - 1u)];
+                }
+                const uint32_t region = lds_words / 4u;
+                uint32_t *const mine = bits + wave * region, *const starts = starts_of[wave];
+                if (lane < kWaveEntries / 32u) starts[lane] = 0u;
+                __builtin_amdgcn_wave_barrier();
+                const uint32_t at_row = own - start;
+                if (lane < 16u && at_row < n) atomicOr(&starts[at_row >> 5], 1u << (at_row & 31u));
+                uint32_t lo = ~0u, hi = 0u;
+#pragma unroll
+                for (uint32_t k = 0; k < kEach; ++k) {
+                    if (k * 64u >= n) break;
+                    lo = min(lo, col[k]);
+                    hi = max(hi, col[k]);
+                    if (COPY && k * 64u + lane < n) { to.cols[uint64_t(start) + k * 64u + lane] = col[k]; to.vals[uint64_t(start) + k * 64u + lane] = val[k]; }
+                }
+                lo = uint32_t(__builtin_amdgcn_readlane(int(wave_scan<~0u>(lo, [](uint32_t a, uint32_t b) { return min(a, b); })), 63));
+                hi = uint32_t(__builtin_amdgcn_readlane(int(wave_scan<0u>(hi, [](uint32_t a, uint32_t b) { return max(a, b); })), 63));
+                const uint32_t longest = uint32_t(__builtin_amdgcn_readlane(
+                    int(wave_scan<0u>(lane < 16u ? next - own : 0u, [](uint32_t a, uint32_t b) { return max(a, b); })), 63));
+                const uint32_t reach = hi - lo, words = reach / 32u + 1u;
+                const bool fits = reach < max_span, maps = fits && 5u * words <= region;
+                const uint32_t log = 32u - uint32_t(__builtin_clz(max(2u * n - 1u, 1u)));          // of the table
+                const uint32_t clear = maps ? 5u * words : fits ? 1u << log : 0u;
+                for (uint32_t w = lane; w < clear; w += 64u) mine[w] = 0u;
+                __builtin_amdgcn_wave_barrier();
+                const uint32_t s1 = row_start(4) - start, s2 = row_start(8) - start, s3 = row_start(12) - start;
+                uint32_t range = 0, unsorted = 0, stored = 0, active = 0, pairs[4] = {}, front = 0;
+#pragma unroll
+                for (uint32_t k = 0; k < kEach; ++k) {
+                    if (k * 64u >= n) break;
+                    const uint32_t i = k * 64u + lane, at = col[k] - lo;
+                    const uint32_t before = uint32_t(__builtin_amdgcn_update_dpp(int(front), int(col[k]), 0x138, 0xf, 0xf, false));       // wave_shr:1
+                    front = uint32_t(__builtin_amdgcn_readlane(int(col[k]), 63));
+                    const uint32_t strip = (i >= s1 ? 1u : 0u) + (i >= s2 ? 1u : 0u) + (i >= s3 ? 1u : 0u);
+                    bool first = false, pair = false;
+                    if (i < n) {
+                        range |= col[k] >= K ? 1u : 0u;
+                        unsorted |= before >= col[k] && !(starts[i >> 5] >> (i & 31u) & 1u) ? 1u : 0u;
+                        if (maps) {
+                            const uint32_t bit = 1u << (at & 31u);
+                            first = !(atomicOr(&mine[at >> 5], bit) & bit);
+                            pair = !(atomicOr(&mine[(1u + strip) * words + (at >> 5)], bit) & bit);
+                        } else if (fits) {
+                            uint32_t slot = (at * 0x9e3779b1u) >> (32u - log), held;
+                            while ((held = atomicCAS(&mine[slot], 0u, at + 1u)) != 0u && (held & 0xfffffu) != at + 1u) slot = (slot + 1u) & ((1u << log) - 1u);
+                            first = held == 0u;
+                            pair = !(atomicOr(&mine[slot], 0x100000u << strip) & (0x100000u << strip));
+                        }
+                    }
+                    stored += uint32_t(__popcll(__ballot(i < n && val[k] != 0.0f)));
+                    active += uint32_t(__popcll(__ballot(first)));
+#pragma unroll
+                    for (uint32_t s = 0; s < 4u; ++s) pairs[s] += uint32_t(__popcll(__ballot(pair && strip == s)));
+                }
+                const uint32_t error = (__ballot(range) ? uint32_t(kErrRange) : 0u) | (__ballot(unsorted) ? uint32_t(kErrUnsorted) : 0u);
+                const uint32_t record[12] = {n, longest, active, reach + 1u, pairs[0], pairs[1], pairs[2], pairs[3], stored, error, lo, lo + reach + 1u};
+#pragma unroll
+                for (uint32_t k = 0; k < 12u; ++k) word = lane == k ? record[k] : word;
+            }
+            if (lane < 12u) reinterpret_cast<uint32_t *>(out + p)[lane] = word;
+        }
+    }
+    if (!COPY) return;
+#pragma unroll 1
+    for (uint32_t w = 0; w < 4u; ++w) {                      // the longer panels are copied here, beside their census
+        const uint32_t q = panel_of(w);
+        if (q >= P) continue;
+        const uint32_t begin = min(rowPtr[uint64_t(q) * 16u], nnz), end = min(rowPtr[uint64_t(q) * 16u + 16u], nnz);
+        if (end < begin || end - begin <= kWaveEntries) continue;
+        for (uint64_t i0 = begin; i0 < end; i0 += 8u * kThreads) {
+            uint32_t x[8];
+            float y[8];
+#pragma unroll
+            for (uint32_t k = 0; k < 8u; ++k) { x[k] = cols[min(i0 + k * kThreads + t, end - uint64_t(1))]; y[k] = vals[min(i0 + k * kThreads + t, end - uint64_t(1))]; }
+#pragma unroll
+            for (uint32_t k = 0; k < 8u; ++k)
+                if (i0 + k * kThreads + t < end) { to.cols[i0 + k * kThreads + t] = x[k]; to.vals[i0 + k * kThreads + t] = y[k]; }
+        }
+    }
 }
 
 // Brick tiles of the panels that fit: hdr lines and values (cute_hrpb_retile defines both).  brp: first block of every

@@ -1156,6 +1156,31 @@ struct HostToDevice {
     }
 };
 
+// The census of every panel into `records`; a caller's arrays are copied to d's own.
+void launch_census(const cute_hrpb_dev *d, const uint32_t *rowPtr, const uint32_t *cols, const float *vals, cute_build::PanelCensus *records)
+{
+    const uint32_t P = d->P;
+    const cute_build::CsrCopy to = {d->dRowPtr, d->dCols, d->dCsrVals};
+    const bool copy = rowPtr != d->dRowPtr;
+    if (uint64_t(d->nnz) <= uint64_t(P) * cute_build::kWaveMean) {
+        const uint32_t quarter = (P + 3u) / 4u, skew = uint32_t(uint64_t(quarter) * 3u / 10u),
+                       front = P <= cute_build::kWaveFront ? P : quarter;
+        const uint32_t lds_words = cute_build::wave_census_words(max_span(d));
+        if (copy)
+            CUTE_BUILD_LDS(cute_build::panel_census_waves<true>, panel_grid(front + quarter), lds_words * 4u, rowPtr, cols, vals, P, d->K, d->nnz, max_span(d), lds_words,
+                           quarter, skew, front, to, records);
+        else
+            CUTE_BUILD_LDS(cute_build::panel_census_waves<false>, panel_grid(front + quarter), lds_words * 4u, rowPtr, cols, vals, P, d->K, d->nnz, max_span(d), lds_words,
+                           quarter, skew, front, to, records);
+    } else {
+        const uint32_t lds_words = cute_build::census_words(max_span(d)), share = uint32_t((uint64_t(d->nnz) + P - 1u) / P);
+        if (copy)
+            CUTE_BUILD_LDS(cute_build::panel_census<true>, panel_grid(P), lds_words * 4u, rowPtr, cols, vals, P, d->K, d->nnz, max_span(d), lds_words, share, to, records);
+        else
+            CUTE_BUILD_LDS(cute_build::panel_census<false>, panel_grid(P), lds_words * 4u, rowPtr, cols, vals, P, d->K, d->nnz, max_span(d), lds_words, share, to, records);
+    }
+}
+
 // The common tail of both uploads.  The CSR arrays are on their way to the device (default stream): to d's own, or they are the caller's and
 // the census copies them.  Checks them, counts what
 // the planner wants to know about every panel, and builds the one MFMA layout the planner's default rules would use for
@@ -1169,14 +1194,7 @@ int finish_upload(cute_hrpb_dev *d, int quad_layout, const DeviceContext &c, con
         int rc = pin.alloc((uint64_t(P) + kTilePanels) * sizeof(cute_build::PanelCensus));      // (the loop below asks for records ahead of it)
         if (rc != CUTE_OK) return rc;
         pin.pending = true;
-        const uint32_t lds_words = cute_build::census_words(max_span(d)), share = uint32_t((uint64_t(d->nnz) + P - 1u) / P);
-        const cute_build::CsrCopy to = {d->dRowPtr, d->dCols, d->dCsrVals};
-        if (rowPtr == d->dRowPtr)
-            CUTE_BUILD_LDS(cute_build::panel_census<false>, panel_grid(P), lds_words * 4u, rowPtr, cols, vals, P, d->K, d->nnz, max_span(d), lds_words, share, to,
-                           pin.as<cute_build::PanelCensus>());
-        else
-            CUTE_BUILD_LDS(cute_build::panel_census<true>, panel_grid(P), lds_words * 4u, rowPtr, cols, vals, P, d->K, d->nnz, max_span(d), lds_words, share, to,
-                           pin.as<cute_build::PanelCensus>());
+        launch_census(d, rowPtr, cols, vals, pin.as<cute_build::PanelCensus>());
         rc = check_launch("panel census");
         if (rc == CUTE_OK) rc = pin.wait();
         if (rc != CUTE_OK) return rc;

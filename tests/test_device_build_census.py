@@ -1,4 +1,4 @@
-"""The census of new matrices: a strip's entries held in registers (up to 512) or walked, and the bitmaps of four, two or one strips in LDS
+"""The census of new matrices: panels of up to 512 entries that a wavefront holds, where panels are short on average; else a strip's entries held in registers (up to 512) or walked, and the bitmaps of four, two or one strips in LDS
 at a time, by the panel's column window.  What it counts decides every place in both layouts, so these must equal the host
 builders word for word."""
 import numpy as np
@@ -48,3 +48,43 @@ def test_strips_held_or_walked(cs, torch_cuda, lengths):
         with pytest.raises(cs.CuteError) as err:
             cs.DeviceHRPB(16, K, *(torch_cuda.from_numpy(x.view(np.int32) if x.dtype == np.uint32 else x).cuda() for x in (rp, unsorted, vl)))
         assert err.value.status == -3
+
+
+@pytest.mark.parametrize("sizes,spans,K,P", [
+    ((0, 1, 63, 64, 65, 511, 512, 513), None, 4096, 9),              # bitmaps only; a panel in front each
+    ((512, 512, 300, 512), (9824, 9825, 65536, 2), 65536, 7),        # the last window of five bitmaps, the first of the table
+    ((512, 1, 513, 500), (13088, 131072, 131072, 131073), 400000, 9),
+    ((512, 513, 5000, 0, 511, 49153, 2, 2000), None, 60000, 1024),   # longer panels; one that is counted entry by entry
+    ((512, 513, 5000, 0, 511, 49153, 2, 2000), None, 60000, 1027)])  # four panels to a work-group in front, not a multiple of four
+def test_panels_of_a_wavefront(cs, torch_cuda, sizes, spans, K, P):
+    rng = np.random.default_rng(P + K)
+    more = P - len(sizes)
+    sizes = tuple(sizes) + tuple(int(x) for x in rng.integers(0, 40, more))
+    M, rp, cl, vl = _panels(rng, K, sizes, spans and tuple(spans) + (500,) * more)
+    assert cl.size <= 512 * P                              # short panels on average: this kernel, not the other
+    got = _both_layouts(cs, torch_cuda, M, K, rp, cl, vl, 2).layouts()
+    _check_bricks(cs, got, M, K, rp, cl, vl)
+    _check_quads(cs, got, M, rp, cl, vl)
+
+
+def test_wavefronts_see_every_unsorted_pair(cs, torch_cuda):
+    """Neighbours in a row may stand in two lanes, in two registers of a wavefront, or begin a strip."""
+    K, length = 4096, 32
+    rng = np.random.default_rng(3)
+    rows = [np.sort(rng.choice(K, length, replace=False)) for _ in range(16)]
+    rp = (np.arange(17) * length).astype(np.uint32)
+    cl, vl = np.concatenate(rows).astype(np.uint32), np.ones(16 * length, np.float32)
+    gpu = lambda a: torch_cuda.from_numpy(a.view(np.int32) if a.dtype == np.uint32 else a).cuda()
+    for r in range(16):
+        for i in (1, 17, 31):
+            bad = cl.copy()
+            bad[r * length + i] = bad[r * length + i - 1]
+            with pytest.raises(cs.CuteError) as err:
+                cs.DeviceHRPB(16, K, gpu(rp), gpu(bad), gpu(vl))
+            assert err.value.status == -3
+    far = cl.copy()
+    far[-1] = K
+    with pytest.raises(cs.CuteError) as err:
+        cs.DeviceHRPB(16, K, gpu(rp), gpu(far), gpu(vl))
+    assert err.value.status == -4
+    cs.DeviceHRPB(16, K, gpu(rp), gpu(cl), gpu(vl))
