@@ -38,7 +38,9 @@ constexpr uint32_t kScanBlock = kThreads * kScanItems;      // entries per scan 
 // take 256 threads and up to kPanelFirst (list kernel: kPanelList, whose LDS lets six work-groups share a compute unit instead
 // of three, 60 -> 40 us on the graph above), panels between have a launch that is given their list, or, for the strip lists, a
 // work-group a strip.
-constexpr uint32_t kPanelCap = 4096, kPanelFirst = 2048, kPanelList = 1024;
+// Where no panel has more than kPanelShort entries, 128 threads take one.  With that and LDS for the widest window there is, not for the most that the
+// matrix could have, a compute unit holds 16 panels instead of 4: bricks of a 9-point stencil of 300 x 300 points 31 -> 14 us.
+constexpr uint32_t kPanelCap = 4096, kPanelFirst = 2048, kPanelList = 1024, kPanelShort = 512;
 constexpr uint32_t kPanelSpan = 1u << 17;                   // columns of its window: a bitmap of 16 KB and 8 KB of running counts
 
 enum : uint32_t { kErrRange = 1, kErrUnsorted = 2, kAnyError = kErrRange | kErrUnsorted };
@@ -171,7 +173,7 @@ __device__ __forceinline__ uint32_t row_in_panel(const uint32_t *rp, uint32_t e)
 // ------------------------------------------------------------------------------------------------
 // A panel in LDS.
 // ------------------------------------------------------------------------------------------------
-constexpr uint32_t panel_threads(uint32_t cap) { return cap == kPanelCap ? 512u : 256u; }
+constexpr uint32_t panel_threads(uint32_t cap) { return cap == kPanelCap ? 512u : cap == kPanelShort ? 128u : 256u; }
 struct Two { uint32_t x, y; };
 template <uint32_t CAP> struct PanelLds {
     static constexpr uint32_t kBlock = panel_threads(CAP);

@@ -697,7 +697,9 @@ int check_launch(const char *what);
 
 // The widest column window the panel kernels take on this matrix, and the LDS its bitmap and running counts need.
 inline uint32_t max_span(const cute_hrpb_dev *d) { return std::min(d->K, cute_build::kPanelSpan); }
-inline uint32_t window_lds(const cute_hrpb_dev *d, uint32_t at_least) { return std::max((cute_build::panel_window_words(max_span(d)) + 1u) * 6u, at_least); }
+inline uint32_t window_lds(uint32_t span, uint32_t at_least) { return std::max((cute_build::panel_window_words(span) + 1u) * 6u, at_least); }
+// No panel that the panel kernels take has a wider window: the widest of a tile of panels, which the census loop knows.
+inline uint32_t widest_span(const cute_hrpb_dev *d) { return std::max(1u, std::min(max_span(d), d->widestTile)); }
 constexpr const uint32_t *kAllPanels = nullptr;
 inline bool panel_is_large(const cute_hrpb_dev *d, uint32_t p) { return d->panelNnz[p] > cute_build::kPanelCap || d->panelSpan[p] > max_span(d); }
 
@@ -841,7 +843,7 @@ int build_bricks_on_device(cute_hrpb_dev *d, LargeWork &w)
     int rc = number_large_panels(d, w, nullptr);
     if (rc != CUTE_OK) return rc;
     const uint64_t hdr_words = uint64_t(d->nb) * CUTE_TILED_HDR_WORDS, num_vals = uint64_t(d->nnz) + 64u;
-    const uint32_t count = uint32_t(w.panel.size());
+    const uint32_t count = uint32_t(w.panel.size()), span = widest_span(d);
     Layout lay, tab;
     const uint64_t oBrp = tab.add(uint64_t(d->P) + 1u, 4), oUnit = tab.add(count, 4), oPrefix = tab.add(count + 1u, 4), oCols = tab.add(count, 4);
     const std::vector<uint32_t> medium = panels_between(d, cute_build::kPanelFirst);
@@ -870,12 +872,13 @@ int build_bricks_on_device(cute_hrpb_dev *d, LargeWork &w)
     pin.pending = true;
     if (!in_place)
         CUTE_BUILD(cute_build::copy_words, grid_capped(tab.bytes / 4u), pin.as<const uint32_t>(), Layout::at<uint32_t>(mem.p, oTab), tab.bytes / 4u);
-    CUTE_PANELS(cute_build::panel_bricks<cute_build::kPanelFirst>, cute_build::kPanelFirst, d->P, window_lds(d, (cute_build::kPanelFirst + 1u) * 2u), nullptr,
-                d->dRowPtr, d->dCols, d->dCsrVals, d->P, d->nnz, max_span(d), kAllPanels, table(oBrp), hdr, vals);
-    if (!medium.empty())
-        CUTE_PANELS(cute_build::panel_bricks<cute_build::kPanelCap>, cute_build::kPanelCap, uint32_t(medium.size()),
-                    window_lds(d, (cute_build::kPanelCap + 1u) * 2u), in_place ? side.get() : nullptr, d->dRowPtr, d->dCols, d->dCsrVals, d->P, d->nnz, max_span(d), table(oMedium),
-                    table(oBrp), hdr, vals);
+#define CUTE_PANEL_BRICKS(CAP, COUNT, STREAM, LIST)                                                                                    \
+    CUTE_PANELS(cute_build::panel_bricks<CAP>, CAP, COUNT, window_lds(span, (CAP + 1u) * 2u), STREAM, d->dRowPtr, d->dCols, d->dCsrVals, d->P, d->nnz,  \
+                span, LIST, table(oBrp), hdr, vals)
+    if (d->longestPanel <= cute_build::kPanelShort) CUTE_PANEL_BRICKS(cute_build::kPanelShort, d->P, nullptr, kAllPanels);
+    else CUTE_PANEL_BRICKS(cute_build::kPanelFirst, d->P, nullptr, kAllPanels);
+    if (!medium.empty()) CUTE_PANEL_BRICKS(cute_build::kPanelCap, uint32_t(medium.size()), in_place ? side.get() : nullptr, table(oMedium));
+#undef CUTE_PANEL_BRICKS
     if (count) {
         const uint32_t blocks = prefix[count];
         CUTE_BUILD(cute_build::large_clear, grid_of(uint64_t(blocks) * CUTE_TILED_HDR_WORDS), table(oUnit), table(oPrefix), count, uint32_t(CUTE_TILED_HDR_WORDS), hdr);
@@ -904,7 +907,7 @@ int build_quads_on_device(cute_hrpb_dev *d, LargeWork &w)
     const StripLists lists = strips ? list_strips(d, with_large) : StripLists();
     int rc = with_large ? int(CUTE_OK) : number_large_panels(d, w, nullptr);
     if (rc != CUTE_OK) return rc;
-    const uint32_t count = with_large ? 0u : uint32_t(w.panel.size()), per = strips ? 4u : 1u;
+    const uint32_t count = with_large ? 0u : uint32_t(w.panel.size()), per = strips ? 4u : 1u, span = widest_span(d);
     Layout lay, tab;
     const uint64_t oGroup = tab.add(d->qgp.size(), 4), oBase = tab.add(uint64_t(d->P) + 1u, 4), oUnit = tab.add(count, 4),
                    oPrefix = tab.add(count + 1u, 4), oFirst = tab.add(uint64_t(count) * per, 4), oPairs = tab.add(uint64_t(count) * 4u, 4),
@@ -947,10 +950,11 @@ int build_quads_on_device(cute_hrpb_dev *d, LargeWork &w)
     uint32_t *sums = counts.as<uint32_t>();
     const uint32_t listed = uint32_t(medium.size());
 #define CUTE_PANEL_QUADS(S, CAP, COUNT, LIST, LISTED, STREAM)                                                                         \
-    CUTE_PANELS((cute_build::panel_quads<S, CAP>), CAP, COUNT, window_lds(d, CAP * 8u), STREAM, d->dRowPtr, d->dCols, d->dCsrVals, d->P, d->nnz,  \
-                max_span(d), LIST, LISTED, table(oGroup), table(oBase), uint32_t(stored), recs, packed)
+    CUTE_PANELS((cute_build::panel_quads<S, CAP>), CAP, COUNT, window_lds(span, CAP * 8u), STREAM, d->dRowPtr, d->dCols, d->dCsrVals, d->P, d->nnz,  \
+                span, LIST, LISTED, table(oGroup), table(oBase), uint32_t(stored), recs, packed)
 #define CUTE_BUILD_QUADS(S)                                                                                                           \
-    CUTE_PANEL_QUADS(S, cute_build::kPanelList, (S) ? d->P + listed : d->P, (S) ? table(oMedium) : kAllPanels, (S) ? listed : 0u, nullptr); \
+    if (d->longestPanel <= cute_build::kPanelShort) CUTE_PANEL_QUADS(S, cute_build::kPanelShort, d->P, kAllPanels, 0u, nullptr);            \
+    else CUTE_PANEL_QUADS(S, cute_build::kPanelList, (S) ? d->P + listed : d->P, (S) ? table(oMedium) : kAllPanels, (S) ? listed : 0u, nullptr); \
     if constexpr (!(S))                                                                                                               \
         if (listed) CUTE_PANEL_QUADS(S, cute_build::kPanelCap, listed, table(oMedium), listed, in_place ? side.get() : nullptr);        \
     if (count) {                                                                                                                      \
@@ -966,7 +970,7 @@ int build_quads_on_device(cute_hrpb_dev *d, LargeWork &w)
     }
     // (the strips that take longest go first)
     if (!lists.big.empty()) {
-        const uint32_t words = cute_build::panel_window_words(max_span(d));
+        const uint32_t words = cute_build::panel_window_words(span);
         hipLaunchKernelGGL(cute_build::big_quads, dim3(uint32_t(lists.big.size())), dim3(cute_build::kBigThreads),
                            (cute_build::big_window_words(words) + lists.bigRows + lists.bigSteps) * 4u, in_place ? side.get() : nullptr, d->dRowPtr, d->dCols, d->dCsrVals,
                            table(oBig), words, lists.bigRows, table(oGroup), table(oBase), recs, packed);

@@ -45,6 +45,16 @@ def test_entry_counts(cs, torch_cuda, sizes, quad_layout):
 
 
 @pytest.mark.parametrize("quad_layout", [1, 2])
+@pytest.mark.parametrize("sizes,K,spans", [((512, 511, 127, 128, 129, 0), 4096, None), ((512, 0, 1, 513), 4096, None),
+                                           ((512, 300, 512), 70000, (65536, 32, 33)), ((512, 300, 700), 400000, (131072, 131073, 40))])
+def test_short_panels_and_windows_narrower_than_the_matrix(cs, torch_cuda, sizes, K, spans, quad_layout):
+    M, rp, cl, vl = _panels(np.random.default_rng(sum(sizes) + K), K, sizes, spans)
+    got = _both_layouts(cs, torch_cuda, M, K, rp, cl, vl, quad_layout).layouts()
+    _check_bricks(cs, got, M, K, rp, cl, vl)
+    _check_quads(cs, got, M, rp, cl, vl)
+
+
+@pytest.mark.parametrize("quad_layout", [1, 2])
 def test_column_windows(cs, torch_cuda, quad_layout):
     K = 400000
     spans = (31, 32, 33, 131071, 131072, 131073, 400000, 64)
