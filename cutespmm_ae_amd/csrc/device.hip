@@ -697,7 +697,7 @@ int check_launch(const char *what);
 
 // The widest column window the panel kernels take on this matrix, and the LDS its bitmap and running counts need.
 inline uint32_t max_span(const cute_hrpb_dev *d) { return std::min(d->K, cute_build::kPanelSpan); }
-inline uint32_t window_lds(uint32_t span, uint32_t at_least) { return std::max((cute_build::panel_window_words(span) + 1u) * 6u, at_least); }
+inline uint32_t window_lds(uint32_t span, uint32_t at_least) { return std::max(cute_build::window_room(span) / 2u * 9u, at_least); }
 // No panel that the panel kernels take has a wider window: the widest of a tile of panels, which the census loop knows.
 inline uint32_t widest_span(const cute_hrpb_dev *d) { return std::max(1u, std::min(max_span(d), d->widestTile)); }
 constexpr const uint32_t *kAllPanels = nullptr;
