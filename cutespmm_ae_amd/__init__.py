@@ -28,7 +28,7 @@ ABI_SYMBOLS = [
     "cute_gen_matrix", "cute_gen_dense",
     "cute_hrpb_upload", "cute_hrpb_upload_layout", "cute_hrpb_upload_device_csr", "cute_hrpb_dev_layout_sizes",
     "cute_hrpb_dev_read_layouts", "cute_hrpb_dev_free", "cute_hrpb_dev_bytes", "cute_hrpb_dev_csr",
-    "cute_spmm_plan_create", "cute_spmm_plan_info", "cute_spmm_plan_column_slabs", "cute_spmm_plan_window", "cute_spmm_plan_free", "cute_spmm_run", "cute_spmm_run_static",
+    "cute_spmm_plan_create", "cute_spmm_plan_info", "cute_spmm_plan_column_slabs", "cute_spmm_plan_window", "cute_spmm_plan_row_parts", "cute_spmm_plan_free", "cute_spmm_run", "cute_spmm_run_static",
     "cute_spmm_run_scratch", "cute_spmm_plan_scratch_bytes", "cute_device_layout", "cute_release_idle_memory",
     "cute_csr_spmm_dev", "cute_gpu_csr_spmm", "cute_spmm_time", "cute_csr_spmm_time",
     "cute_device_info",
@@ -204,6 +204,7 @@ def load_library():
     lib.cute_spmm_plan_info.argtypes = [C.c_void_p, C.POINTER(cute_plan_info)]
     lib.cute_spmm_plan_column_slabs.argtypes = [C.c_void_p, u32p, u32p]
     lib.cute_spmm_plan_window.argtypes = [C.c_void_p, u32p]
+    lib.cute_spmm_plan_row_parts.argtypes = [C.c_void_p, u32p]
     lib.cute_spmm_plan_free.argtypes = [C.c_void_p]
     lib.cute_spmm_run.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]
     lib.cute_spmm_run_static.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]
@@ -736,10 +737,17 @@ class SPMM_TC:
         return columns.value
 
     @property
+    def row_parts(self):
+        """Lane groups that share a row of a product of a few columns (``csr_rows_split``); 1: another kernel takes the rows."""
+        parts = C.c_uint32()
+        _check(load_library().cute_spmm_plan_row_parts(self._plan, C.byref(parts)), "cute_spmm_plan_row_parts")
+        return parts.value
+
+    @property
     def kernel_name(self):
         """The kernel that does the plan's main work: the MFMA kernel, or the row kernel of a plan without MFMA panels."""
         info = self.info
-        return (("csr_rows_window" if self.window_columns else "csr_rows_batched") if info["numChunks"] == 0 else
+        return (("csr_rows_window" if self.window_columns else "csr_rows_split" if self.row_parts > 1 else "csr_rows_batched") if info["numChunks"] == 0 else
                 "hrpb_quad_hub_f32" if info["hubRows"] else
                 ("hrpb_quad_rows_f32" if info["fusedLaunch"] else "hrpb_quad_half_f32" if info["slabWidth"] == 32 else "hrpb_quad_f32")
                 if info["mfmaShape"] == 2 else

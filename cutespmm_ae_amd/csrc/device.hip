@@ -275,6 +275,8 @@ struct cute_spmm_plan {
     // slabs of the MFMA part and of the row part when an XCD owns columns instead of rows (cute_dev::xcd_share), else 0
     uint32_t columnSlabs = 0, rowColumnSlabs = 0;
     uint32_t rowBlocksPerXcd = 0;       // longest of those ranges
+    // rows through csr_rows_split: lane groups that share a row (1: not used), a power of two
+    uint32_t rowParts = 1;
     // rows through csr_rows_window: columns of B in its ring (0: not used) and the chains of tiles
     uint32_t windowColumns = 0, windowChains = 0, windowChainTiles = 0;
     bool windowWarm = false;
@@ -1305,6 +1307,30 @@ int make_hub_tables(cute_spmm_plan *p, const cute_hrpb_dev *d, uint32_t hub_rows
     return CUTE_OK;
 }
 
+// How many lane groups share a row in csr_rows_split; 1: another kernel takes the rows.  Up to 8 columns, for rows of 24 entries or more on average, a
+// lane group for three and a half to seven entries each: the four a lane has on their way are then nearly all used.  One row kernel or brick kernel / 4, 8,
+// 16, 32 groups, us from a replayed graph: finite elements (rows of 60), 1 200 rows, N = 1 11.6 / 4.5, 3.2, 2.7, 2.7, 12 000 rows, N = 1 12.9 / 5.0, 3.8, 3.6, 3.6,
+// N = 8 7.1 / 6.1, 4.6, 4.4, 5.1; rows of 32 in a band, 5 120 rows, N = 1 5.3 / 2.8, 2.6, 2.5, 2.7, 102 400 rows, N = 1 8.3 / 7.2, 5.9, 7.7, 10.8, N = 8
+// 11.4 / 10.1, 9.7, 14.9, 26.7, N = 16 15.9 / 15.4, 16.5, 27.4.  Shorter rows gain little or lose: 20 000 rows of 16, N = 3 3.46 / 3.51; 100 000 rows of 8,
+// N = 1 5.1 / 5.4; 9-point stencil of 500 x 500 points, N = 8 6.6 / 9.3.  Nor where one row is much longer than the others, for which the brick kernel cuts its
+// panel: R-MAT graph of 32 768 nodes, N = 1 13.3 / 84, 43, 24, 14.  And the brick kernel, which fetches a row of B once for all rows of a panel, is ahead
+// from three columns on where rows share columns and the launch no longer fits the device at once: finite elements, 48 000 rows, brick kernel / 16
+// groups: N = 1 9.3 / 6.2, N = 3 9.3 / 9.9, N = 8 9.3 / 10.3; 500 000 rows of 32 in a band, N = 8 64.5 / 61.8.
+uint32_t row_parts(const cute_hrpb_dev *d, uint32_t N)
+{
+    if (N > 8u || uint64_t(d->nnz) < 24ull * d->M) return 1u;
+    uint32_t longest = 0, parts = 4;
+    uint64_t active = 0;
+    for (uint32_t q = 0; q < d->P; ++q) {
+        longest = std::max(longest, d->panelMaxRow[q]);
+        active += d->panelCols[q];
+    }
+    while (parts < 16u && uint64_t(d->nnz) >= 7ull * parts * d->M) parts *= 2u;
+    if (N > 2u && uint64_t(d->nnz) >= 2u * active && uint64_t(d->M) * parts * (N > 4u || N == 3u ? 2u : 1u) > 524288u) return 1u;
+    // (a launch has at most 2^32 threads, of which a row takes parts, twice as many from two lanes a group on)
+    return uint64_t(longest) * d->M > 4ull * d->nnz || uint64_t(d->M) * parts * 2u > 0x7fffffffull ? 1u : parts;
+}
+
 // Rows of a plan without MFMA panels through csr_rows_window where that is ahead.  Needs the widest window of a tile to fit the ring,
 // rows of up to 64 entries (the LDS of window_entries) and little padding: a lane waits for the longest of 64 rows.  Then both kernels'
 // times are estimated, in us, and the ring has to be ahead by 15 %.  Fitted on 400 banded matrices drawn
@@ -1488,6 +1514,13 @@ int cute_spmm_plan_column_slabs(const cute_spmm_plan *p, uint32_t *mfma, uint32_
     return CUTE_OK;
 }
 
+int cute_spmm_plan_row_parts(const cute_spmm_plan *p, uint32_t *parts)
+{
+    if (!p) return CUTE_ERR_ARG;
+    if (parts) *parts = p->rowParts;
+    return CUTE_OK;
+}
+
 int cute_spmm_plan_window(const cute_spmm_plan *p, uint32_t *columns)
 {
     if (!p) return CUTE_ERR_ARG;
@@ -1564,6 +1597,8 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
         const uint32_t lists = d->quadRows == 4 ? 4u : 1u;
         return std::max(panelCols[q], (qgp[(q + 1) * lists] - qgp[q * lists]) * 16u);
     };
+    const uint32_t parts = default_bars && t.precision == CUTE_PREC_FP32 && !t.slots && !t.mfma_shape && !t.hub_rows && !t.max_chunk_blocks &&
+                                   !t.brick_groups && !t.pipeline && !t.chunk_order ? row_parts(d, N) : 1u;
     uint64_t reused = 0;                          // entries of panels that go to the MFMA side by the usual bars: reuse, long or uneven rows
     uint32_t n_brick = 0, n_rows = 0, n_empty = 0;
     for (uint32_t q = 0; q < P; ++q) {
@@ -1571,7 +1606,7 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
         bool rows;
         if (nblk == 0) { rows = true; n_empty++; }
         else if (t.path == CUTE_PATH_BRICK) rows = false;
-        else if (t.path == CUTE_PATH_ROWS) rows = true;
+        else if (t.path == CUTE_PATH_ROWS || parts > 1u) rows = true;
         else {
             // Row kernel when a B row fetched by the MFMA side serves hardly more than one nonzero of the
             // panel (the matrix cores then buy nothing) -- unless a row is so long that one lane group
@@ -2142,6 +2177,7 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
     p->info.precision = p->bf16x3 ? uint32_t(CUTE_PREC_BF16X3) : uint32_t(CUTE_PREC_FP32);
     p->info.path = uint32_t(t.path);
     p->columnSlabs = mfma_by_columns ? num_slabs : 0u;
+    p->rowParts = num_row_panels == P && !p->windowColumns ? parts : 1u;
     p->info.mfmaShape = uint32_t(p->shape);
     p->info.hubRows = p->numHub;
     p->info.pipeline = uint32_t(p->pipeline);
@@ -2459,6 +2495,19 @@ int run_with(const cute_spmm_plan *p, const float *dB, float *dC, void *stream, 
         if (p->windowColumns == 16u) { if (p->windowWarm) CUTE_WINDOW_LAUNCH(16, true); else CUTE_WINDOW_LAUNCH(16, false); }
         else { if (p->windowWarm) CUTE_WINDOW_LAUNCH(8, true); else CUTE_WINDOW_LAUNCH(8, false); }
 #undef CUTE_WINDOW_LAUNCH
+    } else if (p->rowParts > 1u) {
+        uint32_t log_lanes = 0;
+        while (uint32_t(p->rows_vec) << log_lanes < N) ++log_lanes;
+        const uint32_t log_parts = uint32_t(__builtin_ctz(p->rowParts));
+        const uint64_t threads = uint64_t(p->d->M) << (log_lanes + log_parts);
+        const uint32_t per_xcd = uint32_t((threads + 256u * cute_dev::kNumXcd - 1u) / (256u * cute_dev::kNumXcd));
+#define CUTE_SPLIT_LAUNCH(VEC)                                                                                                    \
+    hipLaunchKernelGGL(cute_dev::csr_rows_split<VEC>, dim3(per_xcd * cute_dev::kNumXcd), dim3(256), 0, s, p->d->dRowPtr, p->d->dCols, p->d->dCsrVals, dB, dC, \
+                       p->d->M, N, log_lanes, log_parts, per_xcd)
+        if (p->rows_vec == 4) CUTE_SPLIT_LAUNCH(4);
+        else if (p->rows_vec == 2) CUTE_SPLIT_LAUNCH(2);
+        else CUTE_SPLIT_LAUNCH(1);
+#undef CUTE_SPLIT_LAUNCH
     } else if (p->numRows && !rows_launched) {
         launch_rows<true>(p->rows_vec, p->rows_logl, p->dRowList, p->numRows, p->rows_slabs, p->d->dRowPtr, p->d->dCols,
                     p->d->dCsrVals, dB, dC, N, s, &p->rowRanges, p->rowBlocksPerXcd, p->rowColumnSlabs);

@@ -62,7 +62,7 @@ def run_one(path, widths, iters, cache=None, check=True, extras=False):
     return [json.loads(line) for line in proc.stdout.splitlines() if line.startswith("{")]
 
 
-PLAN_KERNELS = ("hrpb_", "csr_rows_batched", "csr_rows_window", "reduce_partials")      # what one step of a plan launches
+PLAN_KERNELS = ("hrpb_", "csr_rows_batched", "csr_rows_window", "csr_rows_split", "reduce_partials")      # what one step of a plan launches
 CSR_KERNEL = "csr_rows<"                                              # the comparison column's kernel
 
 

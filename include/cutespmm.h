@@ -476,6 +476,8 @@ int cute_spmm_plan_column_slabs(const cute_spmm_plan *p, uint32_t *mfma, uint32_
  * entries to it (6 bytes an entry and some padding), as for a late MFMA layout.  Where there is no memory for it the rows gather
  * from memory instead; any other failure is the plan's. */
 int cute_spmm_plan_window(const cute_spmm_plan *p, uint32_t *columns);
+/* Lane groups that share a row of a product of a few columns (csr_rows_split); 1: another kernel takes the rows. */
+int cute_spmm_plan_row_parts(const cute_spmm_plan *p, uint32_t *parts);
 void cute_spmm_plan_free(cute_spmm_plan *p);
 /* dB [K x N], dC [M x N]: device pointers, row-major, 16-byte aligned.  Asynchronous on
  * `stream` (a hipStream_t, NULL = default stream).  C is fully overwritten: the caller
