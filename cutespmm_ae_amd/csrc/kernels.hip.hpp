@@ -886,7 +886,7 @@ __device__ __forceinline__ void quad_chunk(uint32_t chunk, uint32_t block_y, con
 #undef CUTE_QUAD_ROLL_REST
 #undef CUTE_QUAD_MFMA16
     }
-    if (piece) {              // (the partials matrix: rows (piece-1)*16.., same pitch as C)
+    if (!HUB && piece) {      // (the partials matrix: rows (piece-1)*16.., same pitch as C)
         constexpr int E = STRIPS ? 4 : 16;
         float mine[E];
         const f32x4 sum = (acc[0] + acc[1]) + (acc[2] + acc[3]);
@@ -896,19 +896,22 @@ __device__ __forceinline__ void quad_chunk(uint32_t chunk, uint32_t block_y, con
         auto at = [&](uint32_t unit, int e) { return __umul24(unit * uint32_t(E) + uint32_t(e), N * 4u) + offset; };
         store_piece(cut, piece, block_y, mine, at, [&](int) { return FULL || column < N; }, partials, C);
     } else if (live) {
-        char *out_base = reinterpret_cast<char *>(C);
+        // (pieces of a hub plan are added up by reduce_partials: store_piece here takes hrpb_quad_hub_f32<true> from 64 to 65 vector registers, and a
+        // compute unit then holds one of its work-groups instead of two)
+        char *out_base = reinterpret_cast<char *>(HUB && piece ? partials : C);
+        const uint32_t unit = HUB && piece ? piece - 1u : panel;
         if (STRIPS) {
             // all 16 pairs of a group belong to one 4-row strip; the four accumulators only break
             // the dependency chain and are summed here
             const f32x4 sum = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-            uint32_t off = __umul24(panel * 4u, row_pitch) + n * 4u;
+            uint32_t off = __umul24(unit * 4u, row_pitch) + n * 4u;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 __builtin_nontemporal_store(sum[i], reinterpret_cast<float *>(out_base + off));
                 off += row_pitch;
             }
         } else {
-            uint32_t off = __umul24(panel * 16u, row_pitch) + n * 4u;
+            uint32_t off = __umul24(unit * 16u, row_pitch) + n * 4u;
 #pragma unroll
             for (int rg = 0; rg < 4; ++rg)
 #pragma unroll

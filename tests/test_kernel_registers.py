@@ -7,10 +7,10 @@ import re
 import cutespmm_ae_amd as cs
 
 
-def _kernels():
+def _kernels(field=b"vgpr_spill_count"):
     blob = open(cs.LIB_PATH, "rb").read()
     found = {}
-    for m in re.finditer(rb"\.vgpr_spill_count(.)", blob, re.S):
+    for m in re.finditer(rb"\." + field + rb"(.)", blob, re.S):
         names = list(re.finditer(rb"\.symbol(?:\xd9.|\xda..|[\xa0-\xbf])(_Z\w+)\.kd", blob[max(0, m.start() - 2048):m.start()], re.S))
         assert names, "a kernel without a symbol"
         found[names[-1].group(1).decode()] = m.group(1)[0]       # a small integer is one byte
@@ -21,3 +21,10 @@ def test_no_kernel_spills_vector_registers():
     kernels = _kernels()
     assert len(kernels) > 100 and any("hrpb_quad_rows_f32" in k for k in kernels), len(kernels)
     assert {k: n for k, n in kernels.items() if n} == {}
+
+
+def test_two_work_groups_of_the_hub_kernel_fit_a_compute_unit():
+    """Its work-groups are sixteen wavefronts and the launch starts two a compute unit: eight wavefronts a SIMD, 64 registers.  (Off the grid of 64
+    columns it has always taken 65.)"""
+    hub = {k: n for k, n in _kernels(b"vgpr_count").items() if "hrpb_quad_hub_f32ILb1E" in k}
+    assert list(hub.values()) == [64], hub
