@@ -2195,7 +2195,7 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
 
 namespace {
 
-template <int VEC, int NG, bool FULL, bool COLUMNS>
+template <int VEC, int NG, bool FULL, bool COLUMNS, bool CUT>
 void launch_brick_full(const cute_spmm_plan *p, const float *dB, float *dC, float *partials, const cute_dev::CutPieces *cut, hipStream_t s)
 {
     const uint32_t groups = (p->info.numChunks + cute_dev::kWavesPerGroup - 1) / cute_dev::kWavesPerGroup;
@@ -2203,24 +2203,31 @@ void launch_brick_full(const cute_spmm_plan *p, const float *dB, float *dC, floa
     const dim3 grid(per_xcd * cute_dev::kNumXcd, p->info.numSlabs), block(cute_dev::kWaveSize * cute_dev::kWavesPerGroup);
     if (p->bf16x3) {
         if constexpr (VEC == 4)
-            hipLaunchKernelGGL((cute_dev::hrpb_brick_bf16x3<NG, FULL, COLUMNS>), grid, block, 0, s, p->dChunks, p->info.numChunks, per_xcd,
+            hipLaunchKernelGGL((cute_dev::hrpb_brick_bf16x3<NG, FULL, COLUMNS, CUT>), grid, block, 0, s, p->dChunks, p->info.numChunks, per_xcd,
                                p->d->dHdr, p->d->dVals, uint32_t(p->d->numVals), dB, dC, partials, p->info.N, p->columnSlabs, cut);
     } else if (p->pipeline == 1)
-        hipLaunchKernelGGL((cute_dev::hrpb_brick_f32_rolling<VEC, NG, FULL, COLUMNS>), grid, block, 0, s, p->dChunks,
+        hipLaunchKernelGGL((cute_dev::hrpb_brick_f32_rolling<VEC, NG, FULL, COLUMNS, CUT>), grid, block, 0, s, p->dChunks,
                            p->info.numChunks, per_xcd, p->d->dHdr, p->d->dVals, uint32_t(p->d->numVals), dB, dC, partials, p->info.N, p->columnSlabs, cut);
     else
         hipLaunchKernelGGL((cute_dev::hrpb_brick_f32<VEC, NG, FULL>), grid, block, 0, s, p->dChunks, p->info.numChunks,
                            per_xcd, p->d->dHdr, p->d->dVals, dB, dC, partials, p->info.N, p->columnSlabs);
 }
 
+template <int VEC, int NG, bool CUT>
+void launch_brick_as(const cute_spmm_plan *p, const float *dB, float *dC, float *partials, const cute_dev::CutPieces *cut, hipStream_t s)
+{
+    const bool full = p->info.N % p->info.slabWidth == 0;
+    if (p->columnSlabs && full) launch_brick_full<VEC, NG, true, true, CUT>(p, dB, dC, partials, cut, s);
+    else if (p->columnSlabs) launch_brick_full<VEC, NG, false, true, CUT>(p, dB, dC, partials, cut, s);
+    else if (full) launch_brick_full<VEC, NG, true, false, CUT>(p, dB, dC, partials, cut, s);
+    else launch_brick_full<VEC, NG, false, false, CUT>(p, dB, dC, partials, cut, s);
+}
+
 template <int VEC, int NG>
 void launch_brick(const cute_spmm_plan *p, const float *dB, float *dC, float *partials, const cute_dev::CutPieces *cut, hipStream_t s)
 {
-    const bool full = p->info.N % p->info.slabWidth == 0;
-    if (p->columnSlabs && full) launch_brick_full<VEC, NG, true, true>(p, dB, dC, partials, cut, s);
-    else if (p->columnSlabs) launch_brick_full<VEC, NG, false, true>(p, dB, dC, partials, cut, s);
-    else if (full) launch_brick_full<VEC, NG, true, false>(p, dB, dC, partials, cut, s);
-    else launch_brick_full<VEC, NG, false, false>(p, dB, dC, partials, cut, s);
+    if (p->numFixups) launch_brick_as<VEC, NG, true>(p, dB, dC, partials, cut, s);
+    else launch_brick_as<VEC, NG, false>(p, dB, dC, partials, cut, s);
 }
 
 template <int VEC, bool BATCHED>
@@ -2365,18 +2372,24 @@ void launch_brick_rows_as(const cute_spmm_plan *p, const float *dB, float *dC, f
     const uint32_t rows_per_slab = p->rowBlocksPerXcd * cute_dev::kNumXcd;
     const uint64_t brick_blocks = uint64_t(grid.x) * grid.y, row_blocks = uint64_t(rows_per_slab) * p->rows_slabs;
     const dim3 flat(uint32_t(brick_blocks + row_blocks)), block(cute_dev::kWaveSize * cute_dev::kWavesPerGroup);
-#define CUTE_BRICK_ROWS(F, COLUMNS)                                                                                       \
-    hipLaunchKernelGGL((cute_dev::hrpb_brick_rows_f32<VEC, NG, F, LOG_L, COLUMNS>), flat, block, 0, s, grid.x, uint32_t(brick_blocks),  \
+#define CUTE_BRICK_ROWS_AS(F, COLUMNS, CUT)                                                                               \
+    hipLaunchKernelGGL((cute_dev::hrpb_brick_rows_f32<VEC, NG, F, LOG_L, COLUMNS, CUT>), flat, block, 0, s, grid.x, uint32_t(brick_blocks),  \
                        p->dChunks, p->info.numChunks, per_xcd, p->d->dHdr, p->d->dVals, uint32_t(p->d->numVals), p->dRowList, \
                        p->numRows, rows_per_slab, p->rowRanges, p->columnSlabs, p->rowColumnSlabs, p->d->dRowPtr, p->d->dCols, p->d->dCsrVals,                    \
                        dB, dC, partials, N, cut)
+#define CUTE_BRICK_ROWS(F, COLUMNS)                               \
+    {                                                             \
+        if (p->numFixups) CUTE_BRICK_ROWS_AS(F, COLUMNS, true);   \
+        else CUTE_BRICK_ROWS_AS(F, COLUMNS, false);               \
+    }
     constexpr bool wide = LOG_L >= 5;            // a launch by columns has 128 columns or more
     const bool full = N % (16u * VEC * NG) == 0;
-    if (wide && p->columnSlabs && full) CUTE_BRICK_ROWS(true, wide);
-    else if (wide && p->columnSlabs) CUTE_BRICK_ROWS(false, wide);
-    else if (full) CUTE_BRICK_ROWS(true, false);
-    else CUTE_BRICK_ROWS(false, false);
+    if (wide && p->columnSlabs && full) CUTE_BRICK_ROWS(true, wide)
+    else if (wide && p->columnSlabs) CUTE_BRICK_ROWS(false, wide)
+    else if (full) CUTE_BRICK_ROWS(true, false)
+    else CUTE_BRICK_ROWS(false, false)
 #undef CUTE_BRICK_ROWS
+#undef CUTE_BRICK_ROWS_AS
 }
 
 bool launch_brick_rows(const cute_spmm_plan *p, const float *dB, float *dC, float *partials, const cute_dev::CutPieces *cut, hipStream_t s)
@@ -2426,29 +2439,34 @@ int run_with(const cute_spmm_plan *p, const float *dB, float *dC, void *stream, 
         const uint32_t groups = (p->info.numChunks + cute_dev::kWavesPerGroup - 1) / cute_dev::kWavesPerGroup;
         const uint32_t per_xcd = (groups + cute_dev::kNumXcd - 1) / cute_dev::kNumXcd;
         const dim3 grid(per_xcd * cute_dev::kNumXcd, p->info.numSlabs), block(cute_dev::kWaveSize * cute_dev::kWavesPerGroup);
-        const bool full = N % 64u == 0, strips = p->d->quadRows == 4;
+        const bool full = N % 64u == 0, strips = p->d->quadRows == 4, pieces = p->numFixups != 0;
         // mixed plan: quad chunks and sparse rows in one launch (instantiated for 4-float lanes and 4..64 lanes per row)
         const uint32_t rows_per_slab = p->rowBlocksPerXcd * cute_dev::kNumXcd;
         const uint64_t row_blocks = uint64_t(rows_per_slab) * p->rows_slabs, quad_blocks = uint64_t(grid.x) * grid.y;
         if (p->info.fusedLaunch && quad_blocks + row_blocks < 0x7fffffffull) {
-#define CUTE_FUSED_LAUNCH(F, S, LL, COLUMNS)                                                                              \
-    hipLaunchKernelGGL((cute_dev::hrpb_quad_rows_f32<F, S, LL, COLUMNS>), dim3(uint32_t(quad_blocks + row_blocks)), block, 0, s,     \
+#define CUTE_FUSED_LAUNCH_AS(F, S, LL, COLUMNS, CUT)                                                                      \
+    hipLaunchKernelGGL((cute_dev::hrpb_quad_rows_f32<F, S, LL, COLUMNS, CUT>), dim3(uint32_t(quad_blocks + row_blocks)), block, 0, s,     \
                        grid.x, uint32_t(quad_blocks), p->dHeads, p->info.numChunks, per_xcd, p->d->dQRecs, p->d->dQVals,   \
                        uint32_t(p->d->numQuadVals),                                                                  \
                        p->dRowList, p->numRows, rows_per_slab, p->rowRanges, p->columnSlabs, p->rowColumnSlabs, p->d->dRowPtr, p->d->dCols, p->d->dCsrVals, dB, dC,    \
                        partials, N, cut)
+#define CUTE_FUSED_LAUNCH(F, S, LL, COLUMNS)                                    \
+    {                                                                           \
+        if (pieces) CUTE_FUSED_LAUNCH_AS(F, S, LL, COLUMNS, true);              \
+        else CUTE_FUSED_LAUNCH_AS(F, S, LL, COLUMNS, false);                    \
+    }
 #define CUTE_FUSED_LL(F, S)                                                     \
     switch (p->rows_logl) {                                                     \
-        case 0: CUTE_FUSED_LAUNCH(F, S, 0, false); break;                       \
-        case 1: CUTE_FUSED_LAUNCH(F, S, 1, false); break;                       \
-        case 2: CUTE_FUSED_LAUNCH(F, S, 2, false); break;                       \
-        case 3: CUTE_FUSED_LAUNCH(F, S, 3, false); break;                       \
+        case 0: CUTE_FUSED_LAUNCH(F, S, 0, false) break;                        \
+        case 1: CUTE_FUSED_LAUNCH(F, S, 1, false) break;                        \
+        case 2: CUTE_FUSED_LAUNCH(F, S, 2, false) break;                        \
+        case 3: CUTE_FUSED_LAUNCH(F, S, 3, false) break;                        \
         case 4:   /* by columns: sixteen lanes a row */                         \
-            if (p->columnSlabs) CUTE_FUSED_LAUNCH(F, S, 4, true);               \
-            else CUTE_FUSED_LAUNCH(F, S, 4, false);                             \
-            break;                             \
-        case 5: CUTE_FUSED_LAUNCH(F, S, 5, false); break;                       \
-        default: CUTE_FUSED_LAUNCH(F, S, 6, false); break;                             \
+            if (p->columnSlabs) CUTE_FUSED_LAUNCH(F, S, 4, true)                \
+            else CUTE_FUSED_LAUNCH(F, S, 4, false)                              \
+            break;                                                              \
+        case 5: CUTE_FUSED_LAUNCH(F, S, 5, false) break;                        \
+        default: CUTE_FUSED_LAUNCH(F, S, 6, false) break;                       \
     }
             if (full && strips) { CUTE_FUSED_LL(true, true) }
             else if (full) { CUTE_FUSED_LL(true, false) }
@@ -2456,26 +2474,31 @@ int run_with(const cute_spmm_plan *p, const float *dB, float *dC, void *stream, 
             else { CUTE_FUSED_LL(false, false) }
 #undef CUTE_FUSED_LL
 #undef CUTE_FUSED_LAUNCH
+#undef CUTE_FUSED_LAUNCH_AS
             rows_launched = true;
         } else if (p->halfLists) {
-            if (strips)
-                hipLaunchKernelGGL(cute_dev::hrpb_quad_half_f32<true>, grid, block, 0, s, p->dHeads, p->info.numChunks, per_xcd, p->d->dQRecs,
-                                   p->d->dQVals, uint32_t(p->d->numQuadVals), dB, dC, partials, N, p->columnSlabs, cut);
-            else
-                hipLaunchKernelGGL(cute_dev::hrpb_quad_half_f32<false>, grid, block, 0, s, p->dHeads, p->info.numChunks, per_xcd, p->d->dQRecs,
-                                   p->d->dQVals, uint32_t(p->d->numQuadVals), dB, dC, partials, N, p->columnSlabs, cut);
+#define CUTE_HALF_LAUNCH(S, CUT)                                                                                         \
+    hipLaunchKernelGGL((cute_dev::hrpb_quad_half_f32<S, CUT>), grid, block, 0, s, p->dHeads, p->info.numChunks, per_xcd, p->d->dQRecs, \
+                       p->d->dQVals, uint32_t(p->d->numQuadVals), dB, dC, partials, N, p->columnSlabs, cut)
+            if (strips && pieces) CUTE_HALF_LAUNCH(true, true);
+            else if (strips) CUTE_HALF_LAUNCH(true, false);
+            else if (pieces) CUTE_HALF_LAUNCH(false, true);
+            else CUTE_HALF_LAUNCH(false, false);
+#undef CUTE_HALF_LAUNCH
         } else {
-#define CUTE_QUAD_LAUNCH(F, S)                                                                                          \
-    if (p->columnSlabs)                                                                                                 \
-        hipLaunchKernelGGL((cute_dev::hrpb_quad_f32<F, S, true>), grid, block, 0, s, p->dHeads, p->info.numChunks, per_xcd,  \
-                           p->d->dQRecs, p->d->dQVals, uint32_t(p->d->numQuadVals), dB, dC, partials, N, p->columnSlabs, cut);   \
-    else                                                                                                                \
-        hipLaunchKernelGGL((cute_dev::hrpb_quad_f32<F, S, false>), grid, block, 0, s, p->dHeads, p->info.numChunks, per_xcd, \
-                           p->d->dQRecs, p->d->dQVals, uint32_t(p->d->numQuadVals), dB, dC, partials, N, 0u, cut)
+#define CUTE_QUAD_LAUNCH_AS(F, S, COLUMNS, CUT)                                                                          \
+    hipLaunchKernelGGL((cute_dev::hrpb_quad_f32<F, S, COLUMNS, CUT>), grid, block, 0, s, p->dHeads, p->info.numChunks, per_xcd, \
+                       p->d->dQRecs, p->d->dQVals, uint32_t(p->d->numQuadVals), dB, dC, partials, N, p->columnSlabs, cut)
+#define CUTE_QUAD_LAUNCH(F, S)                                                  \
+    if (p->columnSlabs && pieces) CUTE_QUAD_LAUNCH_AS(F, S, true, true);        \
+    else if (p->columnSlabs) CUTE_QUAD_LAUNCH_AS(F, S, true, false);            \
+    else if (pieces) CUTE_QUAD_LAUNCH_AS(F, S, false, true);                    \
+    else CUTE_QUAD_LAUNCH_AS(F, S, false, false)
             if (full && strips) { CUTE_QUAD_LAUNCH(true, true); }
             else if (full) { CUTE_QUAD_LAUNCH(true, false); }
             else if (strips) { CUTE_QUAD_LAUNCH(false, true); }
             else { CUTE_QUAD_LAUNCH(false, false); }
+#undef CUTE_QUAD_LAUNCH_AS
 #undef CUTE_QUAD_LAUNCH
         }
     } else if (p->info.numChunks) {

@@ -215,7 +215,9 @@ __device__ __forceinline__ BrickItem brick_item(const uint4 *__restrict__ chunks
 // counter returns to zero by itself (atomicInc wraps), so the next launch finds it as this one did.  What a piece stores for
 // others, and what it reads of theirs, passes by the XCD's own L2 (agent-scope accesses): counting in then needs the stores to have
 // arrived, not the write-back of everything the L2 holds that a device-wide release is on this part (which made counting in 1.1 to 5.5
-// times slower than a second launch).
+// times slower than a second launch).  A plan without cut panels runs the kernels that are compiled without any of this (CUT = false): the branch and
+// the registers behind it cost 0.5 to 1 % of a short launch (9-point stencil of 200 x 200 points, N = 101, 11.37 -> 11.45 us; hrpb_quad_half_f32 46 -> 50
+// vector registers).
 // With a second launch (reduce_partials), as calls whose scratch comes without counters and kernels that are no plan's default have it, and
 // without, us: R-MAT graph of 131 072 nodes, N = 64 45.0 / 44.0; 65 536 nodes, N = 47 26.6 / 23.9.
 // ---------------------------------------------------------------------------------------
@@ -494,12 +496,12 @@ __device__ __forceinline__ void brick_store_piece(const BrickItem &it, const f32
 }
 
 // C tile of one item, addressed like the loads: 32-bit byte offsets from a scalar base.
-template <int VEC, int NG, bool FULL>
+template <int VEC, int NG, bool FULL, bool CUT>
 __device__ __forceinline__ void brick_store_lean(const BrickItem &it, const f32x4 (&acc)[NG][VEC], float *__restrict__ C,
                                                  float *__restrict__ partials, uint32_t N, uint32_t lane, const CutPieces *__restrict__ cut)
 {
     typedef typename Vec<VEC>::type V;
-    if (it.piece) return brick_store_piece<VEC, NG, FULL>(it, acc, C, partials, N, cut);
+    if (CUT && it.piece) return brick_store_piece<VEC, NG, FULL>(it, acc, C, partials, N, cut);
     char *out_base = reinterpret_cast<char *>(C);
     const uint32_t row0 = it.panel * 16u + (lane >> 4) * 4u;
 #pragma unroll
@@ -523,7 +525,7 @@ __device__ __forceinline__ void brick_store_lean(const BrickItem &it, const f32x
 // budget is small enough that a launch of short panels is resident as a whole.  Padding-only
 // bricks skip their MFMAs.  NG = 2 lets one wavefront cover two column groups, which halves the
 // header traffic and shares the A-side index arithmetic between them.
-template <int VEC, int NG, bool FULL>
+template <int VEC, int NG, bool FULL, bool CUT>
 __device__ __forceinline__ void brick_rolling_body(uint32_t block_x, uint32_t block_y, const uint4 *__restrict__ chunks,
                                                    uint32_t num_chunks, uint32_t groups_per_xcd,
                                                    const uint32_t *__restrict__ hdr, const float *__restrict__ vals,
@@ -546,7 +548,7 @@ __device__ __forceinline__ void brick_rolling_body(uint32_t block_x, uint32_t bl
         for (int v = 0; v < VEC; ++v) acc[ng][v] = f32x4(0.0f);
 
     uint32_t blk = it.start;
-    if (blk < end) {
+    if (__builtin_expect(blk < end, true)) {     // (an empty item's code would stand in front of everybody's first fetch)
         V b[4][NG];
         float a[4];
         uint64_t bitmap[4];
@@ -554,6 +556,7 @@ __device__ __forceinline__ void brick_rolling_body(uint32_t block_x, uint32_t bl
         {
             const LeanHeader h0 = load_lean_header(hdr, blk, lane);
             h1 = load_lean_header(hdr, min(blk + 1, end - 1), lane);
+            __builtin_amdgcn_sched_barrier(0);       // both lines are asked for before the first is waited for (9-point stencil of 200 x 200 points, N = 101: 9.75 -> 9.5 us)
             // h1's load must be complete before the loop is entered.  The wait in front of its first use in
             // the loop is compiled once for both ways into the loop; were the load still in flight here (the
             // compiler would sink it behind the operand loads below), that wait would allow only two younger
@@ -596,16 +599,16 @@ __device__ __forceinline__ void brick_rolling_body(uint32_t block_x, uint32_t bl
                     acc[ng][v] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], vec_get<VEC>(b[j][ng], v), acc[ng][v], 0, 0, 0);
         }
     }
-    brick_store_lean<VEC, NG, FULL>(it, acc, C, partials, N, lane, cut);
+    brick_store_lean<VEC, NG, FULL, CUT>(it, acc, C, partials, N, lane, cut);
 }
 
-template <int VEC, int NG, bool FULL, bool COLUMNS>
+template <int VEC, int NG, bool FULL, bool COLUMNS, bool CUT>
 __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, (NG == 1 ? 8 : 4)) void hrpb_brick_f32_rolling(
     const uint4 *__restrict__ chunks, uint32_t num_chunks, uint32_t groups_per_xcd, const uint32_t *__restrict__ hdr,
     const float *__restrict__ vals, uint32_t zero_index, const float *__restrict__ B, float *__restrict__ C,
     float *__restrict__ partials, uint32_t N, uint32_t column_slabs, const CutPieces *__restrict__ cut)
 {
-    brick_rolling_body<VEC, NG, FULL>(blockIdx.x, blockIdx.y, chunks, num_chunks, groups_per_xcd, hdr, vals, zero_index, B, C,
+    brick_rolling_body<VEC, NG, FULL, CUT>(blockIdx.x, blockIdx.y, chunks, num_chunks, groups_per_xcd, hdr, vals, zero_index, B, C,
                                       partials, N, COLUMNS ? column_slabs : 0u, cut);
 }
 
@@ -668,7 +671,7 @@ __device__ __forceinline__ void mfma_block_bf16x3(const Bf16Operands<NG> &o, f32
         }
 }
 
-template <int NG, bool FULL, bool COLUMNS>
+template <int NG, bool FULL, bool COLUMNS, bool CUT>
 __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, (NG == 1 ? 6 : 4)) void hrpb_brick_bf16x3(
     const uint4 *__restrict__ chunks, uint32_t num_chunks, uint32_t groups_per_xcd, const uint32_t *__restrict__ hdr,
     const float *__restrict__ vals, uint32_t zero_index, const float *__restrict__ B, float *__restrict__ C,
@@ -690,7 +693,7 @@ __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, (NG == 1 ? 6 : 4)) void 
         for (int v = 0; v < VEC; ++v) acc[ng][v] = f32x4(0.0f);
 
     uint32_t blk = it.start;
-    if (blk < end) {
+    if (__builtin_expect(blk < end, true)) {     // (an empty item's code would stand in front of everybody's first fetch)
         f32x4 b[4][NG];
         float a[4];
         LeanHeader h1;
@@ -718,7 +721,7 @@ __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, (NG == 1 ? 6 : 4)) void 
         split_block<NG>(o, a, b);
         mfma_block_bf16x3<NG>(o, acc);
     }
-    brick_store_lean<VEC, NG, FULL>(it, acc, C, partials, N, lane, cut);
+    brick_store_lean<VEC, NG, FULL, CUT>(it, acc, C, partials, N, lane, cut);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -760,13 +763,13 @@ __device__ __forceinline__ float quad_load_b(const float *__restrict__ B, uint32
     return *reinterpret_cast<const float *>(reinterpret_cast<const char *>(B) + (__umul24(col, row_pitch) + col_off));
 }
 
-template <bool FULL, bool STRIPS, bool HUB>
+template <bool FULL, bool STRIPS, bool HUB, bool CUT>
 __device__ __forceinline__ void quad_chunk(uint32_t chunk, uint32_t block_y, const uint32_t *__restrict__ heads,
                                            const uint32_t *__restrict__ qrecs, const float *__restrict__ qvals, uint32_t zero_index,
                                            const float *__restrict__ B, float *__restrict__ C, float *__restrict__ partials,
                                            uint32_t N, const CutPieces *__restrict__ cut, const float *hub);
 
-template <bool FULL, bool STRIPS>
+template <bool FULL, bool STRIPS, bool CUT>
 __device__ __forceinline__ void quad_body(uint32_t block_x, uint32_t block_y, const uint32_t *__restrict__ heads,
                                           uint32_t num_chunks, uint32_t groups_per_xcd, const uint32_t *__restrict__ qrecs,
                                           const float *__restrict__ qvals, uint32_t zero_index,
@@ -777,10 +780,10 @@ __device__ __forceinline__ void quad_body(uint32_t block_x, uint32_t block_y, co
     const uint32_t x = xcd_share(block_x, block_y, column_slabs);
     const uint32_t chunk = (x * groups_per_xcd + block_x / kNumXcd) * kWavesPerGroup + wave;
     if (chunk >= num_chunks) return;
-    quad_chunk<FULL, STRIPS, false>(chunk, block_y, heads, qrecs, qvals, zero_index, B, C, partials, N, cut, nullptr);
+    quad_chunk<FULL, STRIPS, false, CUT>(chunk, block_y, heads, qrecs, qvals, zero_index, B, C, partials, N, cut, nullptr);
 }
 
-template <bool FULL, bool STRIPS, bool HUB>
+template <bool FULL, bool STRIPS, bool HUB, bool CUT>
 __device__ __forceinline__ void quad_chunk(uint32_t chunk, uint32_t block_y, const uint32_t *__restrict__ heads,
                                            const uint32_t *__restrict__ qrecs, const float *__restrict__ qvals, uint32_t zero_index,
                                            const float *__restrict__ B, float *__restrict__ C, float *__restrict__ partials,
@@ -886,7 +889,7 @@ __device__ __forceinline__ void quad_chunk(uint32_t chunk, uint32_t block_y, con
 #undef CUTE_QUAD_ROLL_REST
 #undef CUTE_QUAD_MFMA16
     }
-    if (!HUB && piece) {      // (the partials matrix: rows (piece-1)*16.., same pitch as C)
+    if (CUT && !HUB && piece) {      // (the partials matrix: rows (piece-1)*16.., same pitch as C)
         constexpr int E = STRIPS ? 4 : 16;
         float mine[E];
         const f32x4 sum = (acc[0] + acc[1]) + (acc[2] + acc[3]);
@@ -924,13 +927,13 @@ __device__ __forceinline__ void quad_chunk(uint32_t chunk, uint32_t block_y, con
     }
 }
 
-template <bool FULL, bool STRIPS, bool COLUMNS>
+template <bool FULL, bool STRIPS, bool COLUMNS, bool CUT>
 __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, 8) void hrpb_quad_f32(
     const uint32_t *__restrict__ heads, uint32_t num_chunks, uint32_t groups_per_xcd, const uint32_t *__restrict__ qrecs,
     const float *__restrict__ qvals, uint32_t zero_index, const float *__restrict__ B, float *__restrict__ C,
     float *__restrict__ partials, uint32_t N, uint32_t column_slabs, const CutPieces *__restrict__ cut)
 {
-    quad_body<FULL, STRIPS>(blockIdx.x, blockIdx.y, heads, num_chunks, groups_per_xcd, qrecs, qvals, zero_index, B, C,
+    quad_body<FULL, STRIPS, CUT>(blockIdx.x, blockIdx.y, heads, num_chunks, groups_per_xcd, qrecs, qvals, zero_index, B, C,
                             partials, N, COLUMNS ? column_slabs : 0u, cut);
 }
 
@@ -958,7 +961,7 @@ __device__ __forceinline__ float add_halves(float lo, float hi)
     return __uint_as_float(s[0]) + __uint_as_float(s[1]);
 }
 
-template <bool STRIPS>
+template <bool STRIPS, bool CUT>
 __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, 8) void hrpb_quad_half_f32(
     const uint32_t *__restrict__ heads, uint32_t num_chunks, uint32_t groups_per_xcd, const uint32_t *__restrict__ qrecs,
     const float *__restrict__ qvals, uint32_t zero_index, const float *__restrict__ B, float *__restrict__ C,
@@ -977,6 +980,7 @@ __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, 8) void hrpb_quad_half_f
     uint32_t ca[kQuadRecordWords], cb[kQuadRecordWords];       // as in quad_chunk
 #pragma unroll
     for (int p = 0; p < kQuadRecordWords; ++p) ca[p] = head[4 + p];
+    asm volatile("" ::"s"(ca[11]), "s"(ca[12]), "s"(ca[15]), "s"(ca[16]), "s"(ca[17]), "s"(ca[18]));
 
     const uint32_t n = slab * kHalf + (lane & (kHalf - 1));
     const bool live = n < N;
@@ -1051,18 +1055,26 @@ __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, 8) void hrpb_quad_half_f
 #undef CUTE_HALF_ROLL_REST
 #undef CUTE_HALF_MFMA8
     }
-    // the lane's rows of the tile: rows `half` and up, for the halves' sums of rows i and i + E
+    // a lane's rows of the tile: those from first_row on, each the halves' sums of rows e and e + E
     constexpr int E = STRIPS ? 2 : 8;
     const uint32_t first_row = upper & uint32_t(E);
     const f32x4 sum = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-    float mine[E];
+    auto row = [&](int e) { return STRIPS ? add_halves(sum[e], sum[(e + 2) % 4]) : add_halves(acc[e / 4][e % 4], acc[(e / 4 + 2) % 4][e % 4]); };
+    if (CUT && piece) {
+        float mine[E];
 #pragma unroll
-    for (int e = 0; e < E; ++e) mine[e] = STRIPS ? add_halves(sum[e], sum[(e + 2) % 4]) : add_halves(acc[e / 4][e % 4], acc[(e / 4 + 2) % 4][e % 4]);
-    auto at = [&](uint32_t unit, int e) { return __umul24(unit * uint32_t(2 * E) + first_row + uint32_t(e), row_pitch) + col_off; };
-    if (piece) store_piece(cut, piece, slab, mine, at, [&](int) { return live; }, partials, C);
-    else if (live)
+        for (int e = 0; e < E; ++e) mine[e] = row(e);
+        auto at = [&](uint32_t unit, int e) { return __umul24(unit * uint32_t(2 * E) + first_row + uint32_t(e), row_pitch) + col_off; };
+        store_piece(cut, piece, slab, mine, at, [&](int) { return live; }, partials, C);
+        return;
+    }
+    uint32_t off = __umul24(panel * uint32_t(2 * E) + first_row, row_pitch) + n * 4u;
 #pragma unroll
-        for (int e = 0; e < E; ++e) __builtin_nontemporal_store(mine[e], reinterpret_cast<float *>(reinterpret_cast<char *>(C) + at(panel, e)));
+    for (int e = 0; e < E; ++e) {
+        const float v = row(e);
+        if (live) __builtin_nontemporal_store(v, reinterpret_cast<float *>(reinterpret_cast<char *>(C) + off));
+        off += row_pitch;
+    }
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1092,7 +1104,7 @@ __global__ __launch_bounds__(kWaveSize *kHubWaves) void hrpb_quad_hub_f32(
     // consecutive chunks of the list (longest first) go to different work-groups
     const uint32_t stride = gridDim.x * kHubWaves;
     for (uint32_t chunk = wave * gridDim.x + blockIdx.x; chunk < num_chunks; chunk += stride)
-        quad_chunk<FULL, true, true>(chunk, blockIdx.y, heads, qrecs, qvals, zero_index, B, C, partials, N, nullptr, hub);
+        quad_chunk<FULL, true, true, true>(chunk, blockIdx.y, heads, qrecs, qvals, zero_index, B, C, partials, N, nullptr, hub);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1649,7 +1661,7 @@ __global__ __launch_bounds__(1024) void csr_rows_window(const uint4 *__restrict_
 // leave idle.  Blocks [0, quad_blocks) are the quad kernel's 2-D grid flattened (x fastest, so the
 // XCD of a block is still x % 8); the rest are the row kernel's blocks, dealt to the XCDs in
 // contiguous ranges like the row kernel's own launch does.
-template <bool FULL, bool STRIPS, int LOG_L, bool COLUMNS>
+template <bool FULL, bool STRIPS, int LOG_L, bool COLUMNS, bool CUT>
 __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, 8) void hrpb_quad_rows_f32(
     uint32_t quad_blocks_x, uint32_t quad_blocks, const uint32_t *__restrict__ heads, uint32_t num_chunks,
     uint32_t groups_per_xcd, const uint32_t *__restrict__ qrecs, const float *__restrict__ qvals, uint32_t zero_index,
@@ -1659,7 +1671,7 @@ __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, 8) void hrpb_quad_rows_f
 {
     static_assert(kWaveSize * kWavesPerGroup == 256, "both bodies are written for 256-thread blocks");
     if (blockIdx.x < quad_blocks) {
-        quad_body<FULL, STRIPS>(blockIdx.x % quad_blocks_x, blockIdx.x / quad_blocks_x, heads, num_chunks, groups_per_xcd,
+        quad_body<FULL, STRIPS, CUT>(blockIdx.x % quad_blocks_x, blockIdx.x / quad_blocks_x, heads, num_chunks, groups_per_xcd,
                                 qrecs, qvals, zero_index, B, C, partials, N, COLUMNS ? column_slabs : 0u, cut);
     } else {   // quad_blocks is a multiple of the XCD count, so the XCD of a row block is (its index) % 8 as well
         const uint32_t rb = blockIdx.x - quad_blocks;
@@ -1673,7 +1685,7 @@ __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, 8) void hrpb_quad_rows_f
 }
 
 // The same for a plan that pairs the rolling brick kernel with the row kernel.
-template <int VEC, int NG, bool FULL, int LOG_L, bool COLUMNS>
+template <int VEC, int NG, bool FULL, int LOG_L, bool COLUMNS, bool CUT>
 __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, (NG == 1 ? 8 : 4)) void hrpb_brick_rows_f32(
     uint32_t brick_blocks_x, uint32_t brick_blocks, const uint4 *__restrict__ chunks, uint32_t num_chunks,
     uint32_t groups_per_xcd, const uint32_t *__restrict__ hdr, const float *__restrict__ tile_vals, uint32_t zero_index,
@@ -1682,7 +1694,7 @@ __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, (NG == 1 ? 8 : 4)) void 
     const float *__restrict__ B, float *__restrict__ C, float *__restrict__ partials, uint32_t N, const CutPieces *__restrict__ cut)
 {
     if (blockIdx.x < brick_blocks) {
-        brick_rolling_body<VEC, NG, FULL>(blockIdx.x % brick_blocks_x, blockIdx.x / brick_blocks_x, chunks, num_chunks,
+        brick_rolling_body<VEC, NG, FULL, CUT>(blockIdx.x % brick_blocks_x, blockIdx.x / brick_blocks_x, chunks, num_chunks,
                                           groups_per_xcd, hdr, tile_vals, zero_index, B, C, partials, N, COLUMNS ? column_slabs : 0u, cut);
     } else {
         const uint32_t rb = blockIdx.x - brick_blocks;

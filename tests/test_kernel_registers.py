@@ -28,3 +28,10 @@ def test_two_work_groups_of_the_hub_kernel_fit_a_compute_unit():
     columns it has always taken 65.)"""
     hub = {k: n for k, n in _kernels(b"vgpr_count").items() if "hrpb_quad_hub_f32ILb1E" in k}
     assert list(hub.values()) == [64], hub
+
+
+def test_plans_without_cut_panels_carry_no_registers_for_pieces():
+    """The kernels are compiled without the pieces of cut panels as well (the last template argument); 32-column lists take 46 registers that way."""
+    half = {k: n for k, n in _kernels(b"vgpr_count").items() if "hrpb_quad_half_f32" in k}
+    uncut = [n for k, n in half.items() if re.search(r"ILb[01]ELb0EE", k)]
+    assert len(half) == 4 and len(uncut) == 2 and max(uncut) <= 46, half
