@@ -222,6 +222,7 @@ __device__ __forceinline__ BrickItem brick_item(const uint4 *__restrict__ chunks
 // without, us: R-MAT graph of 131 072 nodes, N = 64 45.0 / 44.0; 65 536 nodes, N = 47 26.6 / 23.9.
 // ---------------------------------------------------------------------------------------
 constexpr uint32_t kPiecesAtOnce = 8;
+constexpr uint32_t kEightsOfOne = 2;          // up to so many eights the last piece of all adds them up, and nobody an eight
 
 struct CutPieces {             // in device memory: an argument more would be in registers from a wavefront's start
     const uint4 *of_piece;     // {first piece of the unit, pieces, first counter, unit}
@@ -229,8 +230,24 @@ struct CutPieces {             // in device memory: an argument more would be in
     uint64_t slabs;
 };
 
-__device__ __forceinline__ void store_shared(float *p, float x) { __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-__device__ __forceinline__ float load_shared(const float *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+// Loads and stores of W columns with the scope bit that the compiler gives agent-scope atomics (sc1), which the language has for single words only.  A word
+// a lane, bricks of two or four columns left every line in pieces that memory has to put together: R-MAT graph of 32 768 nodes and 9 edges a node, N = 84, bf16x3
+// 58.9 us, 16 384 nodes and 4 edges, N = 24 13.5; with whole vectors 35.6 ... 36.5 and 8.9 ... 9.3 (a second launch instead: 36.5 and 9.5).
+constexpr int kAgentScope = 16;
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t shared_tiles(float *partials) { return __builtin_amdgcn_make_buffer_rsrc(partials, 0, ~0u, 0x00020000); }
+template <int W> __device__ __forceinline__ typename Vec<W>::type load_shared(float *partials, uint32_t at, uint32_t further)
+{
+    if constexpr (W == 4) return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(shared_tiles(partials), at, further, kAgentScope));
+    else if constexpr (W == 2) return __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(shared_tiles(partials), at, further, kAgentScope));
+    else return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(shared_tiles(partials), at, further, kAgentScope));
+}
+template <int W> __device__ __forceinline__ void store_shared(float *partials, uint32_t at, const typename Vec<W>::type &x)
+{
+    if constexpr (W == 4) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), shared_tiles(partials), at, 0, kAgentScope);
+    else if constexpr (W == 2) __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, x), shared_tiles(partials), at, 0, kAgentScope);
+    else __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x), shared_tiles(partials), at, 0, kAgentScope);
+}
 
 // The lane, without a register that holds it: what the end of a piece needs is not kept through its main loop.
 __device__ __forceinline__ uint32_t lane_again() { return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
@@ -246,35 +263,59 @@ __device__ __forceinline__ bool last_to_arrive(uint32_t *counter, uint32_t membe
     return last;
 }
 
-// sum (of `count` values so far), then value(0) .. value(n - 1) one after the other; n is up to kPiecesAtOnce
-template <class Value> __device__ __forceinline__ float add_pieces(float sum, bool none_so_far, uint32_t n, Value value)
+// sum (of the values so far), then v[0] .. v[n - 1] one after the other
+template <class T> __device__ __forceinline__ T add_pieces(T sum, bool none_so_far, uint32_t n, const T (&v)[kPiecesAtOnce])
 {
-    float v[kPiecesAtOnce];
-#pragma unroll
-    for (uint32_t k = 0; k < kPiecesAtOnce; ++k) v[k] = value(min(k, n - 1u));
 #pragma unroll
     for (uint32_t k = 0; k < kPiecesAtOnce; ++k) {
-        const float next = k == 0u && none_so_far ? v[0] : sum + v[k];
+        const T next = k == 0u && none_so_far ? v[0] : sum + v[k];
         sum = k < n ? next : sum;
     }
     return sum;
 }
 
-// A lane's part of the tile of a piece: E elements, at(unit, e) the byte offset of element e of tile (or panel, or strip) `unit`.
-// Near the last column two lanes, or two elements of one, hold the same sum: owned(e) is true for one of them.  (The sums of an eight
-// stand where its first tile does, so a place that was read again after it was written would count twice.)
-template <int E, class At, class Owned>
-__device__ __forceinline__ void store_piece(const CutPieces *__restrict__ cut, uint32_t piece, uint32_t slab, const float (&mine)[E], At at, Owned owned,
-                                            float *__restrict__ partials, float *__restrict__ C)
+// A lane's part of the tile of a piece: E vectors of W columns, at(unit, e) the byte offset of vector e of tile (or panel, or strip) `unit`.  Near the last
+// column two lanes, or two vectors of one, hold the same columns: the last own(e) of a vector are the lane's.  (The sums of an eight
+// stand where its first tile does, so a place that was read again after it was written would count twice.)  pitch: bytes from a tile to the next; ragged: a
+// vector may be partly owned.
+template <int W, int E, class At, class Own>
+__device__ __forceinline__ void store_piece(const CutPieces *__restrict__ cut, uint32_t piece, uint32_t slab, const typename Vec<W>::type (&mine)[E], At at, Own own,
+                                            uint32_t pitch, bool ragged, float *__restrict__ partials, float *__restrict__ C)
 {
-    char *const tiles = reinterpret_cast<char *>(partials);
-    auto element = [&](uint32_t tile, int e) { return reinterpret_cast<float *>(tiles + at(tile, e)); };
+    typedef typename Vec<W>::type V;
+    float *tiles = partials;
+    asm volatile("" : "+s"(tiles));        // other wavefronts write here too: not the argument that nothing else points to
+    auto put = [&](uint32_t unit, int e, const V &v, auto whole, auto word) {
+        const uint32_t n = own(e);
+        if (n == uint32_t(W)) whole(at(unit, e), v);
+        if constexpr (W > 1)
+            if (ragged)
+#pragma unroll
+                for (int j = 1; j < W; ++j)
+                    if (n < uint32_t(W) && uint32_t(W - j) <= n) word(at(unit, e) + uint32_t(j) * 4u, vec_get<W>(v, j));
+    };
+    auto to_tile = [&](uint32_t tile, int e, const V &v) {
+        put(tile, e, v, [&](uint32_t to, const V &x) { store_shared<W>(tiles, to, x); }, [&](uint32_t to, float x) { store_shared<1>(tiles, to, x); });
+    };
+    auto to_c = [&](uint32_t unit, int e, const V &v) {
+        char *const c = reinterpret_cast<char *>(C);
+        put(unit, e, v, [&](uint32_t to, const V &x) { store_vec_streaming<W>(x, c + to); },
+            [&](uint32_t to, float x) { __builtin_nontemporal_store(x, reinterpret_cast<float *>(c + to)); });
+    };
+    // (a fence behind a few stores, or the addresses of all of them take registers first)
+    if (!cut) {               // a second launch reads them; columns that two lanes hold get the same bits twice
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            if (own(e)) store_vec_streaming<W>(mine[e], reinterpret_cast<char *>(partials) + at(piece - 1u, e));
+            if (W > 1 || e % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+        }
+        return;
+    }
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-        if (owned(e)) store_shared(element(piece - 1u, e), mine[e]);
-        if (e % 4 == 3) __builtin_amdgcn_sched_barrier(0);     // (or the addresses of all of them take registers first)
+        to_tile(piece - 1u, e, mine[e]);
+        if (W > 1 || e % 4 == 3) __builtin_amdgcn_sched_barrier(0);
     }
-    if (!cut) return;
     const uint4 of = cut->of_piece[piece - 1u];
     uint32_t *const counters = cut->counters + slab;
     const uint32_t slabs = uint32_t(cut->slabs);
@@ -282,37 +323,56 @@ __device__ __forceinline__ void store_piece(const CutPieces *__restrict__ cut, u
                    counter = __builtin_amdgcn_readfirstlane(of.z), unit = __builtin_amdgcn_readfirstlane(of.w);
     const uint32_t eights = (pieces + kPiecesAtOnce - 1u) / kPiecesAtOnce, eight = (piece - 1u - first) / kPiecesAtOnce,
                    tile0 = first + eight * kPiecesAtOnce, members = min(kPiecesAtOnce, pieces - eight * kPiecesAtOnce);
-    if (!last_to_arrive(counters + size_t(counter + eight) * slabs, members)) return;
-    // (one loop for every E, a few elements a turn: the tile is not held in registers again)
-    constexpr int kTurn = E <= 4 ? E : 2;
-    auto to_c = [&](int e, float x) { __builtin_nontemporal_store(x, reinterpret_cast<float *>(reinterpret_cast<char *>(C) + at(unit, e))); };
+    // (one loop for every E, a few words of a lane a turn: the tile is not held in registers again)
+    constexpr int kTurn = W == 4 && E == 4 ? 1 : W == 1 && E == 4 ? 4 : 2;
+    static_assert(E % kTurn == 0, "whole turns");
+    // the turn's vectors of n tiles, `apart` bytes from one to the next, added up: all are on their way before the first is added
+    auto add_all = [&](int e0, V (&sum)[kTurn], bool none_so_far, uint32_t n, uint32_t tile, uint32_t apart) {
+        V v[kTurn][kPiecesAtOnce];
+        uint32_t further = 0;          // (behind the last the same again)
+#pragma unroll
+        for (uint32_t k = 0; k < kPiecesAtOnce; ++k) {
+#pragma unroll
+            for (int e = 0; e < kTurn; ++e) v[e][k] = load_shared<W>(tiles, at(tile, e0 + e), further);
+            further += k + 1u < n ? apart : 0u;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int e = 0; e < kTurn; ++e) sum[e] = add_pieces(sum[e], none_so_far, n, v[e]);
+    };
+    const bool by_eights = eights > kEightsOfOne;
+    if (by_eights) {
+        if (!last_to_arrive(counters + size_t(counter + eight) * slabs, members)) return;
 #pragma unroll 1
-    for (int e0 = 0; e0 < E; e0 += kTurn) {
-        float sum[kTurn];
+        for (int e0 = 0; e0 < E; e0 += kTurn) {
+            V sum[kTurn];
 #pragma unroll
-        for (int e = 0; e < kTurn; ++e) sum[e] = add_pieces(0.0f, true, members, [&](uint32_t k) { return load_shared(element(tile0 + k, e0 + e)); });
+            for (int e = 0; e < kTurn; ++e) sum[e] = V(0.0f);
+            add_all(e0, sum, true, members, tile0, pitch);
 #pragma unroll
-        for (int e = 0; e < kTurn; ++e)
-            if (owned(e0 + e)) {
-                if (eights == 1u) to_c(e0 + e, sum[e]);
-                else store_shared(element(tile0, e0 + e), sum[e]);
-            }
+            for (int e = 0; e < kTurn; ++e) to_tile(tile0, e0 + e, sum[e]);
+        }
     }
-    if (eights == 1u || !last_to_arrive(counters + size_t(counter + eights) * slabs, eights)) return;
+    if (!last_to_arrive(counters + size_t(counter + eights) * slabs, by_eights ? eights : pieces)) return;
+    // the sums of the eights, or what they are the sums of
+    const uint32_t of_all = by_eights ? eights : pieces, apart = by_eights ? kPiecesAtOnce * pitch : pitch, step = by_eights ? kPiecesAtOnce * kPiecesAtOnce : kPiecesAtOnce;
 #pragma unroll 1
     for (int e0 = 0; e0 < E; e0 += kTurn) {
-        float sum[kTurn];
+        V sum[kTurn];
 #pragma unroll
-        for (int e = 0; e < kTurn; ++e) sum[e] = 0.0f;
+        for (int e = 0; e < kTurn; ++e) sum[e] = V(0.0f);
+        uint32_t tile = first;
 #pragma unroll 1
-        for (uint32_t base = 0; base < eights; base += kPiecesAtOnce)
+        for (uint32_t base = 0; base < of_all; base += kPiecesAtOnce, tile += step) {
+            V part[kTurn];
 #pragma unroll
-            for (int e = 0; e < kTurn; ++e)
-                sum[e] = add_pieces(sum[e], base == 0u, min(kPiecesAtOnce, eights - base),
-                                    [&](uint32_t k) { return load_shared(element(first + (base + k) * kPiecesAtOnce, e0 + e)); });
+            for (int e = 0; e < kTurn; ++e) part[e] = sum[e];
+            add_all(e0, part, !by_eights || base == 0u, min(kPiecesAtOnce, of_all - base), tile, apart);
 #pragma unroll
-        for (int e = 0; e < kTurn; ++e)
-            if (owned(e0 + e)) to_c(e0 + e, sum[e]);
+            for (int e = 0; e < kTurn; ++e) sum[e] = by_eights || base == 0u ? part[e] : sum[e] + part[e];
+        }
+#pragma unroll
+        for (int e = 0; e < kTurn; ++e) to_c(unit, e0 + e, sum[e]);
     }
 }
 
@@ -486,13 +546,17 @@ __device__ __forceinline__ void brick_store_piece(const BrickItem &it, const f32
                                                   float *__restrict__ partials, uint32_t N, const CutPieces *__restrict__ cut)
 {
     const uint32_t lane = lane_again(), col0 = it.slab * (16u * VEC * NG) + (lane & 15u) * VEC;
-    float mine[NG * 4 * VEC];
+    typename Vec<VEC>::type mine[NG * 4];        // four rows of each column group
 #pragma unroll
-    for (int e = 0; e < NG * 4 * VEC; ++e) mine[e] = acc[e / (4 * VEC)][e % VEC][e / VEC % 4];
-    auto first_of = [&](int e) { return col0 + uint32_t(e / (4 * VEC)) * 16u * VEC; };
-    auto column = [&](int e) { return (FULL ? first_of(e) : first_column<VEC>(first_of(e), N)) + uint32_t(e % VEC); };
-    auto at = [&](uint32_t unit, int e) { return __umul24(unit * 16u + (lane >> 4) * 4u + uint32_t(e / VEC % 4), N * 4u) + column(e) * 4u; };
-    store_piece(cut, it.piece, it.slab, mine, at, [&](int e) { return FULL || column(e) >= first_of(e); }, partials, C);
+    for (int e = 0; e < NG * 4; ++e)
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) vec_set<VEC>(mine[e], v, acc[e / 4][v][e % 4]);
+    auto column = [&](int e) { return col0 + uint32_t(e / 4) * 16u * VEC; };
+    auto at = [&](uint32_t unit, int e) {
+        return __umul24(unit * 16u + (lane >> 4) * 4u + uint32_t(e % 4), N * 4u) + (FULL ? column(e) : first_column<VEC>(column(e), N)) * 4u;
+    };
+    auto own = [&](int e) -> uint32_t { return FULL ? uint32_t(VEC) : column(e) < N ? min(N - column(e), uint32_t(VEC)) : 0u; };
+    store_piece<VEC>(cut, it.piece, it.slab, mine, at, own, 64u * N, !FULL && N % uint32_t(VEC) != 0u, partials, C);
 }
 
 // C tile of one item, addressed like the loads: 32-bit byte offsets from a scalar base.
@@ -502,6 +566,7 @@ __device__ __forceinline__ void brick_store_lean(const BrickItem &it, const f32x
 {
     typedef typename Vec<VEC>::type V;
     if (CUT && it.piece) return brick_store_piece<VEC, NG, FULL>(it, acc, C, partials, N, cut);
+    if (CUT) lane = lane_again();
     char *out_base = reinterpret_cast<char *>(C);
     const uint32_t row0 = it.panel * 16u + (lane >> 4) * 4u;
 #pragma unroll
@@ -897,7 +962,7 @@ __device__ __forceinline__ void quad_chunk(uint32_t chunk, uint32_t block_y, con
         for (int e = 0; e < E; ++e) mine[e] = STRIPS ? sum[e] : acc[e / 4][e % 4];
         const uint32_t column = block_y * kWaveSize + lane_again(), offset = min(column, N - 1u) * 4u;
         auto at = [&](uint32_t unit, int e) { return __umul24(unit * uint32_t(E) + uint32_t(e), N * 4u) + offset; };
-        store_piece(cut, piece, block_y, mine, at, [&](int) { return FULL || column < N; }, partials, C);
+        store_piece<1>(cut, piece, block_y, mine, at, [&](int) { return FULL || column < N ? 1u : 0u; }, uint32_t(E) * N * 4u, false, partials, C);
     } else if (live) {
         // (pieces of a hub plan are added up by reduce_partials: store_piece here takes hrpb_quad_hub_f32<true> from 64 to 65 vector registers, and a
         // compute unit then holds one of its work-groups instead of two)
@@ -1065,7 +1130,7 @@ __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, 8) void hrpb_quad_half_f
 #pragma unroll
         for (int e = 0; e < E; ++e) mine[e] = row(e);
         auto at = [&](uint32_t unit, int e) { return __umul24(unit * uint32_t(2 * E) + first_row + uint32_t(e), row_pitch) + col_off; };
-        store_piece(cut, piece, slab, mine, at, [&](int) { return live; }, partials, C);
+        store_piece<1>(cut, piece, slab, mine, at, [&](int) { return live ? 1u : 0u; }, uint32_t(2 * E) * row_pitch, false, partials, C);
         return;
     }
     uint32_t off = __umul24(panel * uint32_t(2 * E) + first_row, row_pitch) + n * 4u;
@@ -1240,11 +1305,17 @@ __global__ __launch_bounds__(kWaveSize *kReduceWaves) void reduce_partials(const
     const bool valid = e < tile;
     const float *src = partials + size_t(fx.y) * tile + (valid ? e : 0u);
     float total = 0.0f;
+    auto sum_of = [&](uint32_t piece0) {
+        const uint32_t n = min(kPiecesAtOnce, pieces - piece0);
+        float v[kPiecesAtOnce];
+#pragma unroll
+        for (uint32_t k = 0; k < kPiecesAtOnce; ++k) v[k] = src[size_t(piece0 + min(k, n - 1u)) * tile];
+        return add_pieces(0.0f, true, n, v);
+    };
     for (uint32_t base = 0; base < eights; base += G) {               // (a block works on one unit: the rounds are the same for all of it)
         const uint32_t eight = base + g, piece0 = eight * kPiecesAtOnce;
         float sum = 0.0f;
-        if (eight < eights)
-            sum = add_pieces(0.0f, true, min(kPiecesAtOnce, pieces - piece0), [&](uint32_t k) { return src[size_t(piece0 + k) * tile]; });
+        if (eight < eights) sum = sum_of(piece0);
         if (G == 1u) { total = sum; break; }
         sums[wave][lane] = sum;
         __syncthreads();
@@ -1376,7 +1447,9 @@ __device__ __forceinline__ void rows_batched_body(uint32_t block_id, uint32_t sl
         }
         if (AHEAD) mine = next;
     }
-    if (live) store_vec_streaming<VEC>(acc, C + size_t(row) * N + c0);
+    // (narrow groups work it out again: kept through the loop it took the register of the row's number in one of the fused kernels, which went to scratch)
+    const uint32_t column = slab * L * VEC + (AHEAD ? t : lane_again() & (L - 1)) * VEC;
+    if (AHEAD ? live : column < N) store_vec_streaming<VEC>(acc, C + size_t(row) * N + first_column<VEC>(column, N));
 }
 
 template <int VEC, int LOG_L, int BATCH, bool COLUMNS>

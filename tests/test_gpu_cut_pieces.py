@@ -70,3 +70,10 @@ def test_pieces_in_a_graph(cs, torch_cuda):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(eager, dC)
+
+
+@pytest.mark.parametrize("pieces,N", [(9, 5), (20, 6), (9, 24), (17, 27), (9, 65), (9, 66), (17, 67), (70, 68), (9, 129), (17, 131), (9, 257)])
+def test_vectors_at_the_last_columns(cs, orc, torch_cuda, pieces, N):
+    """Tiles travel by vectors of two and four columns.  A vector that would pass the last column is moved back over columns of the lane, the column group
+    or the slab before it: only what is its own may be written, or sums that stand in a first tile already count twice."""
+    test_pieces_add_up_alike(cs, orc, torch_cuda, pieces, N, 1)
