@@ -1933,10 +1933,19 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
             // A graph's bricks, which it has below 32 columns, are bound by their matrix work and are cut like a launch that does not fill the device
             // and is bound by its longest item: at twice the target, into pieces of one (17/10/16 51.0, 39.2, 39.2, 30.3; 16/8/16 19.7, 18.2,
             // 18.1, 18.1).  Wider bricks keep six shares and four: bf16x3 loses (16/10/128 85.4, 88.0, 88.2, 102), in fp32 they are
-            // those of even panels.  So do plans whose finer cut's tiles would not fit cute_spmm_run_static's scratch.
+            // those of even panels.  So do plans whose finer cut's tiles would not fit cute_spmm_run_static's scratch.  Who adds the pieces up does not
+            // turn the rule round: run_scratch, hub and pipelined plans, with a second launch, at six into fours / four into twos: 16/10/47 26.3, 24.2 and
+            // 17/10/64 45.9, 45.3 by run_scratch, 16/10/47 61.5, 42.9 and 17/10/64 91.5, 91.9 with 128 hub rows, 17/10/16 60.9, 36.7 pipelined.
+            // Lists of two column slabs: most strips to be cut are the few lengths of a graph's hub panels, and where two shares make four pieces of one
+            // (a work-group each) a launch of strips of more than 12 groups a share took up to 1.18 times the time of the coarser cut; twos of three shares do not, nor five fourths.
+            // us at six into fours, four into twos, now: 16/12/128 64.0, 75.7, 55.2; 16/9/101 53.1, 61.2, 47.0; 16/8/128 41.6, 43.0, 35.2; 15/12/128 28.0, 27.4,
+            // 23.2; 17/8/112 105, 88.0, 80.6; 17/8/128 78.3, 79.5, 78.7; 16/7/80 34.9, 28.9, 30.2.  With three slabs and more it gains and loses alike (16/12/144 91.6, 72.9, 76.6;
+            // 16/9/160 57.6 to 63.0; 16/6/200 0.77 times), and nothing was slower than with the coarser cut.
             const bool finer = attempt == 0 && (p->shape == 2 || N < 32u);
-            const uint32_t limit = uint32_t(std::max<uint64_t>(2u * uint64_t(target), (finer ? (p->shape == 2 ? 4u : 0u) : 6u) * share));
-            const uint32_t piece = limit > 2u * target ? uint32_t((finer ? 2u : 4u) * share) : target;
+            const bool two_slabs = finer && p->shape == 2 && num_slabs == 2u && share > 8u;
+            const uint64_t least_cut = two_slabs ? 3u : finer ? (p->shape == 2 ? 4u : 0u) : 6u;
+            const uint32_t limit = uint32_t(std::max<uint64_t>(2u * uint64_t(target), least_cut * share));
+            const uint32_t piece = limit <= 2u * target ? target : uint32_t(two_slabs && share > 12u ? share * 5u / 4u : (finer ? 2u : 4u) * share);
             chunks.resize(std::max<size_t>(chunks.capacity(), 64u));
             size_t at = 0;
             for (uint32_t q = 0; q < num_units; ++q) {
@@ -1968,7 +1977,8 @@ int cute_spmm_plan_create(cute_hrpb_dev *d, uint32_t N, const cute_tunables *tn,
         const bool lean = p->shape == 2 || p->pipeline == 1;
         const uint64_t tile_rows = uint64_t(n_pieces) * (CUTE_TM >> upp_log);
         const bool fits = !lean || !n_pieces || cute_offsets_fit(d->M, d->K, N, 0, tile_rows) == 1;
-        if (attempt == 0 && (!fits || tile_rows * N * sizeof(float) > uint64_t(CUTE_STATIC_SCRATCH_BYTES))) continue;
+        // (with the default cut there are at most as many pieces as wavefronts, 32 MiB of tiles; max_chunk_blocks can add to them)
+        if (attempt == 0 && !t.slots && (p->shape == 2 || N < 32u) && (!fits || tile_rows * N * sizeof(float) > uint64_t(CUTE_STATIC_SCRATCH_BYTES))) continue;
         if (fits) break;
         if (attempt == 2 || t.mfma_shape == 2 || t.pipeline == 1) { delete p; return CUTE_ERR_SHAPE; }   // the caller forced a fast kernel
         attempt = 1;
