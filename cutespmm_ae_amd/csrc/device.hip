@@ -1316,6 +1316,12 @@ int make_hub_tables(cute_spmm_plan *p, const cute_hrpb_dev *d, uint32_t hub_rows
 // panel: R-MAT graph of 32 768 nodes, N = 1 13.3 / 84, 43, 24, 14.  And the brick kernel, which fetches a row of B once for all rows of a panel, is ahead
 // from three columns on where rows share columns and the launch no longer fits the device at once: finite elements, 48 000 rows, brick kernel / 16
 // groups: N = 1 9.3 / 6.2, N = 3 9.3 / 9.9, N = 8 9.3 / 10.3; 500 000 rows of 32 in a band, N = 8 64.5 / 61.8.
+// Nor, up to 55 entries a row, between launches that leave wavefront slots free (190 000 lanes) and matrices so large that the row kernel is slow, where a group
+// more a row is more wavefronts and loads for the same entries: rows in a wide band, which share few columns, with two lanes a group (3 and 5 to 8 columns) or short
+// rows and N = 4; bands of any width with two lanes where the groups' last turn leaves a lane in seven or more idle; columns at random, none shared, for N = 1 alone.
+// Row kernel / groups: two lanes, N = 8, band of 400, 64 000 rows of 24 5.25 / 5.91, of 48 8.55 / 9.59, of 32 (every lane busy) 6.60 / 6.44, 128 000 of 24 8.51 / 10.05; band of
+// 2 048, N = 5, 64 000 of 48 9.61 / 12.08, 32 000 of 32, N = 7 5.38 / 6.13; N = 4, 128 000 of 24 8.27 / 9.45, band of 800, 72 000 of 30 7.93 / 5.26; random, 64 000 of 32,
+// N = 1 8.72 / 9.83, N = 5 13.2 / 12.2.  Beyond: band of 400, N = 8, 256 000 rows of 32 30.1 / 24.2.
 uint32_t row_parts(const cute_hrpb_dev *d, uint32_t N)
 {
     if (N > 8u || uint64_t(d->nnz) < 24ull * d->M) return 1u;
@@ -1326,7 +1332,16 @@ uint32_t row_parts(const cute_hrpb_dev *d, uint32_t N)
         active += d->panelCols[q];
     }
     while (parts < 16u && uint64_t(d->nnz) >= 7ull * parts * d->M) parts *= 2u;
-    if (N > 2u && uint64_t(d->nnz) >= 2u * active && uint64_t(d->M) * parts * (N > 4u || N == 3u ? 2u : 1u) > 524288u) return 1u;
+    const bool two = N > 4u || N == 3u;
+    const uint64_t nnz = d->nnz, lanes = uint64_t(d->M) * parts * (two ? 2u : 1u);
+    if (N > 2u && nnz >= 2u * active && lanes > 524288u) return 1u;
+    if (parts < 16u && lanes > 190000u) {
+        const uint64_t turn = 4u * uint64_t(parts) * d->M, turns = (nnz + turn - 1u) / turn;
+        const bool idle = 20u * nnz < 17u * turns * turn;
+        const bool random = 50u * nnz < 51u * active, wide = !random && 10u * nnz < 11u * active;
+        if (two ? !random && (wide || (idle && (parts == 4u || lanes > 524288u))) && (parts == 4u || lanes < 2000000u)
+                : N == 4u ? wide && parts == 4u && nnz < 4000000u : N == 1u && random && nnz < 2300000u) return 1u;
+    }
     // (a launch has at most 2^32 threads, of which a row takes parts, twice as many from two lanes a group on)
     return uint64_t(longest) * d->M > 4ull * d->nnz || uint64_t(d->M) * parts * 2u > 0x7fffffffull ? 1u : parts;
 }

@@ -44,3 +44,20 @@ def test_padding_reads_nothing_and_rows_are_written_once(cs, orc, torch_cuda):
     assert plan.row_parts == 8
     plan.run(torch.from_numpy(B).cuda(), C)
     assert np.array_equal(C.cpu().numpy(), orc.spmm_csr(rp, cl, vl, B))
+
+
+@pytest.mark.parametrize("kind,rows,per_row,span,N,parts", [(5, 16000, 24, 400, 8, 4), (5, 64000, 24, 400, 8, 1), (5, 64000, 24, 400, 4, 4), (5, 32000, 32, 400, 7, 8), (5, 32000, 32, 2048, 7, 1),
+                                                            (5, 64000, 48, 400, 3, 1), (5, 128000, 24, 2048, 4, 1), (5, 64000, 24, 2048, 2, 4), (1, 64000, 32, 0, 1, 1), (1, 16000, 32, 0, 1, 8),
+                                                            (5, 128000, 32, 400, 8, 8), (5, 96000, 48, 400, 6, 1),
+                                                            (5, 64000, 32, 400, 8, 8), (5, 72000, 30, 800, 4, 8), (1, 64000, 24, 0, 5, 4), (1, 64000, 24, 0, 2, 4)])
+def test_the_route_over_the_sizes(cs, orc, torch_cuda, kind, rows, per_row, span, N, parts):
+    """Groups share rows while the launch leaves slots free, or from four million entries on; in between it depends on the lanes and on shared columns."""
+    torch = torch_cuda
+    A = cs.gen_matrix(kind, 5, rows, per_row, span)
+    vals = (np.arange(len(A.vals)) % 7 - 3).astype(np.float32)
+    plan = cs.SPMM_TC(cs.HRPB(A.M, A.K, A.rowPtr, A.cols, vals), N)
+    assert plan.row_parts == parts
+    B = np.random.default_rng(N).integers(-4, 5, (A.K, N)).astype(np.float32)
+    C = torch.full((A.M, N), float("nan"), device="cuda")
+    plan.run(torch.from_numpy(B).cuda(), C)
+    assert np.array_equal(C.cpu().numpy(), orc.spmm_csr(A.rowPtr, A.cols, vals, B))
