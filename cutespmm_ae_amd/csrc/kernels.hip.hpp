@@ -216,7 +216,7 @@ __device__ __forceinline__ BrickItem brick_item(const uint4 *__restrict__ chunks
 // others, and what it reads of theirs, passes by the XCD's own L2 (agent-scope accesses): counting in then needs the stores to have
 // arrived, not the write-back of everything the L2 holds that a device-wide release is on this part (which made counting in 1.1 to 5.5
 // times slower than a second launch).  A plan without cut panels runs the kernels that are compiled without any of this (CUT = false): the branch and
-// the registers behind it cost 0.5 to 1 % of a short launch (9-point stencil of 200 x 200 points, N = 101, 11.37 -> 11.45 us; hrpb_quad_half_f32 46 -> 50
+// the registers behind it cost 0.5 to 1 % of a short launch (9-point stencil of 200 x 200 points, N = 101, 9.54 -> 9.65 us; hrpb_quad_half_f32 46 -> 50
 // vector registers).
 // With a second launch (reduce_partials), as calls whose scratch comes without counters and kernels that are no plan's default have it, and
 // without, us: R-MAT graph of 131 072 nodes, N = 64 45.0 / 44.0; 65 536 nodes, N = 47 26.6 / 23.9.
@@ -324,7 +324,7 @@ __device__ __forceinline__ void store_piece(const CutPieces *__restrict__ cut, u
     const uint32_t eights = (pieces + kPiecesAtOnce - 1u) / kPiecesAtOnce, eight = (piece - 1u - first) / kPiecesAtOnce,
                    tile0 = first + eight * kPiecesAtOnce, members = min(kPiecesAtOnce, pieces - eight * kPiecesAtOnce);
     // (one loop for every E, a few words of a lane a turn: the tile is not held in registers again)
-    constexpr int kTurn = W == 4 && E == 4 ? 1 : W == 1 && E == 4 ? 4 : 2;
+    constexpr int kTurn = W == 4 ? 1 : W == 1 && E == 4 ? 4 : 2;
     static_assert(E % kTurn == 0, "whole turns");
     // the turn's vectors of n tiles, `apart` bytes from one to the next, added up: all are on their way before the first is added
     auto add_all = [&](int e0, V (&sum)[kTurn], bool none_so_far, uint32_t n, uint32_t tile, uint32_t apart) {
@@ -590,7 +590,10 @@ __device__ __forceinline__ void brick_store_lean(const BrickItem &it, const f32x
 // budget is small enough that a launch of short panels is resident as a whole.  Padding-only
 // bricks skip their MFMAs.  NG = 2 lets one wavefront cover two column groups, which halves the
 // header traffic and shares the A-side index arithmetic between them.
-template <int VEC, int NG, bool FULL, bool CUT>
+// AHEAD: an item's first two header lines are asked for together, which is 1 to 2 % where B comes from the caches and loses 4 % where it comes from HBM: 9-point
+// stencils, us without / with, 200 x 200 points, N = 101 9.54 / 9.34, 256 x 256, N = 128 12.95 / 12.5, 300 x 300, N = 512 78.0 / 77.0, 352 x 352 107.9 / 109.8,
+// 396 x 396 147.0 / 153.7.
+template <int VEC, int NG, bool FULL, bool AHEAD, bool CUT>
 __device__ __forceinline__ void brick_rolling_body(uint32_t block_x, uint32_t block_y, const uint4 *__restrict__ chunks,
                                                    uint32_t num_chunks, uint32_t groups_per_xcd,
                                                    const uint32_t *__restrict__ hdr, const float *__restrict__ vals,
@@ -621,7 +624,7 @@ __device__ __forceinline__ void brick_rolling_body(uint32_t block_x, uint32_t bl
         {
             const LeanHeader h0 = load_lean_header(hdr, blk, lane);
             h1 = load_lean_header(hdr, min(blk + 1, end - 1), lane);
-            __builtin_amdgcn_sched_barrier(0);       // both lines are asked for before the first is waited for (9-point stencil of 200 x 200 points, N = 101: 9.75 -> 9.5 us)
+            if (AHEAD) __builtin_amdgcn_sched_barrier(0);       // both lines are asked for before the first is waited for
             // h1's load must be complete before the loop is entered.  The wait in front of its first use in
             // the loop is compiled once for both ways into the loop; were the load still in flight here (the
             // compiler would sink it behind the operand loads below), that wait would allow only two younger
@@ -667,13 +670,13 @@ __device__ __forceinline__ void brick_rolling_body(uint32_t block_x, uint32_t bl
     brick_store_lean<VEC, NG, FULL, CUT>(it, acc, C, partials, N, lane, cut);
 }
 
-template <int VEC, int NG, bool FULL, bool COLUMNS, bool CUT>
+template <int VEC, int NG, bool FULL, bool COLUMNS, bool AHEAD, bool CUT>
 __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, (NG == 1 ? 8 : 4)) void hrpb_brick_f32_rolling(
     const uint4 *__restrict__ chunks, uint32_t num_chunks, uint32_t groups_per_xcd, const uint32_t *__restrict__ hdr,
     const float *__restrict__ vals, uint32_t zero_index, const float *__restrict__ B, float *__restrict__ C,
     float *__restrict__ partials, uint32_t N, uint32_t column_slabs, const CutPieces *__restrict__ cut)
 {
-    brick_rolling_body<VEC, NG, FULL, CUT>(blockIdx.x, blockIdx.y, chunks, num_chunks, groups_per_xcd, hdr, vals, zero_index, B, C,
+    brick_rolling_body<VEC, NG, FULL, AHEAD, CUT>(blockIdx.x, blockIdx.y, chunks, num_chunks, groups_per_xcd, hdr, vals, zero_index, B, C,
                                       partials, N, COLUMNS ? column_slabs : 0u, cut);
 }
 
@@ -1767,7 +1770,7 @@ __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, (NG == 1 ? 8 : 4)) void 
     const float *__restrict__ B, float *__restrict__ C, float *__restrict__ partials, uint32_t N, const CutPieces *__restrict__ cut)
 {
     if (blockIdx.x < brick_blocks) {
-        brick_rolling_body<VEC, NG, FULL, CUT>(blockIdx.x % brick_blocks_x, blockIdx.x / brick_blocks_x, chunks, num_chunks,
+        brick_rolling_body<VEC, NG, FULL, true, CUT>(blockIdx.x % brick_blocks_x, blockIdx.x / brick_blocks_x, chunks, num_chunks,
                                           groups_per_xcd, hdr, tile_vals, zero_index, B, C, partials, N, COLUMNS ? column_slabs : 0u, cut);
     } else {
         const uint32_t rb = blockIdx.x - brick_blocks;
