@@ -1324,26 +1324,27 @@ int make_hub_tables(cute_spmm_plan *p, const cute_hrpb_dev *d, uint32_t hub_rows
 // N = 1 8.72 / 9.83, N = 5 13.2 / 12.2.  Beyond: band of 400, N = 8, 256 000 rows of 32 30.1 / 24.2.
 uint32_t row_parts(const cute_hrpb_dev *d, uint32_t N)
 {
-    if (N > 8u || uint64_t(d->nnz) < 24ull * d->M) return 1u;
+    const uint64_t nnz = d->nnz, M = d->M;
+    if (N > 8u || nnz < 24u * M) return 1u;
     uint32_t longest = 0, parts = 4;
     uint64_t active = 0;
     for (uint32_t q = 0; q < d->P; ++q) {
         longest = std::max(longest, d->panelMaxRow[q]);
         active += d->panelCols[q];
     }
-    while (parts < 16u && uint64_t(d->nnz) >= 7ull * parts * d->M) parts *= 2u;
+    while (parts < 16u && nnz >= 7u * parts * M) parts *= 2u;
     const bool two = N > 4u || N == 3u;
-    const uint64_t nnz = d->nnz, lanes = uint64_t(d->M) * parts * (two ? 2u : 1u);
+    const uint64_t lanes = M * parts * (two ? 2u : 1u);
     if (N > 2u && nnz >= 2u * active && lanes > 524288u) return 1u;
     if (parts < 16u && lanes > 190000u) {
-        const uint64_t turn = 4u * uint64_t(parts) * d->M, turns = (nnz + turn - 1u) / turn;
+        const uint64_t turn = 4u * parts * M, turns = (nnz + turn - 1u) / turn;
         const bool idle = 20u * nnz < 17u * turns * turn;
         const bool random = 50u * nnz < 51u * active, wide = !random && 10u * nnz < 11u * active;
         if (two ? !random && (wide || (idle && (parts == 4u || lanes > 524288u))) && (parts == 4u || lanes < 2000000u)
                 : N == 4u ? wide && parts == 4u && nnz < 4000000u : N == 1u && random && nnz < 2300000u) return 1u;
     }
     // (a launch has at most 2^32 threads, of which a row takes parts, twice as many from two lanes a group on)
-    return uint64_t(longest) * d->M > 4ull * d->nnz || uint64_t(d->M) * parts * 2u > 0x7fffffffull ? 1u : parts;
+    return longest * M > 4u * nnz || M * parts * 2u > 0x7fffffffu ? 1u : parts;
 }
 
 // Rows of a plan without MFMA panels through csr_rows_window where that is ahead.  Needs the widest window of a tile to fit the ring,
@@ -2230,15 +2231,10 @@ void launch_brick_full(const cute_spmm_plan *p, const float *dB, float *dC, floa
         if constexpr (VEC == 4)
             hipLaunchKernelGGL((cute_dev::hrpb_brick_bf16x3<NG, FULL, COLUMNS, CUT>), grid, block, 0, s, p->dChunks, p->info.numChunks, per_xcd,
                                p->d->dHdr, p->d->dVals, uint32_t(p->d->numVals), dB, dC, partials, p->info.N, p->columnSlabs, cut);
-    } else if (p->pipeline == 1) {
-#define CUTE_ROLLING_LAUNCH(AHEAD) \
-    hipLaunchKernelGGL((cute_dev::hrpb_brick_f32_rolling<VEC, NG, FULL, COLUMNS, AHEAD, CUT>), grid, block, 0, s, p->dChunks, p->info.numChunks, per_xcd, \
-                       p->d->dHdr, p->d->dVals, uint32_t(p->d->numVals), dB, dC, partials, p->info.N, p->columnSlabs, cut)
-        // B fits the Infinity Cache with an eighth to spare (B of 184 and 254 MB: the 300 x 300 and 352 x 352 points measured at the kernel)
-        if (uint64_t(p->d->K) * p->info.N * sizeof(float) * 8u <= context().cache_bytes * 7u) CUTE_ROLLING_LAUNCH(true);
-        else CUTE_ROLLING_LAUNCH(false);
-#undef CUTE_ROLLING_LAUNCH
-    } else
+    } else if (p->pipeline == 1)
+        hipLaunchKernelGGL((cute_dev::hrpb_brick_f32_rolling<VEC, NG, FULL, COLUMNS, CUT>), grid, block, 0, s, p->dChunks,
+                           p->info.numChunks, per_xcd, p->d->dHdr, p->d->dVals, uint32_t(p->d->numVals), dB, dC, partials, p->info.N, p->columnSlabs, cut);
+    else
         hipLaunchKernelGGL((cute_dev::hrpb_brick_f32<VEC, NG, FULL>), grid, block, 0, s, p->dChunks, p->info.numChunks,
                            per_xcd, p->d->dHdr, p->d->dVals, dB, dC, partials, p->info.N, p->columnSlabs);
 }

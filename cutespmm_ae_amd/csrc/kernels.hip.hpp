@@ -590,10 +590,7 @@ __device__ __forceinline__ void brick_store_lean(const BrickItem &it, const f32x
 // budget is small enough that a launch of short panels is resident as a whole.  Padding-only
 // bricks skip their MFMAs.  NG = 2 lets one wavefront cover two column groups, which halves the
 // header traffic and shares the A-side index arithmetic between them.
-// AHEAD: an item's first two header lines are asked for together, which is 1 to 2 % where B comes from the caches and loses 4 % where it comes from HBM: 9-point
-// stencils, us without / with, 200 x 200 points, N = 101 9.54 / 9.34, 256 x 256, N = 128 12.95 / 12.5, 300 x 300, N = 512 78.0 / 77.0, 352 x 352 107.9 / 109.8,
-// 396 x 396 147.0 / 153.7.
-template <int VEC, int NG, bool FULL, bool AHEAD, bool CUT>
+template <int VEC, int NG, bool FULL, bool CUT>
 __device__ __forceinline__ void brick_rolling_body(uint32_t block_x, uint32_t block_y, const uint4 *__restrict__ chunks,
                                                    uint32_t num_chunks, uint32_t groups_per_xcd,
                                                    const uint32_t *__restrict__ hdr, const float *__restrict__ vals,
@@ -616,15 +613,19 @@ __device__ __forceinline__ void brick_rolling_body(uint32_t block_x, uint32_t bl
         for (int v = 0; v < VEC; ++v) acc[ng][v] = f32x4(0.0f);
 
     uint32_t blk = it.start;
-    if (__builtin_expect(blk < end, true)) {     // (an empty item's code would stand in front of everybody's first fetch)
+    if (blk < end) {
         V b[4][NG];
         float a[4];
         uint64_t bitmap[4];
         LeanHeader h1, h2;
         {
-            const LeanHeader h0 = load_lean_header(hdr, blk, lane);
+            LeanHeader h0 = load_lean_header(hdr, blk, lane);
             h1 = load_lean_header(hdr, min(blk + 1, end - 1), lane);
-            if (AHEAD) __builtin_amdgcn_sched_barrier(0);       // both lines are asked for before the first is waited for
+            // h1 is asked for before h0's scalars are waited for (the compiler had moved it behind them, a round trip later).  Tied to a scalar, and no fence: what
+            // comes after keeps its order.  With a fence for it the operand loads mix with what they wait for: rows of odd widths are 4 % faster, 200 x 200 points,
+            // N = 101 11.4 -> 10.9 us, but 256 x 256, N = 128 13.6 -> 13.8, finite elements of 232 nodes, N = 512 10.6 -> 11.4, from HBM 396 x 396 points, N = 512
+            // 147 -> 154, and in some variants the loop then waits for nearly all loads.
+            asm volatile("" : "+s"(h0.bitmap[0])::"memory");
             // h1's load must be complete before the loop is entered.  The wait in front of its first use in
             // the loop is compiled once for both ways into the loop; were the load still in flight here (the
             // compiler would sink it behind the operand loads below), that wait would allow only two younger
@@ -670,13 +671,13 @@ __device__ __forceinline__ void brick_rolling_body(uint32_t block_x, uint32_t bl
     brick_store_lean<VEC, NG, FULL, CUT>(it, acc, C, partials, N, lane, cut);
 }
 
-template <int VEC, int NG, bool FULL, bool COLUMNS, bool AHEAD, bool CUT>
+template <int VEC, int NG, bool FULL, bool COLUMNS, bool CUT>
 __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, (NG == 1 ? 8 : 4)) void hrpb_brick_f32_rolling(
     const uint4 *__restrict__ chunks, uint32_t num_chunks, uint32_t groups_per_xcd, const uint32_t *__restrict__ hdr,
     const float *__restrict__ vals, uint32_t zero_index, const float *__restrict__ B, float *__restrict__ C,
     float *__restrict__ partials, uint32_t N, uint32_t column_slabs, const CutPieces *__restrict__ cut)
 {
-    brick_rolling_body<VEC, NG, FULL, AHEAD, CUT>(blockIdx.x, blockIdx.y, chunks, num_chunks, groups_per_xcd, hdr, vals, zero_index, B, C,
+    brick_rolling_body<VEC, NG, FULL, CUT>(blockIdx.x, blockIdx.y, chunks, num_chunks, groups_per_xcd, hdr, vals, zero_index, B, C,
                                       partials, N, COLUMNS ? column_slabs : 0u, cut);
 }
 
@@ -761,14 +762,15 @@ __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, (NG == 1 ? 6 : 4)) void 
         for (int v = 0; v < VEC; ++v) acc[ng][v] = f32x4(0.0f);
 
     uint32_t blk = it.start;
-    if (__builtin_expect(blk < end, true)) {     // (an empty item's code would stand in front of everybody's first fetch)
+    if (blk < end) {
         f32x4 b[4][NG];
         float a[4];
         LeanHeader h1;
         {
-            const LeanHeader h0 = load_lean_header(hdr, blk, lane);
+            LeanHeader h0 = load_lean_header(hdr, blk, lane);
             h1 = load_lean_header(hdr, min(blk + 1, end - 1), lane);
-            asm volatile("" ::"v"(h1.cols[0]), "v"(h1.cols[1]), "v"(h1.cols[2]), "v"(h1.cols[3]));   // as in the fp32 kernel
+            asm volatile("" : "+s"(h0.bitmap[0])::"memory");                                         // as in the fp32 kernel
+            asm volatile("" ::"v"(h1.cols[0]), "v"(h1.cols[1]), "v"(h1.cols[2]), "v"(h1.cols[3]));
 #pragma unroll
             for (int j = 0; j < 4; ++j) load_brick_lean<VEC, NG, FULL>(b[j], a[j], j, h0, vals, zero_index, B, row_pitch, col_offs);
         }
@@ -1770,7 +1772,7 @@ __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, (NG == 1 ? 8 : 4)) void 
     const float *__restrict__ B, float *__restrict__ C, float *__restrict__ partials, uint32_t N, const CutPieces *__restrict__ cut)
 {
     if (blockIdx.x < brick_blocks) {
-        brick_rolling_body<VEC, NG, FULL, true, CUT>(blockIdx.x % brick_blocks_x, blockIdx.x / brick_blocks_x, chunks, num_chunks,
+        brick_rolling_body<VEC, NG, FULL, CUT>(blockIdx.x % brick_blocks_x, blockIdx.x / brick_blocks_x, chunks, num_chunks,
                                           groups_per_xcd, hdr, tile_vals, zero_index, B, C, partials, N, COLUMNS ? column_slabs : 0u, cut);
     } else {
         const uint32_t rb = blockIdx.x - brick_blocks;
