@@ -88,3 +88,34 @@ def test_wavefronts_see_every_unsorted_pair(cs, torch_cuda):
         cs.DeviceHRPB(16, K, gpu(rp), gpu(far), gpu(vl))
     assert err.value.status == -4
     cs.DeviceHRPB(16, K, gpu(rp), gpu(cl), gpu(vl))
+
+
+def test_two_threads_build_graphs_at_one_time(cs, torch_cuda):
+    """The lists of a graph's long strips are built on a side stream that all threads share: each thread gets the layout that one alone gets."""
+    import threading
+
+    def build(seed):
+        A = cs.gen_matrix(4, seed, 15, 10, 0)
+        dev = [torch_cuda.from_numpy(np.array(x) if x.dtype == np.float32 else np.array(x).view(np.int32)).cuda() for x in (A.rowPtr, A.cols, A.vals)]
+        return lambda: cs.DeviceHRPB(A.M, A.K, *dev, quad_layout=2).layouts()
+
+    makers = [build(5), build(6)]
+    alone = [make() for make in makers]
+    got, barrier = [[], []], threading.Barrier(2)
+
+    def work(i):
+        for _ in range(6):
+            barrier.wait(timeout=60)
+            got[i].append(makers[i]())
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for i in range(2):
+        assert len(got[i]) == 6
+        for one in got[i]:
+            assert one.keys() == alone[i].keys()
+            assert all(np.array_equal(one[k], alone[i][k], equal_nan=True) if isinstance(one[k], np.ndarray) and one[k].dtype.kind == "f" else
+                       np.array_equal(one[k], alone[i][k]) for k in one)
