@@ -2231,10 +2231,17 @@ void launch_brick_full(const cute_spmm_plan *p, const float *dB, float *dC, floa
         if constexpr (VEC == 4)
             hipLaunchKernelGGL((cute_dev::hrpb_brick_bf16x3<NG, FULL, COLUMNS, CUT>), grid, block, 0, s, p->dChunks, p->info.numChunks, per_xcd,
                                p->d->dHdr, p->d->dVals, uint32_t(p->d->numVals), dB, dC, partials, p->info.N, p->columnSlabs, cut);
-    } else if (p->pipeline == 1)
-        hipLaunchKernelGGL((cute_dev::hrpb_brick_f32_rolling<VEC, NG, FULL, COLUMNS, CUT>), grid, block, 0, s, p->dChunks,
-                           p->info.numChunks, per_xcd, p->d->dHdr, p->d->dVals, uint32_t(p->d->numVals), dB, dC, partials, p->info.N, p->columnSlabs, cut);
-    else
+    } else if (p->pipeline == 1) {
+#define CUTE_ROLLING_LAUNCH(TOGETHER) \
+    hipLaunchKernelGGL((cute_dev::hrpb_brick_f32_rolling<VEC, NG, FULL, COLUMNS, TOGETHER, CUT>), grid, block, 0, s, p->dChunks, p->info.numChunks, per_xcd, \
+                       p->d->dHdr, p->d->dVals, uint32_t(p->d->numVals), dB, dC, partials, p->info.N, p->columnSlabs, cut)
+        // An item's first two header lines together where B is small, one after the other where the launch is long and memory is the bound.  9-point stencils, us
+        // together / after: 300 x 300 points, N = 64 (B of 23 MB) 9.5 / 9.7, 256 x 256, N = 128 (34) 13.30 / 13.43; 396 x 396, N = 256 (160) 68.8 / 66.5, 300 x 300, N = 512
+        // (184) 80.3 / 78.0, 352 x 352 111.0 / 107.2, 508 x 508 238.0 / 235.3; 600 x 600, N = 100 (144) 75.5 both, finite elements level.
+        if (uint64_t(p->d->K) * p->info.N * sizeof(float) * 8u <= context().cache_bytes * 3u) CUTE_ROLLING_LAUNCH(true);
+        else CUTE_ROLLING_LAUNCH(false);
+#undef CUTE_ROLLING_LAUNCH
+    } else
         hipLaunchKernelGGL((cute_dev::hrpb_brick_f32<VEC, NG, FULL>), grid, block, 0, s, p->dChunks, p->info.numChunks,
                            per_xcd, p->d->dHdr, p->d->dVals, dB, dC, partials, p->info.N, p->columnSlabs);
 }

@@ -590,7 +590,7 @@ __device__ __forceinline__ void brick_store_lean(const BrickItem &it, const f32x
 // budget is small enough that a launch of short panels is resident as a whole.  Padding-only
 // bricks skip their MFMAs.  NG = 2 lets one wavefront cover two column groups, which halves the
 // header traffic and shares the A-side index arithmetic between them.
-template <int VEC, int NG, bool FULL, bool CUT>
+template <int VEC, int NG, bool FULL, bool TOGETHER, bool CUT>
 __device__ __forceinline__ void brick_rolling_body(uint32_t block_x, uint32_t block_y, const uint4 *__restrict__ chunks,
                                                    uint32_t num_chunks, uint32_t groups_per_xcd,
                                                    const uint32_t *__restrict__ hdr, const float *__restrict__ vals,
@@ -621,11 +621,11 @@ __device__ __forceinline__ void brick_rolling_body(uint32_t block_x, uint32_t bl
         {
             LeanHeader h0 = load_lean_header(hdr, blk, lane);
             h1 = load_lean_header(hdr, min(blk + 1, end - 1), lane);
-            // h1 is asked for before h0's scalars are waited for (the compiler had moved it behind them, a round trip later).  Tied to a scalar, and no fence: what
+            // TOGETHER: h1 is asked for before h0's scalars are waited for (the compiler moves it behind them, a round trip later).  Tied to a scalar, and no fence: what
             // comes after keeps its order.  With a fence for it the operand loads mix with what they wait for: rows of odd widths are 4 % faster, 200 x 200 points,
             // N = 101 11.4 -> 10.9 us, but 256 x 256, N = 128 13.6 -> 13.8, finite elements of 232 nodes, N = 512 10.6 -> 11.4, from HBM 396 x 396 points, N = 512
             // 147 -> 154, and in some variants the loop then waits for nearly all loads.
-            asm volatile("" : "+s"(h0.bitmap[0])::"memory");
+            if constexpr (TOGETHER) asm volatile("" : "+s"(h0.bitmap[0])::"memory");
             // h1's load must be complete before the loop is entered.  The wait in front of its first use in
             // the loop is compiled once for both ways into the loop; were the load still in flight here (the
             // compiler would sink it behind the operand loads below), that wait would allow only two younger
@@ -671,13 +671,13 @@ __device__ __forceinline__ void brick_rolling_body(uint32_t block_x, uint32_t bl
     brick_store_lean<VEC, NG, FULL, CUT>(it, acc, C, partials, N, lane, cut);
 }
 
-template <int VEC, int NG, bool FULL, bool COLUMNS, bool CUT>
+template <int VEC, int NG, bool FULL, bool COLUMNS, bool TOGETHER, bool CUT>
 __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, (NG == 1 ? 8 : 4)) void hrpb_brick_f32_rolling(
     const uint4 *__restrict__ chunks, uint32_t num_chunks, uint32_t groups_per_xcd, const uint32_t *__restrict__ hdr,
     const float *__restrict__ vals, uint32_t zero_index, const float *__restrict__ B, float *__restrict__ C,
     float *__restrict__ partials, uint32_t N, uint32_t column_slabs, const CutPieces *__restrict__ cut)
 {
-    brick_rolling_body<VEC, NG, FULL, CUT>(blockIdx.x, blockIdx.y, chunks, num_chunks, groups_per_xcd, hdr, vals, zero_index, B, C,
+    brick_rolling_body<VEC, NG, FULL, TOGETHER, CUT>(blockIdx.x, blockIdx.y, chunks, num_chunks, groups_per_xcd, hdr, vals, zero_index, B, C,
                                       partials, N, COLUMNS ? column_slabs : 0u, cut);
 }
 
@@ -1772,7 +1772,7 @@ __global__ __launch_bounds__(kWaveSize *kWavesPerGroup, (NG == 1 ? 8 : 4)) void 
     const float *__restrict__ B, float *__restrict__ C, float *__restrict__ partials, uint32_t N, const CutPieces *__restrict__ cut)
 {
     if (blockIdx.x < brick_blocks) {
-        brick_rolling_body<VEC, NG, FULL, CUT>(blockIdx.x % brick_blocks_x, blockIdx.x / brick_blocks_x, chunks, num_chunks,
+        brick_rolling_body<VEC, NG, FULL, true, CUT>(blockIdx.x % brick_blocks_x, blockIdx.x / brick_blocks_x, chunks, num_chunks,
                                           groups_per_xcd, hdr, tile_vals, zero_index, B, C, partials, N, COLUMNS ? column_slabs : 0u, cut);
     } else {
         const uint32_t rb = blockIdx.x - brick_blocks;
